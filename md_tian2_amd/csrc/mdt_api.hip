@@ -21,9 +21,12 @@ size_t mdt_replica_smem(int N, int cap, bool nbr_lds);
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
                               const BatchView &bv, int add_fin, hipStream_t st);
 hipError_t mdt_launch_estimators(int ntraj, const PropConst *pc, const BatchView &bv, double *out, hipStream_t st);
-hipError_t mdt_launch_traj(int ntraj, size_t smem, const PropConst *pc, const BatchView &bv, const double *cjk,
-                           const long long *cjk_off, const uint32_t *step_base, uint32_t step_prev, uint32_t step,
-                           int flags, int block, bool classical, hipStream_t st, int t_base = 0);
+hipError_t mdt_launch_traj_classical(int ntraj, const PropConst *pc, const BatchView &bv, const uint32_t *step_base,
+                                     uint32_t step_prev, uint32_t step, int flags, int block, hipStream_t st,
+                                     int t_base);
+hipError_t mdt_launch_prop(int ntraj, int maxP, const PropConst *pc, const BatchView &bv, const double *cjk,
+                           const long long *cjk_off, const PropChunk *chunks, int nchunk, double *com, bool com_on,
+                           const uint32_t *step_base, uint32_t step_prev, uint32_t step, int flags, hipStream_t st);
 hipError_t mdt_launch_advance(uint32_t *step_base, uint32_t n, int set, hipStream_t st);
 size_t mdt_mixed_smem(int nmax, int pmax);
 hipError_t mdt_launch_mixed(int tpa, int block, int ntraj, size_t smem, const EmtConst *ec, const PropConst *pc,
@@ -247,6 +250,10 @@ struct mdt_batch {
     uint32_t obs_step0 = 0;
     int no_com = 0;  // mdt_batch_set_com_removal(b, 0)
     double *d_est = nullptr;  // MDT_NEST per trajectory
+    // k_prop's chunks (built for chunk_mode, the bead mode) and their COM partial sums
+    PropChunk *d_chunk = nullptr;
+    double *d_com = nullptr;
+    int nchunk = 0, chunk_mode = -1;
 
     // k_replica's pair-term arithmetic: mode 1 is full FP32 pair terms when
     // the EMT types' stiffness allows (EmtConst::fp32_ok), else only the
@@ -527,7 +534,7 @@ int mdt_batch_destroy(mdt_batch *b) {
                     b->d_tproj, b->d_tid, b->d_x, b->d_v, b->d_a, b->d_f, b->d_dens, b->d_epot,
                     b->d_cjk, b->d_status, b->d_pc, b->d_step, b->d_nnG, b->d_nnC,
                     b->d_nnflag, b->d_nnF, b->d_judge, b->d_mix, b->d_mix_nbr, b->d_mix_ref, b->d_mix_fold, b->d_mix_cnt, b->d_mix_valid, b->d_obs, b->d_done, b->d_est, b->d_eta,
-                    b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey, b->d_step_h, b->d_ident};
+                    b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey, b->d_step_h, b->d_ident, b->d_chunk, b->d_com};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
@@ -937,6 +944,37 @@ static int check_mixed(mdt_batch *b) {
     return 0;
 }
 
+// k_prop's chunk table for the current bead mode
+static int build_chunks(mdt_batch *b) {
+    if (b->chunk_mode == b->bead_mode) return 0;
+    std::vector<PropChunk> ch;
+    for (int t = 0; t < b->ntraj; ++t) {
+        const int N = b->N[t], P = b->P[t];
+        const bool mix = b->bead_mode == MDT_BEADS_MIXED && P > 1;
+        const int first = (int)ch.size();
+        if (mix) ch.push_back(PropChunk{t, 0, 1, P, 0, 0});
+        const int nb = mix ? 1 : P, na = MDT_CHUNK / nb;
+        for (int i = mix ? 1 : 0; i < N; i += na) ch.push_back(PropChunk{t, i, std::min(na, N - i), nb, 0, 0});
+        for (size_t k = first; k < ch.size(); ++k) {
+            ch[k].first = first;
+            ch[k].count = (int)ch.size() - first;
+        }
+    }
+    if (b->d_chunk) (void)hipFree(b->d_chunk);
+    if (b->d_com) (void)hipFree(b->d_com);
+    b->d_chunk = nullptr;
+    b->d_com = nullptr;
+    b->chunk_mode = -1;
+    int rc = dalloc(&b->d_chunk, ch.size()) | dalloc(&b->d_com, 4 * ch.size());
+    if (rc) return rc;
+    HIPCHK(hipMemcpy(b->d_chunk, ch.data(), sizeof(PropChunk) * ch.size(), hipMemcpyHostToDevice));
+    b->nchunk = (int)ch.size();
+    b->chunk_mode = b->bead_mode;
+    return 0;
+}
+
+static bool traj_classical(const mdt_batch *b);
+
 static int ensure_ready(mdt_batch *b, bool need_prop) {
     if (b->pes == 1 && !b->ctx->have_nn) return fail(MDT_ESTATE, "no network (call mdt_nn_params_set)");
     if (b->pes == 0 && !b->ctx->have_params) return fail(MDT_ESTATE, "no EMT parameters (call mdt_emt_params_set)");
@@ -958,6 +996,10 @@ static int ensure_ready(mdt_batch *b, bool need_prop) {
     }
     b->pc.mixed = b->bead_mode == 1 ? 1 : 0;
     b->pc.no_com = b->no_com;
+    if (!traj_classical(b)) {
+        int rc = build_chunks(b);
+        if (rc) return rc;
+    }
     return push_pc(b);
 }
 
@@ -1356,10 +1398,8 @@ static int launch_judge(mdt_batch *b, hipStream_t st) {
     return launch_replicas(b, jb, 0, st);
 }
 
-// LDS of k_traj: the P x P normal-mode matrix, three atom lists (uint16)
-// and one flag byte per atom
-// k_traj's workgroup: the largest trajectory's atoms rounded up to whole
-// waves, at most 256 threads (every loop of k_traj strides by blockDim.x)
+// k_traj_classical's workgroup: the largest trajectory's atoms rounded up to
+// whole waves, at most 256 threads
 static int traj_block(const mdt_batch *b) {
     const int w = ((b->maxN + 63) / 64) * 64;
     return w < 64 ? 64 : (w > 256 ? 256 : w);
@@ -1371,17 +1411,26 @@ static bool traj_classical(const mdt_batch *b) {
     return b->allP1 && b->maxN <= traj_block(b) && !b->pc.any_pile && !b->pc.any_andersen;
 }
 
-static size_t traj_smem(const mdt_batch *b) {
-    return sizeof(double) * b->maxP * b->maxP + 7 * (size_t)b->maxN + 16;
+// the propagators of every trajectory (flags of k_prop)
+static int launch_prop(mdt_batch *b, const BatchView &bv, const uint32_t *step_base, uint32_t prev, uint32_t step,
+                       int flags) {
+    mdt_context *c = b->ctx;
+    if (traj_classical(b)) {
+        HIPCHK(mdt_launch_traj_classical(b->ntraj, b->d_pc, bv, step_base, prev, step, flags, traj_block(b), c->stream, 0));
+        return 0;
+    }
+    const bool com = (b->pc.any_andersen || b->pc.any_pile) && !b->no_com;
+    HIPCHK(mdt_launch_prop(b->ntraj, b->maxP, b->d_pc, bv, b->d_cjk, b->d_cjkoff, b->d_chunk, b->nchunk, b->d_com, com,
+                           step_base, prev, step, flags, c->stream));
+    return 0;
 }
 
 static int launch_force(mdt_batch *b) {
     mdt_context *c = b->ctx;
     const BatchView bv = b->view();
     if (!b->allP1) {
-        const size_t ts = traj_smem(b);
-        HIPCHK(mdt_launch_traj(b->ntraj, ts, b->d_pc, bv, b->d_cjk, b->d_cjkoff, nullptr, b->step, b->step, 4,
-                               traj_block(b), false, c->stream));
+        int rc = launch_prop(b, bv, nullptr, b->step, b->step, 4);
+        if (rc) return rc;
     }
     return launch_pes(b, bv, b->allP1 ? 0 : 1, c->stream);
 }
@@ -1550,25 +1599,20 @@ int mdt_batch_compute_forces(mdt_batch *b) {
 static int enqueue_steps(mdt_batch *b, int nsteps, const uint32_t *step_base, uint32_t first, bool events) {
     mdt_context *c = b->ctx;
     const BatchView bv = b->view();
-    const size_t ts = traj_smem(b);
-    const bool classical = traj_classical(b);
+    int rc;
     const int rp = b->allP1 ? 0 : 4;
     for (int s = 0; s < nsteps; ++s) {
         const uint32_t prev = first + s, st = first + s + 1;
         const int flags = (s > 0 ? 1 : 0) | 2 | rp;
-        HIPCHK(mdt_launch_traj(b->ntraj, ts, b->d_pc, bv, b->d_cjk, b->d_cjkoff, step_base, prev, st, flags,
-                               traj_block(b), classical, c->stream));
+        if ((rc = launch_prop(b, bv, step_base, prev, st, flags))) return rc;
         if (events) HIPCHK(hipEventRecord(b->evf[2 * s], c->stream));
-        int rc = launch_pes(b, bv, b->allP1 ? 0 : 1, c->stream);
-        if (rc) return rc;
+        if ((rc = launch_pes(b, bv, b->allP1 ? 0 : 1, c->stream))) return rc;
         if (events) HIPCHK(hipEventRecord(b->evf[2 * s + 1], c->stream));
         if (b->pes == 1 && b->judge_interval > 0 && c->have_params && (st % (uint32_t)b->judge_interval) == 0 &&
             !step_base && (rc = launch_judge(b, c->stream)))
             return rc;
     }
-    if (nsteps > 0)
-        HIPCHK(mdt_launch_traj(b->ntraj, ts, b->d_pc, bv, b->d_cjk, b->d_cjkoff, step_base, first + nsteps,
-                               first + nsteps, 1, traj_block(b), classical, c->stream));
+    if (nsteps > 0) return launch_prop(b, bv, step_base, first + nsteps, first + nsteps, 1);
     return 0;
 }
 
@@ -1609,13 +1653,12 @@ static int enqueue_half(mdt_batch *b, int h, int nsteps, const uint32_t *step_ba
     for (int s = 0; s < nsteps; ++s) {
         const uint32_t prev = first + s, stp = first + s + 1;
         const int flags = (s > 0 ? 1 : 0) | 2;
-        HIPCHK(mdt_launch_traj(t1 - t0, 0, b->d_pc, bv, b->d_cjk, b->d_cjkoff, step_base, prev, stp, flags,
-                               traj_block(b), true, st, t0));
+        HIPCHK(mdt_launch_traj_classical(t1 - t0, b->d_pc, bv, step_base, prev, stp, flags, traj_block(b), st, t0));
         HIPCHK(mdt_launch_replica(k.tpa, t1 - t0, k.block, k.smem, c->d_ec, b->d_pc, v, 0, st));
     }
     if (nsteps > 0)
-        HIPCHK(mdt_launch_traj(t1 - t0, 0, b->d_pc, bv, b->d_cjk, b->d_cjkoff, step_base, first + nsteps,
-                               first + nsteps, 1, traj_block(b), true, st, t0));
+        HIPCHK(mdt_launch_traj_classical(t1 - t0, b->d_pc, bv, step_base, first + nsteps, first + nsteps, 1,
+                                         traj_block(b), st, t0));
     return 0;
 }
 

@@ -95,6 +95,17 @@ struct PropConst {
     int no_com;  // 1: no remove_com_velocity after propagate_1 (an extension; see mdt_batch_set_com_removal)
 };
 
+// A run of one trajectory's atoms with all their beads: the work of one
+// workgroup of the propagators (k_prop).  In the mixed bead model the
+// projectile's beads are a chunk of their own and the classical atoms'
+// chunks have nb = 1.
+struct PropChunk {
+    int t;             // trajectory
+    int i0, na, nb;    // atoms i0 .. i0 + na - 1, beads per atom (na nb <= 256)
+    int first, count;  // the trajectory's chunks: first .. first + count - 1
+};
+#define MDT_CHUNK 256
+
 struct BatchView {
     int ntraj, nrep;
     int nbcap;      // neighbour-list capacity per atom
@@ -129,9 +140,9 @@ struct BatchView {
     int judge_mod, judge_phase;
     // trajectory observation (collect_trajectory_characteristics,
     // src/trajectory_info.f90:47-263; the exit test of src/md_tian2.f90:88-92)
-    // when obs != NULL: after each step's propagate_2 k_traj updates
+    // when obs != NULL: after each step's propagate_2 the propagators update
     // obs[t], and a trajectory whose projectile beads are all above
-    // obs_ul or all below obs_ll is frozen (done[t] set: k_traj and the
+    // obs_ul or all below obs_ll is frozen (done[t] set: the propagators and the
     // force kernels skip it from then on)
     // mixed bead mode, per listed trajectory (slot = position in the list):
     // the classical atoms' lists are kept across steps (Verlet skin) when

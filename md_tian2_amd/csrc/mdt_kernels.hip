@@ -19,9 +19,9 @@
 //            fixed point; then set_acceleration.
 //   Fixed-point integer accumulation is associative, so results are bitwise
 //   reproducible whatever order the lanes' atomics land in.
-// k_traj: one workgroup per trajectory: propagate_2 of the previous step,
-//   propagate_1, COM removal and (P > 1) the ring-polymer free step
-//   (src/md_algo.f90:37-106, src/rpmd.f90:309-452).
+// k_traj_classical (one-bead batches) and k_prop / k_com_ring (the others):
+//   propagate_2 of the previous step, propagate_1, COM removal and (P > 1)
+//   the ring-polymer free step (src/md_algo.f90:37-106, src/rpmd.f90:309-452).
 #include <hip/hip_runtime.h>
 
 #include "mdt_device.h"
@@ -975,9 +975,6 @@ __global__ void __launch_bounds__(MAXB, 4)
 }
 
 // ---------------------------------------------------------------------------
-// P > 1 trajectory kernel: [propagate_2 of the previous step] then
-// [propagate_1 + COM removal] then [ring-polymer free step] for one
-// trajectory per workgroup.  cjk (P x P, column-major cjk(j,k)) in global.
 // collect_trajectory_characteristics after propagate_2 of step step_prev
 // (src/trajectory_info.f90:47-263) for trajectory t: centroids, the
 // projectile (atom 0) against every other atom (min image).  Reads x, v and
@@ -1076,7 +1073,7 @@ __device__ bool traj_observe(const PropConst &pc, const int *s_proj, const Batch
 #undef OX
 }
 
-// The propagator updates shared by k_traj and k_traj_classical, in the
+// The propagator updates shared by k_prop and k_traj_classical, in the
 // reference's operation order with FMA contraction off (the pragma's flag
 // stays on the instructions after inlining): both kernels then give
 // bitwise the same states, whatever code surrounds the updates.
@@ -1107,8 +1104,21 @@ __device__ __forceinline__ double verlet_x(double x, double dt, double vn) {
     return x + dt * vn;
 }
 
-// flags bit0: propagate_2, bit1: propagate_1, bit2: ring-polymer step
-// (trajectories with P == 1 only get f = 0 from bit2, as calc_force zeroes f).
+// ---------------------------------------------------------------------------
+// The propagators of batches with ring polymers, PILE or Andersen atoms or
+// one-bead slabs of more than 256 atoms.  One lane per atom-bead; a
+// workgroup holds every bead of a run of atoms (PropChunk, at most 256
+// atom-beads), so that all couplings but one -- the branch test of
+// langevin_1 over an atom's beads, the spring forces, the normal-mode
+// transforms -- stay inside it, and a trajectory spreads over as many
+// workgroups as it has work for.  The one coupling across atoms,
+// remove_com_velocity, takes the chunks' partial sums to a second launch.
+//
+// flags bit0: propagate_2, bit1: propagate_1, bit2: ring-polymer step (atoms
+// with one bead only get f = 0 from it, as calc_force zeroes f), bit3: the COM
+// velocity is removed after propagate_1 (k_com_ring follows, which also
+// takes the transforms of the ring-polymer step, since those read the
+// corrected velocities).
 // step_base (graph replays): when non-null, *step_base is added to both step
 // numbers, which are then offsets within the captured chunk.
 // Mixed bead mode (pc.mixed): atoms of non-projectile types are classical --
@@ -1116,399 +1126,447 @@ __device__ __forceinline__ double verlet_x(double x, double dt, double vn) {
 // Langevin / Andersen temperature is kB T / m, PILE acts on their single
 // mode, positions advance in propagate_1 and the ring-polymer step skips
 // them; in the COM sum a classical atom counts as P identical beads.
+//
+// Memory bound: about 200 B per atom-bead and launch.  64 trajectories of
+// H/Pt 8x8x6 with 32 beads (788k atom-beads, 3136 chunks) take 46 us in
+// k_prop and 33 us in k_com_ring, against 511 us with one workgroup of 256
+// lanes per trajectory (64 of 256 CUs, x and v through global memory between
+// the phases); 192 uneven H/Au trajectories 38 against 401 us; 384 mixed
+// trajectories of H/Pt 6x6x4 14 + 10 against 41 us.
 // ---------------------------------------------------------------------------
-// Four waves per SIMD: the register allocation is held to 128 VGPRs (a
-// 16-byte spill); measured 66 -> 58 us per launch on 4096 H/Au 6x6x4
-// trajectories against the unbounded 133-VGPR build at three waves.
+
+// The chunk of this workgroup.  Workgroups go round the 8 XCDs in launch
+// order, so consecutive chunks -- which share cache lines, their rows of
+// [bead][component][atom] being short -- are given to one XCD.
+__device__ __forceinline__ int chunk_of_block(int nchunk) {
+    const int per = (nchunk + 7) >> 3;
+    return ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+}
+
+// C (P x P, column-major cjk(j,k)) to LDS in columns of P + 1 entries: the
+// forward transform reads down a column per lane, and columns P apart would
+// share their banks.  Every lane calls it; the caller synchronises.
+__device__ __forceinline__ void load_cjk(double *C, const double *cjk, int P, int lane, int nthr) {
+    for (int k = lane; k < P * P; k += nthr) C[(k / P) * (P + 1) + k % P] = cjk[k];
+}
+
+// The exact free step of one atom's ring polymer (do_ring_polymer_step,
+// rpmd.f90:309-452) on x, v of the lane's atom-bead: forward transform and
+// harmonic rotation of mode k = the lane's bead, then back.  s_x, s_v:
+// 3 x 256 LDS words each, holding the chunk's x and v ([component][slot],
+// slot = bead na + atom of the chunk); on: the lane's atom takes part.
+// Every lane of the block calls it; x and v of fixed components stay.
+__device__ __forceinline__ void ring_transform(double (*s_x)[256], double (*s_v)[256], const double *C, bool on, int a,
+                                               int k, int na, int P, double mass, double temp_k, double dt, uint8_t fb,
+                                               double x[3], double v[3]) {
+    const int lane = threadIdx.x;
+    const int ld = P + 1;
+    double p[3] = {0.0, 0.0, 0.0}, q[3] = {0.0, 0.0, 0.0};
+    if (on) {
+        for (int j = 0; j < P; ++j) {
+            const double cj = C[j + ld * k];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                p[c] = p[c] + (mass * s_v[c][j * na + a]) * cj;
+                q[c] = q[c] + s_x[c][j * na + a] * cj;
+            }
+        }
+        const double betaN = 1.0 / (MDT_KB * temp_k * P);
+        const double twown = 2.0 / betaN / MDT_HBAR;
+        double p1 = 1.0, p2 = 0.0, p3 = dt / mass, p4 = 1.0;
+        const int fk = (k <= P / 2) ? k : P - k;  // mirrored modes share a frequency
+        if (fk > 0) {
+            const double wk = twown * sin(fk * (MDT_PI / P));
+            const double wt = wk * dt, wm = wk * mass;
+            const double cw = cos(wt), sw = sin(wt);
+            p1 = cw;
+            p2 = -wm * sw;
+            p3 = sw / wm;
+            p4 = cw;
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double pn = p[c] * p1 + q[c] * p2;
+            q[c] = p[c] * p3 + q[c] * p4;
+            p[c] = pn;
+        }
+    }
+    __syncthreads();
+    if (on)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            s_v[c][lane] = p[c];
+            s_x[c][lane] = q[c];
+        }
+    __syncthreads();
+    if (on) {
+        double rr[3] = {0.0, 0.0, 0.0}, vv[3] = {0.0, 0.0, 0.0};
+        for (int j = 0; j < P; ++j) {
+            const double cj = C[k + ld * j];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                rr[c] = rr[c] + s_x[c][j * na + a] * cj;
+                vv[c] = vv[c] + s_v[c][j * na + a] * cj / mass;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (!(fb >> c & 1)) {
+                x[c] = rr[c];
+                v[c] = vv[c];
+            }
+    }
+}
+
+// 4 waves per SIMD: the registers of langevin_1's normals and coefficients
+// held to 128.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-k_traj(const PropConst *__restrict__ pcg, BatchView bv,
-                                              const double *cjk_all, const long long *cjk_off,
-                                              const uint32_t *step_base, uint32_t step_prev, uint32_t step,
-                                              int flags) {
+k_prop(const PropConst *__restrict__ pcg, BatchView bv, const double *cjk_all, const long long *cjk_off,
+       const PropChunk *__restrict__ chunks, int nchunk, double *__restrict__ com, const uint32_t *step_base,
+       uint32_t step_prev, uint32_t step, int flags) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ int s_algo[MDT_MAXT], s_proj[MDT_MAXT];
-    __shared__ double red[4];
+    __shared__ double s_x[3][256], s_v[3][256];
+    __shared__ int s_small[256];
+    __shared__ double s_com[4][4];
     const PropConst &pc = *pcg;
-    const int t = blockIdx.x;
+    const int w = chunk_of_block(nchunk);
+    if (w >= nchunk) return;  // whole block: uniform
+    const PropChunk ch = chunks[w];
+    const int t = ch.t, na = ch.na, nb = ch.nb;
     if (bv.done && bv.done[t]) return;  // frozen trajectory (whole block: uniform)
-    const int N = bv.traj_N[t];
-    const int P = bv.traj_P[t];
+    const int N = bv.traj_N[t], P = bv.traj_P[t];
     const long long soff = bv.traj_soff[t];
-    const long long poff = soff / 3;
     const long long aoff = bv.traj_aoff[t];
     const uint32_t tid = bv.traj_id[t];
     const double tsurf = bv.tsurf[t], tproj = bv.tproj[t];
     const double dt = pc.dt;
-    const double *cjk = cjk_all + cjk_off[t];
-    const int nthr = blockDim.x, lane = threadIdx.x;
-    if (step_base) {
+    const int lane = threadIdx.x, nthr = blockDim.x;
+    if (step_base) {  // graph replays: step numbers are offsets from the device counter
         const uint32_t s0 = *step_base;
         step_prev += s0;
         step += s0;
     }
-    // LDS: C (P x P) | ring-polymer atom lists: PILE, transformed (not
-    // Langevin), Langevin (spring force) | big flags
-    double *C = (double *)smem_raw;
-    uint16_t *l_pile = (uint16_t *)(C + P * P), *l_tr = l_pile + N, *l_lan = l_tr + N;
-    uint8_t *big = (uint8_t *)(l_lan + N);
-    __shared__ int s_cnt[3];
-    for (int k = lane; k < P * P; k += nthr) C[k] = cjk[k];
-    for (int k = lane; k < MDT_MAXT; k += nthr) {
-        s_algo[k] = pc.algo[k];
-        s_proj[k] = pc.is_proj[k];
-    }
-    if (lane < 3) s_cnt[lane] = 0;
+    double *C = (double *)smem_raw;  // P (P + 1), loaded where the chunk transforms
+    const bool act = lane < na * nb;
+    const int b = lane / na, a_ = lane - b * na;  // bead, atom of the chunk
+    const int i = ch.i0 + a_;
+    const long long xi = soff + (long long)b * 3 * N + i;             // component 0; + N per component
+    const long long pi = soff / 3 + (long long)b * N + i;
+    int ty = 0, algo = MDT_PROP_VERLET;
+    uint8_t fb = 7;
+    double mass = 1.0, dn = 0.0;
+    double x[3] = {0.0, 0.0, 0.0}, v[3] = {0.0, 0.0, 0.0}, a[3] = {0.0, 0.0, 0.0}, v0[3] = {0.0, 0.0, 0.0};
     int bad_local = 0;
-#define XI(c, b, i) (soff + ((long long)(b) * 3 + (c)) * N + (i))
-#define PI_(b, i) (poff + (long long)(b) * N + (i))
-    __syncthreads();
-    // beads of atom type ty: P, or 1 for a classical atom in mixed mode
-#define PT(ty) ((pc.mixed && !s_proj[ty]) ? 1 : P)
-    // atom-bead slots in use: every atom's P beads, or in the mixed model
-    // (atom 0 the only ring polymer) P beads of atom 0 and bead 0 of the rest
-    const bool mix = pc.mixed && P > 1;
-    const int nab = mix ? P + N - 1 : N * P;
-#define AB(q, i, b)                       \
-    if (mix) {                            \
-        i = (q) < P ? 0 : (q) - P + 1;    \
-        b = (q) < P ? (q) : 0;            \
-    } else {                              \
-        i = (q) % N;                      \
-        b = (q) / N;                      \
-    }
-    __shared__ double s_rmin[4];
-    __shared__ int s_done;
-    // ring-polymer atoms (P > 1 beads) by propagator; list order is free
-    // (every task below is independent of the others)
-    if (P > 1)
-        for (int i = lane; i < N; i += nthr) {
-            const int ty = bv.type[aoff + i];
-            if (PT(ty) == 1) continue;
-            const int a = s_algo[ty];
-            if (a == MDT_PROP_PILE) l_pile[atomicAdd(&s_cnt[0], 1)] = (uint16_t)i;
-            if (a == MDT_PROP_LANGEVIN)
-                l_lan[atomicAdd(&s_cnt[2], 1)] = (uint16_t)i;
-            else
-                l_tr[atomicAdd(&s_cnt[1], 1)] = (uint16_t)i;
+    if (act) {
+        ty = bv.type[aoff + i];
+        algo = pc.algo[ty];
+        fb = bv.fixed[pi];
+        mass = bv.mass[aoff + i];
+        dn = bv.dens[pi];
+        const bool ring = (flags & 4) && nb > 1;  // the spring forces and transforms read every bead's x
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            v0[c] = v[c] = bv.v[xi + (long long)c * N];
+            if (ring || ((flags & 2) && !(fb >> c & 1))) x[c] = bv.x[xi + (long long)c * N];
+            if ((flags & 3) && !(fb >> c & 1)) a[c] = bv.a[xi + (long long)c * N];
         }
-    __syncthreads();
-    const int n_pile = s_cnt[0], n_tr = s_cnt[1], n_lan = s_cnt[2];
-    // langevin_2 of the previous step and langevin_1 of this one read the
-    // same friction (dens after ldfa), temperature and branch, so their
-    // coefficients are equal: with one atom-bead slot per lane (nab <= nthr)
-    // the lane keeps them in LDS from the first for the second
-    const bool one_slot = nab <= nthr;
-    __shared__ LanCoef s_lan[256];
+    }
+    const bool lan = act && algo == MDT_PROP_LANGEVIN;
+    const double temp_k = pc.is_proj[ty] ? tproj : tsurf;
+    LanCoef L;
     bool have_l = false;
-
-    if (flags & 1) {
-        // ldfa for Langevin atoms, per bead (md_algo.f90:97)
-        for (int q = lane; q < nab; q += nthr) {
-            int i, b;
-            AB(q, i, b);
-            const int ty = bv.type[aoff + i];
-            if (s_algo[ty] == MDT_PROP_LANGEVIN) {
-                int bad = 0;
-                bv.dens[PI_(b, i)] = ldfa(bv.dens[PI_(b, i)], bv.mass[aoff + i], &bad);
-                if (bad) bad_local |= MDT_ST_NEG_DENSITY;
-            }
+    if (flags & 3) {
+        if ((flags & 1) && lan) {
+            int bad = 0;
+            dn = ldfa(dn, mass, &bad);  // per bead (md_algo.f90:97)
+            if (bad) bad_local |= MDT_ST_NEG_DENSITY;
+            bv.dens[pi] = dn;
         }
-        __syncthreads();
-        for (int i = lane; i < N; i += nthr) {
-            int all = 1;
-            const int pb = PT(bv.type[aoff + i]);
-            for (int b = 0; b < pb; ++b)
-                if (!lan_big(bv.dens[PI_(b, i)], dt)) all = 0;
-            big[i] = (uint8_t)all;
+        // the branch test of langevin_1 / langevin_2: every bead of the atom (md_algo.f90:176)
+        bool big = lan_big(dn, dt);
+        if (nb > 1) {
+            if (lane < na) s_small[lane] = 0;
+            __syncthreads();
+            if (act && !big) s_small[a_] = 1;  // benign race: every writer stores 1
+            __syncthreads();
+            big = act && !s_small[a_];
         }
-        __syncthreads();
-        for (int q = lane; q < nab; q += nthr) {
-            int i, b;
-            AB(q, i, b);
-            const int ty = bv.type[aoff + i];
-            const uint8_t fb = bv.fixed[PI_(b, i)];
-            const double mass = bv.mass[aoff + i];
-            if (s_algo[ty] == MDT_PROP_LANGEVIN) {
-                const double temp = MDT_KB * PT(ty) * (s_proj[ty] ? tproj : tsurf) / mass;
-                const bool exact = big[i] && temp > MDT_TOLERANCE;
-                const LanCoef L = lan_coef(bv.dens[PI_(b, i)], dt, temp, exact);
-                if (one_slot) {
-                    s_lan[lane] = L;
-                    have_l = true;
-                }
-                const double w = lan_w(L);
-                for (int c = 0; c < 3; ++c) {
-                    // the deviate of this step's langevin_1, kept by propagate_1
-                    // (mdt_normal(seed, tid, step_prev, MDT_STREAM_LANGEVIN, i P + b, c))
-                    const double eta = bv.eta[XI(c, b, i)];
-                    const double v = bv.v[XI(c, b, i)];
-                    bv.v[XI(c, b, i)] = (fb >> c & 1) ? 0.0 : lan_v2(L, w, v, bv.a[XI(c, b, i)], eta);
-                }
-            } else {
-                for (int c = 0; c < 3; ++c) {
-                    const double v = bv.v[XI(c, b, i)];
-                    bv.v[XI(c, b, i)] = (fb >> c & 1) ? 0.0 : verlet_v(v, dt, bv.a[XI(c, b, i)]);
-                }
-            }
-        }
-        __syncthreads();
-    }
-
-    if ((flags & 1) && bv.obs) {
-        // frozen after this step: no propagate_1 / ring-polymer step
-        if (traj_observe(pc, s_proj, bv, t, N, P, soff, aoff, lane, nthr, step_prev, s_rmin, &s_done)) {
-            if (bad_local) atomicOr(&bv.status[t], bad_local);
-            return;
+        if (lan) {
+            const double temp = MDT_KB * nb * temp_k / mass;
+            L = lan_coef(dn, dt, temp, big && temp > MDT_TOLERANCE);
+            have_l = true;
         }
     }
-
-    if (flags & 2) {
-        // the branch test of langevin_1 over all beads (md_algo.f90:176)
-        for (int i = lane; i < N; i += nthr) {
-            int all = 1;
-            const int pb = PT(bv.type[aoff + i]);
-            for (int b = 0; b < pb; ++b)
-                if (!lan_big(bv.dens[PI_(b, i)], dt)) all = 0;
-            big[i] = (uint8_t)all;
+    if ((flags & 1) && act) {  // propagate_2 of step step_prev
+        if (lan) {
+            const double w2 = lan_w(L);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)  // the deviate of that step's langevin_1, kept by propagate_1
+                v[c] = (fb >> c & 1) ? 0.0 : lan_v2(L, w2, v[c], a[c], bv.eta[xi + (long long)c * N]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[c] = (fb >> c & 1) ? 0.0 : verlet_v(v[c], dt, a[c]);
         }
-        __syncthreads();
-        // pile_thermostat per atom (md_algo.f90:440-502)
-        if (pc.any_pile) {
-            // one-bead atoms: thread per (atom, component)
-            if (P == 1 || mix)
-                for (int q = lane; q < N * 3; q += nthr) {
-                    const int i = q / 3, c = q % 3;
-                    const int ty = bv.type[aoff + i];
-                    if (s_algo[ty] != MDT_PROP_PILE || PT(ty) != 1) continue;
-                    const double mass = bv.mass[aoff + i];
-                    const double betaN = 1.0 / (MDT_KB * (s_proj[ty] ? tproj : tsurf));
-                    const double c1 = exp(-0.5 * dt * (1 / pc.pile_tau));
+    }
+    bool have_c = false;
+    if (flags & 2) {  // propagate_1 of step step
+        // pile_thermostat (md_algo.f90:440-502)
+        if (pc.any_pile && nb == 1 && act && algo == MDT_PROP_PILE) {
+            const double betaN = 1.0 / (MDT_KB * temp_k);
+            const double c1 = exp(-0.5 * dt * (1 / pc.pile_tau));
+            const double c2 = sqrt(1 - c1 * c1);
+            for (int c = 0; c < 3; ++c) {
+                const double z = mdt_normal(pc.seed, tid, step, MDT_STREAM_PILE, (uint32_t)(i * P), (uint32_t)c);
+                const double np = c1 * (mass * v[c]) + sqrt(mass / betaN) * c2 * z;
+                v[c] = (fb >> c & 1) ? 0.0 : np / mass;
+            }
+        }
+        if (pc.any_pile && nb > 1) {
+            const bool pile = act && algo == MDT_PROP_PILE;
+            if (__syncthreads_or(pile)) {
+                load_cjk(C, cjk_all + cjk_off[t], P, lane, nthr);
+                have_c = true;
+                const int k = b, ld = P + 1;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) s_v[c][lane] = v[c];
+                __syncthreads();
+                double acc[3] = {0.0, 0.0, 0.0};
+                if (pile) {
+                    for (int j = 0; j < P; ++j) {
+                        const double cj = C[j + ld * k];
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) acc[c] = acc[c] + (mass * s_v[c][j * na + a_]) * cj;
+                    }
+                    const double betaN = 1.0 / (MDT_KB * temp_k * P);
+                    double g;
+                    if (k == 0) {
+                        g = 1 / pc.pile_tau;
+                    } else {
+                        const double wn = 1 / betaN / MDT_HBAR;
+                        const double wk = 2 * wn * sin(k * MDT_PI / P);
+                        g = 2 * wk;
+                    }
+                    const double c1 = exp(-0.5 * dt * g);
                     const double c2 = sqrt(1 - c1 * c1);
-                    const double z = mdt_normal(pc.seed, tid, step, MDT_STREAM_PILE, (uint32_t)(i * P), (uint32_t)c);
-                    const double np = c1 * (mass * bv.v[XI(c, 0, i)]) + sqrt(mass / betaN) * c2 * z;
-                    const uint8_t fb = bv.fixed[PI_(0, i)];
-                    bv.v[XI(c, 0, i)] = (fb >> c & 1) ? 0.0 : np / mass;
+                    double z[3];
+                    mdt_normal3(pc.seed, tid, step, MDT_STREAM_PILE, (uint32_t)(i * P + k), z);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) acc[c] = c1 * acc[c] + sqrt(mass / betaN) * c2 * z[c];
                 }
-            // ring polymers: thread per (atom, component, mode); the thermostatted
-            // normal-mode momenta go through f (rewritten by calc_force after this)
-            for (int q = lane; q < n_pile * 3 * P; q += nthr) {
-                const int k = q % P, c = (q / P) % 3, i = l_pile[q / (3 * P)];
-                const int ty = bv.type[aoff + i];
-                const double mass = bv.mass[aoff + i];
-                const double betaN = 1.0 / (MDT_KB * (s_proj[ty] ? tproj : tsurf) * P);
-                double acc = 0.0;
-                for (int j = 0; j < P; ++j) acc = acc + (mass * bv.v[XI(c, j, i)]) * C[j + P * k];
-                double g;
-                if (k == 0) {
-                    g = 1 / pc.pile_tau;
-                } else {
-                    const double wn = 1 / betaN / MDT_HBAR;
-                    const double wk = 2 * wn * sin(k * MDT_PI / P);
-                    g = 2 * wk;
+                __syncthreads();
+#pragma unroll
+                for (int c = 0; c < 3; ++c) s_v[c][lane] = acc[c];
+                __syncthreads();
+                if (pile) {
+                    double ap[3] = {0.0, 0.0, 0.0};
+                    for (int j = 0; j < P; ++j) {
+                        const double cj = C[b + ld * j];
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) ap[c] = ap[c] + s_v[c][j * na + a_] * cj;
+                    }
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) v[c] = (fb >> c & 1) ? 0.0 : ap[c] / mass;
                 }
-                const double c1 = exp(-0.5 * dt * g);
-                const double c2 = sqrt(1 - c1 * c1);
-                const double z = mdt_normal(pc.seed, tid, step, MDT_STREAM_PILE, (uint32_t)(i * P + k), (uint32_t)c);
-                bv.f[XI(c, k, i)] = c1 * acc + sqrt(mass / betaN) * c2 * z;
+                __syncthreads();  // s_v is used again below
             }
-            __syncthreads();
-            for (int q = lane; q < n_pile * 3 * P; q += nthr) {
-                const int b = q % P, c = (q / P) % 3, i = l_pile[q / (3 * P)];
-                const double mass = bv.mass[aoff + i];
-                const uint8_t fb = bv.fixed[PI_(b, i)];
-                double ap = 0.0;
-                if (!(fb >> c & 1))
-                    for (int k = 0; k < P; ++k) ap = ap + bv.f[XI(c, k, i)] * C[b + P * k];
-                bv.v[XI(c, b, i)] = ap / mass;
-            }
-            __syncthreads();
         }
-        for (int q = lane; q < nab; q += nthr) {
-            int i, b;
-            AB(q, i, b);
-            const int ty = bv.type[aoff + i];
-            const int pb = PT(ty);
-            const int algo = s_algo[ty];
-            const uint8_t fb = bv.fixed[PI_(b, i)];
-            const double mass = bv.mass[aoff + i];
-            if (algo == MDT_PROP_LANGEVIN) {
-                LanCoef L;
-                if (have_l) {
-                    L = s_lan[lane];
-                } else {
-                    const double temp = MDT_KB * pb * (s_proj[ty] ? tproj : tsurf) / mass;
-                    const bool exact = big[i] && temp > MDT_TOLERANCE;
-                    L = lan_coef(bv.dens[PI_(b, i)], dt, temp, exact);
-                }
+        if (lan) {
+            if (fb != 7) {  // a fixed component uses no deviate
                 double z[3];
                 mdt_normal3(pc.seed, tid, step, MDT_STREAM_LANGEVIN, (uint32_t)(i * P + b), z);
+#pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     const double eta = z[c];
-                    bv.eta[XI(c, b, i)] = eta;  // langevin_2 of this step takes the same deviate
-                    const double r = bv.x[XI(c, b, i)], v = bv.v[XI(c, b, i)], a = bv.a[XI(c, b, i)];
                     if (!(fb >> c & 1)) {
-                        bv.x[XI(c, b, i)] = lan_x1(L, dt, r, v, a, eta);
-                        bv.v[XI(c, b, i)] = lan_v1(L, v, a, eta);
+                        bv.eta[xi + (long long)c * N] = eta;  // langevin_2 of this step takes the same deviate
+                        const double r = x[c], vo = v[c];
+                        x[c] = lan_x1(L, dt, r, vo, a[c], eta);
+                        v[c] = lan_v1(L, vo, a[c], eta);
                     } else {
-                        bv.v[XI(c, b, i)] = 0.0;
-                    }
-                }
-            } else if (algo == MDT_PROP_VERLET || algo == MDT_PROP_ANDERSEN || algo == MDT_PROP_PILE) {
-                for (int c = 0; c < 3; ++c) {
-                    const double v = bv.v[XI(c, b, i)];
-                    const double vn = (fb >> c & 1) ? 0.0 : verlet_v(v, dt, bv.a[XI(c, b, i)]);
-                    bv.v[XI(c, b, i)] = vn;
-                    if (pb == 1 && !(fb >> c & 1)) bv.x[XI(c, b, i)] = verlet_x(bv.x[XI(c, b, i)], dt, vn);
-                }
-                if (algo == MDT_PROP_ANDERSEN) {
-                    const double ibetaN = pb * MDT_KB * (s_proj[ty] ? tproj : tsurf);
-                    const double sigma = sqrt(ibetaN / mass);
-                    const double u = mdt_uniform(pc.seed, tid, step, MDT_STREAM_ANDERSEN_U, (uint32_t)(i * P + b), 0u);
-                    if (u < dt / pc.andersen_time) {
-                        double z[3];
-                        mdt_normal3(pc.seed, tid, step, MDT_STREAM_ANDERSEN_V, (uint32_t)(i * P + b), z);
-                        for (int c = 0; c < 3; ++c)
-                            if (!(fb >> c & 1)) bv.v[XI(c, b, i)] = z[c] * sigma + 0.0;
+                        v[c] = 0.0;
                     }
                 }
             } else {
-                bad_local |= MDT_ST_BAD_PROP;
+                v[0] = v[1] = v[2] = 0.0;
             }
+        } else if (act && (algo == MDT_PROP_VERLET || algo == MDT_PROP_ANDERSEN || algo == MDT_PROP_PILE)) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double vn = (fb >> c & 1) ? 0.0 : verlet_v(v[c], dt, a[c]);
+                v[c] = vn;
+                if (nb == 1 && !(fb >> c & 1)) x[c] = verlet_x(x[c], dt, vn);
+            }
+            if (algo == MDT_PROP_ANDERSEN) {
+                const double sigma = sqrt(nb * MDT_KB * temp_k / mass);
+                const double u = mdt_uniform(pc.seed, tid, step, MDT_STREAM_ANDERSEN_U, (uint32_t)(i * P + b), 0u);
+                if (u < dt / pc.andersen_time) {
+                    double z[3];
+                    mdt_normal3(pc.seed, tid, step, MDT_STREAM_ANDERSEN_V, (uint32_t)(i * P + b), z);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                        if (!(fb >> c & 1)) v[c] = z[c] * sigma + 0.0;
+                }
+            }
+        } else if (act) {
+            bad_local |= MDT_ST_BAD_PROP;
         }
-        __syncthreads();
-        if ((pc.any_andersen || pc.any_pile) && !pc.no_com) {
-            // remove_com_velocity, closed form of the 1000 iterations
-            if (lane < 64) {
-                double ax = 0, ay = 0, az = 0, am = 0;
-                for (int i = lane; i < N; i += 64) {
-                    const double m = bv.mass[aoff + i];
-                    double bx = 0, by = 0, bz = 0;
-                    const int pb = PT(bv.type[aoff + i]);
-                    for (int b = 0; b < pb; ++b) {
-                        bx += bv.v[XI(0, b, i)];
-                        by += bv.v[XI(1, b, i)];
-                        bz += bv.v[XI(2, b, i)];
-                    }
-                    if (pb == 1 && P > 1) {  // a classical atom stands for P identical beads
-                        bx *= P;
-                        by *= P;
-                        bz *= P;
-                    }
-                    ax += bx * m;
-                    ay += by * m;
-                    az += bz * m;
-                    am += m;
-                }
-                for (int o = 32; o > 0; o >>= 1) {
-                    ax += __shfl_xor(ax, o, 64);
-                    ay += __shfl_xor(ay, o, 64);
-                    az += __shfl_xor(az, o, 64);
-                    am += __shfl_xor(am, o, 64);
-                }
-                if (lane == 0) {
-                    red[0] = ax;
-                    red[1] = ay;
-                    red[2] = az;
-                    red[3] = am;
-                }
+        if (flags & 8) {  // this chunk's part of remove_com_velocity's sums, in a fixed order
+            double s[4];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) s[c] = act ? v[c] * mass * (P / nb) : 0.0;  // classical: P identical beads
+            s[3] = act && b == 0 ? mass : 0.0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                for (int o = 32; o > 0; o >>= 1) s[c] += __shfl_xor(s[c], o, 64);
+                if ((lane & 63) == 0) s_com[lane >> 6][c] = s[c];
             }
             __syncthreads();
-            const double fac = (1.0 - pow(1.0 - 1.0 / N, 1000.0)) / red[3] / P;
-            for (int q = lane; q < nab; q += nthr) {
-                int i, b;
-                AB(q, i, b);
-                bv.v[XI(0, b, i)] -= red[0] * fac;
-                bv.v[XI(1, b, i)] -= red[1] * fac;
-                bv.v[XI(2, b, i)] -= red[2] * fac;
-            }
-            __syncthreads();
+            if (lane < 4) com[4 * (long long)w + lane] = s_com[0][lane] + s_com[1][lane] + s_com[2][lane] + s_com[3][lane];
         }
     }
-
+    bool moved = (flags & 2) != 0;
     if (flags & 4) {
-        if (P == 1) {
-            for (int q = lane; q < 3 * N; q += nthr) bv.f[soff + q] = 0.0;
-        } else {
-            // do_ring_polymer_step (rpmd.f90:309-452)
-            const double kt = MDT_KB * tproj * P / MDT_HBAR;
-            const double m1 = bv.mass[aoff + 0];
-            const double prefactor = -1 * m1 * (kt * kt);
-            const double piN = MDT_PI / P;
-            if (mix)  // classical atoms: no ring polymer, f = 0
-                for (int q = lane; q < (N - 1) * 3; q += nthr) bv.f[XI(q % 3, 0, 1 + q / 3)] = 0.0;
-            // Langevin atoms: the step is reverted; spring force with m(1) and
-            // Tproj (rpmd.f90:418-435)
-            for (int q = lane; q < n_lan * 3 * P; q += nthr) {
-                const int b = q % P, c = (q / P) % 3, i = l_lan[q / (3 * P)];
+        double f[3] = {0.0, 0.0, 0.0};
+        if (nb > 1) {
+            const bool tr = act && !lan && !(flags & 8);
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                s_x[c][lane] = x[c];
+                s_v[c][lane] = v[c];
+            }
+            const bool any_tr = __syncthreads_or(tr);
+            if (lan) {
+                // the step is reverted; spring force with m(1) and Tproj (rpmd.f90:418-435)
+                const double kt = MDT_KB * tproj * P / MDT_HBAR;
+                const double prefactor = -1 * bv.mass[aoff + 0] * (kt * kt);
                 const int pv = b == 0 ? P - 1 : b - 1, nx = b == P - 1 ? 0 : b + 1;
-                bv.f[XI(c, b, i)] = prefactor * (2 * bv.x[XI(c, b, i)] - bv.x[XI(c, pv, i)] - bv.x[XI(c, nx, i)]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    f[c] = prefactor * (2 * x[c] - s_x[c][pv * na + a_] - s_x[c][nx * na + a_]);
             }
-            // the other ring polymers: thread per (atom, component, mode) for the
-            // forward transform and the exact harmonic rotation, whose results
-            // go through a (momenta) and f (positions) -- calc_force zeroes
-            // both (force.f90:49-50) -- then per (atom, component, bead) back
-            for (int q = lane; q < n_tr * 3 * P; q += nthr) {
-                const int k = q % P, c = (q / P) % 3, i = l_tr[q / (3 * P)];
-                const int ty = bv.type[aoff + i];
-                const double mass = bv.mass[aoff + i];
-                double ap = 0.0, aq = 0.0;
-                for (int j = 0; j < P; ++j) {
-                    ap = ap + (mass * bv.v[XI(c, j, i)]) * C[j + P * k];
-                    aq = aq + bv.x[XI(c, j, i)] * C[j + P * k];
+            if (any_tr) {
+                if (!have_c) {
+                    load_cjk(C, cjk_all + cjk_off[t], P, lane, nthr);
+                    __syncthreads();
                 }
-                const double betaN = 1.0 / (MDT_KB * (s_proj[ty] ? tproj : tsurf) * P);
-                const double twown = 2.0 / betaN / MDT_HBAR;
-                double p1 = 1.0, p2 = 0.0, p3 = dt / mass, p4 = 1.0;
-                const int fk = (k <= P / 2) ? k : P - k;  // mirrored modes share a frequency
-                if (fk > 0) {
-                    const double wk = twown * sin(fk * piN);
-                    const double wt = wk * dt, wm = wk * mass;
-                    const double cw = cos(wt), sw = sin(wt);
-                    p1 = cw;
-                    p2 = -wm * sw;
-                    p3 = sw / wm;
-                    p4 = cw;
-                }
-                bv.a[XI(c, k, i)] = ap * p1 + aq * p2;
-                bv.f[XI(c, k, i)] = ap * p3 + aq * p4;
-            }
-            __syncthreads();
-            for (int q = lane; q < n_tr * 3 * P; q += nthr) {
-                const int b = q % P, c = (q / P) % 3, i = l_tr[q / (3 * P)];
-                const uint8_t fb = bv.fixed[PI_(b, i)];
-                if (fb >> c & 1) continue;
-                const double mass = bv.mass[aoff + i];
-                double rr = 0.0, vv = 0.0;
-                for (int k = 0; k < P; ++k) {
-                    rr = rr + bv.f[XI(c, k, i)] * C[b + P * k];
-                    vv = vv + bv.a[XI(c, k, i)] * C[b + P * k] / mass;
-                }
-                bv.x[XI(c, b, i)] = rr;
-                bv.v[XI(c, b, i)] = vv;
-            }
-            __syncthreads();
-            for (int q = lane; q < n_tr * 3 * P; q += nthr) {
-                const int b = q % P, c = (q / P) % 3, i = l_tr[q / (3 * P)];
-                bv.f[XI(c, b, i)] = 0.0;
-                bv.a[XI(c, b, i)] = 0.0;
+                ring_transform(s_x, s_v, C, tr, a_, b, na, P, mass, temp_k, dt, fb, x, v);
+                moved = moved || tr;
             }
         }
+        if (act)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) bv.f[xi + (long long)c * N] = f[c];
     }
-#undef XI
-#undef PI_
-#undef PT
-#undef AB
+    if (act)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const bool fixc = fb >> c & 1;
+            // a fixed component's v is written only when it was not 0 already
+            if (((flags & 3) || moved) && (!fixc || v0[c] != v[c])) bv.v[xi + (long long)c * N] = v[c];
+            if (moved && !fixc) bv.x[xi + (long long)c * N] = x[c];
+        }
     if (bad_local) atomicOr(&bv.status[t], bad_local);
 }
 
+// remove_com_velocity (the closed form of its 1000 iterations) from the
+// chunks' partial sums, then the transforms of the ring-polymer step.
+__global__ void __launch_bounds__(256)
+k_com_ring(const PropConst *__restrict__ pcg, BatchView bv, const double *cjk_all, const long long *cjk_off,
+           const PropChunk *__restrict__ chunks, int nchunk, const double *__restrict__ com, int flags) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double s_x[3][256], s_v[3][256];
+    const PropConst &pc = *pcg;
+    const int w = chunk_of_block(nchunk);
+    if (w >= nchunk) return;  // whole block: uniform
+    const PropChunk ch = chunks[w];
+    const int t = ch.t, na = ch.na, nb = ch.nb;
+    if (bv.done && bv.done[t]) return;  // frozen trajectory (whole block: uniform)
+    const int N = bv.traj_N[t], P = bv.traj_P[t];
+    const long long soff = bv.traj_soff[t];
+    const long long aoff = bv.traj_aoff[t];
+    const int lane = threadIdx.x, nthr = blockDim.x;
+    double *C = (double *)smem_raw;
+    const bool act = lane < na * nb;
+    const int b = lane / na, a_ = lane - b * na;
+    const int i = ch.i0 + a_;
+    const long long xi = soff + (long long)b * 3 * N + i;
+    double x[3] = {0.0, 0.0, 0.0}, v[3] = {0.0, 0.0, 0.0};
+    if (act)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] = bv.v[xi + (long long)c * N];
+    __shared__ double s_sub[3];
+    if (lane < 64) {  // the trajectory's partial sums, in an order of its own chunks only
+        double sum[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int q = lane; q < ch.count; q += 64)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sum[c] += com[4 * (long long)(ch.first + q) + c];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            for (int o = 32; o > 0; o >>= 1) sum[c] += __shfl_xor(sum[c], o, 64);
+        if (lane == 0) {
+            const double fac = (1.0 - pow(1.0 - 1.0 / N, 1000.0)) / sum[3] / P;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) s_sub[c] = sum[c] * fac;
+        }
+    }
+    __syncthreads();
+    if (act)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] -= s_sub[c];
+    const int ty = act ? bv.type[aoff + i] : 0;
+    const bool tr = (flags & 4) && nb > 1 && act && pc.algo[ty] != MDT_PROP_LANGEVIN;
+    if (__syncthreads_or(tr)) {
+        load_cjk(C, cjk_all + cjk_off[t], P, lane, nthr);
+        uint8_t fb = 7;
+        double mass = 1.0;
+        if (tr) {
+            fb = bv.fixed[soff / 3 + (long long)b * N + i];
+            mass = bv.mass[aoff + i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                x[c] = bv.x[xi + (long long)c * N];
+                s_x[c][lane] = x[c];
+                s_v[c][lane] = v[c];
+            }
+        }
+        __syncthreads();
+        ring_transform(s_x, s_v, C, tr, a_, b, na, P, mass, pc.is_proj[ty] ? bv.tproj[t] : bv.tsurf[t], pc.dt, fb, x, v);
+        if (tr)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                if (!(fb >> c & 1)) bv.x[xi + (long long)c * N] = x[c];
+    }
+    if (act)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) bv.v[xi + (long long)c * N] = v[c];
+}
+
+// traj_observe between propagate_2 and propagate_1 of k_prop, one workgroup
+// per trajectory
+__global__ void __launch_bounds__(256)
+k_observe(const PropConst *__restrict__ pcg, BatchView bv, const uint32_t *step_base, uint32_t step_prev) {
+    __shared__ int s_proj[MDT_MAXT];
+    __shared__ double s_rmin[4];
+    __shared__ int s_done;
+    const PropConst &pc = *pcg;
+    const int t = blockIdx.x;
+    if (bv.done && bv.done[t]) return;  // frozen trajectory (whole block: uniform)
+    if (step_base) step_prev += *step_base;
+    for (int k = threadIdx.x; k < MDT_MAXT; k += blockDim.x) s_proj[k] = pc.is_proj[k];
+    __syncthreads();
+    traj_observe(pc, s_proj, bv, t, bv.traj_N[t], bv.traj_P[t], bv.traj_soff[t], bv.traj_aoff[t], threadIdx.x,
+                 blockDim.x, step_prev, s_rmin, &s_done);
+}
+
 // ---------------------------------------------------------------------------
-// k_traj_classical: k_traj for batches of classical trajectories (P = 1)
-// with every atom on its own lane and no PILE or Andersen atoms (no COM
-// removal): each lane keeps its atom's state in registers from propagate_2
-// through propagate_1 and the force reset, reading and writing each array
-// once; the only barriers are the observer's.  Same arithmetic, in the same
-// order, as k_traj; a kernel of its own so that k_traj's ring-polymer code
-// does not set its register budget.
+// k_traj_classical: the propagators of batches of classical trajectories
+// (P = 1) with every atom on its own lane and no PILE or Andersen atoms (no
+// COM removal): each lane keeps its atom's state in registers from
+// propagate_2 through propagate_1 and the force reset, reading and writing
+// each array once; the only barriers are the observer's, which runs inside.
+// Same arithmetic, in the same order, as k_prop; a kernel of its own so that
+// k_prop's ring-polymer code does not set its register budget.
 __global__ void __launch_bounds__(256)
 k_traj_classical(const PropConst *__restrict__ pcg, BatchView bv, const uint32_t *step_base, uint32_t step_prev,
                  uint32_t step, int flags, int t_base) {
@@ -2318,17 +2376,36 @@ hipError_t mdt_launch_mixed(int tpa, int block, int ntraj, size_t smem, const Em
     return hipGetLastError();
 }
 
-// classical: every trajectory has P = 1 and at most `block` atoms, and no
-// atom type uses PILE or Andersen (k_traj_classical)
-hipError_t mdt_launch_traj(int ntraj, size_t smem, const PropConst *pc, const BatchView &bv, const double *cjk,
-                           const long long *cjk_off, const uint32_t *step_base, uint32_t step_prev, uint32_t step,
-                           int flags, int block, bool classical, hipStream_t st, int t_base) {
-    if (classical)
-        hipLaunchKernelGGL(k_traj_classical, dim3(ntraj), dim3(block), 0, st, pc, bv, step_base, step_prev, step,
-                           flags, t_base);
-    else
-        hipLaunchKernelGGL(k_traj, dim3(ntraj), dim3(block), smem, st, pc, bv, cjk, cjk_off, step_base, step_prev,
+// classical batches: every trajectory has P = 1 and at most `block` atoms,
+// and no atom type uses PILE or Andersen (k_traj_classical)
+hipError_t mdt_launch_traj_classical(int ntraj, const PropConst *pc, const BatchView &bv, const uint32_t *step_base,
+                                     uint32_t step_prev, uint32_t step, int flags, int block, hipStream_t st,
+                                     int t_base) {
+    hipLaunchKernelGGL(k_traj_classical, dim3(ntraj), dim3(block), 0, st, pc, bv, step_base, step_prev, step, flags,
+                       t_base);
+    return hipGetLastError();
+}
+
+// the other batches, over the chunk table.  With observation the frozen
+// trajectories are decided between propagate_2 and propagate_1; with COM
+// removal (com_on) propagate_1 and the transforms are two launches.
+hipError_t mdt_launch_prop(int ntraj, int maxP, const PropConst *pc, const BatchView &bv, const double *cjk,
+                           const long long *cjk_off, const PropChunk *chunks, int nchunk, double *com, bool com_on,
+                           const uint32_t *step_base, uint32_t step_prev, uint32_t step, int flags, hipStream_t st) {
+    const size_t smem = maxP > 1 ? sizeof(double) * maxP * (maxP + 1) : 0;
+    const dim3 g(((nchunk + 7) / 8) * 8), blk(256);
+    if ((flags & 1) && bv.obs) {
+        hipLaunchKernelGGL(k_prop, g, blk, smem, st, pc, bv, cjk, cjk_off, chunks, nchunk, com, step_base, step_prev,
+                           step, 1);
+        hipLaunchKernelGGL(k_observe, dim3(ntraj), blk, 0, st, pc, bv, step_base, step_prev);
+        flags &= ~1;
+    }
+    if ((flags & 2) && com_on) flags |= 8;
+    if (flags & 7)
+        hipLaunchKernelGGL(k_prop, g, blk, smem, st, pc, bv, cjk, cjk_off, chunks, nchunk, com, step_base, step_prev,
                            step, flags);
+    if (flags & 8)
+        hipLaunchKernelGGL(k_com_ring, g, blk, smem, st, pc, bv, cjk, cjk_off, chunks, nchunk, com, flags);
     return hipGetLastError();
 }
 

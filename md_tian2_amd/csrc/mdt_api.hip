@@ -35,8 +35,7 @@ size_t mdt_nene_smem(int N);
 size_t mdt_nene_radial_smem(int N);
 int mdt_nene_cap();
 hipError_t mdt_nene_attributes(hipFuncAttributes *fa, int radial);
-size_t mdt_nn_frame_smem(int N);
-hipError_t mdt_launch_nn_frame(int nblocks, size_t smem, const NnConst *M, const NnTrainView &tv, const int *frames,
+hipError_t mdt_launch_nn_frame(int nblocks, int maxN, size_t lds_limit, const NnConst *M, const NnTrainView &tv, const int *frames,
                                int mode, double cEw, double cFw, hipStream_t st);
 hipError_t mdt_launch_nn_mlp(int ntiles, const NnConst *M, const NnTrainView &tv, const int4 *tiles,
                              const int *rows, hipStream_t st);
@@ -44,7 +43,7 @@ hipError_t mdt_launch_nn_grad(int nblocks, const NnConst *M, const NnTrainView &
                               const int *rows, float *partials, hipStream_t st);
 hipError_t mdt_launch_nn_adam(NnConst *M, const float *partials, int W, float *grad, float *am, float *av, float lr,
                               float beta1, float beta2, float eps, int step, int mode, hipStream_t st);
-hipError_t mdt_launch_nene(int nrep, size_t smem, const NnConst *M, const BatchView &bv, float *G, float *C,
+hipError_t mdt_launch_nene(int nrep, int nmax, size_t lds_limit, const NnConst *M, const BatchView &bv, float *G, float *C,
                            int *rep_flag, double *fpes, int maxN, int add_fin, int skip_extrap, int radial,
                            uint16_t *nbr, uint8_t *nbr_cnt, uint32_t *nbr_ref, int *nbr_key, double skin_bohr,
                            hipStream_t st, int images);
@@ -1370,7 +1369,7 @@ static int launch_pes(mdt_batch *b, const BatchView &bv, int add_fin, hipStream_
             v.rep_list = k.d_reps;
             hipStream_t s2 = st;
             if ((rc = fork_stream(fk, &s2))) return rc;
-            HIPCHK(mdt_launch_nene(k.nrep, nn_smem(c, k.nmax), c->d_nn, v, b->d_nnG, b->d_nnC, b->d_nnflag,
+            HIPCHK(mdt_launch_nene(k.nrep, k.nmax, b->lds_limit, c->d_nn, v, b->d_nnG, b->d_nnC, b->d_nnflag,
                                    b->d_nnF, b->maxN, add_fin, 1, nn_radial(c), b->d_nnNbr, b->d_nnCnt, b->d_nnRef,
                                    b->d_nnKey, b->list_skin / MDT_BOHR2ANG, s2, nn_images(b, k)));
         }
@@ -2103,6 +2102,41 @@ int mdt_compute_emt_noalloc(mdt_context *ctx, int natoms, int nbeads, const int3
 // NENE surrogate (src/pes_nene_mod.f90: read_nene :123-5759, compute_nene
 // :7145-7368)
 // ---------------------------------------------------------------------------
+// the factored form of each element's angular functions (NnConst::f_*)
+static void factor_angular(NnConst &M) {
+    for (int e = 0; e < M.nelem; ++e) {
+        const int na = M.na[e];
+        int ok = na > 0 && na <= 16, nb = 0, nu = 0, used = 0;  // used: bit per slot
+        for (int k = 0; k < na && ok; ++k) {
+            if (M.a_e1[e][k] != M.a_e1[e][0] || M.a_e2[e][k] != M.a_e2[e][0]) ok = 0;
+            int n = 0, m = 0;
+            while (n < nb && M.f_etal2[e][n] != M.a_etal2[e][k]) ++n;
+            while (m < nu && !(M.f_lam[e][m] == M.a_lam[e][k] && M.f_zp[e][m] == M.a_zp[e][k])) ++m;
+            if (n == 4 || m == 4) {
+                ok = 0;
+                break;
+            }
+            if (n == nb) {
+                M.f_etal2[e][nb] = M.a_etal2[e][k];
+                M.f_eta[e][nb] = M.a_etal2[e][k] * (1.0f / 1.4426950408889634f);
+                ++nb;
+            }
+            if (m == nu) {
+                M.f_lam[e][nu] = M.a_lam[e][k];
+                M.f_zp[e][nu] = M.a_zp[e][k];
+                M.f_zl[e][nu] = (float)(1 << M.a_zp[e][k]) * M.a_lam[e][k];
+                ++nu;
+            }
+            const int slot = 4 * n + m;
+            if (used >> slot & 1) ok = 0;  // two functions on one slot
+            used |= 1 << slot;
+            M.f_slot[e][k] = slot;
+        }
+        M.f_ok[e] = ok;
+        M.f_mask[e] = na > 0 ? 1 << M.a_e1[e][0] | 1 << M.a_e2[e][0] : 0;
+    }
+}
+
 int mdt_nn_params_set(mdt_context *ctx, int nelem, const int32_t *elem_of_type, int ntypes, const int32_t *nsf,
                       const int32_t *sf_type, const int32_t *sf_e1, const int32_t *sf_e2, const double *eta,
                       const double *rs, const double *lambda, const double *zeta, const double *rc,
@@ -2153,6 +2187,7 @@ int mdt_nn_params_set(mdt_context *ctx, int nelem, const int32_t *elem_of_type, 
                 if (nr >= NN_MAXR) return bail(MDT_EUNSUP, "element %d: too many radial functions", e);
                 M->r_el[e][nr] = sf_e1[q];
                 M->r_eta[e][nr] = (float)eta[q];
+                M->r_ce[e][nr] = (float)(-eta[q] * 1.4426950408889634);
                 M->r_rs[e][nr] = (float)rs[q];
                 ++nr;
             } else if (sf_type[q] == 3) {
@@ -2213,6 +2248,7 @@ int mdt_nn_params_set(mdt_context *ctx, int nelem, const int32_t *elem_of_type, 
     }
     M->nh1 = nh1;
     M->nh2 = nh2;
+    factor_angular(*M);
     M->radial_only = 1;
     for (int e = 0; e < nelem; ++e) {
         if (M->na[e] > 0) M->radial_only = 0;
@@ -2342,7 +2378,7 @@ int mdt_compute_nene(mdt_context *ctx, int natoms, int nbeads, const int32_t *id
     if ((rc = ensure_nn(b))) return rc;
     if ((rc = ensure_ready(b, false))) return rc;
     HIPCHK(hipMemsetAsync(b->d_status, 0, sizeof(int) * b->ntraj, ctx->stream));
-    HIPCHK(mdt_launch_nene(b->nrep, nn_smem(ctx, b->maxN), ctx->d_nn, b->view(), b->d_nnG, b->d_nnC, b->d_nnflag,
+    HIPCHK(mdt_launch_nene(b->nrep, b->maxN, b->lds_limit, ctx->d_nn, b->view(), b->d_nnG, b->d_nnC, b->d_nnflag,
                            b->d_nnF, b->maxN, 0, 0, nn_radial(ctx), b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey,
                            b->list_skin / MDT_BOHR2ANG, ctx->stream, 1));
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -2567,7 +2603,7 @@ int mdt_nn_train_create(mdt_context *ctx, int nframes, const int32_t *natoms, co
     HIPCHK(hipMemset(tr->d_G, 0, sizeof(float) * rowsK));
     // descriptors of every frame (they depend on the positions only)
     hipStream_t st = ctx->stream;
-    HIPCHK(mdt_launch_nn_frame(nframes, mdt_nn_frame_smem(tr->maxN), ctx->d_nn, tr->view(), tr->d_frames, 0, 0.0,
+    HIPCHK(mdt_launch_nn_frame(nframes, tr->maxN, ctx->lds_limit, ctx->d_nn, tr->view(), tr->d_frames, 0, 0.0,
                                0.0, st));
     HIPCHK(hipStreamSynchronize(st));
     *out = tr;
@@ -2620,7 +2656,7 @@ static int run_minibatch(mdt_nntrain *tr, int m, double wE, double wF, int mode,
     const int nf = tr->fr_off[m + 1] - tr->fr_off[m];
     const int t0 = tr->tl_off[m], nt = tr->tl_off[m + 1] - t0;
     HIPCHK(mdt_launch_nn_mlp(nt, c->d_nn, tv, tr->d_tiles + t0, tr->d_rows, st));
-    HIPCHK(mdt_launch_nn_frame(nf, mdt_nn_frame_smem(tr->maxN), c->d_nn, tv, tr->d_frames + tr->fr_off[m], 1,
+    HIPCHK(mdt_launch_nn_frame(nf, tr->maxN, c->lds_limit, c->d_nn, tv, tr->d_frames + tr->fr_off[m], 1,
                                wE / nf, wF / (3.0 * tr->natoms_mb[m]), st));
     if (mode < 0) return 0;  // evaluation only
     const int nb = grad_blocks(tr, nt), W = nb * 4;
@@ -2733,7 +2769,7 @@ int mdt_nn_train_loss_grad(mdt_nntrain *tr, int nsel, const int32_t *frames, dou
     if (e1 == hipSuccess) e1 = hipMemcpy(df, frames, sizeof(int) * nsel, hipMemcpyHostToDevice);
     if (e1 == hipSuccess) e1 = mdt_launch_nn_mlp((int)tiles.size(), c->d_nn, tv, dt, dr, st);
     if (e1 == hipSuccess)
-        e1 = mdt_launch_nn_frame(nsel, mdt_nn_frame_smem(tr->maxN), c->d_nn, tv, df, 1, wE / nsel, wF / (3.0 * nat), st);
+        e1 = mdt_launch_nn_frame(nsel, tr->maxN, c->lds_limit, c->d_nn, tv, df, 1, wE / nsel, wF / (3.0 * nat), st);
     if (e1 == hipSuccess)
         e1 = hipMemsetAsync(tr->d_partials, 0, sizeof(float) * (size_t)W * NN_MAXE * NN_NPAR, st);
     if (e1 == hipSuccess)

@@ -218,11 +218,23 @@ struct NnConst {
     int nr[NN_MAXE], na[NN_MAXE];    // radial / angular functions per element (inputs 0..nr-1, nr..nr+na-1)
     int r_el[NN_MAXE][NN_MAXR];      // neighbour element of radial function
     float r_eta[NN_MAXE][NN_MAXR], r_rs[NN_MAXE][NN_MAXR];
+    float r_ce[NN_MAXE][NN_MAXR];    // -eta log2(e)
     int a_e1[NN_MAXE][NN_MAXA], a_e2[NN_MAXE][NN_MAXA];
     float a_etal2[NN_MAXE][NN_MAXA];  // eta log2(e)
     float a_lam[NN_MAXE][NN_MAXA];
     float a_norm[NN_MAXE][NN_MAXA];   // 2^(1 - zeta)
     int a_zp[NN_MAXE][NN_MAXA];       // zeta = 2^a_zp (1, 2, 4, 8 or 16)
+    // factored angular sums: an element whose angular functions share one
+    // neighbour-pair class, take at most 4 distinct eta and 4 distinct
+    // (lambda, zeta), and map one-to-one onto (eta, (lambda, zeta)) slots
+    // accumulates per neighbour pair the outer product of B_n = exp(-eta_n
+    // (rij^2 + rik^2 + rjk^2)) and u_m = (1 + lambda_m cos)^zeta_m; function
+    // k is norm_k * slot f_slot = 4 n + m.  f_mask: bits of the class's
+    // elements; f_zl = zeta lambda
+    int f_ok[NN_MAXE], f_mask[NN_MAXE];
+    float f_etal2[NN_MAXE][4], f_eta[NN_MAXE][4], f_lam[NN_MAXE][4], f_zl[NN_MAXE][4];
+    int f_zp[NN_MAXE][4];
+    int f_slot[NN_MAXE][NN_MAXA];
     float smul[NN_MAXE][NN_K1], sadd[NN_MAXE][NN_K1];  // network input x = G smul + sadd
     float dfac[NN_MAXE][NN_K1];                         // dE/dG = dE/dx dfac
     float glo[NN_MAXE][NN_K1], ghi[NN_MAXE][NN_K1];     // extrapolation bounds min - 1e-4, max + 1e-4

@@ -3,24 +3,25 @@
 // evaluates (src/pes_nene_mod.f90:7145-7368; RuNNer getshortatomic,
 // atomsymfunction2, atomsymfunction3Andi, getcutoff type 1, calconenn).
 //
-// k_nene: calc_force with the network, one workgroup (256 lanes) per
-// replica (trajectory t, bead b):
-//   stage    fractional coordinates (FP64) and element of every atom in LDS;
-//   pass G   centre atoms in chunks of 16 (16 lanes each): build the chunk's
-//            neighbour lists within rc over all periodic images (ordered,
-//            two-pass count/write, no atomics) with d, 1/r, fc, dfc in LDS,
-//            then radial sums over neighbours and angular sums over
-//            neighbour pairs; raw G to the replica's scratch rows; values
-//            outside [min - 1e-4, max + 1e-4] flag the replica;
+// k_nene_g / k_nene_f: calc_force with the network, one workgroup per
+// replica (trajectory t, bead b), one wavefront per centre atom at a time:
+//   stage    fractional coordinates (2^-32 fixed point) and element of every
+//            atom in LDS;
+//   pass G   the centre's neighbour list within rc over all periodic images
+//            (ordered, no atomics) with d, 1/r, fc, dfc in LDS, then radial
+//            sums over neighbours and angular sums over neighbour pairs; raw
+//            G to the replica's scratch rows; values outside [min - 1e-4,
+//            max + 1e-4] flag the replica;
 //   network  per element, 16-atom tiles per wavefront on
-//            v_mfma_f32_16x16x32_bf16 with operands split into bf16 hi + lo
-//            parts (three products per tile, FP32 accumulation: ~16-bit
-//            operand precision); forward to the atomic energy, backward to
-//            c = dE/dG (scaling factor folded in), written to scratch;
-//   pass F   the same chunks again: dE/dr = sum_k c_k dG_k/dr contracted
-//            per neighbour / neighbour pair, +F on the centre in registers,
-//            the neighbours' shares into fixed-point LDS accumulators
-//            (order-independent: bitwise reproducible);
+//            v_mfma_f32_16x16x32_bf16 with operands split into three bf16
+//            parts (six products per tile, FP32 accumulation: FP32 operand
+//            precision); forward to the atomic energy, backward to c =
+//            dE/dG (scaling factor folded in), written to scratch;
+//   pass F   the lists again: dE/dr = sum_k c_k dG_k/dr contracted per
+//            neighbour / neighbour pair, the neighbours' shares into
+//            fixed-point LDS accumulators (order-independent: bitwise
+//            reproducible), minus their sum on the centre;
+// Networks without angular functions run k_nene_rg / k_nene_rf instead.
 //   output   f, a = f/m (fixed components 0), epot (fixed-order sum).
 // Positions arrive in Angstrom (FP64) and are converted to Bohr; energy
 // and forces leave in eV and eV/Angstrom, as compute_nene adds them
@@ -30,7 +31,10 @@
 #include "mdt_device.h"
 
 #define NN_TPA 16
-#define NN_CA 16             // centre atoms per chunk (256 lanes / 16)
+#define NN_CA 16             // centre atoms per chunk of the radial kernels (256 lanes / 16)
+#define NN_KB 16             // generic angular functions summed at a time
+#define NN_RB 8              // radial functions at a time
+#define NN_FB 4              // distinct exponents and powers of the factored angular sums
 #define NN_CAP 96            // neighbours within rc per atom (fcc Au at 6.5 A: 78)
 #define NN_BLOCK 256
 #define NN_L2E 1.4426950408889634f
@@ -61,28 +65,6 @@ struct NnView {
     float skin;         // Bohr
 };
 
-// symmetry-function tables every lane indexes by element (LDS copy)
-struct NnSfTab {
-    int nr[NN_MAXE], na[NN_MAXE];
-    int8_t r_el[NN_MAXE][NN_MAXR];
-    float r_eta[NN_MAXE][NN_MAXR], r_rs[NN_MAXE][NN_MAXR];
-    int8_t a_cls[NN_MAXE][NN_MAXA];  // neighbour-pair class e1 * NN_MAXE + e2 (e1 <= e2)
-    float a_eta[NN_MAXE][NN_MAXA], a_etal2[NN_MAXE][NN_MAXA], a_lam[NN_MAXE][NN_MAXA], a_norm[NN_MAXE][NN_MAXA];
-    int8_t a_zp[NN_MAXE][NN_MAXA];
-    // factored angular sums: an element whose angular functions share one
-    // neighbour-pair class, take at most NN_FB distinct eta and NN_FB
-    // distinct (lambda, zeta), and map one-to-one onto (eta, (lambda,
-    // zeta)) slots accumulates per triplet the outer product of
-    // B_n = exp(-eta_n (rij^2 + rik^2 + rjk^2)) and u_m = (1 + lambda_m
-    // cos)^zeta_m; function k is norm_k * slot (n_k, m_k)
-    int f_ok[NN_MAXE], f_cls[NN_MAXE], f_nb[NN_MAXE], f_nu[NN_MAXE];
-    float f_etal2[NN_MAXE][4], f_eta[NN_MAXE][4], f_lam[NN_MAXE][4];
-    int f_zp[NN_MAXE][4];
-    int8_t f_slot[NN_MAXE][NN_MAXA];  // n * NN_FB + m
-};
-#define NN_FB 4
-static_assert(NN_FB * NN_FB == NN_TPA, "one slot of the factored angular sums per lane of a centre's group");
-
 __device__ __forceinline__ float act_f(int code, float z, float *d1) {
     if (code == 1) {
         const float h = tanhf(z);
@@ -107,6 +89,41 @@ __device__ __forceinline__ void cutoff(float pi_rc, float r, float *fc, float *d
     *dfc = -0.5f * pi_rc * s;
 }
 
+// The same as a polynomial in s = 2 r^2 / rc^2 - 1 in [-1, 1] (cos is even in
+// r, so neither r nor a sine is needed; Chebyshev interpolation of 0.5 (1 +
+// cos(pi sqrt((s + 1) / 2))), 6e-11 at degree 7 and 4e-15 at degree 9):
+// *fc, and *dfr = dfc/ds = dfc/dr rc^2 / (4 r).
+__device__ __forceinline__ void cut_poly(float s, float *fc, float *dfr) {
+    const float a[8] = {0.197150066f, -0.441896469f, 0.297287184f, -0.0577822716f,
+                        0.00555029732f, -0.000320913322f, 1.24524271e-05f, -3.46419213e-07f};
+    float p = a[7], d = 0.f;
+#pragma unroll
+    for (int k = 6; k >= 0; --k) {
+        d = d * s + p;
+        p = p * s + a[k];
+    }
+    *fc = p;
+    *dfr = d;
+}
+__constant__ double c_cut9[10] = {0.19715006646059666, -0.44189646865659865, 0.29728718197212139, -0.057782271571948658,
+                                 0.0055503064048013544, -0.00032091347134881624, 1.2437897731294723e-05, -3.4618099399447157e-07,
+                                 7.2647468318809416e-09, -1.1911074904169539e-10};
+__device__ __forceinline__ void cut_poly(double s, double *fc, double *dfr) {
+    // the coefficients are loaded here at every call: kept in registers over
+    // the centres' loop they would cost the pair loops 20
+    int z = 0;
+    asm volatile("" : "+s"(z));
+    const double *a = c_cut9 + z;
+    double p = a[9], d = 0.0;
+#pragma unroll
+    for (int k = 8; k >= 0; --k) {
+        d = d * s + p;
+        p = p * s + a[k];
+    }
+    *fc = p;
+    *dfr = d;
+}
+
 __device__ __forceinline__ void split8(const float v[8], bf16x8 &hi, bf16x8 &lo) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -114,6 +131,35 @@ __device__ __forceinline__ void split8(const float v[8], bf16x8 &hi, bf16x8 &lo)
         hi[j] = h;
         lo[j] = (__bf16)(v[j] - (float)h);
     }
+}
+
+// v as three bf16 parts of 8 bits each: all 24 bits of an FP32 operand
+struct Bf3 {
+    bf16x8 h, m, l;
+};
+__device__ __forceinline__ Bf3 split24(const float v[8]) {
+    Bf3 r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const __bf16 h = (__bf16)v[j];
+        const float v1 = v[j] - (float)h;
+        const __bf16 m = (__bf16)v1;
+        r.h[j] = h;
+        r.m[j] = m;
+        r.l[j] = (__bf16)(v1 - (float)m);
+    }
+    return r;
+}
+
+// D += A B to FP32 operand precision: the six products above 2^-24
+__device__ __forceinline__ f32x4 mfma6(const Bf3 &a, const Bf3 &b, f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, b.h, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.l, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.h, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.m, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.h, c, 0, 0, 0);
+    return c;
 }
 
 // D += A B with A, B given as bf16 hi + lo: hi*hi + hi*lo + lo*hi
@@ -134,6 +180,16 @@ __device__ __forceinline__ void fxadd(unsigned long long *acc, double x, int *ba
     atomicAdd(acc, (unsigned long long)(long long)rint(y));
 }
 
+// fxadd on a register
+__device__ __forceinline__ void fxput(unsigned long long *acc, double x, int *bad) {
+    const double y = x * NN_FSCALE;
+    if (!(fabs(y) < 9.0e18)) {
+        *bad |= MDT_ST_FIXED_OVERFLOW;
+        return;
+    }
+    *acc += (unsigned long long)(long long)rint(y);
+}
+
 // x * 2^32 from an FP32 x as a 64-bit fixed-point addend: floor(x) and the
 // 32-bit fraction (x - floor(x)) 2^32, both exact in FP32 for |x| < 2^31
 // (exact when x has no bits below 2^-32, truncated below that)
@@ -147,21 +203,37 @@ __device__ __forceinline__ void fxadd32(unsigned long long *acc, float x, int *b
     atomicAdd(acc, ((unsigned long long)(uint32_t)(int)fl << 32) + lo);
 }
 
-// per-chunk neighbour data (structure of arrays)
-struct ChunkNbr {
-    float dx[NN_CA * NN_CAP], dy[NN_CA * NN_CAP], dz[NN_CA * NN_CAP];
-    float fc[NN_CA * NN_CAP], dfc[NN_CA * NN_CAP];
-    uint16_t j[NN_CA * NN_CAP];
-    uint8_t el[NN_CA * NN_CAP];
-    int cnt[NN_CA];
+// x * 2^32 rounded to nearest as a 64-bit fixed-point addend, |x| < 2^19:
+// adding 1.5 2^52 leaves the rounded value in the low mantissa bits
+#define NN_MAGIC 6755399441055744.0
+__device__ __forceinline__ unsigned long long fix32(float x) {
+    return (unsigned long long)(__double_as_longlong(fma((double)x, NN_FSCALE, NN_MAGIC)) - __double_as_longlong(NN_MAGIC));
+}
+#define NN_FIX32_MAX 5.0e5f
+
+// Neighbours of one centre, one list per wavefront.  p: the vector (Bohr)
+// and the neighbour's index | element << 16 | 1 << element << 20; q: 1/r,
+// r^2, fc, dfc / r.  queue: pairs of entries (p | q << 8) waiting to be
+// evaluated.  The words after it hold, per entry, the fixed-point force (x,
+// y, z; pass F) or g_j - g_i (the Jacobian-vector product).
+struct WaveNbr {
+    float4 p[NN_CAP], q[NN_CAP];
+    uint16_t queue[128];
+};
+struct WaveNbrF : WaveNbr {
+    unsigned long long acc[3][NN_CAP];
 };
 
-// r and 1/r of a neighbour entry (from its vector: one reciprocal square root)
-__device__ __forceinline__ void nbr_rir(const ChunkNbr &L, int e, float *r, float *ir) {
-    const float x = L.dx[e], y = L.dy[e], z = L.dz[e];
-    const float r2 = x * x + y * y + z * z;
-    *ir = __builtin_amdgcn_rsqf(r2);
-    *r = r2 * *ir;
+__device__ __forceinline__ int nbr_j(const float4 &p) { return __float_as_int(p.w) & 0xFFFF; }
+__device__ __forceinline__ int nbr_el(const float4 &p) { return (__float_as_int(p.w) >> 16) & 15; }
+__device__ __forceinline__ int nbr_mask(const float4 &p) { return __float_as_int(p.w) >> 20; }
+
+// orders a wavefront's LDS writes before its later LDS reads (buffers
+// private to one wavefront)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 }  // namespace
@@ -173,37 +245,37 @@ __device__ __forceinline__ uint32_t frac_fix(double f) {
     return (uint32_t)(unsigned long long)(f * 4294967296.0);
 }
 
-// Neighbour list of centre i (16 lanes; i < 0: none) within rc over all
-// periodic images: lane `sub` tests atoms n = sub, sub+16, ...; hits are
-// counted, prefix-summed over the 16 lanes and passed to put(pos, n, ex, ey,
+// Neighbour list of centre i (W lanes; i < 0: none) within rc over all
+// periodic images: lane `sub` tests atoms n = sub, sub+W, ...; hits are
+// counted, prefix-summed over the W lanes and passed to put(pos, n, ex, ey,
 // ez, r2) in (lane, n, image) order (vector in Bohr).  Returns the number of
 // hits (in every lane of the group); more than NN_CAP set the overflow flag
 // and only the first NN_CAP are passed.  ux, uy, uz: the atoms' fractional
 // coordinates (frac_fix).
-template <class Put>
+template <int W = NN_TPA, class Put>
 __device__ int build_images(float rc2, const uint32_t *ux, const uint32_t *uy, const uint32_t *uz, const double h[9],
                             const int *imax, float wx, float wy, float wz, int N, int i, int lane, int *bad,
                             Put put) {
-    const int sub = lane % NN_TPA;
+    const int sub = lane % W;
     int cnt = 0, tot = 0;
     for (int pass = 0; pass < 2; ++pass) {
         int base = 0;
         if (pass == 1) {
-            // exclusive prefix of the 16 lanes' counts
+            // exclusive prefix of the W lanes' counts
             int incl = cnt;
 #pragma unroll
-            for (int o = 1; o < NN_TPA; o <<= 1) {
-                const int y = __shfl_up(incl, o, NN_TPA);
+            for (int o = 1; o < W; o <<= 1) {
+                const int y = __shfl_up(incl, o, W);
                 if (sub >= o) incl += y;
             }
             base = incl - cnt;
-            tot = __shfl(incl, NN_TPA - 1, NN_TPA);
+            tot = __shfl(incl, W - 1, W);
             if (tot > NN_CAP) *bad |= MDT_ST_NBR_OVERFLOW;
         }
         int pos = base;
         if (i >= 0) {
             const long long xi = ux[i], yi = uy[i], zi = uz[i];
-            for (int n = sub; n < N; n += NN_TPA) {
+            for (int n = sub; n < N; n += W) {
                 const double f0 = (double)((long long)ux[n] - xi) * 0x1p-32;  // in (-1, 1)
                 const double f1 = (double)((long long)uy[n] - yi) * 0x1p-32;
                 const double f2 = (double)((long long)uz[n] - zi) * 0x1p-32;
@@ -234,28 +306,54 @@ __device__ int build_images(float rc2, const uint32_t *ux, const uint32_t *uy, c
     return tot;
 }
 
-// Builds the neighbour lists of centre atoms k0 .. k0+NN_CA-1 (16 lanes per
-// centre) with d, fc, dfc, the neighbour and its element per entry.
-__device__ void build_chunk(float rc2, float pi_rc, ChunkNbr &L, const uint32_t *ux, const uint32_t *uy,
-                            const uint32_t *uz, const uint8_t *elem, const double h[9], const int *imax, float wx,
-                            float wy, float wz, int N, int k0, int lane, int *bad) {
-    const int c = lane / NN_TPA, sub = lane % NN_TPA;
-    const int i = k0 + c;
-    const int tot = build_images(rc2, ux, uy, uz, h, imax, wx, wy, wz, N, i < N ? i : -1, lane, bad,
-                                 [&](int pos, int n, double ex, double ey, double ez, double r2) {
-                                     const int e = c * NN_CAP + pos;
-                                     const float rr = (float)sqrt(r2);
-                                     float fcv, dfcv;
-                                     cutoff(pi_rc, rr, &fcv, &dfcv);
-                                     L.dx[e] = (float)ex;
-                                     L.dy[e] = (float)ey;
-                                     L.dz[e] = (float)ez;
-                                     L.fc[e] = fcv;
-                                     L.dfc[e] = dfcv;
-                                     L.j[e] = (uint16_t)n;
-                                     L.el[e] = elem[n];
-                                 });
-    if (sub == 0) L.cnt[c] = tot < NN_CAP ? tot : NN_CAP;
+// The neighbour list of centre i on one wavefront: every image of an atom
+// within rc, by the minimum image where the cut-off sphere fits the cell
+// (w < 1/2 on every axis: one pass, hits compacted in atom order by a
+// ballot), else by the image search.  Returns the number of entries.
+__device__ __forceinline__ int build_list(float rc2, WaveNbr &L, const uint32_t *ux, const uint32_t *uy,
+                          const uint32_t *uz, const uint8_t *elem, const double *s_h, const int *imax, float wx,
+                          float wy, float wz, int N, int i, int l, int *bad) {
+    const double two_rc2 = 2.0 / (double)rc2;
+    auto put = [&](int e, int n, double ex, double ey, double ez, double r2) {
+        const double y = __builtin_amdgcn_rsq(r2);
+        const double ir = fma(y * 0.5, fma(-(r2 * y), y, 1.0), y);
+        double fcv, dfr;
+        cut_poly(r2 * two_rc2 - 1.0, &fcv, &dfr);
+        const int el = elem[n];
+        L.p[e] = make_float4((float)ex, (float)ey, (float)ez, __int_as_float(n | el << 16 | 1 << (20 + el)));
+        L.q[e] = make_float4((float)ir, (float)r2, (float)fcv, (float)(2.0 * two_rc2 * dfr));
+    };
+    int tot = 0;
+    wave_lds_sync();  // the previous centre's reads are done; the cell (LDS) is read once per list
+    double h[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) h[k] = s_h[k];
+    if (wx < 0.4999f && wy < 0.4999f && wz < 0.4999f) {
+        const uint32_t xi = ux[i], yi = uy[i], zi = uz[i];
+        const unsigned long long below = l == 0 ? 0ull : ~0ull >> (64 - l);
+        for (int n0 = 0; n0 < N; n0 += 64) {
+            const int n = n0 + l;
+            double ex = 0.0, ey = 0.0, ez = 0.0, r2 = 1e300;
+            if (n < N && n != i) {
+                const double g0 = (double)(int)(ux[n] - xi) * 0x1p-32, g1 = (double)(int)(uy[n] - yi) * 0x1p-32,
+                             g2 = (double)(int)(uz[n] - zi) * 0x1p-32;
+                ex = h[0] * g0 + h[3] * g1 + h[6] * g2;
+                ey = h[1] * g0 + h[4] * g1 + h[7] * g2;
+                ez = h[2] * g0 + h[5] * g1 + h[8] * g2;
+                r2 = ex * ex + ey * ey + ez * ez;
+            }
+            const bool in = r2 <= (double)rc2;
+            const unsigned long long m = __ballot(in);
+            const int pos = tot + __popcll(m & below);
+            if (in && pos < NN_CAP) put(pos, n, ex, ey, ez, r2);
+            tot += __popcll(m);
+        }
+        if (tot > NN_CAP) *bad |= MDT_ST_NBR_OVERFLOW;
+    } else {
+        tot = build_images<64>(rc2, ux, uy, uz, h, imax, wx, wy, wz, N, i, l, bad, put);
+    }
+    wave_lds_sync();
+    return tot < NN_CAP ? tot : NN_CAP;
 }
 
 template <int WIDTH>
@@ -284,22 +382,21 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
     f32x4 z1[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
+        if (ks * 32 >= nin) break;  // wavefront-uniform
         float av[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int k = ks * 32 + kg + j;
             av[j] = (atomA >= 0 && k < nin) ? Grep[(size_t)atomA * NN_K1 + k] * M.smul[ee][k] + M.sadd[ee][k] : 0.f;
         }
-        bf16x8 ah, al;
-        split8(av, ah, al);
+        const Bf3 a = split24(av);
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             float bv[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) bv[j] = M.W1[ee][ks * 32 + kg + j][nt * 16 + nB];
-            bf16x8 bh, bl;
-            split8(bv, bh, bl);
-            z1[nt] = mfma3(ah, al, bh, bl, z1[nt]);
+            const Bf3 b = split24(bv);
+            z1[nt] = mfma6(a, b, z1[nt]);
         }
     }
     float h1[2][4], d1[2][4];
@@ -318,17 +415,15 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
     for (int j = 0; j < 8; ++j) av2[j] = T[rA * 33 + kg + j];
     __syncthreads();
     // ---- layer 2 ----
-    bf16x8 ah, al;
-    split8(av2, ah, al);
+    Bf3 a = split24(av2);
     f32x4 z2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         float bv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) bv[j] = M.W2[ee][kg + j][nt * 16 + nB];
-        bf16x8 bh, bl;
-        split8(bv, bh, bl);
-        z2[nt] = mfma3(ah, al, bh, bl, z2[nt]);
+        const Bf3 b = split24(bv);
+        z2[nt] = mfma6(a, b, z2[nt]);
     }
     float h2[2][4], d2[2][4];
 #pragma unroll
@@ -356,7 +451,7 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
 #pragma unroll
     for (int j = 0; j < 8; ++j) av2[j] = T[rA * 33 + kg + j];
     __syncthreads();
-    split8(av2, ah, al);
+    a = split24(av2);
     // dE/dh1 = delta2 W2^T
     f32x4 g1[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -364,9 +459,8 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
         float bv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) bv[j] = M.W2[ee][nt * 16 + nB][kg + j];
-        bf16x8 bh, bl;
-        split8(bv, bh, bl);
-        g1[nt] = mfma3(ah, al, bh, bl, g1[nt]);
+        const Bf3 b = split24(bv);
+        g1[nt] = mfma6(a, b, g1[nt]);
     }
     // delta1 = dE/dz1 -> A layout
 #pragma unroll
@@ -377,17 +471,17 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
 #pragma unroll
     for (int j = 0; j < 8; ++j) av2[j] = T[rA * 33 + kg + j];
     __syncthreads();
-    split8(av2, ah, al);
+    a = split24(av2);
     // dE/dx = delta1 W1^T, four 16-column tiles of the 64 inputs
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
+        if (nt * 16 >= nin) break;  // wavefront-uniform
         float bv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) bv[j] = M.W1[ee][nt * 16 + nB][kg + j];
-        bf16x8 bh, bl;
-        split8(bv, bh, bl);
+        const Bf3 b = split24(bv);
         f32x4 dx = {0.f, 0.f, 0.f, 0.f};
-        dx = mfma3(ah, al, bh, bl, dx);
+        dx = mfma6(a, b, dx);
         const int k = nt * 16 + nB;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -397,530 +491,555 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
     }
 }
 
-// Symmetry functions of the chunk's centre atoms (16 lanes each) into
-// Grep rows; *extrap set when a value leaves [min - 1e-4, max + 1e-4].
-__device__ void g_chunk(const NnConst &Mc, const NnSfTab &S, const ChunkNbr &L, const uint8_t *elem, int N, int k0,
-                        int lane,
-                        float rc2, float pi_rc, float *Grep, int *extrapp) {
-    const int c = lane / NN_TPA, sub = lane % NN_TPA;
-    int extrap = 0;
-    struct {
-        float rc2, pi_rc;
-    } M{rc2, pi_rc};
-    const int i = k0 + c;
-    const int cnt = L.cnt[c];
-    const int e = (i < N) ? elem[i] : 0;
-    const int nr = (i < N) ? S.nr[e] : 0, na = (i < N) ? S.na[e] : 0;
-    const int base = c * NN_CAP;
-    float g[NN_MAXR > NN_MAXA ? NN_MAXR : NN_MAXA];
-    // radial (atomsymfunction2: exp(-eta (r - rs)^2) fc(r))
-#pragma unroll
-    for (int k = 0; k < NN_MAXR; ++k) g[k] = 0.f;
-    for (int p = sub; p < cnt; p += NN_TPA) {
-        float r, irp;
-        nbr_rir(L, base + p, &r, &irp);
-        const float fcv = L.fc[base + p];
-        const int ep = L.el[base + p];
-#pragma unroll
-        for (int k = 0; k < NN_MAXR; ++k)
-            if (k < nr && ep == S.r_el[e][k]) {
-                const float dr = r - S.r_rs[e][k];
-                g[k] += __builtin_amdgcn_exp2f(-S.r_eta[e][k] * NN_L2E * dr * dr) * fcv;
-            }
-    }
-#pragma unroll
-    for (int k = 0; k < NN_MAXR; ++k) {
-        const float v = sum_group<NN_TPA>(g[k]);
-        if (i < N && k < nr && sub == (k & (NN_TPA - 1))) {
-            Grep[(size_t)i * NN_K1 + k] = v;
-            if (v < Mc.glo[e][k] || v > Mc.ghi[e][k]) extrap = 1;
+// ---------------------------------------------------------------------------
+// Networks with angular functions: one wavefront per centre atom.
+// What bounds them is the neighbour pairs (1.6 k per atom of a 6.5 A list),
+// of which only about 47 % are within rc of each other.  A loop over the pairs with
+// a test inside runs at that share of its lanes, and a triangular loop over
+// 16 lanes loses more at its ends; so the wavefront tests pairs 64 at a time
+// and queues those that count, and evaluates the queue 64 at a time with
+// every lane at work.  With one centre per wavefront every parameter of its
+// functions is wavefront-uniform (scalar registers, no tables in LDS).
+// H/Au 6x6x4, 512 replicas: k_nene_g 1017 -> 439 us, k_nene_f 1570 -> 615 us,
+// issuing vector instructions 85 % of the time; the training gradient over
+// 256 frames of 37 atoms: k_nn_frame 2240 -> 167 us.  The error against FP64
+// fell too (forces 2.1e-5 -> 3.3e-6 relative, gradient 2.7e-3 -> 3.9e-4): the
+// cut-off without the hardware's sine and cosine, and the network's
+// operands split in three bf16 parts instead of two (mfma6).
+// ---------------------------------------------------------------------------
+
+// Evaluates body(pq, on) for the pairs of entries pq = p | q << 8 within rc of
+// each other whose elements are exactly those of `mask` (0: any), 64 at a time
+// (on: the lane has a pair; lanes without one are given some pair).
+// Pairs go by their circular distance d = 1, 2, ... (q = p + d mod cnt), so
+// that a batch holds a neighbour in few lanes: pass F adds to both
+// neighbours' words.
+template <class Body>
+__device__ __forceinline__ void for_pairs(WaveNbr &L, int cnt, int mask, float rc2, int l, Body body) {
+    if (cnt < 2) return;
+    const int total = cnt * (cnt - 1) / 2;
+    const int sd = 64 / cnt, sp = 64 - sd * cnt;
+    const unsigned long long below = l == 0 ? 0ull : ~0ull >> (64 - l);
+    int d = l / cnt, p = l - d * cnt, nq = 0;
+    ++d;
+    for (int t0 = 0; t0 < total; t0 += 64) {
+        bool in = t0 + l < total;
+        int q = p + d;
+        q -= q >= cnt ? cnt : 0;
+        if (in) {
+            const float4 a = L.p[p], b = L.p[q];
+            const float cx = b.x - a.x, cy = b.y - a.y, cz = b.z - a.z;
+            const int m = (__float_as_int(a.w) | __float_as_int(b.w)) >> 20;
+            in = !(cx * cx + cy * cy + cz * cz > rc2) && (mask == 0 || m == mask);
+        }
+        const unsigned long long bal = __ballot(in);
+        if (in) L.queue[nq + __popcll(bal & below)] = (uint16_t)(p | q << 8);
+        nq += __popcll(bal);
+        p += sp;
+        d += sd;
+        if (p >= cnt) {
+            p -= cnt;
+            ++d;
+        }
+        if (nq >= 64) {
+            nq -= 64;
+            wave_lds_sync();
+            const int pq = L.queue[nq + l];
+            body(pq, true);
+            wave_lds_sync();
         }
     }
-    // angular (atomsymfunction3Andi): pairs p < q of the neighbour list
-    if (i < N && S.f_ok[e]) {
-        // factored form: per triplet NN_FB exponentials and NN_FB powers,
-        // their outer product accumulated per slot
-        const int fcls = S.f_cls[e], nb = S.f_nb[e], nu = S.f_nu[e];
-        float etl[NN_FB], lam[NN_FB];
-        int zp[NN_FB];
+    if (nq > 0) {
+        wave_lds_sync();
+        const int pq = L.queue[l < nq ? l : 0];
+        body(pq, l < nq);
+        wave_lds_sync();
+    }
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+// One halving step of sum_halving: lanes i and i ^ (2 s - 1) each keep the half
+// of the values that their bit s selects.
+template <int s, int n>
+__device__ __forceinline__ void halve(float (&v)[n], int l) {
+    constexpr int ctrl = s == 8 ? 0x140 : s == 4 ? 0x141 : s == 2 ? 0x1B : 0xB1;  // mirrors of 16, 8, 4, 2 lanes
+    const bool up = (l & s) != 0;
+#pragma unroll
+    for (int q = 0; q < s; ++q) {
+        const float give = up ? v[q] : v[q + s];
+        const float keep = up ? v[q + s] : v[q];
+        v[q] = keep + dpp_f<ctrl>(give);
+    }
+    if constexpr (s > 1) halve<s / 2>(v, l);
+}
+
+// Sums of v[0..n-1], n = 8 or 16, over the wavefront: by halving within a row
+// of 16 lanes (n - 1 exchanges on the vector ALU), then over the rows.  Lane
+// l returns the sum of v[l % n].
+template <int n>
+__device__ __forceinline__ float sum_halving(float (&v)[n], int l) {
+    static_assert(n == 8 || n == 16, "a row of 16 lanes");
+    halve<n / 2>(v, l);
+    float r = v[0];
+    if constexpr (n == 8) r += dpp_f<0x128>(r);  // lane i ^ 8
+    r += __shfl_xor(r, 16, 64);
+    r += __shfl_xor(r, 32, 64);
+    return r;
+}
+
+// wavefront-uniform float of lane k
+__device__ __forceinline__ float lane_f(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }
+
+// geometry of one neighbour pair shared by the passes; dfr: dfc/dr / r of the
+// third side, k2 = 2 / rc^2
+struct PairGeo {
+    float ia, ib, cth, Sd, fa, fb, fcc, dfr, cx, cy, cz;
+};
+__device__ __forceinline__ PairGeo pair_geo(const float4 &a, const float4 &a2, const float4 &b, const float4 &b2,
+                                            float k2) {
+    PairGeo g;
+    g.cx = b.x - a.x;
+    g.cy = b.y - a.y;
+    g.cz = b.z - a.z;
+    const float c2 = g.cx * g.cx + g.cy * g.cy + g.cz * g.cz;
+    g.ia = a2.x;
+    g.ib = b2.x;
+    g.fa = a2.z;
+    g.fb = b2.z;
+    g.cth = (a.x * b.x + a.y * b.y + a.z * b.z) * g.ia * g.ib;
+    float d;
+    cut_poly(c2 * k2 - 1.0f, &g.fcc, &d);
+    g.dfr = 2.f * k2 * d;
+    g.Sd = a2.y + b2.y + c2;
+    return g;
+}
+
+// Parameters of NN_RB radial functions k0 .. k0 + NN_RB - 1 of element e in
+// scalar registers, loaded together (a load per function inside a loop would
+// wait for each; entries past the element's last function are not used).
+struct RadBlock {
+    float rs[NN_RB], ce[NN_RB];  // shift, -eta log2(e)
+    int el[NN_RB];
+    __device__ __forceinline__ RadBlock(const NnConst &M, int e, int k0) {
+#pragma unroll
+        for (int k = 0; k < NN_RB; ++k) {
+            rs[k] = M.r_rs[e][k0 + k];
+            ce[k] = M.r_ce[e][k0 + k];
+            el[k] = M.r_el[e][k0 + k];
+        }
+    }
+};
+static_assert(NN_MAXR % NN_RB == 0, "whole blocks");
+
+// the factored angular sums' parameters of element e, in scalar registers
+// over the pair loop (whose fences would have them loaded again)
+struct AngFactors {
+    float etl[NN_FB], eta[NN_FB], lam[NN_FB], zl[NN_FB];
+    int zp[NN_FB];
+    __device__ __forceinline__ AngFactors(const NnConst &M, int e) {
 #pragma unroll
         for (int q = 0; q < NN_FB; ++q) {
-            etl[q] = S.f_etal2[e][q];
-            lam[q] = S.f_lam[e][q];
-            zp[q] = S.f_zp[e][q];
+            etl[q] = M.f_etal2[e][q];
+            eta[q] = M.f_eta[e][q];
+            lam[q] = M.f_lam[e][q];
+            zl[q] = M.f_zl[e][q];
+            zp[q] = M.f_zp[e][q];
         }
+    }
+};
+
+// x^zeta and x^(zeta - 1), zeta = 2^zp with zp wavefront-uniform
+__device__ __forceinline__ void pow_zeta(float x, int zp, float *pw, float *pm) {
+    float p = x, m = 1.f;
+    for (int z = 0; z < zp; ++z) {
+        m *= p;
+        p *= p;
+    }
+    *pw = p;
+    *pm = m;
+}
+
+// Symmetry functions of centre i (element e) into its row Grow; *extrap set
+// when a value leaves [min - 1e-4, max + 1e-4].
+__device__ __forceinline__ void g_centre(const NnConst &M, WaveNbr &L, int cnt, int e, int l, float *Grow, int *extrapp) {
+    const int nr = M.nr[e], na = M.na[e];
+    const float rc2 = M.rc2, k2 = 2.0f / M.rc2;
+    int extrap = 0;
+    // radial (atomsymfunction2: exp(-eta (r - rs)^2) fc(r))
+    for (int k0 = 0; k0 < nr; k0 += NN_RB) {
+        RadBlock R(M, e, k0);
+        float g[NN_RB];
+#pragma unroll
+        for (int k = 0; k < NN_RB; ++k) g[k] = 0.f;
+        for (int n = l; n < cnt; n += 64) {
+            const float4 q = L.q[n];
+            const float r = q.y * q.x, fcv = q.z;
+            const int el = nbr_el(L.p[n]);
+#pragma unroll
+            for (int k = 0; k < NN_RB; ++k) {
+                const float dr = r - R.rs[k];
+                const float t = __builtin_amdgcn_exp2f(R.ce[k] * dr * dr) * fcv;
+                g[k] += el == R.el[k] ? t : 0.f;
+            }
+        }
+        const float v = sum_halving<NN_RB>(g, l);
+        const int k = k0 + l;
+        if (l < NN_RB && k < nr) {
+            Grow[k] = v;
+            if (v < M.glo[e][k] || v > M.ghi[e][k]) extrap = 1;
+        }
+    }
+    // angular (atomsymfunction3Andi): pairs of neighbours
+    if (M.f_ok[e]) {
+        // factored form: per pair NN_FB exponentials and NN_FB powers, their
+        // outer product accumulated per slot
         float acc[NN_FB * NN_FB];
 #pragma unroll
         for (int q = 0; q < NN_FB * NN_FB; ++q) acc[q] = 0.f;
-        for (int p = sub; p < cnt; p += NN_TPA) {
-            const float ax_ = L.dx[base + p], ay_ = L.dy[base + p], az_ = L.dz[base + p];
-            float ra, ia;
-            nbr_rir(L, base + p, &ra, &ia);
-            const float fa = L.fc[base + p];
-            const int ep = L.el[base + p];
-            for (int q = p + 1; q < cnt; ++q) {
-                const float bx = L.dx[base + q], by = L.dy[base + q], bz = L.dz[base + q];
-                const float cx = bx - ax_, cy = by - ay_, cz = bz - az_;
-                const float rc2v = cx * cx + cy * cy + cz * cz;
-                if (rc2v > M.rc2) continue;
-                const int eq = L.el[base + q];
-                const int cls = ep < eq ? ep * NN_MAXE + eq : eq * NN_MAXE + ep;
-                if (cls != fcls) continue;
-                const float rb2 = bx * bx + by * by + bz * bz;
-                const float ib = __builtin_amdgcn_rsqf(rb2), rb = rb2 * ib;
-                const float cth = (ax_ * bx + ay_ * by + az_ * bz) * ia * ib;
-                float fcc, dfcc;
-                cutoff(M.pi_rc, sqrtf(rc2v), &fcc, &dfcc);
-                const float Cf = fa * L.fc[base + q] * fcc;
-                const float Sd = ra * ra + rb * rb + rc2v;
-                float u[NN_FB];
+        const AngFactors F(M, e);
+        for_pairs(L, cnt, M.f_mask[e], rc2, l, [&](int pq, bool on) {
+            const int p = pq & 255, q = pq >> 8;
+            const PairGeo g = pair_geo(L.p[p], L.q[p], L.p[q], L.q[q], k2);
+            const float Cf = on ? g.fa * g.fb * g.fcc : 0.f;
+            float u[NN_FB];
 #pragma unroll
-                for (int m = 0; m < NN_FB; ++m) {
-                    const float x = 1.0f + lam[m] * cth;
-                    float pw = x;
-#pragma unroll
-                    for (int z = 0; z < 4; ++z) pw = z < zp[m] ? pw * pw : pw;  // zeta <= 16
-                    u[m] = (m < nu && x > 0.f) ? pw * Cf : 0.f;
-                }
-#pragma unroll
-                for (int n = 0; n < NN_FB; ++n) {
-                    const float B = n < nb ? __builtin_amdgcn_exp2f(-etl[n] * Sd) : 0.f;
-#pragma unroll
-                    for (int m = 0; m < NN_FB; ++m) acc[n * NN_FB + m] += B * u[m];
-                }
+            for (int m = 0; m < NN_FB; ++m) {
+                float pw, pm;
+                pow_zeta(fmaxf(1.0f + F.lam[m] * g.cth, 0.f), F.zp[m], &pw, &pm);
+                u[m] = pw * Cf;
             }
-        }
-        // slot q's sum to lane q of the group; function k reads its slot's lane
-        float mine = 0.f;
 #pragma unroll
-        for (int q = 0; q < NN_FB * NN_FB; ++q) {
-            const float v = sum_group<NN_TPA>(acc[q]);
-            mine = (sub == q) ? v : mine;
-        }
-#pragma unroll 1
-        for (int k = 0; k < NN_MAXA; ++k) {
-            const float v = __shfl(mine, (lane & ~(NN_TPA - 1)) + S.f_slot[e][k < na ? k : 0], 64);
-            if (k < na && sub == (k & (NN_TPA - 1))) {
-                const float g4 = v * S.a_norm[e][k];
-                Grep[(size_t)i * NN_K1 + nr + k] = g4;
-                if (g4 < Mc.glo[e][nr + k] || g4 > Mc.ghi[e][nr + k]) extrap = 1;
+            for (int n = 0; n < NN_FB; ++n) {
+                const float B = __builtin_amdgcn_exp2f(-F.etl[n] * g.Sd);
+#pragma unroll
+                for (int m = 0; m < NN_FB; ++m) acc[n * NN_FB + m] += B * u[m];
             }
+        });
+        const float v = sum_halving<NN_FB * NN_FB>(acc, l);  // lane l: slot l % 16
+        const float g4 = __shfl(v, l < na ? M.f_slot[e][l & 31] : 0, 64) * M.a_norm[e][l & 31];
+        if (l < na) {
+            Grow[nr + l] = g4;
+            if (g4 < M.glo[e][nr + l] || g4 > M.ghi[e][nr + l]) extrap = 1;
         }
     } else {
-        // generic form: every function per triplet (no pair loop for an
-        // element without angular functions)
+        // generic form: NN_KB functions at a time, each evaluated per pair
+        for (int k0 = 0; k0 < na; k0 += NN_KB) {
+            float g[NN_KB];
 #pragma unroll
-    for (int k = 0; k < NN_MAXA; ++k) g[k] = 0.f;
-    for (int p = sub; p < (na > 0 ? cnt : 0); p += NN_TPA) {
-        const float ax_ = L.dx[base + p], ay_ = L.dy[base + p], az_ = L.dz[base + p];
-        float ra, ia;
-        nbr_rir(L, base + p, &ra, &ia);
-        const float fa = L.fc[base + p];
-        const int ep = L.el[base + p];
-        for (int q = p + 1; q < cnt; ++q) {
-            const float bx = L.dx[base + q], by = L.dy[base + q], bz = L.dz[base + q];
-            const float cx = bx - ax_, cy = by - ay_, cz = bz - az_;
-            const float rc2v = cx * cx + cy * cy + cz * cz;
-            if (rc2v > M.rc2) continue;
-            const float rb2 = bx * bx + by * by + bz * bz;
-            const float ib = __builtin_amdgcn_rsqf(rb2), rb = rb2 * ib;
-            const int eq = L.el[base + q];
-            const int cls = ep < eq ? ep * NN_MAXE + eq : eq * NN_MAXE + ep;
-            const float cth = (ax_ * bx + ay_ * by + az_ * bz) * ia * ib;
-            float fcc, dfcc;
-            cutoff(M.pi_rc, sqrtf(rc2v), &fcc, &dfcc);
-            const float Cf = fa * L.fc[base + q] * fcc;
-            const float Sd = ra * ra + rb * rb + rc2v;
-            float B = 0.f, etaprev = -1.f;
+            for (int k = 0; k < NN_KB; ++k) g[k] = 0.f;
+            for_pairs(L, cnt, 0, rc2, l, [&](int pq, bool on) {
+                const int p = pq & 255, q = pq >> 8;
+                const float4 a = L.p[p], b = L.p[q];
+                const PairGeo pg = pair_geo(a, L.q[p], b, L.q[q], k2);
+                const float Cf = on ? pg.fa * pg.fb * pg.fcc : 0.f;
+                const int ea = nbr_el(a), eb = nbr_el(b);
+                const int lo = min(ea, eb), hi = max(ea, eb);
 #pragma unroll
-            for (int k = 0; k < NN_MAXA; ++k)
-                if (k < na && cls == S.a_cls[e][k]) {
-                    const float x = 1.0f + S.a_lam[e][k] * cth;
-                    if (x > 0.f) {
-                        float pw = x;
-                        for (int z = 0; z < S.a_zp[e][k]; ++z) pw *= pw;
-                        if (S.a_etal2[e][k] != etaprev) {
-                            etaprev = S.a_etal2[e][k];
-                            B = __builtin_amdgcn_exp2f(-etaprev * Sd);
-                        }
-                        g[k] += S.a_norm[e][k] * pw * B * Cf;
+                for (int k = 0; k < NN_KB; ++k)
+                    if (k0 + k < na) {  // wavefront-uniform
+                        const int kk = k0 + k;
+                        const bool mine = lo == M.a_e1[e][kk] && hi == M.a_e2[e][kk];
+                        float pw, pm;
+                        pow_zeta(fmaxf(1.0f + M.a_lam[e][kk] * pg.cth, 0.f), M.a_zp[e][kk], &pw, &pm);
+                        const float t = M.a_norm[e][kk] * pw * __builtin_amdgcn_exp2f(-M.a_etal2[e][kk] * pg.Sd) * Cf;
+                        g[k] += mine ? t : 0.f;
                     }
-                }
+            });
+            const float v = sum_halving<NN_KB>(g, l);
+            const int k = k0 + l;
+            if (l < NN_KB && k < na) {
+                Grow[nr + k] = v;
+                if (v < M.glo[e][nr + k] || v > M.ghi[e][nr + k]) extrap = 1;
+            }
         }
-    }
-#pragma unroll
-    for (int k = 0; k < NN_MAXA; ++k) {
-        const float v = sum_group<NN_TPA>(g[k]);
-        if (i < N && k < na && sub == (k & (NN_TPA - 1))) {
-            Grep[(size_t)i * NN_K1 + nr + k] = v;
-            if (v < Mc.glo[e][nr + k] || v > Mc.ghi[e][nr + k]) extrap = 1;
-        }
-    }
     }
     if (extrap) *extrapp = 1;
 }
 
-// dE/dr of the chunk's centre atoms' symmetry functions with coefficients
-// cb = dE/dG (VJP): centre force in registers, neighbours' shares into the
-// fixed-point accumulators ax, ay, az (Hartree/Bohr).
-__device__ void force_chunk(const NnSfTab &S, const ChunkNbr &L, const float (*cb)[NN_K1], float (*Wsh)[NN_FB * NN_FB],
-                            const uint8_t *elem, int N, int k0, int lane, float rc2, float pi_rc,
-                            unsigned long long *ax, unsigned long long *ay, unsigned long long *az, int *badp) {
-    const int c = lane / NN_TPA, sub = lane % NN_TPA;
+// dE/dr of the centre's symmetry functions with coefficients dE/dG (row
+// Crow).  The partial derivatives of a pair's term by its three distances
+// and the angle give, on neighbour p (vector a) and q (vector b),
+//   F_p = -(A b + B_p a),  F_q = -(A a + B_q b),
+//   A   = tc / (ra rb) - (ts + uc),
+//   B_p = -tc cos / ra^2 + ts + u_a + (ts + uc)   (B_q alike),
+// added to the neighbours' words in 2^32 fixed point (wavefront-private LDS;
+// integers, so the order does not matter).  The centre takes minus the sum
+// of its neighbours' forces, exactly.  ax, ay, az: the atoms' accumulators.
+__device__ __forceinline__ void force_centre(const NnConst &M, WaveNbrF &L, int cnt, int i, int e, int l, const float *Crow,
+                             unsigned long long *ax, unsigned long long *ay, unsigned long long *az, int *badp) {
+    const int nr = M.nr[e], na = M.na[e];
+    const float rc2 = M.rc2, k2 = 2.0f / M.rc2;
     int bad = 0;
-    struct {
-        float rc2, pi_rc;
-    } M{rc2, pi_rc};
-    const int i = k0 + c;
-    const int cnt = L.cnt[c];
-    const int e = (i < N) ? elem[i] : 0;
-    const int nr = (i < N) ? S.nr[e] : 0, na = (i < N) ? S.na[e] : 0;
-    const int base = c * NN_CAP;
-    float Fi0 = 0.f, Fi1 = 0.f, Fi2 = 0.f;  // force on the centre (Hartree/Bohr)
-    // radial: dG/dr = (-2 eta (r - rs) fc + dfc) exp(-eta (r - rs)^2)
-    for (int p = sub; p < cnt; p += NN_TPA) {
-        float r, ir;
-        nbr_rir(L, base + p, &r, &ir);
-        const float fcv = L.fc[base + p], dfcv = L.dfc[base + p];
-        const int ep = L.el[base + p];
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < NN_MAXR; ++k)
-            if (k < nr && ep == S.r_el[e][k]) {
-                const float dr = r - S.r_rs[e][k];
-                const float ex = __builtin_amdgcn_exp2f(-S.r_eta[e][k] * NN_L2E * dr * dr);
-                s += cb[c][k] * ex * (dfcv - 2.f * S.r_eta[e][k] * dr * fcv);
+    const float ck = l < nr + na ? Crow[l] : 0.f;  // lane k: dE/dG_k
+    const float ckr = l < nr ? ck : 0.f;
+    for (int n = l; n < cnt; n += 64) L.acc[0][n] = L.acc[1][n] = L.acc[2][n] = 0ull;
+    auto add = [&](int pq, bool on, const float4 &a, const float4 &b, const PairGeo &g, float Sg, float Sc, float Ss) {
+        const int p = pq & 255, q = pq >> 8;
+        const float Cf = g.fa * g.fb * g.fcc;
+        const float tc = Cf * Sc, ts = -2.f * Cf * Ss;
+        const float tsuc = ts + Sg * g.fa * g.fb * g.dfr;
+        const float A = tc * g.ia * g.ib - tsuc;
+        const float tcc = tc * g.cth;
+        const float Bp = ts + tsuc + Sg * L.q[p].w * g.fb * g.fcc - tcc * g.ia * g.ia;
+        const float Bq = ts + tsuc + Sg * L.q[q].w * g.fa * g.fcc - tcc * g.ib * g.ib;
+        const float fp0 = -(A * b.x + Bp * a.x), fp1 = -(A * b.y + Bp * a.y), fp2 = -(A * b.z + Bp * a.z);
+        const float fq0 = -(A * a.x + Bq * b.x), fq1 = -(A * a.y + Bq * b.y), fq2 = -(A * a.z + Bq * b.z);
+        const float big = fabsf(fp0) + fabsf(fp1) + fabsf(fp2) + fabsf(fq0) + fabsf(fq1) + fabsf(fq2);
+        if (__all(big < NN_FIX32_MAX)) {  // NaN takes the other way, to the overflow flag
+            if (on) {
+                atomicAdd(&L.acc[0][p], fix32(fp0));
+                atomicAdd(&L.acc[1][p], fix32(fp1));
+                atomicAdd(&L.acc[2][p], fix32(fp2));
+                atomicAdd(&L.acc[0][q], fix32(fq0));
+                atomicAdd(&L.acc[1][q], fix32(fq1));
+                atomicAdd(&L.acc[2][q], fix32(fq2));
             }
-        const float v0 = s * L.dx[base + p] * ir, v1 = s * L.dy[base + p] * ir, v2 = s * L.dz[base + p] * ir;
-        Fi0 += v0;
-        Fi1 += v1;
-        Fi2 += v2;
-        const int j = L.j[base + p];
-        fxadd(&ax[j], -(double)v0, &bad);
-        fxadd(&ay[j], -(double)v1, &bad);
-        fxadd(&az[j], -(double)v2, &bad);
-    }
-    // angular
-    const bool fast = i < N && S.f_ok[e];
-    float W[NN_FB * NN_FB], etl[NN_FB], eta[NN_FB], lam[NN_FB];
-    int zp[NN_FB];
-    int fcls = -1, nb = 0, nu = 0;
-    {
-        // W(n, m) = sum over the functions on slot (n, m) of dE/dG_k norm_k,
-        // lane `sub` of each centre's group computing slot sub (every lane
-        // of the block passes the barrier)
-        float wq = 0.f;
-        if (fast)
-            for (int k = 0; k < na; ++k)
-                if (S.f_slot[e][k] == sub) wq += cb[c][nr + k] * S.a_norm[e][k];
-        Wsh[c][sub] = wq;
-        __syncthreads();
-    }
-    if (fast) {
-        fcls = S.f_cls[e];
-        nb = S.f_nb[e];
-        nu = S.f_nu[e];
-#pragma unroll
-        for (int q = 0; q < NN_FB; ++q) {
-            etl[q] = S.f_etal2[e][q];
-            eta[q] = S.f_eta[e][q];
-            lam[q] = S.f_lam[e][q];
-            zp[q] = S.f_zp[e][q];
+        } else if (on) {
+            fxadd(&L.acc[0][p], (double)fp0, &bad);
+            fxadd(&L.acc[1][p], (double)fp1, &bad);
+            fxadd(&L.acc[2][p], (double)fp2, &bad);
+            fxadd(&L.acc[0][q], (double)fq0, &bad);
+            fxadd(&L.acc[1][q], (double)fq1, &bad);
+            fxadd(&L.acc[2][q], (double)fq2, &bad);
         }
+    };
+    if (M.f_ok[e]) {
+        // W(n, m) = sum over the functions on slot (n, m) of dE/dG_k norm_k
+        float wl = 0.f, W[NN_FB * NN_FB];
+        for (int k = 0; k < na; ++k) wl += M.f_slot[e][k] == l ? lane_f(ck, nr + k) * M.a_norm[e][k] : 0.f;
 #pragma unroll
-        for (int q = 0; q < NN_FB * NN_FB; ++q) W[q] = Wsh[c][q];
-    }
-    for (int p = sub; p < (na > 0 ? cnt : 0); p += NN_TPA) {
-        const float ax_ = L.dx[base + p], ay_ = L.dy[base + p], az_ = L.dz[base + p];
-        float ra, ia;
-        nbr_rir(L, base + p, &ra, &ia);
-        const float fa = L.fc[base + p], dfa = L.dfc[base + p];
-        const int ep = L.el[base + p];
-        float Fj0 = 0.f, Fj1 = 0.f, Fj2 = 0.f;
-        for (int q = p + 1; q < cnt; ++q) {
-            const float bx = L.dx[base + q], by = L.dy[base + q], bz = L.dz[base + q];
-            const float cx = bx - ax_, cy = by - ay_, cz = bz - az_;
-            const float rc2v = cx * cx + cy * cy + cz * cz;
-            if (rc2v > M.rc2) continue;
-            const int eq = L.el[base + q];
-            const int cls = ep < eq ? ep * NN_MAXE + eq : eq * NN_MAXE + ep;
-            if (fast && cls != fcls) continue;
-            const float rb2 = bx * bx + by * by + bz * bz;
-            const float ib = __builtin_amdgcn_rsqf(rb2), rb = rb2 * ib;
-            const float fb = L.fc[base + q], dfb = L.dfc[base + q];
-            const float cth = (ax_ * bx + ay_ * by + az_ * bz) * ia * ib;
-            const float ircc = __builtin_amdgcn_rsqf(rc2v), rcc = rc2v * ircc;
-            float fcc, dfcc;
-            cutoff(M.pi_rc, rcc, &fcc, &dfcc);
-            const float Cf = fa * fb * fcc;
-            const float Sd = ra * ra + rb * rb + rc2v;
+        for (int q = 0; q < NN_FB * NN_FB; ++q) W[q] = lane_f(wl, q);
+        wave_lds_sync();
+        const AngFactors F(M, e);
+        for_pairs(L, cnt, M.f_mask[e], rc2, l, [&](int pq, bool on) {
+            const float4 a = L.p[pq & 255], b = L.p[pq >> 8];
+            const PairGeo g = pair_geo(a, L.q[pq & 255], b, L.q[pq >> 8], k2);
+            // Sg = sum B_n W(n,m) u_m, Sc = sum B_n W(n,m) du_m/dcos, Ss = sum eta_n B_n W(n,m) u_m
+            float u[NN_FB], du[NN_FB];
+#pragma unroll
+            for (int m = 0; m < NN_FB; ++m) {
+                const float x = 1.0f + F.lam[m] * g.cth;
+                float pw, pm;
+                pow_zeta(x, F.zp[m], &pw, &pm);
+                u[m] = x > 0.f ? pw : 0.f;
+                du[m] = x > 0.f ? F.zl[m] * pm : 0.f;
+            }
             float Sg = 0.f, Sc = 0.f, Ss = 0.f;
-            if (fast) {
-                // Sg = sum B_n W(n,m) u_m, Sc = sum B_n W(n,m) du_m/dcos,
-                // Ss = sum eta_n B_n W(n,m) u_m
-                float u[NN_FB], du[NN_FB];
+#pragma unroll
+            for (int n = 0; n < NN_FB; ++n) {
+                const float B = __builtin_amdgcn_exp2f(-F.etl[n] * g.Sd);
+                float t = 0.f, td = 0.f;
 #pragma unroll
                 for (int m = 0; m < NN_FB; ++m) {
-                    const float x = 1.0f + lam[m] * cth;
-                    float pw = x, pm = 1.f;  // x^zeta, x^(zeta-1); zeta <= 16
-#pragma unroll
-                    for (int z = 0; z < 4; ++z) {
-                        const bool go = z < zp[m];
-                        pm = go ? pm * pw : pm;
-                        pw = go ? pw * pw : pw;
-                    }
-                    const bool on = m < nu && x > 0.f;
-                    u[m] = on ? pw : 0.f;
-                    du[m] = on ? (float)(1 << zp[m]) * lam[m] * pm : 0.f;
+                    t += W[n * NN_FB + m] * u[m];
+                    td += W[n * NN_FB + m] * du[m];
                 }
-#pragma unroll
-                for (int n = 0; n < NN_FB; ++n) {
-                    const float B = n < nb ? __builtin_amdgcn_exp2f(-etl[n] * Sd) : 0.f;
-                    float t = 0.f, td = 0.f;
-#pragma unroll
-                    for (int m = 0; m < NN_FB; ++m) {
-                        t += W[n * NN_FB + m] * u[m];
-                        td += W[n * NN_FB + m] * du[m];
-                    }
-                    Sg += B * t;
-                    Sc += B * td;
-                    Ss += eta[n] * B * t;
-                }
-            } else {
-                float B = 0.f, etaprev = -1.f;
-#pragma unroll
-                for (int k = 0; k < NN_MAXA; ++k)
-                    if (k < na && cls == S.a_cls[e][k]) {
-                        const float lamk = S.a_lam[e][k];
-                        const float x = 1.0f + lamk * cth;
-                        if (x > 0.f) {
-                            float pw = x, pm = 1.f;  // x^zeta, x^(zeta-1)
-                            for (int z = 0; z < S.a_zp[e][k]; ++z) {
-                                pm *= pw;
-                                pw *= pw;
-                            }
-                            if (S.a_etal2[e][k] != etaprev) {
-                                etaprev = S.a_etal2[e][k];
-                                B = __builtin_amdgcn_exp2f(-etaprev * Sd);
-                            }
-                            const float ck = cb[c][nr + k] * S.a_norm[e][k] * B;
-                            const float zeta = (float)(1 << S.a_zp[e][k]);
-                            Sg += ck * pw;
-                            Sc += ck * zeta * lamk * pm;
-                            Ss += ck * S.a_eta[e][k] * pw;
-                        }
-                    }
+                Sg += B * t;
+                Sc += B * td;
+                Ss += F.eta[n] * (B * t);
             }
-            if (Sg == 0.f && Sc == 0.f) continue;
-            const float iab = ia * ib;
-            const float tc = Cf * Sc, ts = -2.f * Cf * Ss;
-            const float ua = Sg * dfa * fb * fcc * ia, ub = Sg * fa * dfb * fcc * ib;
-            const float uc = Sg * fa * fb * dfcc * ircc;
-            const float ga0 = tc * (bx * iab - cth * ax_ * ia * ia) + ts * ax_ + ua * ax_;
-            const float ga1 = tc * (by * iab - cth * ay_ * ia * ia) + ts * ay_ + ua * ay_;
-            const float ga2 = tc * (bz * iab - cth * az_ * ia * ia) + ts * az_ + ua * az_;
-            const float gb0 = tc * (ax_ * iab - cth * bx * ib * ib) + ts * bx + ub * bx;
-            const float gb1 = tc * (ay_ * iab - cth * by * ib * ib) + ts * by + ub * by;
-            const float gb2 = tc * (az_ * iab - cth * bz * ib * ib) + ts * bz + ub * bz;
-            const float gc0 = (ts + uc) * cx, gc1 = (ts + uc) * cy, gc2 = (ts + uc) * cz;
-            Fi0 += ga0 + gb0;
-            Fi1 += ga1 + gb1;
-            Fi2 += ga2 + gb2;
-            Fj0 -= ga0 - gc0;
-            Fj1 -= ga1 - gc1;
-            Fj2 -= ga2 - gc2;
-            const int kq = L.j[base + q];
-            fxadd(&ax[kq], -(double)(gb0 + gc0), &bad);
-            fxadd(&ay[kq], -(double)(gb1 + gc1), &bad);
-            fxadd(&az[kq], -(double)(gb2 + gc2), &bad);
-        }
-        const int j = L.j[base + p];
-        fxadd(&ax[j], (double)Fj0, &bad);
-        fxadd(&ay[j], (double)Fj1, &bad);
-        fxadd(&az[j], (double)Fj2, &bad);
+            add(pq, on, a, b, g, Sg, Sc, Ss);
+        });
+    } else if (na > 0) {
+        wave_lds_sync();
+        for_pairs(L, cnt, 0, rc2, l, [&](int pq, bool on) {
+            const float4 a = L.p[pq & 255], b = L.p[pq >> 8];
+            const PairGeo g = pair_geo(a, L.q[pq & 255], b, L.q[pq >> 8], k2);
+            const int ea = nbr_el(a), eb = nbr_el(b);
+            const int lo = min(ea, eb), hi = max(ea, eb);
+            float Sg = 0.f, Sc = 0.f, Ss = 0.f;
+            for (int k = 0; k < na; ++k) {
+                const float x = 1.0f + M.a_lam[e][k] * g.cth;
+                const bool mine = x > 0.f && lo == M.a_e1[e][k] && hi == M.a_e2[e][k];
+                float pw, pm;
+                pow_zeta(x, M.a_zp[e][k], &pw, &pm);
+                const float c = mine ? lane_f(ck, nr + k) * M.a_norm[e][k] *
+                                           __builtin_amdgcn_exp2f(-M.a_etal2[e][k] * g.Sd)
+                                     : 0.f;
+                Sg += c * pw;
+                Sc += c * (float)(1 << M.a_zp[e][k]) * M.a_lam[e][k] * pm;
+                Ss += c * (M.a_etal2[e][k] * (1.0f / NN_L2E)) * pw;
+            }
+            if (__all(Sg == 0.f && Sc == 0.f)) return;
+            add(pq, on, a, b, g, Sg, Sc, Ss);
+        });
     }
-    const float S0 = sum_group<NN_TPA>(Fi0), S1 = sum_group<NN_TPA>(Fi1), S2 = sum_group<NN_TPA>(Fi2);
-    if (i < N && sub == 0) {
-        fxadd(&ax[i], (double)S0, &bad);
-        fxadd(&ay[i], (double)S1, &bad);
-        fxadd(&az[i], (double)S2, &bad);
+    wave_lds_sync();
+    // radial: dG/dr = (-2 eta (r - rs) fc + dfc) exp(-eta (r - rs)^2); then the
+    // neighbours' sums to their atoms and minus their total to the centre
+    long long t0 = 0, t1 = 0, t2 = 0;
+    for (int n0 = 0; n0 < cnt; n0 += 64) {
+        const int n = n0 + l < cnt ? n0 + l : 0;
+        const bool on = n0 + l < cnt;
+        const float4 p = L.p[n], q = L.q[n];
+        const float r = q.y * q.x, fcv = q.z, dfcv = q.w * r;
+        const int el = nbr_el(p);
+        float s = 0.f;
+        for (int k0 = 0; k0 < nr; k0 += NN_RB) {
+            RadBlock R(M, e, k0);
+#pragma unroll
+            for (int k = 0; k < NN_RB; ++k) {
+                const float dr = r - R.rs[k];
+                const float ex = __builtin_amdgcn_exp2f(R.ce[k] * dr * dr);
+                // d/dr exp(ce dr^2 ln 2) = 2 ln 2 ce dr exp
+                const float t = lane_f(ckr, k0 + k) * ex * (dfcv + (2.f / NN_L2E) * R.ce[k] * dr * fcv);
+                s += el == R.el[k] ? t : 0.f;
+            }
+        }
+        s *= -q.x;  // on the neighbour: -dE/dr along the unit vector
+        const float v0 = s * p.x, v1 = s * p.y, v2 = s * p.z;
+        const bool ok = fabsf(v0) + fabsf(v1) + fabsf(v2) < NN_FIX32_MAX;
+        unsigned long long f0 = L.acc[0][n], f1 = L.acc[1][n], f2 = L.acc[2][n];
+        if (ok) {
+            f0 += fix32(v0);
+            f1 += fix32(v1);
+            f2 += fix32(v2);
+        } else if (on) {
+            fxput(&f0, (double)v0, &bad);
+            fxput(&f1, (double)v1, &bad);
+            fxput(&f2, (double)v2, &bad);
+        }
+        if (on) {
+            const int j = nbr_j(p);
+            atomicAdd(&ax[j], f0);
+            atomicAdd(&ay[j], f1);
+            atomicAdd(&az[j], f2);
+            t0 -= (long long)f0;
+            t1 -= (long long)f1;
+            t2 -= (long long)f2;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        t0 += __shfl_xor(t0, o, 64);
+        t1 += __shfl_xor(t1, o, 64);
+        t2 += __shfl_xor(t2, o, 64);
+    }
+    if (l == 0) {
+        atomicAdd(&ax[i], (unsigned long long)t0);
+        atomicAdd(&ay[i], (unsigned long long)t1);
+        atomicAdd(&az[i], (unsigned long long)t2);
     }
     if (bad) *badp |= bad;
 }
 
-// u_ik = sum_a dG_ik/dr_a . g_a for the chunk's centre atoms i (the
-// Jacobian-vector product of the training gradient; g per atom in LDS).
-// Per neighbour pair: g_j - g_i projected on the pair direction; per
-// neighbour triple: the three difference vectors dotted with the angular
-// function's partial vectors, shared over all functions of the triple.
-// Result scaled by -dfac (u = dLoss/d(dE/dx)) into Urep rows.
-__device__ void jvp_chunk(const NnSfTab &S, const ChunkNbr &L, const uint8_t *elem, int N, int k0, int lane,
-                          float rc2, float pi_rc, const float *gx, const float *gy, const float *gz,
-                          const float (*dfac)[NN_K1], float *Urep) {
-    const int c = lane / NN_TPA, sub = lane % NN_TPA;
-    const int i = k0 + c;
-    const int cnt = L.cnt[c];
-    const int e = (i < N) ? elem[i] : 0;
-    const int nr = (i < N) ? S.nr[e] : 0, na = (i < N) ? S.na[e] : 0;
-    const int base = c * NN_CAP;
-    const float gix = (i < N) ? gx[i] : 0.f, giy = (i < N) ? gy[i] : 0.f, giz = (i < N) ? gz[i] : 0.f;
-    float P[NN_MAXR > NN_MAXA ? NN_MAXR : NN_MAXA];
+// u_k = sum_a dG_k/dr_a . g_a of centre i (the Jacobian-vector product of the
+// training gradient; g per atom in LDS), scaled by -dfac (u = dLoss/d(dE/dx))
+// into its row Urow.  Per neighbour pair the three difference vectors dotted
+// with the angular functions' partial vectors, shared by all functions.
+__device__ __forceinline__ void jvp_centre(const NnConst &M, WaveNbrF &L, int cnt, int i, int e, int l, const float *gx,
+                           const float *gy, const float *gz, float *Urow) {
+    const int nr = M.nr[e], na = M.na[e];
+    const float rc2 = M.rc2, k2 = 2.0f / M.rc2;
+    float4 *gd = (float4 *)&L.acc[0][0];  // g_j - g_i per entry
+    const float gix = gx[i], giy = gy[i], giz = gz[i];
+    for (int n = l; n < cnt; n += 64) {
+        const int j = nbr_j(L.p[n]);
+        gd[n] = make_float4(gx[j] - gix, gy[j] - giy, gz[j] - giz, 0.f);
+    }
+    wave_lds_sync();
+    for (int k0 = 0; k0 < nr; k0 += NN_RB) {
+        RadBlock R(M, e, k0);
+        float P[NN_RB];
 #pragma unroll
-    for (int k = 0; k < NN_MAXR; ++k) P[k] = 0.f;
-    for (int p = sub; p < cnt; p += NN_TPA) {
-        float r, ir;
-        nbr_rir(L, base + p, &r, &ir);
-        const float fcv = L.fc[base + p], dfcv = L.dfc[base + p];
-        const int j = L.j[base + p];
-        const float proj = (L.dx[base + p] * (gx[j] - gix) + L.dy[base + p] * (gy[j] - giy) +
-                            L.dz[base + p] * (gz[j] - giz)) * ir;
-        const int ep = L.el[base + p];
+        for (int k = 0; k < NN_RB; ++k) P[k] = 0.f;
+        for (int n = l; n < cnt; n += 64) {
+            const float4 p = L.p[n], q = L.q[n], d = gd[n];
+            const int el = nbr_el(p);
+            const float r = q.y * q.x, fcv = q.z, dfcv = q.w * r;
+            const float proj = (p.x * d.x + p.y * d.y + p.z * d.z) * q.x;
 #pragma unroll
-        for (int k = 0; k < NN_MAXR; ++k)
-            if (k < nr && ep == S.r_el[e][k]) {
-                const float dr = r - S.r_rs[e][k];
-                const float ex = __builtin_amdgcn_exp2f(-S.r_eta[e][k] * NN_L2E * dr * dr);
-                P[k] += ex * (dfcv - 2.f * S.r_eta[e][k] * dr * fcv) * proj;
+            for (int k = 0; k < NN_RB; ++k) {
+                const float dr = r - R.rs[k];
+                const float ex = __builtin_amdgcn_exp2f(R.ce[k] * dr * dr);
+                const float t = ex * (dfcv + (2.f / NN_L2E) * R.ce[k] * dr * fcv) * proj;
+                P[k] += el == R.el[k] ? t : 0.f;
             }
+        }
+        const float v = sum_halving<NN_RB>(P, l);
+        const int k = k0 + l;
+        if (l < NN_RB && k < nr) Urow[k] = -M.dfac[e][k] * v;
     }
+    // cos, S = ra^2 + rb^2 + rc^2 and the cut-off product along g
+    auto along = [&](int pq, const float4 &a, const float4 &b, const PairGeo &g, float *dcosD, float *SD, float *FD) {
+        const int p = pq & 255, q = pq >> 8;
+        const float4 Da = gd[p], Db = gd[q];
+        const float aD = a.x * Da.x + a.y * Da.y + a.z * Da.z;   // a . (g_p - g_i)
+        const float bD = b.x * Db.x + b.y * Db.y + b.z * Db.z;   // b . (g_q - g_i)
+        const float cD = g.cx * (Db.x - Da.x) + g.cy * (Db.y - Da.y) + g.cz * (Db.z - Da.z);
+        const float bDa = b.x * Da.x + b.y * Da.y + b.z * Da.z;
+        const float aDb = a.x * Db.x + a.y * Db.y + a.z * Db.z;
+        *dcosD = (bDa + aDb) * g.ia * g.ib - g.cth * (aD * g.ia * g.ia + bD * g.ib * g.ib);
+        *SD = aD + bD + cD;
+        *FD = L.q[p].w * g.fb * g.fcc * aD + g.fa * L.q[q].w * g.fcc * bD + g.fa * g.fb * g.dfr * cD;
+    };
+    if (M.f_ok[e]) {
+        float acc[NN_FB * NN_FB];
 #pragma unroll
-    for (int k = 0; k < NN_MAXR; ++k) {
-        const float v = sum_group<NN_TPA>(P[k]);
-        if (i < N && k < nr && sub == (k & (NN_TPA - 1))) Urep[(size_t)i * NN_K1 + k] = -dfac[e][k] * v;
-    }
+        for (int q = 0; q < NN_FB * NN_FB; ++q) acc[q] = 0.f;
+        const AngFactors F(M, e);
+        for_pairs(L, cnt, M.f_mask[e], rc2, l, [&](int pq, bool on) {
+            const float4 a = L.p[pq & 255], b = L.p[pq >> 8];
+            const PairGeo g = pair_geo(a, L.q[pq & 255], b, L.q[pq >> 8], k2);
+            float dcosD, SD, FD;
+            along(pq, a, b, g, &dcosD, &SD, &FD);
+            const float Cf = g.fa * g.fb * g.fcc;
+            const float CdcosD = on ? Cf * dcosD : 0.f, CSD = on ? -2.f * Cf * SD : 0.f, FDon = on ? FD : 0.f;
+            float u[NN_FB], du[NN_FB];
 #pragma unroll
-    for (int k = 0; k < NN_MAXA; ++k) P[k] = 0.f;
-    for (int p = sub; p < (na > 0 ? cnt : 0); p += NN_TPA) {
-        const float ax_ = L.dx[base + p], ay_ = L.dy[base + p], az_ = L.dz[base + p];
-        float ra, ia;
-        nbr_rir(L, base + p, &ra, &ia);
-        const float fa = L.fc[base + p], dfa = L.dfc[base + p];
-        const int ep = L.el[base + p];
-        const int jp = L.j[base + p];
-        const float Dja0 = gx[jp] - gix, Dja1 = gy[jp] - giy, Dja2 = gz[jp] - giz;
-        for (int q = p + 1; q < cnt; ++q) {
-            const float bx = L.dx[base + q], by = L.dy[base + q], bz = L.dz[base + q];
-            const float cx = bx - ax_, cy = by - ay_, cz = bz - az_;
-            const float rc2v = cx * cx + cy * cy + cz * cz;
-            if (rc2v > rc2) continue;
-            const float rb2 = bx * bx + by * by + bz * bz;
-            const float ib = __builtin_amdgcn_rsqf(rb2), rb = rb2 * ib;
-            const float fb = L.fc[base + q], dfb = L.dfc[base + q];
-            const int eq = L.el[base + q];
-            const int cls = ep < eq ? ep * NN_MAXE + eq : eq * NN_MAXE + ep;
-            const int kq = L.j[base + q];
-            const float Dka0 = gx[kq] - gix, Dka1 = gy[kq] - giy, Dka2 = gz[kq] - giz;
-            const float Dkj0 = Dka0 - Dja0, Dkj1 = Dka1 - Dja1, Dkj2 = Dka2 - Dja2;
-            const float cth = (ax_ * bx + ay_ * by + az_ * bz) * ia * ib;
-            const float ircc = __builtin_amdgcn_rsqf(rc2v), rcc = rc2v * ircc;
-            float fcc, dfcc;
-            cutoff(pi_rc, rcc, &fcc, &dfcc);
-            const float Cf = fa * fb * fcc;
-            const float Sd = ra * ra + rb * rb + rc2v;
-            const float iab = ia * ib;
-            const float aD = ax_ * Dja0 + ay_ * Dja1 + az_ * Dja2;   // a . Dja
-            const float bD = bx * Dka0 + by * Dka1 + bz * Dka2;      // b . Dka
-            const float cD = cx * Dkj0 + cy * Dkj1 + cz * Dkj2;      // c . Dkj
-            const float bDa = bx * Dja0 + by * Dja1 + bz * Dja2;     // b . Dja
-            const float aDb = ax_ * Dka0 + ay_ * Dka1 + az_ * Dka2;  // a . Dka
-            const float dcosD = (bDa * iab - cth * aD * ia * ia) + (aDb * iab - cth * bD * ib * ib);
-            const float SD = aD + bD + cD;
-            const float FD = dfa * fb * fcc * aD * ia + fa * dfb * fcc * bD * ib + fa * fb * dfcc * cD * ircc;
-            float B = 0.f, etaprev = -1.f;
+            for (int m = 0; m < NN_FB; ++m) {
+                const float x = 1.0f + F.lam[m] * g.cth;
+                float pw, pm;
+                pow_zeta(x, F.zp[m], &pw, &pm);
+                u[m] = x > 0.f ? pw : 0.f;
+                du[m] = x > 0.f ? F.zl[m] * pm * CdcosD : 0.f;
+            }
 #pragma unroll
-            for (int k = 0; k < NN_MAXA; ++k)
-                if (k < na && cls == S.a_cls[e][k]) {
-                    const float lam = S.a_lam[e][k];
-                    const float x = 1.0f + lam * cth;
-                    if (x > 0.f) {
-                        float pw = x, pm = 1.f;
-                        for (int z = 0; z < S.a_zp[e][k]; ++z) {
-                            pm *= pw;
-                            pw *= pw;
-                        }
-                        if (S.a_etal2[e][k] != etaprev) {
-                            etaprev = S.a_etal2[e][k];
-                            B = __builtin_amdgcn_exp2f(-etaprev * Sd);
-                        }
-                        const float zeta = (float)(1 << S.a_zp[e][k]);
-                        P[k] += S.a_norm[e][k] * B *
-                                (zeta * lam * pm * Cf * dcosD - 2.f * S.a_eta[e][k] * pw * Cf * SD + pw * FD);
+            for (int n = 0; n < NN_FB; ++n) {
+                const float B = __builtin_amdgcn_exp2f(-F.etl[n] * g.Sd);
+                const float B2 = B * (FDon + F.eta[n] * CSD);
+#pragma unroll
+                for (int m = 0; m < NN_FB; ++m) acc[n * NN_FB + m] += B * du[m] + B2 * u[m];
+            }
+        });
+        const float v = sum_halving<NN_FB * NN_FB>(acc, l);  // lane l: slot l % 16
+        const float pk = __shfl(v, l < na ? M.f_slot[e][l & 31] : 0, 64) * M.a_norm[e][l & 31];
+        if (l < na) Urow[nr + l] = -M.dfac[e][nr + l] * pk;
+    } else {
+        for (int k0 = 0; k0 < na; k0 += NN_KB) {
+            float P[NN_KB];
+#pragma unroll
+            for (int k = 0; k < NN_KB; ++k) P[k] = 0.f;
+            for_pairs(L, cnt, 0, rc2, l, [&](int pq, bool on) {
+                const float4 a = L.p[pq & 255], b = L.p[pq >> 8];
+                const PairGeo g = pair_geo(a, L.q[pq & 255], b, L.q[pq >> 8], k2);
+                float dcosD, SD, FD;
+                along(pq, a, b, g, &dcosD, &SD, &FD);
+                const float Cf = g.fa * g.fb * g.fcc;
+                const int ea = nbr_el(a), eb = nbr_el(b);
+                const int lo = min(ea, eb), hi = max(ea, eb);
+#pragma unroll
+                for (int k = 0; k < NN_KB; ++k)
+                    if (k0 + k < na) {  // wavefront-uniform
+                        const int kk = k0 + k;
+                        const float x = 1.0f + M.a_lam[e][kk] * g.cth;
+                        const bool mine = on && x > 0.f && lo == M.a_e1[e][kk] && hi == M.a_e2[e][kk];
+                        float pw, pm;
+                        pow_zeta(x, M.a_zp[e][kk], &pw, &pm);
+                        const float B = __builtin_amdgcn_exp2f(-M.a_etal2[e][kk] * g.Sd);
+                        const float t = M.a_norm[e][kk] * B *
+                                        ((float)(1 << M.a_zp[e][kk]) * M.a_lam[e][kk] * pm * Cf * dcosD -
+                                         2.f * (M.a_etal2[e][kk] * (1.0f / NN_L2E)) * pw * Cf * SD + pw * FD);
+                        P[k] += mine ? t : 0.f;
                     }
-                }
+            });
+            const float v = sum_halving<NN_KB>(P, l);
+            const int k = k0 + l;
+            if (l < NN_KB && k < na) Urow[nr + k] = -M.dfac[e][nr + k] * v;
         }
-    }
-#pragma unroll
-    for (int k = 0; k < NN_MAXA; ++k) {
-        const float v = sum_group<NN_TPA>(P[k]);
-        if (i < N && k < na && sub == (k & (NN_TPA - 1))) Urep[(size_t)i * NN_K1 + nr + k] = -dfac[e][nr + k] * v;
-    }
-}
-
-// LDS copy of the symmetry-function tables (the extrapolation bounds are read
-// from the constants, once per atom)
-__device__ void load_sftab(NnSfTab &S, const NnConst &M, int lane) {
-    for (int k = lane; k < NN_MAXE; k += NN_BLOCK) {
-        S.nr[k] = M.nr[k];
-        S.na[k] = M.na[k];
-    }
-    for (int k = lane; k < NN_MAXE * NN_MAXR; k += NN_BLOCK) {
-        const int e = k / NN_MAXR, q = k % NN_MAXR;
-        S.r_el[e][q] = M.r_el[e][q];
-        S.r_eta[e][q] = M.r_eta[e][q];
-        S.r_rs[e][q] = M.r_rs[e][q];
-    }
-    for (int k = lane; k < NN_MAXE * NN_MAXA; k += NN_BLOCK) {
-        const int e = k / NN_MAXA, q = k % NN_MAXA;
-        S.a_cls[e][q] = M.a_e1[e][q] * NN_MAXE + M.a_e2[e][q];
-        S.a_etal2[e][q] = M.a_etal2[e][q];
-        S.a_eta[e][q] = M.a_etal2[e][q] * (1.0f / NN_L2E);
-        S.a_lam[e][q] = M.a_lam[e][q];
-        S.a_norm[e][q] = M.a_norm[e][q];
-        S.a_zp[e][q] = M.a_zp[e][q];
-    }
-    // factored angular tables, one lane per element (from M: no dependence
-    // on the copies above)
-    if (lane < NN_MAXE) {
-        const int e = lane, na = M.na[e];
-        int ok = na > 0, nb = 0, nu = 0, cls = na > 0 ? M.a_e1[e][0] * NN_MAXE + M.a_e2[e][0] : -1;
-        int used = 0;  // bit per slot
-        for (int k = 0; k < na && ok; ++k) {
-            if (M.a_e1[e][k] * NN_MAXE + M.a_e2[e][k] != cls) ok = 0;
-            int n = 0, m = 0;
-            while (n < nb && S.f_etal2[e][n] != M.a_etal2[e][k]) ++n;
-            if (n == nb) {
-                if (nb == NN_FB) {
-                    ok = 0;
-                    break;
-                }
-                S.f_etal2[e][nb] = M.a_etal2[e][k];
-                S.f_eta[e][nb] = M.a_etal2[e][k] * (1.0f / NN_L2E);
-                ++nb;
-            }
-            while (m < nu && !(S.f_lam[e][m] == M.a_lam[e][k] && S.f_zp[e][m] == M.a_zp[e][k])) ++m;
-            if (m == nu) {
-                if (nu == NN_FB) {
-                    ok = 0;
-                    break;
-                }
-                S.f_lam[e][nu] = M.a_lam[e][k];
-                S.f_zp[e][nu] = M.a_zp[e][k];
-                ++nu;
-            }
-            const int slot = n * NN_FB + m;
-            if (used >> slot & 1) ok = 0;  // two functions on one slot
-            used |= 1 << slot;
-            S.f_slot[e][k] = slot;
-        }
-        for (int n = nb; n < NN_FB; ++n) S.f_etal2[e][n] = S.f_eta[e][n] = 0.f;
-        for (int m = nu; m < NN_FB; ++m) {
-            S.f_lam[e][m] = 0.f;
-            S.f_zp[e][m] = 0;
-        }
-        S.f_ok[e] = ok;
-        S.f_cls[e] = cls;
-        S.f_nb[e] = nb;
-        S.f_nu[e] = nu;
     }
 }
 
@@ -959,18 +1078,17 @@ __device__ void group_elements(const uint8_t *elem, int N, int ne_model, uint16_
     }
 }
 
-// The network on every atom of the replica (per element, 16-atom tiles, one
-// per wavefront per round: atomic energies to Ea, c = dE/dG rows to Crep)
+// The network on every atom of the replica (wavefront w's transpose buffer at
+// T0 + w Tstride; per element, 16-atom tiles, one per wavefront per round: atomic energies to Ea, c = dE/dG rows to Crep)
 // and the replica's energy [eV] to *epot (fixed-order sum).  Every lane of
 // the block calls this (barriers inside).
 __device__ void network_energy(const NnConst &M, const int *s_ne, const uint16_t *elist, int (*rowsb)[16],
-                               float (*T)[16 * 33], const float *Grep, float *Crep, double *Ea, int N, int lane,
-                               double *epot) {
+                               unsigned char *T0, size_t Tstride, const float *Grep, float *Crep, double *Ea, int N,
+                               int lane, int nwaves, double *epot) {
     const int wave = lane >> 6;
     const int ne_model = M.nelem;
     int ntiles = 0;
     for (int e = 0; e < ne_model; ++e) ntiles += (s_ne[e] + 15) / 16;
-    const int nwaves = NN_BLOCK / 64;
     for (int r0 = 0; r0 < ntiles; r0 += nwaves) {
         const int tile = r0 + wave;
         int e = -1, first = 0, cntE = 0, tl = tile;
@@ -993,7 +1111,7 @@ __device__ void network_energy(const NnConst &M, const int *s_ne, const uint16_t
             rowsb[wave][rr] = (e >= 0 && rr < cntE) ? (int)elist[first + rr] : -1;
         }
         __syncthreads();
-        mlp_tile(M, e, rowsb[wave], Grep, Crep, Ea, T[wave], lane);
+        mlp_tile(M, e, rowsb[wave], Grep, Crep, Ea, (float *)(T0 + wave * Tstride), lane);
         __syncthreads();
     }
     if (lane < 64) {
@@ -1009,9 +1127,9 @@ __device__ void network_energy(const NnConst &M, const int *s_ne, const uint16_t
 // (fixed components 0), dens = 0 (no EMT density).
 __device__ void write_forces(const BatchView &bv, const NnView &nv, const unsigned long long *ax,
                              const unsigned long long *ay, const unsigned long long *az, int N, long long roff,
-                             long long doff, long long aoff, int add_fin, int lane) {
+                             long long doff, long long aoff, int add_fin, int lane, int nthr) {
     const double fconv = NN_HA2EV / NN_BOHR2ANG;
-    for (int i = lane; i < N; i += NN_BLOCK) {
+    for (int i = lane; i < N; i += nthr) {
         double F[3] = {(double)(long long)ax[i] * NN_FISCALE * fconv, (double)(long long)ay[i] * NN_FISCALE * fconv,
                        (double)(long long)az[i] * NN_FISCALE * fconv};
         nv.fpes[roff + i] = F[0];
@@ -1037,18 +1155,9 @@ __device__ void write_forces(const BatchView &bv, const NnView &nv, const unsign
 // Pass G and the network: raw G rows, c = dE/dG rows, the replica's energy
 // and extrapolation flag.  A replica outside the training range leaves
 // with its flag set when skip_extrap (k_nene_f skips it too).
-__global__ void __launch_bounds__(NN_BLOCK) k_nene_g(const NnConst *__restrict__ Mg, BatchView bv, NnView nv,
-                                                     int skip_extrap) {
+__global__ void __launch_bounds__(1024) k_nene_g(const NnConst *__restrict__ Mg, BatchView bv, NnView nv, int skip_extrap) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ NnSfTab S;
-    // the neighbour cache of pass G and the network's transposes share LDS
-    __shared__ union {
-        ChunkNbr L;
-        float T[NN_BLOCK / 64][16 * 33];
-    } U;
-    ChunkNbr &L = U.L;
-    float(*T)[16 * 33] = U.T;
-    __shared__ int rowsb[NN_BLOCK / 64][16];
+    __shared__ int rowsb[16][16];
     __shared__ int s_ne[NN_MAXE];
     const NnConst &M = *Mg;
     const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : (int)blockIdx.x;  // size-class launches
@@ -1059,28 +1168,32 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nene_g(const NnConst *__restrict__
     const long long soff = bv.traj_soff[t];
     const long long roff = soff + (long long)b * 3 * N;
     const long long aoff = bv.traj_aoff[t];
-    const int lane = threadIdx.x;
-    const int wave = lane >> 6;
+    const int lane = threadIdx.x, nthr = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(lane >> 6), l = lane & 63, nwaves = nthr >> 6;
     float *Grep = nv.G + (size_t)rep * nv.maxN * NN_K1;
     float *Crep = nv.C + (size_t)rep * nv.maxN * NN_K1;
     int bad = 0, extrap = 0;
 
-    // dynamic LDS: Ea (double N) | ux uy uz (u32 N each) | elist (u16 N) | elem (u8 N)
-    double *Ea = (double *)smem_raw;
+    // dynamic LDS: per wavefront a neighbour list, later the network's
+    // transpose buffer | Ea (double N) | ux uy uz (u32 N each) | elist (u16 N) | elem (u8 N)
+    WaveNbr &L = *(WaveNbr *)(smem_raw + wave * sizeof(WaveNbr));
+    static_assert(sizeof(WaveNbr) >= 16 * 33 * sizeof(float), "the transpose buffer fits the list's words");
+    double *Ea = (double *)(smem_raw + nwaves * sizeof(WaveNbr));
     uint32_t *ux = (uint32_t *)(Ea + N), *uy = ux + N, *uz = uy + N;
     uint16_t *elist = (uint16_t *)(uz + N);
     uint8_t *elem = (uint8_t *)(elist + N);
 
-    // ---- tables ----
     const int ne_model = M.nelem;
-    load_sftab(S, M, lane);
     double h[9], ih[9];
     float w[3];
     int imax[3];
     cell_setup(M, bv.cell + 9 * t, bv.icell + 9 * t, h, ih, w, imax);
+    __shared__ double s_h[9];
+    if (lane == 0)
+        for (int k = 0; k < 9; ++k) s_h[k] = h[k];
 
     // ---- stage ----
-    for (int i = lane; i < N; i += NN_BLOCK) {
+    for (int i = lane; i < N; i += nthr) {
         const int ty = bv.type[aoff + i];
         const int e = M.elem_of_type[ty];
         if (e < 0 || e >= ne_model) bad |= MDT_ST_BAD_PROP;
@@ -1098,12 +1211,10 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nene_g(const NnConst *__restrict__
     group_elements(elem, N, ne_model, elist, s_ne, lane);
     __syncthreads();
 
-    // ---- pass G: symmetry functions ----
-    for (int k0 = 0; k0 < N; k0 += NN_CA) {
-        build_chunk(M.rc2, M.pi_rc, L, ux, uy, uz, elem, h, imax, w[0], w[1], w[2], N, k0, lane, &bad);
-        __syncthreads();
-        g_chunk(M, S, L, elem, N, k0, lane, M.rc2, M.pi_rc, Grep, &extrap);
-        __syncthreads();
+    // ---- pass G: symmetry functions, a centre per wavefront ----
+    for (int i = wave; i < N; i += nwaves) {
+        const int cnt = build_list(M.rc2, L, ux, uy, uz, elem, s_h, imax, w[0], w[1], w[2], N, i, l, &bad);
+        g_centre(M, L, cnt, __builtin_amdgcn_readfirstlane(elem[i]), l, Grep + (size_t)i * NN_K1, &extrap);
     }
 
     // replicas outside the training range go to the EMT fallback untouched
@@ -1117,20 +1228,17 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nene_g(const NnConst *__restrict__
         return;
     }
 
-    network_energy(M, s_ne, elist, rowsb, T, Grep, Crep, Ea, N, lane, &bv.epot[bv.traj_eoff[t] + b]);
+    network_energy(M, s_ne, elist, rowsb, smem_raw, sizeof(WaveNbr), Grep, Crep, Ea, N, lane, nwaves,
+                   &bv.epot[bv.traj_eoff[t] + b]);
     if (extrap) bad |= MDT_ST_NN_EXTRAPOLATION;
     if (bad) atomicOr(&bv.status[t], bad);
 }
 
 // Pass F and the outputs: dE/dr from the c rows of k_nene_g, f (+ the
 // forces already in f when add_fin), a = f/m, dens = 0.
-__global__ void __launch_bounds__(NN_BLOCK) k_nene_f(const NnConst *__restrict__ Mg, BatchView bv, NnView nv,
-                                                     int add_fin, int skip_extrap) {
+__global__ void __launch_bounds__(1024) k_nene_f(const NnConst *__restrict__ Mg, BatchView bv, NnView nv, int add_fin,
+                                                 int skip_extrap) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ NnSfTab S;
-    __shared__ ChunkNbr L;
-    __shared__ float cb[NN_CA][NN_K1];
-    __shared__ float Wsh[NN_CA][NN_FB * NN_FB];
     const NnConst &M = *Mg;
     const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : (int)blockIdx.x;  // size-class launches
     if (skip_extrap && nv.rep_flag[rep]) return;  // whole block: uniform
@@ -1142,22 +1250,26 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nene_f(const NnConst *__restrict__
     const long long roff = soff + (long long)b * 3 * N;
     const long long doff = soff / 3 + (long long)b * N;
     const long long aoff = bv.traj_aoff[t];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x, nthr = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(lane >> 6), l = lane & 63, nwaves = nthr >> 6;
     const float *Crep = nv.C + (size_t)rep * nv.maxN * NN_K1;
     int bad = 0;
 
-    // dynamic LDS: ax ay az (u64 N each) | ux uy uz (u32 N) | elem (u8 N)
-    unsigned long long *ax = (unsigned long long *)smem_raw, *ay = ax + N, *az = ay + N;
+    // dynamic LDS: per wavefront a neighbour list | ax ay az (u64 N each) | ux uy uz (u32 N) | elem (u8 N)
+    WaveNbrF &L = *(WaveNbrF *)(smem_raw + wave * sizeof(WaveNbrF));
+    unsigned long long *ax = (unsigned long long *)(smem_raw + nwaves * sizeof(WaveNbrF)), *ay = ax + N, *az = ay + N;
     uint32_t *ux = (uint32_t *)(az + N), *uy = ux + N, *uz = uy + N;
     uint8_t *elem = (uint8_t *)(uz + N);
 
     const int ne_model = M.nelem;
-    load_sftab(S, M, lane);
     double h[9], ih[9];
     float w[3];
     int imax[3];
     cell_setup(M, bv.cell + 9 * t, bv.icell + 9 * t, h, ih, w, imax);
-    for (int i = lane; i < N; i += NN_BLOCK) {
+    __shared__ double s_h[9];
+    if (lane == 0)
+        for (int k = 0; k < 9; ++k) s_h[k] = h[k];
+    for (int i = lane; i < N; i += nthr) {
         const int e = M.elem_of_type[bv.type[aoff + i]];
         elem[i] = (uint8_t)(e < 0 || e >= ne_model ? 0 : e);
         const double r0 = bv.x[roff + i], r1 = bv.x[roff + N + i], r2 = bv.x[roff + 2 * N + i];
@@ -1171,20 +1283,13 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nene_f(const NnConst *__restrict__
     }
     __syncthreads();
 
-    // ---- pass F: forces ----
-    for (int k0 = 0; k0 < N; k0 += NN_CA) {
-        build_chunk(M.rc2, M.pi_rc, L, ux, uy, uz, elem, h, imax, w[0], w[1], w[2], N, k0, lane, &bad);
-        for (int q = lane; q < NN_CA * NN_K1; q += NN_BLOCK) {
-            const int ci = q / NN_K1, k = q % NN_K1;
-            const int i = k0 + ci;
-            cb[ci][k] = (i < N && k < S.nr[elem[i]] + S.na[elem[i]]) ? Crep[(size_t)i * NN_K1 + k] : 0.f;
-        }
-        __syncthreads();
-        force_chunk(S, L, cb, Wsh, elem, N, k0, lane, M.rc2, M.pi_rc, ax, ay, az, &bad);
-        __syncthreads();
+    // ---- pass F: forces, a centre per wavefront ----
+    for (int i = wave; i < N; i += nwaves) {
+        const int cnt = build_list(M.rc2, L, ux, uy, uz, elem, s_h, imax, w[0], w[1], w[2], N, i, l, &bad);
+        force_centre(M, L, cnt, i, __builtin_amdgcn_readfirstlane(elem[i]), l, Crep + (size_t)i * NN_K1, ax, ay, az, &bad);
     }
-
-    write_forces(bv, nv, ax, ay, az, N, roff, doff, aoff, add_fin, lane);
+    __syncthreads();
+    write_forces(bv, nv, ax, ay, az, N, roff, doff, aoff, add_fin, lane, nthr);
     if (bad) atomicOr(&bv.status[t], bad);
 }
 
@@ -1670,14 +1775,6 @@ __device__ __forceinline__ float act_fast(int code, float z, float *d1) {
     return z;
 }
 
-// orders a wavefront's LDS writes before its later LDS reads (the transpose
-// buffers of mlp_tile_w are private to one wavefront)
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // mlp_tile for one wavefront on its own (no block barriers): the same
 // products on v_mfma_f32_16x16x32_bf16 with hi/lo split operands; the
 // second 32-input block of layer 1 and the dE/dx tiles past the element's
@@ -2039,7 +2136,7 @@ __global__ void __launch_bounds__(NN_BLOCK, 4) k_nene_rf(const NnConst *__restri
             __syncthreads();
         }
     }
-    write_forces(bv, nv, ax, ay, az, N, roff, doff, aoff, add_fin, lane);
+    write_forces(bv, nv, ax, ay, az, N, roff, doff, aoff, add_fin, lane, NN_BLOCK);
     if (bad) atomicOr(&bv.status[t], bad);
 }
 
@@ -2058,33 +2155,31 @@ __global__ void __launch_bounds__(NN_BLOCK, 4) k_nene_rf(const NnConst *__restri
 // k_nn_frame: mode 0 writes the raw symmetry functions of every atom of the
 // frame; mode 1 computes the frame's forces from C, its energy from Eatom,
 // the loss parts, cE = dL/dE and U rows.
-__global__ void __launch_bounds__(NN_BLOCK) k_nn_frame(const NnConst *__restrict__ Mg, NnTrainView tv,
-                                                       const int *frames, int mode, double cEw, double cFw) {
+__global__ void __launch_bounds__(1024) k_nn_frame(const NnConst *__restrict__ Mg, NnTrainView tv, const int *frames,
+                                                   int mode, double cEw, double cFw) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ NnSfTab S;
-    __shared__ ChunkNbr L;
-    __shared__ float cb[NN_CA][NN_K1];
-    __shared__ float Wsh[NN_CA][NN_FB * NN_FB];
-    __shared__ float sdfac[NN_MAXE][NN_K1];
-    __shared__ double red[NN_BLOCK / 64];
+    __shared__ double red[16];
     const NnConst &M = *Mg;
     const int f = frames[blockIdx.x];
     const int N = tv.fr_natoms[f];
     const long long ao = tv.fr_aoff[f];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x, nthr = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(lane >> 6), l = lane & 63, nwaves = nthr >> 6;
     int bad = 0, extrap = 0;
-    // dynamic LDS: ax ay az (u64 N) | ux uy uz (u32 N) | gx gy gz (float N) | elem (u8 N)
-    unsigned long long *ax = (unsigned long long *)smem_raw, *ay = ax + N, *az = ay + N;
+    // dynamic LDS: per wavefront a neighbour list | ax ay az (u64 N) | ux uy uz (u32 N) | gx gy gz (float N) | elem (u8 N)
+    WaveNbrF &L = *(WaveNbrF *)(smem_raw + wave * sizeof(WaveNbrF));
+    unsigned long long *ax = (unsigned long long *)(smem_raw + nwaves * sizeof(WaveNbrF)), *ay = ax + N, *az = ay + N;
     uint32_t *ux = (uint32_t *)(az + N), *uy = ux + N, *uz = uy + N;
     float *gx = (float *)(uz + N), *gy = gx + N, *gz = gy + N;
     uint8_t *elem = (uint8_t *)(gz + N);
-    load_sftab(S, M, lane);
-    for (int k = lane; k < NN_MAXE * NN_K1; k += NN_BLOCK) sdfac[k / NN_K1][k % NN_K1] = M.dfac[k / NN_K1][k % NN_K1];
     double h[9], ih[9];
     float w[3];
     int imax[3];
     cell_setup(M, tv.fr_cell + 9 * f, tv.fr_icell + 9 * f, h, ih, w, imax);
-    for (int i = lane; i < N; i += NN_BLOCK) {
+    __shared__ double s_h[9];
+    if (lane == 0)
+        for (int k = 0; k < 9; ++k) s_h[k] = h[k];
+    for (int i = lane; i < N; i += nthr) {
         const int e = M.elem_of_type[tv.type[ao + i]];
         elem[i] = (uint8_t)(e < 0 ? 0 : e);
         const double *r = tv.pos + 3 * (ao + i);
@@ -2099,31 +2194,23 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nn_frame(const NnConst *__restrict
     __syncthreads();
     float *Grow = tv.G + (size_t)ao * NN_K1;
     if (mode == 0) {
-        for (int k0 = 0; k0 < N; k0 += NN_CA) {
-            build_chunk(M.rc2, M.pi_rc, L, ux, uy, uz, elem, h, imax, w[0], w[1], w[2], N, k0, lane, &bad);
-            __syncthreads();
-            g_chunk(M, S, L, elem, N, k0, lane, M.rc2, M.pi_rc, Grow, &extrap);
-            __syncthreads();
+        for (int i = wave; i < N; i += nwaves) {
+            const int cnt = build_list(M.rc2, L, ux, uy, uz, elem, s_h, imax, w[0], w[1], w[2], N, i, l, &bad);
+            g_centre(M, L, cnt, __builtin_amdgcn_readfirstlane(elem[i]), l, Grow + (size_t)i * NN_K1, &extrap);
         }
         return;
     }
     // forces with the current network (C rows from k_nn_mlp)
     const float *Crow = tv.C + (size_t)ao * NN_K1;
-    for (int k0 = 0; k0 < N; k0 += NN_CA) {
-        build_chunk(M.rc2, M.pi_rc, L, ux, uy, uz, elem, h, imax, w[0], w[1], w[2], N, k0, lane, &bad);
-        for (int q = lane; q < NN_CA * NN_K1; q += NN_BLOCK) {
-            const int ci = q / NN_K1, k = q % NN_K1;
-            const int i = k0 + ci;
-            cb[ci][k] = (i < N && k < S.nr[elem[i]] + S.na[elem[i]]) ? Crow[(size_t)i * NN_K1 + k] : 0.f;
-        }
-        __syncthreads();
-        force_chunk(S, L, cb, Wsh, elem, N, k0, lane, M.rc2, M.pi_rc, ax, ay, az, &bad);
-        __syncthreads();
+    for (int i = wave; i < N; i += nwaves) {
+        const int cnt = build_list(M.rc2, L, ux, uy, uz, elem, s_h, imax, w[0], w[1], w[2], N, i, l, &bad);
+        force_centre(M, L, cnt, i, __builtin_amdgcn_readfirstlane(elem[i]), l, Crow + (size_t)i * NN_K1, ax, ay, az, &bad);
     }
+    __syncthreads();
     // residuals: g = dL/dF (per Hartree/Bohr), force loss part
     const double fconv = NN_HA2EV / NN_BOHR2ANG;
     double lf = 0.0;
-    for (int i = lane; i < N; i += NN_BLOCK) {
+    for (int i = lane; i < N; i += nthr) {
         const double F[3] = {(double)(long long)ax[i] * NN_FISCALE * fconv,
                              (double)(long long)ay[i] * NN_FISCALE * fconv,
                              (double)(long long)az[i] * NN_FISCALE * fconv};
@@ -2139,7 +2226,7 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nn_frame(const NnConst *__restrict
     __syncthreads();
     if (lane == 0) {
         double sF = 0.0, E = 0.0;
-        for (int q = 0; q < NN_BLOCK / 64; ++q) sF += red[q];
+        for (int q = 0; q < nwaves; ++q) sF += red[q];
         for (int i = 0; i < N; ++i) E += tv.Eatom[ao + i];
         const double dE = (NN_HA2EV * E - tv.Eref[f]) / N;
         tv.loss[2 * f] = cEw * dE * dE;
@@ -2148,11 +2235,9 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nn_frame(const NnConst *__restrict
     }
     // Jacobian-vector product
     float *Urow = tv.U + (size_t)ao * NN_K1;
-    for (int k0 = 0; k0 < N; k0 += NN_CA) {
-        build_chunk(M.rc2, M.pi_rc, L, ux, uy, uz, elem, h, imax, w[0], w[1], w[2], N, k0, lane, &bad);
-        __syncthreads();
-        jvp_chunk(S, L, elem, N, k0, lane, M.rc2, M.pi_rc, gx, gy, gz, sdfac, Urow);
-        __syncthreads();
+    for (int i = wave; i < N; i += nwaves) {
+        const int cnt = build_list(M.rc2, L, ux, uy, uz, elem, s_h, imax, w[0], w[1], w[2], N, i, l, &bad);
+        jvp_centre(M, L, cnt, i, __builtin_amdgcn_readfirstlane(elem[i]), l, gx, gy, gz, Urow + (size_t)i * NN_K1);
     }
 }
 
@@ -2446,16 +2531,26 @@ __global__ void __launch_bounds__(NN_BLOCK) k_nn_grad(const NnConst *__restrict_
     if (cur >= 0) acc_flush(acc, partials + ((size_t)gw * NN_MAXE + cur) * NN_NPAR, l);
 }
 
-// fixed-order reduction of the partials; mode 0 writes the gradient to grad
-// (padded layout, NN_MAXE x NN_NPAR), mode 1 also applies Adam to NnConst
-__global__ void k_nn_adam(NnConst *Mg, const float *partials, int W, float *grad, float *am, float *av, float lr,
-                          float beta1, float beta2, float eps, int step, int mode) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= NN_MAXE * NN_NPAR) return;
+// Fixed-order reduction of the partials; mode 0 writes the gradient to grad
+// (padded layout, NN_MAXE x NN_NPAR), mode 1 also applies Adam to NnConst.
+// 64 parameters to a workgroup, each summed by 4 wavefronts over every
+// fourth partial: one lane walking all 296 of a minibatch of 9.5 k atoms
+// waited for each load (74 us, now below 10).
+__global__ void __launch_bounds__(256) k_nn_adam(NnConst *Mg, const float *__restrict__ partials, int W, float *grad,
+                                                 float *am, float *av, float lr, float beta1, float beta2, float eps,
+                                                 int step, int mode) {
+    __shared__ double part[4][64];
+    const int idx = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
     const int e = idx / NN_NPAR, p = idx % NN_NPAR;
-    if (e >= Mg->nelem) return;
+    const bool on = idx < NN_MAXE * NN_NPAR && e < Mg->nelem;
     double g = 0.0;
-    for (int w = 0; w < W; ++w) g += (double)partials[((size_t)w * NN_MAXE + e) * NN_NPAR + p];
+    if (on)
+#pragma unroll 8
+        for (int w = slice; w < W; w += 4) g += (double)partials[((size_t)w * NN_MAXE + e) * NN_NPAR + p];
+    part[slice][threadIdx.x & 63] = g;
+    __syncthreads();
+    if (!on || slice > 0) return;
+    g = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
     const int nin = Mg->nr[e] + Mg->na[e], n1 = Mg->nh1, n2 = Mg->nh2;
     float *par;
     bool real;
@@ -2493,11 +2588,25 @@ __global__ void k_nn_adam(NnConst *Mg, const float *partials, int W, float *grad
     *par -= lr * mh / (sqrtf(vh) + eps);
 }
 
-size_t mdt_nn_frame_smem(int N) { return (size_t)N * (3 * 8 + 3 * 4 + 3 * 4 + 1) + 16; }
+// Wavefronts per workgroup of the kernels that give each centre atom a
+// wavefront: 8, or 16 for launches of at most a workgroup per CU; halved
+// while the workgroup's LDS does not fit or half the wavefronts would have no
+// atom.  Measured with 4 / 8 / 16 wavefronts, H/Au 6x6x4 with the angular
+// network, ms per step: 200 replicas 1.38 / 0.78 / 0.54, 512 replicas 1.54 /
+// 1.06 / 1.09, 2000 replicas 3.99 / 3.96 / 4.28; one replica's call 1421 /
+// 885 / 677 us; the training gradient over 256 frames 634 / 461 / 396 us.
+static int centre_waves(int nblocks, int N, size_t per_wave, size_t per_atom, size_t lds_limit) {
+    int nw = nblocks > 256 ? 8 : 16;
+    while (nw > 4 && (nw > (N + 1) / 2 || nw * per_wave + N * per_atom + 2048 > lds_limit)) nw >>= 1;
+    return nw;
+}
 
-hipError_t mdt_launch_nn_frame(int nblocks, size_t smem, const NnConst *M, const NnTrainView &tv, const int *frames,
-                               int mode, double cEw, double cFw, hipStream_t st) {
-    hipLaunchKernelGGL(k_nn_frame, dim3(nblocks), dim3(NN_BLOCK), smem, st, M, tv, frames, mode, cEw, cFw);
+hipError_t mdt_launch_nn_frame(int nblocks, int maxN, size_t lds_limit, const NnConst *M, const NnTrainView &tv,
+                               const int *frames, int mode, double cEw, double cFw, hipStream_t st) {
+    const size_t per_atom = 3 * 8 + 3 * 4 + 3 * 4 + 1;
+    const int nw = centre_waves(nblocks, maxN, sizeof(WaveNbrF), per_atom, lds_limit);
+    const size_t smem = nw * sizeof(WaveNbrF) + maxN * per_atom + 16;
+    hipLaunchKernelGGL(k_nn_frame, dim3(nblocks), dim3(64 * nw), smem, st, M, tv, frames, mode, cEw, cFw);
     return hipGetLastError();
 }
 
@@ -2517,15 +2626,15 @@ hipError_t mdt_launch_nn_grad(int nblocks, const NnConst *M, const NnTrainView &
 hipError_t mdt_launch_nn_adam(NnConst *M, const float *partials, int W, float *grad, float *am, float *av, float lr,
                               float beta1, float beta2, float eps, int step, int mode, hipStream_t st) {
     const int n = NN_MAXE * NN_NPAR;
-    hipLaunchKernelGGL(k_nn_adam, dim3((n + 255) / 256), dim3(256), 0, st, M, partials, W, grad, am, av, lr, beta1,
+    hipLaunchKernelGGL(k_nn_adam, dim3((n + 63) / 64), dim3(256), 0, st, M, partials, W, grad, am, av, lr, beta1,
                        beta2, eps, step, mode);
     return hipGetLastError();
 }
 
-// dynamic LDS of the larger of k_nene_g (4 N doubles, u16 + u8 per atom)
-// and k_nene_f (3 N doubles, 3 N u64, u8 per atom)
-// the larger of k_nene_g's (23 B per atom) and k_nene_f's (37 B per atom)
-size_t mdt_nene_smem(int N) { return (size_t)N * (3 * 8 + 3 * 4 + 1) + 16; }
+// dynamic LDS of k_nene_f on nw wavefronts (k_nene_g needs less)
+static size_t nene_smem(int N, int nw) { return nw * sizeof(WaveNbrF) + (size_t)N * (3 * 8 + 3 * 4 + 1) + 16; }
+// at least: 4 wavefronts
+size_t mdt_nene_smem(int N) { return nene_smem(N, 4); }
 
 // neighbour-list capacity per atom of the NN kernels (stored lists of the radial kernels)
 int mdt_nene_cap() { return NN_CAP; }
@@ -2544,15 +2653,18 @@ hipError_t mdt_nene_attributes(hipFuncAttributes *fa, int radial) {
     return hipSuccess;
 }
 
-hipError_t mdt_launch_nene(int nrep, size_t smem, const NnConst *M, const BatchView &bv, float *G, float *C,
+// nmax: the largest replica of the launch
+hipError_t mdt_launch_nene(int nrep, int nmax, size_t lds_limit, const NnConst *M, const BatchView &bv, float *G, float *C,
                            int *rep_flag, double *fpes, int maxN, int add_fin, int skip_extrap, int radial,
                            uint16_t *nbr, uint8_t *nbr_cnt, uint32_t *nbr_ref, int *nbr_key, double skin_bohr,
                            hipStream_t st, int images) {
     NnView nv{G, C, rep_flag, fpes, maxN, nbr, nbr_cnt, nbr_ref, nbr_key, (float)skin_bohr};
+    const int nw = centre_waves(nrep, nmax, sizeof(WaveNbrF), 3 * 8 + 3 * 4 + 1, lds_limit);
+    const size_t smem = radial ? mdt_nene_radial_smem(nmax) : nene_smem(nmax, nw);
     if (radial)  // the image search costs k_nene_rg no occupancy: one instantiation
         hipLaunchKernelGGL(k_nene_rg<true>, dim3(nrep), dim3(NN_BLOCK), smem, st, M, bv, nv, skip_extrap);
     else
-        hipLaunchKernelGGL(k_nene_g, dim3(nrep), dim3(NN_BLOCK), smem, st, M, bv, nv, skip_extrap);
+        hipLaunchKernelGGL(k_nene_g, dim3(nrep), dim3(64 * nw), smem, st, M, bv, nv, skip_extrap);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (radial && images)
@@ -2560,6 +2672,6 @@ hipError_t mdt_launch_nene(int nrep, size_t smem, const NnConst *M, const BatchV
     else if (radial)
         hipLaunchKernelGGL(k_nene_rf<false>, dim3(nrep), dim3(NN_BLOCK), smem, st, M, bv, nv, add_fin, skip_extrap);
     else
-        hipLaunchKernelGGL(k_nene_f, dim3(nrep), dim3(NN_BLOCK), smem, st, M, bv, nv, add_fin, skip_extrap);
+        hipLaunchKernelGGL(k_nene_f, dim3(nrep), dim3(64 * nw), smem, st, M, bv, nv, add_fin, skip_extrap);
     return hipGetLastError();
 }

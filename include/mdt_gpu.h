@@ -209,8 +209,8 @@ int mdt_batch_tune(mdt_batch *b, int tpa, int nbcap, int *tpa_chosen);
  * Launch shape of the k_replica size classes (replicas grouped by atom
  * count; no counterpart in the reference, which has no GPU launch): up to
  * `max` classes, 6 int32 each -- largest atom count, replicas, threads per
- * atom, lists kept across launches with the Verlet skin (1: staged in LDS
- * during a launch, 2: read from HBM) or rebuilt every launch (0), threads
+ * atom, lists kept across launches with the Verlet skin (1, or 2 where
+ * that mode was set) or rebuilt every launch (0), threads
  * per workgroup, list capacity per atom.
  * *nclass receives the number of classes (0 in mixed bead mode).
  */
@@ -231,9 +231,8 @@ int mdt_batch_set_wide(mdt_batch *b, int mode);
 /*
  * Neighbour lists of k_replica's size classes (an extension; the reference
  * visits every pair at every call): mode -1 autotuned (default); 0 rebuilt
- * at every launch (in LDS where they fit); 1 kept across launches with the
- * Verlet skin (mdt_batch_set_list_skin) in HBM and staged in LDS during a
- * launch (read from HBM where LDS is too small); 2 kept and read from HBM.
+ * at every launch; 1 or 2 kept across launches with the Verlet skin
+ * (mdt_batch_set_list_skin) and read from HBM (both the same).
  * Forces agree to rounding whichever mode runs.  The next launch
  * configures again.
  */

@@ -8,6 +8,7 @@
 //   P*N arrays (dens, fixed bits) live at traj_soff[t]/3: [bead b][atom i].
 //   Per-atom arrays (type, mass) live at traj_aoff[t]: [atom i].
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #define MDT_MAXT 4
@@ -65,6 +66,7 @@
 // per-(type a, neighbour type n) tables for a gather formulation.
 struct EmtConst {
     int ntypes;
+    int gen;      // counts mdt_emt_params_set calls of the context: lists kept from older constants are rebuilt
     int fp32_ok;  // every EMT type's embedding stiffness 6 V0 kappa / (beta eta2) <= MDT_FP32_STIFF_MAX
     double rcut, acut, cutr;  // cutr = 1.5 * rcut (the reference's hard cut)
     double cut2hi;            // neighbour-list bound on r^2 (cutr^2 widened by 1e-12 rel)
@@ -106,6 +108,15 @@ struct PropChunk {
 };
 #define MDT_CHUNK 256
 
+// k_replica's HBM slot: words per slot and where its parts start (mdt_replica_lists)
+struct ReplicaLists {
+    long long stride, rows, chunk, scan;
+    size_t smem;  // dynamic LDS
+};
+#define REP_FEW 512
+
+#define MDT_FLAT_MAX 4  // atoms of a trajectory outside k_replica's majority type with lists of their own
+
 struct BatchView {
     int ntraj, nrep;
     int nbcap;      // neighbour-list capacity per atom
@@ -126,8 +137,8 @@ struct BatchView {
     double *epot;           // per replica (P per traj, at traj_soff/(3N))
     const long long *traj_eoff;  // offset of a trajectory's epot(1..P)
     int *status;            // per traj
-    uint16_t *nbr_global;   // NULL: neighbour lists in LDS; else nrep * nbr_stride entries
-    long long nbr_stride;   // entries per replica slice (maxN * cap)
+    uint16_t *nbr_global;   // k_mixed's neighbour lists, nbr_stride entries per listed trajectory
+    long long nbr_stride;
     const int *rep_list;    // non-NULL: block k works on replica rep_list[k] (size-class launches)
     const int *only;        // non-NULL: calc_force only on replicas with only[rep] != 0
     const int *skip;        // non-NULL: no calc_force on replicas with skip[rep] != 0
@@ -154,18 +165,20 @@ struct BatchView {
     int *mix_valid;
     double mix_skin;
     long long mix_ns;
-    // k_replica's lists kept across launches (Verlet skin), per block slot of
-    // a size-class launch with lists in HBM: positions at the list build (SoA,
-    // rl_ns per coordinate), list counts and a valid flag; rl_valid NULL: the
-    // lists are rebuilt at every launch
-    // rl_stage != 0: the kept lists live in nbr_global between launches and
-    // are staged in LDS during one (the kernel's LDS-list instantiation)
+    // k_replica: the EMT type whose atoms' pairs its rows hold, every
+    // trajectory having at most MDT_FLAT_MAX atoms of the other EMT type (-1:
+    // rows hold all types); lanes per atom of the list scan
+    int bulk, tpa_shift;
+    // its lists, per block slot of a size-class launch (mdt_replica_lists), and,
+    // for lists kept across launches (Verlet skin): positions at the build
+    // (SoA, rl_ns per coordinate) and a valid word with the generation of the
+    // EMT constants; rl_valid NULL: rebuilt at every launch
+    uint32_t *rl_lists;
+    long long rl_stride, rl_rows, rl_chunk, rl_scan;
     double *rl_ref;
-    uint16_t *rl_cnt;
-    int *rl_valid;
+    int2 *rl_valid;
     double rl_skin;
     long long rl_ns;
-    int rl_stage;
     struct TrajObs *obs;
     int *done;
     double obs_ul, obs_ll, ads_start, ads_end;

@@ -2,23 +2,18 @@
 // md_tian2 propagators.
 //
 // k_replica: calc_force, one workgroup per replica (trajectory t, bead b).
-//   phase 0: stage the replica in LDS, folded into its cell, with fractional
-//            coordinates;
-//   phase 1: TPA lanes per atom scan all atoms with the minimum-image
-//            convention and build an ordered per-atom neighbour list of
-//            (index | periodic-image code << 11), compacted with a wavefront
-//            ballot;
+//   phase 0: stage the replica in LDS;
+//   phase 1: the rows of neighbours, (index | periodic-image code << 11), kept from
+//            an earlier launch or built by a minimum-image scan of all atoms;
 //   phase 2 (pass A): every unordered pair once, by its owner atom:
-//            sigma_k += csig(tk,tn) f_sigma_tn(r) in registers and
-//            sigma_n += csig(tn,tk) f_sigma_tk(r) into a fixed-point LDS
-//            accumulator; then per atom s, dens, E_coh + vref and
+//            sigma_k += csig(tk,tn) f_sigma_tn(r) and sigma_n += csig(tn,tk)
+//            f_sigma_tk(r); then per atom s, dens, E_coh + vref and
 //            G_a = dE/dsigma_a;
 //   phase 3 (pass B): the pair's dE/dr (density part through G of both
 //            atoms, pair-potential part directly) gives +F on the owner and
-//            -F on the partner (Newton's third law), both accumulated in
-//            fixed point; then set_acceleration.
-//   Fixed-point integer accumulation is associative, so results are bitwise
-//   reproducible whatever order the lanes' atomics land in.
+//            -F on the partner (Newton's third law); then set_acceleration.
+//   Every sum is one of integers, or of FP64 multiples of a grid: results are
+//   bitwise reproducible whatever order the lanes' atomics land in.
 // k_traj_classical (one-bead batches) and k_prop / k_com_ring (the others):
 //   propagate_2 of the previous step, propagate_1, COM removal and (P > 1)
 //   the ring-polymer free step (src/md_algo.f90:37-106, src/rpmd.f90:309-452).
@@ -34,19 +29,24 @@
 namespace {
 
 // Tables every lane indexes by atom type: kept in LDS (divergent indices).
-struct LdsTables {
-    double eta2[MDT_MAXT], bs0[MDT_MAXT], kdb[MDT_MAXT], betaeta2[MDT_MAXT];
+struct LdsTypes {
+    double bs0[MDT_MAXT], kdb[MDT_MAXT], betaeta2[MDT_MAXT];
     double e0[MDT_MAXT], lambda[MDT_MAXT], v0[MDT_MAXT], kappa[MDT_MAXT], n0[MDT_MAXT];
     double densc[MDT_MAXT];
+    double etaT[MDT_MAXT], kdbT[MDT_MAXT];  // -eta2, -kdb in mdt_exp_t's unit
     double csig[MDT_MAXT * MDT_MAXT], etad[MDT_MAXT * MDT_MAXT], wv[MDT_MAXT * MDT_MAXT];
-    double csig48[MDT_MAXT * MDT_MAXT];  // csig * 2^48: partner sigma terms in fixed-point units
-    double shift[27 * 3];  // cartesian lattice translation of each image code
     double exptab[MDT_EXP_TAB_N];
-    int owner[MDT_MAXT], pair_on[MDT_MAXT * MDT_MAXT], algo[MDT_MAXT], is_proj[MDT_MAXT];
+    int owner[MDT_MAXT], pair_on[MDT_MAXT * MDT_MAXT];
     // FP32 copies for the single-precision pair terms; *_l2 carry a factor
     // log2(e) so that exp(-a x) = 2^(-a_l2 x)
     float f_eta2l2[MDT_MAXT], f_kdbl2[MDT_MAXT], f_kdb[MDT_MAXT];
     float f_csig[MDT_MAXT * MDT_MAXT], f_etad[MDT_MAXT * MDT_MAXT], f_wv[MDT_MAXT * MDT_MAXT];
+};
+struct LdsTables : LdsTypes {
+    double eta2[MDT_MAXT];
+    double csig48[MDT_MAXT * MDT_MAXT];  // csig * 2^48: partner sigma terms in fixed-point units
+    double shift[27 * 3];  // cartesian lattice translation of each image code
+    int algo[MDT_MAXT], is_proj[MDT_MAXT];
 };
 
 #define MDT_LOG2E 1.4426950408889634
@@ -128,10 +128,8 @@ __device__ __forceinline__ double ldfa(double dens, double mass, int *bad) {
     return fric * convert / MDT_HBAR / mass;
 }
 
-__device__ void load_tables(LdsTables &T, const EmtConst *__restrict__ ec, const PropConst *__restrict__ pc,
-                            const CellRegs &cell, int lane, int nthr) {
+__device__ void load_types(LdsTypes &T, const EmtConst *__restrict__ ec, int lane, int nthr) {
     for (int k = lane; k < MDT_MAXT; k += nthr) {
-        T.eta2[k] = ec->eta2[k];
         T.bs0[k] = ec->betas0[k];
         T.kdb[k] = ec->kappadbeta[k];
         T.betaeta2[k] = ec->betaeta2[k];
@@ -141,16 +139,15 @@ __device__ void load_tables(LdsTables &T, const EmtConst *__restrict__ ec, const
         T.kappa[k] = ec->kappa[k];
         T.n0[k] = ec->n0[k];
         T.densc[k] = ec->densc[k];
+        T.etaT[k] = -ec->eta2[k] * MDT_EXP_K;
+        T.kdbT[k] = -ec->kappadbeta[k] * MDT_EXP_K;
         T.owner[k] = ec->owner[k];
-        T.algo[k] = pc->algo[k];
-        T.is_proj[k] = pc->is_proj[k];
         T.f_eta2l2[k] = (float)(ec->eta2[k] * MDT_LOG2E);
         T.f_kdbl2[k] = (float)(ec->kappadbeta[k] * MDT_LOG2E);
         T.f_kdb[k] = (float)ec->kappadbeta[k];
     }
     for (int k = lane; k < MDT_MAXT * MDT_MAXT; k += nthr) {
         T.csig[k] = ec->csig[k];
-        T.csig48[k] = ec->csig[k] * 281474976710656.0;  // exact (power of two)
         T.etad[k] = ec->etad[k];
         T.wv[k] = ec->wv[k];
         T.pair_on[k] = ec->pair_on[k];
@@ -158,14 +155,29 @@ __device__ void load_tables(LdsTables &T, const EmtConst *__restrict__ ec, const
         T.f_etad[k] = (float)ec->etad[k];
         T.f_wv[k] = (float)ec->wv[k];
     }
+}
+
+__device__ void load_exptab(LdsTypes &T, int lane, int nthr) {
+    const double et[MDT_EXP_TAB_N] = MDT_EXP_TAB_INIT;
+    for (int k = lane; k < MDT_EXP_TAB_N; k += nthr) T.exptab[k] = et[k];
+}
+
+__device__ void load_tables(LdsTables &T, const EmtConst *__restrict__ ec, const PropConst *__restrict__ pc,
+                            const CellRegs &cell, int lane, int nthr) {
+    load_types(T, ec, lane, nthr);
+    for (int k = lane; k < MDT_MAXT; k += nthr) {
+        T.eta2[k] = ec->eta2[k];
+        T.algo[k] = pc->algo[k];
+        T.is_proj[k] = pc->is_proj[k];
+    }
+    for (int k = lane; k < MDT_MAXT * MDT_MAXT; k += nthr) T.csig48[k] = ec->csig[k] * 281474976710656.0;  // exact (power of two)
     for (int c = lane; c < 27; c += nthr) {
         const double m0 = (double)(c % 3 - 1), m1 = (double)((c / 3) % 3 - 1), m2 = (double)(c / 9 - 1);
         T.shift[3 * c + 0] = cell.h[0] * m0 + cell.h[3] * m1 + cell.h[6] * m2;
         T.shift[3 * c + 1] = cell.h[1] * m0 + cell.h[4] * m1 + cell.h[7] * m2;
         T.shift[3 * c + 2] = cell.h[2] * m0 + cell.h[5] * m1 + cell.h[8] * m2;
     }
-    const double et[MDT_EXP_TAB_N] = MDT_EXP_TAB_INIT;
-    for (int k = lane; k < MDT_EXP_TAB_N; k += nthr) T.exptab[k] = et[k];
+    load_exptab(T, lane, nthr);
 }
 
 }  // namespace
@@ -246,7 +258,7 @@ __device__ __forceinline__ void fx_add(unsigned long long *acc, double x, double
 
 // s, embedded density, E_coh + vref and G = dE/dsigma of an atom of type tk
 // with total sigma (src/pes_emt_mod.f90:793-869 and :871-972)
-__device__ __forceinline__ void emt_atom(const LdsTables &T, int tk, double sig, double *Gk, double *Ek, double *dn) {
+__device__ __forceinline__ void emt_atom(const LdsTypes &T, int tk, double sig, double *Gk, double *Ek, double *dn) {
     const double clamp30 = (double)1e-30f;  // pes_emt_mod.f90:793-794
     const double sc = sig > clamp30 ? sig : clamp30;
     const double sl = sc > MDT_TOLERANCE ? sc : MDT_TOLERANCE;
@@ -276,27 +288,119 @@ __device__ __forceinline__ double tie_image(double ia, double ib, double ic, dou
     return rint(x - (s - round(s)));
 }
 
-// Minimum image of the pair (k, n) of a replica staged folded in LDS:
-// d = p_k - p_n - shift[code], code the rounding m of the folded fractional
-// difference (in {-1, 0, 1}^3, the list scan's image code).  The rounding
-// is decided in FP32 from ihf (H^-1, 9 floats, column major; error ~1e-7
-// against the 1e-4 tie window); a component within 1e-4 of +-1/2 takes the
-// reference's image from the FP64 H^-1 ihg and the unfolded positions xr
-// (SoA, N per component), both in global memory, as tie_image does.  Only
-// 9 floats of the cell are read: this runs after both passes, where FP64
-// cell registers kept live would cost the hot loops registers.
-// Returns |d|^2.
-__device__ __forceinline__ double pair_image(const float *ihf, const double *ihg, const double *shift,
-                                             const double *px, const double *py, const double *pz,
-                                             const double *xr, int N, int k, int n, double d[3]) {
-    const double cx = px[k] - px[n], cy = py[k] - py[n], cz = pz[k] - pz[n];
+// One atom of a replica in LDS: position, G = dE/dsigma~ (pass B) and the first
+// accumulator word.  40 bytes, so that random atoms spread over all banks (32
+// would put every x on an eighth of them).
+struct PairRec {
+    double x, y, z, g;
+    unsigned long long w;
+};
+
+// Sums that do not depend on the order of their terms.  A term v is rounded to a
+// multiple of a power of two, the grid: t = v + C with C = 1.5 * 2^52 grids
+// leaves v / grid in t's mantissa, so t's bits less C's are the integer that a
+// 64-bit LDS atomic adds (C's low word is 0: one subtraction), and t - C is the
+// rounded term, whose sums in registers are exact in FP64 (multiples of the grid
+// below 2^53 of them).  Results are bitwise reproducible whatever order the
+// atomics land in, however a row of neighbours is cut into lanes and whichever
+// of its two atoms owns a pair.  (FP64 LDS atomics would save the subtraction, but
+// on random addresses they take 21 cycles a wavefront, 64-bit integer ones 11.)
+//   sigma: 2^-42 (|v| < 512) and 2^-88 for the rest;
+//   forces: 2^-43 eV/A (|v| < 256 eV/A).
+// Larger terms are converted by rint and added by themselves; those beyond 2^63
+// grids, and NaN, are flagged (MDT_ST_FIXED_OVERFLOW) and left out.
+// Energies are summed in registers: 2^-33 eV (sums below 1e6 eV) and 2^-70 for
+// the rest.
+#define MDT_SIG_C1 1536.0                         // 1.5 * 2^(52 - 42)
+#define MDT_SIG_C2 2.1827872842550278e-11         // 1.5 * 2^(52 - 88)
+#define MDT_SIG_FAST 511.0
+#define MDT_FRC_C 768.0                           // 1.5 * 2^(52 - 43)
+#define MDT_FRC_FAST 255.0
+#define MDT_EPR_C1 786432.0                       // 1.5 * 2^(52 - 33)
+#define MDT_EPR_C2 5.7220458984375e-06            // 1.5 * 2^(52 - 70)
+#define MDT_P42 4398046511104.0
+#define MDT_P43 8796093022208.0
+#define MDT_P46 70368744177664.0
+
+// Below this sigma~ (of the near pairs) the words' absolute step shows in a
+// relative sense, and the atom's force scales with sigma~ itself down to the
+// reference's 1e-30 clamp: its sigma~ is summed again over all partners as plain
+// FP64 terms, in an order that depends on the atoms alone.
+#define MDT_SIG_VTINY 2.3283064365386963e-10  // 2^-32
+
+#define MDT_ANY_IMAGE 31   // image code of a kept pair that may round either way
+#define MDT_FLAT_CAP 128   // listed near partners of one such atom (with more it tests every atom in both passes)
+
+// the integer of t = v + C (C's low word is 0)
+__device__ __forceinline__ unsigned long long grid_int(double t, double C) {
+    union {
+        double d;
+        struct {
+            uint32_t lo, hi;
+        } w;
+        unsigned long long u;
+    } a, c;
+    a.d = t;
+    c.d = C;
+    a.w.hi -= c.w.hi;
+    return a.u;
+}
+// v as an integer of grids (scale: grids per unit) and rounded, any size
+__device__ __forceinline__ unsigned long long grid_any(double v, double scale, double *r, int *bad) {
+    double y = rint(v * scale);
+    if (!(fabs(y) < 9.0e18)) {
+        *bad |= MDT_ST_FIXED_OVERFLOW;
+        y = 0.0;
+    }
+    *r = y / scale;
+    return (unsigned long long)(long long)y;
+}
+// the two words of a sigma term below MDT_SIG_FAST; *h, *l: the rounded parts
+__device__ __forceinline__ void sig_words(double v, unsigned long long *u1, unsigned long long *u2, double *h, double *l) {
+    const double t = v + MDT_SIG_C1;
+    *u1 = grid_int(t, MDT_SIG_C1);
+    *h = t - MDT_SIG_C1;
+    const double t2 = (v - *h) + MDT_SIG_C2;
+    *u2 = grid_int(t2, MDT_SIG_C2);
+    *l = t2 - MDT_SIG_C2;
+}
+// a sigma term from MDT_SIG_FAST on: its first word (step 2e-13) is enough;
+// adds it to *p and returns it rounded
+__device__ double sig_large(unsigned long long *p, double v, int *bad) {
+    double h;
+    const unsigned long long u = grid_any(v, MDT_P42, &h, bad);
+    atomicAdd(p, u);
+    return h;
+}
+__device__ __forceinline__ double sig_sum(unsigned long long w1, unsigned long long w2) {
+    return (double)(long long)w1 * (1.0 / MDT_P42) + (double)(long long)w2 * (1.0 / (MDT_P42 * MDT_P46));
+}
+__device__ __forceinline__ double frc_sum(unsigned long long w) { return (double)(long long)w * (1.0 / MDT_P43); }
+// LDS += a sum of rounded terms (a multiple of the grid)
+__device__ __forceinline__ void add_sum(unsigned long long *p, double v, double scale, int *bad) {
+    double r;
+    const unsigned long long u = grid_any(v, scale, &r, bad);
+    atomicAdd(p, u);
+}
+
+// Minimum image of the pair (k, n) of a replica staged in LDS (positions p,
+// fractional components in [-0.2, 1.2)): d = p_k - p_n - shift[code] (4 doubles a code), code
+// the rounding m of the fractional difference (in {-1, 0, 1}^3, the list
+// scan's image code).  The rounding is decided in FP32 from ihf (H^-1, 9
+// floats, column major; error ~1e-7 against the 1e-4 tie window); a component
+// within 1e-4 of +-1/2 takes the reference's image from the FP64 H^-1 ihg and
+// the unfolded positions xr (SoA, N per component), both in global memory, as
+// tie_image does.  Returns |d|^2.
+__device__ __forceinline__ double pair_image(const float *ihf, const double *ihg, const double *shift, const PairRec &pk,
+                                             const PairRec &pn, const double *xr, int N, int k, int n, double d[3],
+                                             int *codep) {
+    const double cx = pk.x - pn.x, cy = pk.y - pn.y, cz = pk.z - pn.z;
     const float ex = (float)cx, ey = (float)cy, ez = (float)cz;
     const float f0 = ihf[0] * ex + ihf[3] * ey + ihf[6] * ez;
     const float f1 = ihf[1] * ex + ihf[4] * ey + ihf[7] * ez;
     const float f2 = ihf[2] * ex + ihf[5] * ey + ihf[8] * ez;
     float m0 = rintf(f0), m1 = rintf(f1), m2 = rintf(f2);
-    const bool t0 = fabsf(fabsf(f0) - 0.5f) < 1e-4f, t1 = fabsf(fabsf(f1) - 0.5f) < 1e-4f,
-               t2 = fabsf(fabsf(f2) - 0.5f) < 1e-4f;
+    const bool t0 = fabsf(f0 - m0) > 0.4999f, t1 = fabsf(f1 - m1) > 0.4999f, t2 = fabsf(f2 - m2) > 0.4999f;
     if (t0 | t1 | t2) {  // rare: the exact fractional difference and the reference's tie rule
         const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
         const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
@@ -305,9 +409,10 @@ __device__ __forceinline__ double pair_image(const float *ihf, const double *ihg
         if (t2) m2 = (float)tie_image(ihg[2], ihg[5], ihg[8], a0, a1, a2, b0, b1, b2, ihg[2] * cx + ihg[5] * cy + ihg[8] * cz);
     }
     const int code = ((int)m0 + 1) + 3 * ((int)m1 + 1) + 9 * ((int)m2 + 1);
-    d[0] = cx - shift[3 * code];
-    d[1] = cy - shift[3 * code + 1];
-    d[2] = cz - shift[3 * code + 2];
+    d[0] = cx - shift[4 * code];
+    d[1] = cy - shift[4 * code + 1];
+    d[2] = cz - shift[4 * code + 2];
+    *codep = code;
     return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
 }
 
@@ -317,45 +422,52 @@ __device__ __forceinline__ double pair_image(const float *ihf, const double *ihg
 // strength-reduced into one induction register per array.
 __device__ __forceinline__ void opaque(int &v) { asm volatile("" : "+v"(v)); }
 
-// Sum of v over the block in a fixed order (butterfly within each wave, then
-// the waves in order through wsum[nthr / 64]); the result is valid in lane 0.
-// Every lane of the block must call it (it synchronises the block).
-__device__ __forceinline__ double block_sum_fixed(double v, double *wsum, int lane, int nthr) {
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((lane & 63) == 0) wsum[lane >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (lane == 0)
-        for (int w = 0; w < (nthr + 63) / 64; ++w) s += wsum[w];
-    __syncthreads();
-    return s;
+    return v;
 }
 
-// The same for four values at once (one pair of barriers); wsum holds 64.
-__device__ __forceinline__ void block_sum4_fixed(double v[4], double *wsum, int lane, int nthr) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
-    if ((lane & 63) == 0)
-        for (int q = 0; q < 4; ++q) wsum[4 * (lane >> 6) + q] = v[q];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        double s = 0.0;
-        if (lane == 0)
-            for (int w = 0; w < (nthr + 63) / 64; ++w) s += wsum[4 * w + q];
-        v[q] = s;
-    }
-    __syncthreads();
+// the same with v's sum over the wavefront (p the same in every lane: left to
+// itself the compiler adds such lanes up one by one)
+__device__ __forceinline__ void add_uniform(unsigned long long *p, double v, double scale, int *bad) {
+    if (__ballot(v != 0.0) == 0) return;  // the wavefront has none
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) add_sum(p, v, scale, bad);
 }
 
 // Pair ownership: each unordered pair is evaluated once, by its owner; the
 // owner alternates with index parity, which gives every atom about half of
-// its neighbours.  The 2^48 fixed point of the partner sigma sums bounds the
-// force error of an isolated atom (sigma ~ 1e-11, the s clamp region) by
-// ~1e-10 eV/A, since that atom's force scales with sigma itself.
+// its neighbours.
 __device__ __forceinline__ bool owns(int k, int n) { return (k < n) != (((k + n) & 1) != 0); }
 
+// calc_force for one replica per workgroup.
+//
+// What bounds it: with enough replicas the issue of vector instructions (about 60 %
+// of the cycles; 165 a pair and lane in both passes together) beside the LDS (45 %:
+// positions, exponential table, atomics), with few of them the latency of its
+// phases.  H/Au 6x6x4, 4096 replicas of 3 k near pairs: 180 us a step with the
+// propagator, 263 before rows were sorted pieces; H/Pt 8x8x6, 2048 replicas: 300 us
+// a launch, 494 before.
+//  * Rows.  The owned half lists hold the near pairs (r <= rnear) of the
+//    atoms of one EMT type, the majority (bv.bulk); their constants are
+//    uniform, so a pair needs no type.  A row is cut into equal pieces, one a
+//    lane, sorted by length, so that a wavefront's lanes end together; the
+//    pieces' sums meet in the order-free words.  The entries lie in HBM in the
+//    order the wavefronts read them, two a word, one word a lane and iteration
+//    (coalesced, and no LDS: a replica of 145 atoms takes 14 KB of it instead of 33).
+//  * Flat lists.  The few atoms of the other EMT type (at most
+//    MDT_FLAT_MAX: the projectile) get the list of their near partners at
+//    every launch, by a minimum-image test of every atom, one partner per lane
+//    in the passes.  They are the fast atoms, so the rows are kept while the
+//    slower ones move.  Universes with more of them (MIXED) hold every pair in
+//    rows and look the types up.
+//  * Kept rows.  They serve until an atom that is in them has moved half the
+//    skin.  Positions stay unfolded (fractional components in [-0.2, 1.2);
+//    others are folded by the fold of the build), so an entry's image code stays
+//    what it was at the build: a launch only reads them.
+//  * The pair terms of two entries are evaluated without a branch between them, so
+//    that one's chain of dependent instructions fills the other's gaps.
 // PREC (arithmetic of the pair terms):
 //   0: FP64 throughout;
 //   1: the cut-off function, the sigma and pair-potential exponentials and
@@ -366,422 +478,466 @@ __device__ __forceinline__ bool owns(int k, int n) { return (k < n) != (((k + n)
 //      1e-5 eV/A, e.g. Pt with V0 = 21.7 eV).
 // In every mode the geometry (differences, r, the exponent arguments
 // r - rcut and r - beta s0, which carry factors up to acut ~ 26/A), the
-// per-atom embedding terms, G and every accumulation stay FP64 / fixed point.
+// per-atom embedding terms, G and every accumulation stay FP64.
 // JUDGE: FP64 EMT forces of the selected replicas compared with
 // bv.judge_f (the network's judge); nothing else is written.
 // MAXB: the largest workgroup of the instantiation, 512, or 1024 for size
 // classes of more than 512 atoms x threads per atom, whose few replicas
 // would otherwise leave each CU two waves per SIMD.
-template <int TPA, bool NBR_LDS, int PREC, bool JUDGE, int MAXB = 512>
+template <bool MIXED, int PREC, bool JUDGE, int MAXB>
 __global__ void __launch_bounds__(MAXB, 4)
     k_replica(const EmtConst *__restrict__ ecg, const PropConst *__restrict__ pcg, BatchView bv, int add_fin) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ LdsTables T;
+    __shared__ LdsTypes T;
+    __shared__ double s_sh[27 * 4];  // lattice translations of the image codes, 32 bytes each
+    __shared__ double s_cell[18];    // H, H^-1
+    __shared__ float s_ihf[9];       // H^-1 in FP32
+    __shared__ double s_ep[2];       // energy words: pair energies - 2 (atoms' energies)
+    __shared__ int s_flat[MDT_FLAT_MAX], s_fcnt[MDT_FLAT_MAX];
+    __shared__ uint16_t s_flist[MIXED ? 1 : MDT_FLAT_MAX * MDT_FLAT_CAP];
+    __shared__ int s_np[64], s_hist[64];  // pieces at each length limit, of each length
+    __shared__ int s_cb[64];              // stream offset of each chunk of 64 pieces
+    __shared__ int s_nflat, s_R, s_slow, s_anyfold;
     const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : (int)blockIdx.x;
-    if (bv.only && !bv.only[rep]) return;                                          // whole block: uniform
-    if (bv.skip && bv.skip[rep]) return;                                           // whole block: uniform
-    if (JUDGE && (rep % bv.judge_mod) != bv.judge_phase) return;                  // whole block: uniform
+    if (bv.only && !bv.only[rep]) return;                          // whole block: uniform
+    if (bv.skip && bv.skip[rep]) return;                           // whole block: uniform
+    if (JUDGE && (rep % bv.judge_mod) != bv.judge_phase) return;   // whole block: uniform
     const int t = bv.rep_traj[rep];
-    const int traj = t;
     if (bv.done && bv.done[t]) return;  // frozen trajectory (whole block: uniform)
     const int b = bv.rep_bead[rep];
     const int N = bv.traj_N[t];
-    const int cap = bv.nbcap < N - 1 ? bv.nbcap : (N > 1 ? N - 1 : 1);
+    const int cap = bv.nbcap < N - 1 ? bv.nbcap : (N > 1 ? N - 1 : 1);  // entries per row
+    const int capg = (bv.nbcap + 7) & ~7;                               // stride of the rows in HBM
     const long long soff = bv.traj_soff[t];
     const long long roff = soff + (long long)b * 3 * N;  // x block of this replica
     const long long doff = soff / 3 + (long long)b * N;   // dens / fixed block
     const long long aoff = bv.traj_aoff[t];
-    const uint32_t tid = bv.traj_id[t];
-    const double tsurf = bv.tsurf[t], tproj = bv.tproj[t];
+    const double *xr = bv.x + roff;
     const int nthr = blockDim.x;
-    const int lane = threadIdx.x;
-    CellRegs cell;
-    load_cell(bv, t, cell);
-    load_tables(T, ecg, pcg, cell, lane, nthr);
+    const int lane = threadIdx.x, wl = lane & 63, wave = lane >> 6, nwaves = nthr >> 6;
+    const int bulk = bv.bulk;
+    load_types(T, ecg, lane, nthr);
+    load_exptab(T, lane, nthr);
+    if (lane < 18) s_cell[lane] = lane < 9 ? bv.cell[9 * t + lane] : bv.icell[9 * t + lane - 9];
+    if (lane < 27) {
+        const double m0 = (double)(lane % 3 - 1), m1 = (double)((lane / 3) % 3 - 1), m2 = (double)(lane / 9 - 1);
+        const double *h = bv.cell + 9 * t;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) s_sh[4 * lane + q] = h[q] * m0 + h[q + 3] * m1 + h[q + 6] * m2;
+    }
+    const double *s_h = s_cell, *s_ih = s_cell + 9;
 
-    // LDS: px py pz | three words A0 A1 A2 | G | E | cnt | nbr | typ | tiny,
-    // where the words hold the fractional coordinates in the scan, the sigma
-    // fixed point (hi, mid, lo) in pass A and the force fixed point (x, y, z)
-    // in pass B.  The lists hold the near pairs (r <= rnear; rnear + skin for
-    // kept lists); the pairs beyond rnear with a tiny atom come from a direct
-    // minimum-image scan of that atom's partners (pair_image).
-    double *px = (double *)smem_raw;
-    double *py = px + N, *pz = py + N;
-    double *sx = pz + N, *sy = sx + N, *sz = sy + N;
-    unsigned long long *shi = (unsigned long long *)sx, *smid = (unsigned long long *)sy;
-    unsigned long long *slo = (unsigned long long *)sz;
-    unsigned long long *fxa = shi, *fya = smid, *fza = slo;
-    double *G = sz + N, *E = G + N;
-    uint16_t *cnt = (uint16_t *)(E + N);
-    uint16_t *nbr = NBR_LDS ? cnt + N : bv.nbr_global + (size_t)blockIdx.x * bv.nbr_stride;
-    // kept lists staged in LDS: their copy between launches
-    uint16_t *nbr_kept = (NBR_LDS && bv.rl_stage) ? bv.nbr_global + (size_t)blockIdx.x * bv.nbr_stride : nbr;
-    uint8_t *typ = (uint8_t *)(cnt + N + (NBR_LDS ? (size_t)N * cap : 0));
+    // LDS: words W2, W3 | records | typ | tiny.  sigma takes two words (record
+    // and W2), forces all three.  W2 and W3 hold the scan's FP32 coordinates.
+    unsigned long long *w2 = (unsigned long long *)smem_raw, *w3 = w2 + N;
+    PairRec *rec = (PairRec *)(w3 + N);
+    uint8_t *typ = (uint8_t *)(rec + N);
     uint8_t *tiny = typ + N;
-    __shared__ int s_anytiny;
-    __shared__ double s_wsum[64];
-    __shared__ float s_ihf[9];  // H^-1 in FP32 for the scan of the tiny atoms' partners
-    if (lane < 9) s_ihf[lane] = (float)bv.icell[9 * t + lane];
+    // HBM, per block slot: the stream of pieces, the piece table (atom | length
+    // << 11), the chunks' offsets in the stream; rows as scanned (those of batches
+    // too small to fill the GPU in LDS: mdt_replica_lists)
+    uint32_t *stream = bv.rl_lists + (long long)blockIdx.x * bv.rl_stride;
+    uint32_t *rows = stream + bv.rl_rows, *chunk = stream + bv.rl_chunk;
+    uint16_t *scan_rows = bv.rl_scan < 0 ? (uint16_t *)(smem_raw + ((58 * N + 7) & ~7)) : (uint16_t *)(stream + bv.rl_scan);
     int bad_local = 0;
-    // Verlet skin (lists in HBM): the lists of this block slot are built with
-    // rnear + skin and kept while no atom moved more than skin / 2 since the
-    // build; a kept list gets every entry's image recomputed from the current
-    // positions (the same rounding and tie rule as the scan).  Only in cells
-    // whose narrowest width exceeds 2 (rnear + skin): there every image
-    // within rnear + skin has fractional components in (-1/2, 1/2), so it is
-    // the rounded image the scan tests, and a pair within rnear now was
-    // listed at the build in that same image.  In narrower cells the rounded
-    // image need not be the nearest, and the lists are rebuilt at every
-    // launch.  (The pairs beyond rnear never come from a list.)
-    const double skin = bv.rl_skin;
-    double wmin = 1e300;
-    for (int q = 0; q < 3; ++q) {
-        const double w = 1.0 / sqrt(cell.ih[q] * cell.ih[q] + cell.ih[q + 3] * cell.ih[q + 3] +
-                                    cell.ih[q + 6] * cell.ih[q + 6]);
-        wmin = w < wmin ? w : wmin;
+
+    // Verlet skin: the rows of this block slot are built with rnear + skin and
+    // kept while no atom in them moved more than skin / 2 since.  A pair's
+    // rounded image is then the build's, unless a fractional component of
+    // the difference lay within skin / width of +-1/2 at the build: such a pair is
+    // listed if any image it can round to lies within rnear + skin, with
+    // the code MDT_ANY_IMAGE, and takes its image at every launch from the
+    // current positions.  (The pairs beyond rnear never come from a row.)
+    const double skin = bv.rl_skin, rnear = ecg->rnear, cutr = ecg->cutr;
+    int2 *valid = bv.rl_valid ? bv.rl_valid + blockIdx.x : nullptr;
+    // x: 0, or 1 | fold << 1 | slow << 2 | row pieces << 3; y: the EMT constants' generation
+    const int kept = valid && valid->y == ecg->gen ? valid->x : 0;
+    bool keep = valid != nullptr;
+    if (keep && !kept) {
+        const double *ih = bv.icell + 9 * t;
+        const double b0 = sqrt(ih[0] * ih[0] + ih[3] * ih[3] + ih[6] * ih[6]) * skin;
+        const double b1 = sqrt(ih[1] * ih[1] + ih[4] * ih[4] + ih[7] * ih[7]) * skin;
+        const double b2 = sqrt(ih[2] * ih[2] + ih[5] * ih[5] + ih[8] * ih[8]) * skin;
+        keep = b0 < 0.05 && b1 < 0.05 && b2 < 0.05;
     }
-    const double rnear = ecg->rnear;
-    const bool keep = (!NBR_LDS || bv.rl_stage) && bv.rl_valid != nullptr && 2.0 * (rnear + skin) < wmin;
     double *ref = keep ? bv.rl_ref + (long long)blockIdx.x * 3 * bv.rl_ns : nullptr;
-    __shared__ int s_reuse;
-    if (lane == 0) s_reuse = keep && bv.rl_valid[blockIdx.x];
-    __syncthreads();
-    if (s_reuse) {  // every thread reads the flag before any clears it
-        double dmax = 0.0;
-        for (int i = lane; i < N; i += nthr) {
-            const double d0 = bv.x[roff + i] - ref[i], d1 = bv.x[roff + N + i] - ref[bv.rl_ns + i],
-                         d2 = bv.x[roff + 2 * N + i] - ref[2 * bv.rl_ns + i];
-            const double d2s = d0 * d0 + d1 * d1 + d2 * d2;
-            dmax = d2s > dmax ? d2s : dmax;
-        }
-        __syncthreads();
-        if (!(dmax <= 0.25 * skin * skin)) s_reuse = 0;  // benign race: every writer stores 0
-    }
-    __syncthreads();
-    const bool reuse = s_reuse != 0;
 
     // ---- phase 0: stage ----
+    if (lane < 9) s_ihf[lane] = (float)bv.icell[9 * t + lane];
+    if (lane < 64) {
+        s_np[lane] = s_hist[lane] = 0;
+        s_cb[lane] = kept && lane < ((kept >> 3) + 63) / 64 ? chunk[lane] : 0;
+    }
+    if (lane == 0) {
+        s_nflat = 0;
+        s_anyfold = 0;
+        s_slow = kept >> 2 & 1;
+        s_R = kept >> 3;
+        s_ep[0] = s_ep[1] = 0.0;
+    }
+    // loads that the passes and the output wait for otherwise: the lane's first
+    // piece, its atom's mass and fixed bits
+    uint32_t info0 = 0, word0 = 0;
+    int off0 = 0;
+    if (kept && lane < kept >> 3) {
+        info0 = rows[lane];
+        off0 = chunk[wave];
+    }
+    double mass0 = 1.0;
+    int fixed0 = 0;
+    if (!JUDGE && lane < N) {
+        mass0 = bv.mass[aoff + lane];
+        fixed0 = bv.fixed[doff + lane];
+    }
+    __syncthreads();  // s_nflat
+    // An atom whose fractional position leaves [-0.2, 1.2) is folded into the
+    // cell; an atom in kept rows as at their build (there, for a fold of zero,
+    // nothing is looked at: kept & 2 tells whether any was not).
+    auto fold = [&](double &x, double &y, double &z, double rx, double ry, double rz, float4 *f) {
+        const double f0 = s_ih[0] * rx + s_ih[3] * ry + s_ih[6] * rz;
+        const double f1 = s_ih[1] * rx + s_ih[4] * ry + s_ih[7] * rz;
+        const double f2 = s_ih[2] * rx + s_ih[5] * ry + s_ih[8] * rz;
+        const double g0 = (f0 >= -0.2 && f0 < 1.2) ? 0.0 : floor(f0);
+        const double g1 = (f1 >= -0.2 && f1 < 1.2) ? 0.0 : floor(f1);
+        const double g2 = (f2 >= -0.2 && f2 < 1.2) ? 0.0 : floor(f2);
+        if (f) *f = make_float4((float)(f0 - g0), (float)(f1 - g1), (float)(f2 - g2), 0.f);
+        if (g0 == 0.0 && g1 == 0.0 && g2 == 0.0) return false;
+        x -= s_h[0] * g0 + s_h[3] * g1 + s_h[6] * g2;
+        y -= s_h[1] * g0 + s_h[4] * g1 + s_h[7] * g2;
+        z -= s_h[2] * g0 + s_h[5] * g1 + s_h[8] * g2;
+        return true;
+    };
+    int moved = 0;
     for (int i = lane; i < N; i += nthr) {
         const int ty = bv.type[aoff + i];
         typ[i] = (uint8_t)ty;
-        const double r[3] = {bv.x[roff + i], bv.x[roff + N + i], bv.x[roff + 2 * N + i]};
-        if (keep && !reuse) {
-            ref[i] = r[0];
-            ref[bv.rl_ns + i] = r[1];
-            ref[2 * bv.rl_ns + i] = r[2];
+        double x = xr[i], y = xr[N + i], z = xr[2 * N + i];
+        const bool rowed = MIXED || ty == bulk;
+        if (kept && rowed) {
+            const double rx = ref[i], ry = ref[bv.rl_ns + i], rz = ref[2 * bv.rl_ns + i];
+            const double d0 = x - rx, d1 = y - ry, d2 = z - rz;
+            if (!(d0 * d0 + d1 * d1 + d2 * d2 <= 0.25 * skin * skin)) moved = 1;
+            if (kept & 2) fold(x, y, z, rx, ry, rz, nullptr);
+        } else if (!rowed) {
+            fold(x, y, z, x, y, z, nullptr);
+            if (T.owner[ty]) {
+                const int q = atomicAdd(&s_nflat, 1);  // the order is free
+                if (q < MDT_FLAT_MAX) {
+                    s_flat[q] = i;
+                    s_fcnt[q] = 0;
+                }
+            }
         }
-        // fold into the cell: fractional in [0, 1)
-        double f0 = cell.ih[0] * r[0] + cell.ih[3] * r[1] + cell.ih[6] * r[2];
-        double f1 = cell.ih[1] * r[0] + cell.ih[4] * r[1] + cell.ih[7] * r[2];
-        double f2 = cell.ih[2] * r[0] + cell.ih[5] * r[1] + cell.ih[8] * r[2];
-        f0 -= floor(f0);
-        f1 -= floor(f1);
-        f2 -= floor(f2);
-        sx[i] = f0;
-        sy[i] = f1;
-        sz[i] = f2;
-        px[i] = cell.h[0] * f0 + cell.h[3] * f1 + cell.h[6] * f2;
-        py[i] = cell.h[1] * f0 + cell.h[4] * f1 + cell.h[7] * f2;
-        pz[i] = cell.h[2] * f0 + cell.h[5] * f1 + cell.h[8] * f2;
+        rec[i].x = x;
+        rec[i].y = y;
+        rec[i].z = z;
+        rec[i].g = 0.0;
+        rec[i].w = w2[i] = w3[i] = 0;
     }
-    __syncthreads();
-    const double acut = ecg->acut, rcut = ecg->rcut, cutr = ecg->cutr, cut2 = ecg->cut2hi;
-    const float acutf = (float)acut, acutl2f = (float)(acut * MDT_LOG2E);
-    const int apb = nthr / TPA;  // atoms per chunk
-    const int wl = lane & 63;
-    const unsigned long long gmask = (TPA >= 64 ? ~0ull : ((1ull << TPA) - 1ull)) << ((wl / TPA) * TPA);
+    if (kept && lane < kept >> 3) word0 = stream[off0 + wl];
+    const bool reuse = !__syncthreads_or(moved) && kept;
     const unsigned long long below = (wl == 0) ? 0ull : ((~0ull) >> (64 - wl));
 
-    // ---- phase 1: owned half neighbour lists (min image, ordered by index) ----
-    // The scan only decides membership: it runs in FP32 on float copies of
-    // the fractional coordinates (in the G/E words, unused until pass A) with
-    // r^2 bound widened by 1e-4 relative; both passes re-check r <= cutr in
-    // FP64.  A fractional difference within 1e-4 of +-1/2 takes its image
-    // from the FP64 rounding, so the chosen image is the FP64 minimum image.
-    // fractional coordinates and type per atom as one float4 (16 B: the G
-    // and E words, 2N doubles); squared distances from the metric H^T H
-    float4 *f4 = (float4 *)G;
-    for (int i = lane; i < N; i += nthr)
-        f4[i] = make_float4((float)sx[i], (float)sy[i], (float)sz[i], __int_as_float((int)typ[i]));
-    int all_on = 1;
-    for (int q = 0; q < ecg->ntypes * ecg->ntypes; ++q)
-        if (!T.pair_on[(q / ecg->ntypes) * MDT_MAXT + q % ecg->ntypes]) all_on = 0;
-    __syncthreads();
-    float g00, g11, g22, g01, g02, g12;  // H^T H, cell vectors = columns of H
-    {
-        const double *h = cell.h;
-        g00 = (float)(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]);
-        g11 = (float)(h[3] * h[3] + h[4] * h[4] + h[5] * h[5]);
-        g22 = (float)(h[6] * h[6] + h[7] * h[7] + h[8] * h[8]);
-        g01 = (float)(2 * (h[0] * h[3] + h[1] * h[4] + h[2] * h[5]));
-        g02 = (float)(2 * (h[0] * h[6] + h[1] * h[7] + h[2] * h[8]));
-        g12 = (float)(2 * (h[3] * h[6] + h[4] * h[7] + h[5] * h[8]));
-    }
-    // the lists hold the near pairs; a kept list is built with rnear + skin,
-    // so a pair now within rnear was listed at the build.  Staged kept lists
-    // (the rows in HBM, a copy in LDS during the launch) hold the whole
-    // rnear + skin rows in HBM and only the entries now within rnear (the
-    // FP32 bound of a build without skin) in LDS, in the same order: the
-    // passes then see the entries of a list built at this launch.
-    const double rn = keep ? rnear + skin : rnear;
-    const float cut2f = (float)(rn * rn * (1.0 + 1e-4));
-    const float near2f = (float)(rnear * rnear * (1.0 + 1e-4));
-    const bool split = NBR_LDS && keep;
-    uint16_t *kcnt = keep ? bv.rl_cnt + (long long)blockIdx.x * bv.rl_ns : nullptr;
-    if (reuse) {  // kept list: the image of every entry from the current positions
+    // ---- phase 1: rows ----
+    // few workgroups and rows for this launch only: they are read where the scan
+    // put them, in LDS, tpa lanes per row (cutting and sorting them costs 6 us)
+    const bool direct = !keep && bv.rl_scan < 0;
+    const int sh = bv.tpa_shift;
+    if (!reuse) {
+        if (lane == 0) s_slow = 0;
+        float4 *f4 = (float4 *)w2;  // fractional coordinates and type
+        for (int i = lane; i < N; i += nthr) {
+            const int ty = typ[i];
+            double x = xr[i], y = xr[N + i], z = xr[2 * N + i];
+            if (keep) {
+                ref[i] = x;
+                ref[bv.rl_ns + i] = y;
+                ref[2 * bv.rl_ns + i] = z;
+            }
+            float4 f;
+            const bool folded = fold(x, y, z, x, y, z, &f);
+            if (!(fabsf(f.x) + fabsf(f.y) + fabsf(f.z) < 1e30f)) bad_local |= MDT_ST_FIXED_OVERFLOW;
+            f.w = __int_as_float(ty);
+            rec[i].x = x;
+            rec[i].y = y;
+            rec[i].z = z;
+            f4[i] = f;
+            if (folded && (MIXED || ty == bulk)) s_anyfold = 1;  // benign race: every writer stores 1
+        }
+        __syncthreads();
+        // The scan only decides membership: FP32 fractional differences, r^2
+        // from the cell metric H^T H with the bound widened by 1e-4; the
+        // passes test r <= rnear in FP64.  A fractional difference within
+        // 1e-4 of +-1/2 takes its image from the reference's expression (in rows
+        // that are kept: MDT_ANY_IMAGE).
+        // tpa lanes per atom; only the owned candidates are visited, in
+        // increasing index: below k those of the other parity (a = (k + 1) / 2
+        // of them), above k those of the same parity.
+        // row lengths go to the record's word
+        float g00, g11, g22, g01, g02, g12;  // H^T H, cell vectors = columns of H
+        {
+            const double *h = bv.cell + 9 * t;
+            g00 = (float)(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]);
+            g11 = (float)(h[3] * h[3] + h[4] * h[4] + h[5] * h[5]);
+            g22 = (float)(h[6] * h[6] + h[7] * h[7] + h[8] * h[8]);
+            g01 = (float)(2 * (h[0] * h[3] + h[1] * h[4] + h[2] * h[5]));
+            g02 = (float)(2 * (h[0] * h[6] + h[1] * h[7] + h[2] * h[8]));
+            g12 = (float)(2 * (h[3] * h[6] + h[4] * h[7] + h[5] * h[8]));
+        }
+        float mg0 = 0.4999f, mg1 = 0.4999f, mg2 = 0.4999f;  // components beyond these can round either way
+        if (keep) {
+            const double *ih = bv.icell + 9 * t;
+            mg0 -= (float)(sqrt(ih[0] * ih[0] + ih[3] * ih[3] + ih[6] * ih[6]) * skin);
+            mg1 -= (float)(sqrt(ih[1] * ih[1] + ih[4] * ih[4] + ih[7] * ih[7]) * skin);
+            mg2 -= (float)(sqrt(ih[2] * ih[2] + ih[5] * ih[5] + ih[8] * ih[8]) * skin);
+        }
+        int all_on = 1;
+        if (MIXED) {
+            for (int q = 0; q < ecg->ntypes * ecg->ntypes; ++q)
+                if (!T.pair_on[(q / ecg->ntypes) * MDT_MAXT + q % ecg->ntypes]) all_on = 0;
+        } else {
+            all_on = T.pair_on[bulk * MDT_MAXT + bulk];
+        }
+        const double rn = keep ? rnear + skin : rnear;
+        const float cut2f = (float)(rn * rn * (1.0 + 1e-4));
+        const int tpa = 1 << sh, apb = nthr >> sh;
+        const unsigned long long gmask = ((1ull << tpa) - 1ull) << ((wl >> sh) << sh);
+        const int mmax = N / 2 + 1;
+        const int sub = lane & (tpa - 1);
         for (int k0 = 0; k0 < N; k0 += apb) {
-            const int k = k0 + lane / TPA;
-            const int sub = lane % TPA;
-            if (k >= N) continue;
-            const int c = kcnt[k];
-            const float4 pk = f4[k];
-            int cn = 0;  // staged: near entries so far
-            for (int e0 = 0; e0 < c; e0 += TPA) {  // the same trip count in the atom's lanes
-                const int e = e0 + sub;
-                bool near = false;
-                uint16_t ent = 0;
-                if (e < c) {
-                    const unsigned q = nbr_kept[(size_t)k * cap + e];
-                    const int n = q & MDT_NBR_IDX_MASK;
+            const int k = k0 + (lane >> sh);
+            const int tk = k < N ? typ[k] : 0;
+            const bool act = k < N && (MIXED || (tk == bulk && all_on));
+            const float4 pk = act ? f4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const int a_lo = (k + 1) >> 1;
+            int c = 0;
+            for (int m0 = 0; m0 < mmax; m0 += tpa) {
+                const int mi = m0 + sub;
+                const int n = mi < a_lo ? ((k + 1) & 1) + 2 * mi : k + 2 + 2 * (mi - a_lo);
+                bool in = false;
+                int code = 0;
+                if (act && n < N) {
                     const float4 pn = f4[n];
-                    const float e0f = pk.x - pn.x, e1f = pk.y - pn.y, e2f = pk.z - pn.z;
-                    float m0f = rintf(e0f), m1f = rintf(e1f), m2f = rintf(e2f);
-                    const bool t0 = fabsf(e0f - m0f) > 0.4999f, t1 = fabsf(e1f - m1f) > 0.4999f,
-                               t2 = fabsf(e2f - m2f) > 0.4999f;
-                    if (t0 | t1 | t2) {
-                        const double *xr = bv.x + roff;
-                        const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
-                        const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
-                        if (t0) m0f = (float)tie_image(cell.ih[0], cell.ih[3], cell.ih[6], a0, a1, a2, b0, b1, b2, sx[k] - sx[n]);
-                        if (t1) m1f = (float)tie_image(cell.ih[1], cell.ih[4], cell.ih[7], a0, a1, a2, b0, b1, b2, sy[k] - sy[n]);
-                        if (t2) m2f = (float)tie_image(cell.ih[2], cell.ih[5], cell.ih[8], a0, a1, a2, b0, b1, b2, sz[k] - sz[n]);
+                    const int tn = __float_as_int(pn.w);
+                    if (MIXED ? (all_on || T.pair_on[tk * MDT_MAXT + tn]) : tn == bulk) {
+                        const float e0 = pk.x - pn.x, e1 = pk.y - pn.y, e2 = pk.z - pn.z;
+                        float m0f = rintf(e0), m1f = rintf(e1), m2f = rintf(e2);
+                        float d0 = e0 - m0f, d1 = e1 - m1f, d2 = e2 - m2f;
+                        const bool t0 = fabsf(d0) > mg0, t1 = fabsf(d1) > mg1, t2 = fabsf(d2) > mg2;
+                        const bool tie = t0 | t1 | t2;
+                        if (tie && !keep) {
+                            const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
+                            const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
+                            const double cx = rec[k].x - rec[n].x, cy = rec[k].y - rec[n].y, cz = rec[k].z - rec[n].z;
+                            const double *ih = s_ih;
+                            if (t0) m0f = (float)tie_image(ih[0], ih[3], ih[6], a0, a1, a2, b0, b1, b2, ih[0] * cx + ih[3] * cy + ih[6] * cz);
+                            if (t1) m1f = (float)tie_image(ih[1], ih[4], ih[7], a0, a1, a2, b0, b1, b2, ih[1] * cx + ih[4] * cy + ih[7] * cz);
+                            if (t2) m2f = (float)tie_image(ih[2], ih[5], ih[8], a0, a1, a2, b0, b1, b2, ih[2] * cx + ih[5] * cy + ih[8] * cz);
+                            d0 = e0 - m0f;
+                            d1 = e1 - m1f;
+                            d2 = e2 - m2f;
+                        }
+                        auto metric = [&](float d0, float d1, float d2) {
+                            return d0 * (g00 * d0 + g01 * d1 + g02 * d2) + d1 * (g11 * d1 + g12 * d2) + g22 * d2 * d2;
+                        };
+                        float r2 = metric(d0, d1, d2);
+                        code = ((int)m0f + 1) + 3 * ((int)m1f + 1) + 9 * ((int)m2f + 1);
+                        if (tie && keep) {
+                            code = MDT_ANY_IMAGE;
+                            for (int q = 1; q < 8; ++q)
+                                r2 = fminf(r2, metric(d0 - (t0 && (q & 1) ? copysignf(1.f, d0) : 0.f),
+                                                      d1 - (t1 && (q & 2) ? copysignf(1.f, d1) : 0.f),
+                                                      d2 - (t2 && (q & 4) ? copysignf(1.f, d2) : 0.f)));
+                        }
+                        in = r2 <= cut2f;
                     }
-                    const int code = ((int)m0f + 1) + 3 * ((int)m1f + 1) + 9 * ((int)m2f + 1);
-                    ent = (uint16_t)(n | (code << MDT_NBR_IDX_BITS));
-                    if (split) {
-                        const float d0 = e0f - m0f, d1 = e1f - m1f, d2 = e2f - m2f;
-                        const float r2 =
-                            d0 * (g00 * d0 + g01 * d1 + g02 * d2) + d1 * (g11 * d1 + g12 * d2) + g22 * d2 * d2;
-                        near = r2 <= near2f;
+                }
+                const unsigned long long m = __ballot(in) & gmask;
+                if (in) {
+                    const int pos = c + __popcll(m & below);
+                    const uint16_t ent = (uint16_t)(n | (code << MDT_NBR_IDX_BITS));
+                    if (pos >= cap) {
+                        bad_local |= MDT_ST_NBR_OVERFLOW;
                     } else {
-                        nbr[(size_t)k * cap + e] = ent;  // the rows in HBM: the image in place
+                        scan_rows[(size_t)k * capg + pos] = ent;
+                        if (code == MDT_ANY_IMAGE) s_slow = 1;  // benign race: every writer stores 1
                     }
                 }
-                if (split) {
-                    const unsigned long long m = __ballot(near) & gmask;
-                    if (near) nbr[(size_t)k * cap + cn + __popcll(m & below)] = ent;
-                    cn += __popcll(m);
-                }
+                c += __popcll(m);
             }
-            if (sub == 0) cnt[k] = (uint16_t)(split ? cn : c);
+            c = c < cap ? c : cap;
+            if (direct) {
+                const uint32_t info = k < N ? (uint32_t)(k | ((c - sub + tpa - 1) >> sh) << MDT_NBR_IDX_BITS) : 0u;
+                if (k < N) rows[(k << sh) + sub] = info;
+                if (k0 == 0) info0 = info;
+            } else if (k < N && sub == 0) {
+                rec[k].w = c;
+            }
+        }
+        __syncthreads();
+        if (direct) {
+            if (lane == 0) s_R = N << sh;
+        } else {
+        // Row table: rows in equal pieces of at most L, the shortest L that gives
+        // at most `lim` pieces -- one per lane, or two where that leaves less
+        // than a quarter of the lanes to split with --, in order of length, so that
+        // a wavefront's lanes have the same (145 atoms on 192 lanes: 57 wavefront
+        // iterations for 49 full ones' worth of pairs, 72 unsorted).
+        {
+            const int magic = 65536 / (wl + 2) + 1;  // x / (wl + 2) for x < 256
+            int np = 0;
+            for (int k = wave; k < N; k += nwaves) {
+                const int c = (int)rec[k].w;
+                np += c > 190 ? 0x10000 : ((c + wl + 1) * magic) >> 16;
+            }
+            atomicAdd(&s_np[wl], np);
+        }
+        __syncthreads();
+        // (few workgroups: the last wavefront is left to the flat lists)
+        const int lim0 = (N + nthr / 4 + nthr - 1) / nthr * nthr - (bv.rl_scan < 0 && nwaves > 3 ? 64 : 0);
+        const int lim = lim0 < N + nthr ? lim0 : N + nthr;
+        const unsigned long long fit = __ballot(s_np[wl] <= lim);
+        const int L = fit ? __builtin_ctzll(fit) + 2 : 4096;  // none fits: one piece per row
+        // pieces of atom k: m of length l + 1 after ns - m of length l
+        auto cut = [&](int k, int &ns, int &l, int &m) {
+            const int c = (int)rec[k].w;
+            ns = (c + L - 1) / L;
+            l = ns ? c / ns : 0;
+            m = c - l * ns;
+        };
+        for (int k = lane; k < N; k += nthr) {
+            int ns, l, m;
+            cut(k, ns, l, m);
+            if (m) atomicAdd(&s_hist[l + 1 < 63 ? l + 1 : 63], m);
+            if (ns > m) atomicAdd(&s_hist[l < 63 ? l : 63], ns - m);
+        }
+        __syncthreads();
+        int off = s_hist[wl];  // pieces of this length or longer
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_down(off, o, 64);
+            if (wl + o < 64) off += y;
+        }
+        if (lane == 0) s_R = off;
+        const int np = s_hist[wl];
+        off -= np;
+        __syncthreads();
+        if (wave == 0) {
+            s_hist[wl] = off;
+            // chunks that start among the pieces of this length: their stream words
+            const int len = wl < 63 ? wl : fit ? L : cap;
+            for (int c = (off + 63) >> 6; 64 * c < off + np; ++c) s_cb[c] = 64 * ((len + 1) >> 1);
+        }
+        __syncthreads();
+        if (wave == 0) {  // offsets
+            int v = s_cb[wl];
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(v, o, 64);
+                if (wl >= o) v += y;
+            }
+            s_cb[wl] = v - s_cb[wl];
+        }
+        __syncthreads();
+        // tpa lanes per atom again, a piece each: the table and, two entries a
+        // word, a word per lane and row of the chunk, the stream
+        for (int k0 = 0; k0 < N; k0 += apb) {
+            const int k = k0 + (lane >> sh);
+            if (k >= N) continue;
+            int ns, l, m;
+            cut(k, ns, l, m);
+            for (int j = sub; j < ns; j += tpa) {
+                const int len = l + (j >= ns - m ? 1 : 0);
+                const int st = j * l + (j > ns - m ? j - (ns - m) : 0);
+                const int p = atomicAdd(&s_hist[len < 63 ? len : 63], 1);  // the order is free
+                rows[p] = (uint32_t)(k | len << MDT_NBR_IDX_BITS);
+                const uint16_t *src = scan_rows + (size_t)k * capg + st;
+                uint32_t *dst = stream + s_cb[p >> 6] + (p & 63);
+                for (int e = 0; e < len; e += 2)
+                    dst[32 * e] = src[e] | (uint32_t)src[e + 1 < len ? e + 1 : e] << 16;
+            }
+        }
+        }
+        __syncthreads();
+        for (int i = lane; i < N; i += nthr) rec[i].w = w2[i] = w3[i] = 0;
+        if (keep) {
+            if (lane < (s_R + 63) / 64) chunk[lane] = s_cb[lane];
+            if (lane == 0)  // read by the next launch
+                *valid = make_int2(1 | (s_anyfold ? 2 : 0) | (s_slow ? 4 : 0) | s_R << 3, ecg->gen);
         }
     }
-    // only the owned candidates are visited, in increasing index: below k
-    // those of the other parity (a = (k + 1) / 2 of them), above k those of
-    // the same parity -- owns(k, n) of every n, without the half of the
-    // lanes that would test and drop the others
-    const int mmax = N / 2 + 1;
-    for (int k0 = 0; k0 < (reuse ? 0 : N); k0 += apb) {
-        const int k = k0 + lane / TPA;
-        const int sub = lane % TPA;
-        const bool act = k < N;
-        const int tk = act ? typ[k] : 0;
-        const float4 pk = act ? f4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-        const int a_lo = (k + 1) >> 1;
-        int c = 0, cn = 0;
-        for (int m0 = 0; m0 < mmax; m0 += TPA) {
-            const int mi = m0 + sub;
-            const int n = mi < a_lo ? ((k + 1) & 1) + 2 * mi : k + 2 + 2 * (mi - a_lo);
-            bool in = false, near = false;
+    // ---- flat lists: the near partners of the atoms outside the majority type ----
+    // (two of those atoms with each other: listed at the lower index)
+    auto flat_pair = [&](int h, int n, double d[3], double &r2, int &code) {
+        if (n == h || !T.pair_on[typ[h] * MDT_MAXT + typ[n]] || (typ[n] != bulk && n < h)) return false;
+        r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[h], rec[n], xr, N, h, n, d, &code);
+        return !(r2 * mdt_rsqrt(r2) > rnear);
+    };
+    const int nflat = MIXED ? 0 : (s_nflat < MDT_FLAT_MAX ? s_nflat : MDT_FLAT_MAX);
+    for (int f = 0; f < nflat; ++f) {
+        for (int n0 = 0; n0 < N; n0 += nthr) {
+            double d[3], r2;
             int code = 0;
-            if (act && n < N) {
-                const float4 pn = f4[n];
-                if (all_on || T.pair_on[tk * MDT_MAXT + __float_as_int(pn.w)]) {
-                    const float e0 = pk.x - pn.x, e1 = pk.y - pn.y, e2 = pk.z - pn.z;
-                    float m0f = rintf(e0), m1f = rintf(e1), m2f = rintf(e2);
-                    float d0 = e0 - m0f, d1 = e1 - m1f, d2 = e2 - m2f;
-                    // within 1e-4 of a half-cell tie: the reference's image, from the unfolded positions
-                    const bool t0 = fabsf(d0) > 0.4999f, t1 = fabsf(d1) > 0.4999f, t2 = fabsf(d2) > 0.4999f;
-                    if (t0 | t1 | t2) {
-                        const double *xr = bv.x + roff;
-                        const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
-                        const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
-                        if (t0) m0f = (float)tie_image(cell.ih[0], cell.ih[3], cell.ih[6], a0, a1, a2, b0, b1, b2, sx[k] - sx[n]);
-                        if (t1) m1f = (float)tie_image(cell.ih[1], cell.ih[4], cell.ih[7], a0, a1, a2, b0, b1, b2, sy[k] - sy[n]);
-                        if (t2) m2f = (float)tie_image(cell.ih[2], cell.ih[5], cell.ih[8], a0, a1, a2, b0, b1, b2, sz[k] - sz[n]);
-                        d0 = e0 - m0f;
-                        d1 = e1 - m1f;
-                        d2 = e2 - m2f;
-                    }
-                    const float r2 = d0 * (g00 * d0 + g01 * d1 + g02 * d2) + d1 * (g11 * d1 + g12 * d2) + g22 * d2 * d2;
-                    in = r2 <= cut2f;
-                    near = r2 <= near2f;
-                    code = ((int)m0f + 1) + 3 * ((int)m1f + 1) + 9 * ((int)m2f + 1);
-                }
-            }
-            const unsigned long long m = __ballot(in) & gmask;
-            const uint16_t ent = (uint16_t)(n | (code << MDT_NBR_IDX_BITS));
-            if (in) {
-                const int pos = c + __popcll(m & below);
-                if (pos < cap)
-                    (split ? nbr_kept : nbr)[(size_t)k * cap + pos] = ent;  // staged: the whole row to HBM
-                else
-                    bad_local |= MDT_ST_NBR_OVERFLOW;
-            }
-            c += __popcll(m);
-            if (split) {  // staged: the near entries to LDS
-                const bool nin = in && near;
-                const unsigned long long mn = __ballot(nin) & gmask;
-                const int pos = cn + __popcll(mn & below);
-                if (nin && pos < cap) nbr[(size_t)k * cap + pos] = ent;
-                cn += __popcll(mn);
-            }
-        }
-        if (act && sub == 0) {
-            const int cc = c < cap ? c : cap;
-            cnt[k] = (uint16_t)(split ? (cn < cap ? cn : cap) : cc);
-            if (keep) kcnt[k] = (uint16_t)cc;
+            const bool in = n0 + lane < N && flat_pair(s_flat[f], n0 + lane, d, r2, code);
+            const unsigned long long m = __ballot(in);
+            int base = 0;
+            if (wl == 0 && m) base = atomicAdd(&s_fcnt[f], __popcll(m));  // the order is free
+            base = __builtin_amdgcn_readfirstlane(base);
+            const int pos = base + __popcll(m & below);
+            if (in && pos < MDT_FLAT_CAP)
+                s_flist[f * MDT_FLAT_CAP + pos] = (uint16_t)((n0 + lane) | (code << MDT_NBR_IDX_BITS));
         }
     }
     __syncthreads();
-    if (keep && !reuse && lane == 0) bv.rl_valid[blockIdx.x] = 1;  // read by the next launch
-    for (int i = lane; i < N; i += nthr) {
-        shi[i] = 0ull;
-        smid[i] = 0ull;
-        slo[i] = 0ull;
+    const int R = s_R;
+    const bool slow = s_slow != 0;  // entries without a fixed image
+    if (!reuse && !direct && lane < R) {
+        info0 = rows[lane];
+        word0 = stream[s_cb[wave] + wl];
     }
-    __syncthreads();
 
-    // ---- phase 2: pass A, sigma ----
-    // the sigma terms of one pair (k, n) at distance r: sigma_k += own in
-    // registers, sigma_n += other into the fixed point
-    auto sigma_pair = [&](int tk, int n, double r, double &sig) {
-        const int tn = typ[n];
-        double own, other48;  // other48: the partner's term times 2^48
+    // ---- pair terms ----
+    const double acut = ecg->acut, rcut = ecg->rcut;
+    const float acutf = (float)acut, acutl2f = (float)(acut * MDT_LOG2E);
+    // exp(acut (r - rcut)) in FP32; the bound (beyond the cut-off) keeps terms that
+    // are multiplied by 0 finite
+    auto cut_exp = [&](double r) { return mdt_exp2f(fminf(acutl2f * (float)(r - rcut), 100.0f)); };
+    // theta and, for its derivative, rt1 = acut e1 theta
+    auto theta = [&](double r, double *rt1) {
+        if constexpr (PREC == 0) {
+            const double e1 = mdt_exp_t((r - rcut) * (acut * MDT_EXP_K), T.exptab);
+            const double th = mdt_rcp(1 + e1);
+            *rt1 = acut * e1 * th;
+            return th;
+        } else {
+            const float e1 = cut_exp(r);
+            const float th = mdt_rcpf(1.0f + e1);
+            *rt1 = (double)(acutf * e1 * th);
+            return (double)th;
+        }
+    };
+    // sigma terms of the pair of types (tk, tn) at r: on k and on n
+    auto sigma_terms = [&](int tk, int tn, double r, double &own, double &other) {
         if constexpr (PREC == 1) {
-            const float e1 = mdt_exp2f(acutl2f * (float)(r - rcut));
+            const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
             const float fsn = th * mdt_exp2f(-T.f_eta2l2[tn] * (float)(r - T.bs0[tn]));
             const float fsk = (tn == tk) ? fsn : th * mdt_exp2f(-T.f_eta2l2[tk] * (float)(r - T.bs0[tk]));
             own = (double)(T.f_csig[tk * MDT_MAXT + tn] * fsn);
-            other48 = (double)(T.f_csig[tn * MDT_MAXT + tk] * fsk) * MDT_W48;
+            other = (double)(T.f_csig[tn * MDT_MAXT + tk] * fsk);
         } else {
-            double th;
-            if constexpr (PREC == 2) {
-                th = (double)mdt_rcpf(1.0f + mdt_exp2f(acutl2f * (float)(r - rcut)));
-            } else {
-                th = mdt_rcp(1 + mdt_exp(acut * (r - rcut), T.exptab));
-            }
-            const double fsn = th * mdt_exp(-T.eta2[tn] * (r - T.bs0[tn]), T.exptab);
-            const double fsk = (tn == tk) ? fsn : th * mdt_exp(-T.eta2[tk] * (r - T.bs0[tk]), T.exptab);
+            double rt1;
+            const double th = theta(r, &rt1);
+            const double fsn = th * mdt_exp_t(T.etaT[tn] * (r - T.bs0[tn]), T.exptab);
+            const double fsk = (tn == tk) ? fsn : th * mdt_exp_t(T.etaT[tk] * (r - T.bs0[tk]), T.exptab);
             own = T.csig[tk * MDT_MAXT + tn] * fsn;
-            other48 = T.csig48[tn * MDT_MAXT + tk] * fsk;
+            other = T.csig[tn * MDT_MAXT + tk] * fsk;
         }
-        sig += own;
-        sig_add_scaled(&shi[n], &smid[n], &slo[n], other48, &bad_local);
     };
-    // one listed pair (entry e of atom k's list), within rnear
-    auto pair_a = [&](int k, int tk, double xk, double yk, double zk, int e, double &sig) {
-        const unsigned q = nbr[(size_t)k * cap + e];
-        const int n = q & MDT_NBR_IDX_MASK, code = q >> MDT_NBR_IDX_BITS;
-        const double dx = (xk - px[n]) - T.shift[3 * code];
-        const double dy = (yk - py[n]) - T.shift[3 * code + 1];
-        const double dz = (zk - pz[n]) - T.shift[3 * code + 2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double r = r2 * mdt_rsqrt(r2);
-        if (r > rnear) return;
-        sigma_pair(tk, n, r, sig);
-    };
-    for (int k0 = 0; k0 < N; k0 += apb) {
-        const int k = k0 + lane / TPA;
-        const int sub = lane % TPA;
-        const bool act = k < N;
-        double sig = 0.0;
-        if (act) {
-            const int tk = typ[k];
-            const double xk = px[k], yk = py[k], zk = pz[k];
-            const int ck = cnt[k];
-            for (int e = sub; e < ck; e += TPA) pair_a(k, tk, xk, yk, zk, e, sig);
-        }
-        sig = group_sum<TPA>(sig);
-        if (act && sub == 0) G[k] = sig;  // own part; the partners' part is in shi/smid/slo
-    }
-    if (lane == 0) s_anytiny = 0;
-    __syncthreads();
-
-    // ---- tiny atoms: sigma~ of the near pairs below MDT_SIG_TINY; then the
-    // pairs beyond rnear of every tiny atom, from a minimum-image scan of
-    // all atoms (a pair of two tiny atoms by its owner) ----
-    for (int k = lane; k < N; k += nthr) {
-        const uint8_t ty = (T.owner[typ[k]] && G[k] + sig_value(shi[k], smid[k], slo[k]) < MDT_SIG_TINY) ? 1 : 0;
-        tiny[k] = ty;
-        if (ty) s_anytiny = 1;  // benign race: every writer stores 1
-    }
-    __syncthreads();
-    const bool anytiny = s_anytiny != 0;
-    // the far partners n of tiny atom t: beyond rnear, within the cut-off
-    auto far_partner = [&](int t, int n, double d[3], double &r, double &ri) {
-        if (n == t || (tiny[n] && !owns(t, n)) || !T.pair_on[typ[t] * MDT_MAXT + typ[n]]) return false;
-        const double r2 = pair_image(s_ihf, bv.icell + 9 * traj, T.shift, px, py, pz, bv.x + roff, N, t, n, d);
-        ri = mdt_rsqrt(r2);
-        r = r2 * ri;
-        return r > rnear && r <= cutr;
-    };
-    // the tiny atoms in index order, 64 flags per ballot (the same mask in
-    // every wave, so the loop and its barriers are uniform over the block)
-    if (anytiny) {
-        for (int t0 = 0; t0 < N; t0 += 64) {
-          unsigned long long tm = __ballot(t0 + wl < N && tiny[t0 + wl] != 0);
-          while (tm) {
-            const int t = t0 + __builtin_ctzll(tm);
-            tm &= tm - 1;
-            const int tt = typ[t];
-            double sig = 0.0;
-            for (int n0 = lane; n0 < N; n0 += nthr) {
-                int n = n0;
-                opaque(n);
-                double d[3], r, ri;
-                if (far_partner(t, n, d, r, ri)) sigma_pair(tt, n, r, sig);
-            }
-            sig = block_sum_fixed(sig, s_wsum, lane, nthr);
-            if (lane == 0) G[t] += sig;
-          }
-        }
-        __syncthreads();
-    }
-
-    // ---- per atom: s, dens, E_coh + vref, G = dE/dsigma ----
-    for (int k = lane; k < N; k += nthr) {
-        const int tk = typ[k];
-        double Gk = 0.0, Ek = 0.0;
-        if (T.owner[tk]) {
-            double dn;
-            emt_atom(T, tk, G[k] + sig_value(shi[k], smid[k], slo[k]), &Gk, &Ek, &dn);
-            if (!JUDGE) bv.dens[doff + k] = dn;  // raw EMT density (pes_emt_mod.f90:855,861)
-        }
-        G[k] = Gk;
-        E[k] = Ek;
-    }
-    __syncthreads();
-    for (int i = lane; i < N; i += nthr) {
-        fxa[i] = 0ull;
-        fya[i] = 0ull;
-        fza[i] = 0ull;
-    }
-    __syncthreads();
-
-    // ---- phase 3: pass B, pair forces and pair energies ----
-    // one listed pair: the pair's dE/dr gives +F on the owner (registers) and
-    // -F on the partner (fixed point); the owner takes the pair energy
-    // the force and energy terms of one pair (k, n), d = r_k - r_n (minimum
-    // image), r = |d|, ri = 1 / r
-    auto force_pair = [&](int tk, int n, double Gk, double dx, double dy, double dz, double r, double ri,
-                          double &fx, double &fy, double &fz, double &ep) {
-        const int tn = typ[n];
+    // dE/dr of the pair: density part through G of both atoms, pair (V) part
+    // directly; and the pair energy
+    auto force_terms = [&](int tk, int tn, double r, double Gk, double Gn, double &c, double &ep) {
         const int kn = tk * MDT_MAXT + tn, nk = tn * MDT_MAXT + tk;
-        double c;
         if constexpr (PREC == 1) {
-            const float e1 = mdt_exp2f(acutl2f * (float)(r - rcut));
+            const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
             const float rt1 = acutf * e1 * th;
             const float drn = (float)(r - T.bs0[tn]);
@@ -796,140 +952,435 @@ __global__ void __launch_bounds__(MAXB, 4)
             const float ta = T.f_csig[kn] * ((T.f_etad[kn] + rt1) * fsn);
             const float tb = T.f_csig[nk] * ((T.f_etad[nk] + rt1) * fsk);
             const float tv = 0.5f * (T.f_wv[kn] * ((T.f_kdb[tn] + rt1) * fvn) + T.f_wv[nk] * ((T.f_kdb[tk] + rt1) * fvk));
-            c = Gk * (double)ta + G[n] * (double)tb + (double)tv;
-            ep += (double)(T.f_wv[kn] * fvn + T.f_wv[nk] * fvk);
+            c = Gk * (double)ta + Gn * (double)tb + (double)tv;
+            ep = (double)(T.f_wv[kn] * fvn + T.f_wv[nk] * fvk);
         } else {
-            double th, rt1;
-            if constexpr (PREC == 2) {
-                const float e1 = mdt_exp2f(acutl2f * (float)(r - rcut));
-                const float thf = mdt_rcpf(1.0f + e1);
-                th = (double)thf;
-                rt1 = (double)(acutf * e1 * thf);
-            } else {
-                const double e1 = mdt_exp(acut * (r - rcut), T.exptab);
-                th = mdt_rcp(1 + e1);
-                rt1 = acut * e1 * th;
-            }
-            const double fsn = th * mdt_exp(-T.eta2[tn] * (r - T.bs0[tn]), T.exptab);
-            const double fvn = th * mdt_exp(-T.kdb[tn] * (r - T.bs0[tn]), T.exptab);
-            // dE/dr of this pair: density part through G, pair (V) part directly
+            double rt1;
+            const double th = theta(r, &rt1);
+            const double drn = r - T.bs0[tn];
+            const double fsn = th * mdt_exp_t(T.etaT[tn] * drn, T.exptab);
+            const double fvn = th * mdt_exp_t(T.kdbT[tn] * drn, T.exptab);
             if (tn == tk) {  // one element: one set of pair constants (kn == nk)
-                c = T.csig[kn] * ((T.etad[kn] + rt1) * fsn) * (Gk + G[n]) + T.wv[kn] * ((T.kdb[tn] + rt1) * fvn);
-                ep += 2.0 * T.wv[kn] * fvn;
+                c = T.csig[kn] * ((T.etad[kn] + rt1) * fsn) * (Gk + Gn) + T.wv[kn] * ((T.kdb[tn] + rt1) * fvn);
+                ep = 2.0 * T.wv[kn] * fvn;
             } else {
-                const double fsk = th * mdt_exp(-T.eta2[tk] * (r - T.bs0[tk]), T.exptab);
-                const double fvk = th * mdt_exp(-T.kdb[tk] * (r - T.bs0[tk]), T.exptab);
-                c = Gk * T.csig[kn] * ((T.etad[kn] + rt1) * fsn) + G[n] * T.csig[nk] * ((T.etad[nk] + rt1) * fsk) +
+                const double drk = r - T.bs0[tk];
+                const double fsk = th * mdt_exp_t(T.etaT[tk] * drk, T.exptab);
+                const double fvk = th * mdt_exp_t(T.kdbT[tk] * drk, T.exptab);
+                c = Gk * T.csig[kn] * ((T.etad[kn] + rt1) * fsn) + Gn * T.csig[nk] * ((T.etad[nk] + rt1) * fsk) +
                     0.5 * (T.wv[kn] * ((T.kdb[tn] + rt1) * fvn) + T.wv[nk] * ((T.kdb[tk] + rt1) * fvk));
-                ep += T.wv[kn] * fvn + T.wv[nk] * fvk;
+                ep = T.wv[kn] * fvn + T.wv[nk] * fvk;
             }
         }
-        // the pair force in fixed-point units (2^42, an exact scaling): the
-        // owner's sums fx, fy, fz are kept in these units too
-        const double crs = c * ri * MDT_F_SCALE;
-        const double gx = crs * dx, gy = crs * dy, gz = crs * dz;
-        fx = fma(-crs, dx, fx);
-        fy = fma(-crs, dy, fy);
-        fz = fma(-crs, dz, fz);
-        fx_add_scaled(&fxa[n], gx, &bad_local);
-        fx_add_scaled(&fya[n], gy, &bad_local);
-        fx_add_scaled(&fza[n], gz, &bad_local);
     };
-    // one listed pair (entry e of atom k's list), within rnear
-    auto pair_b = [&](int k, int tk, double xk, double yk, double zk, double Gk, int e, double &fx, double &fy,
-                      double &fz, double &ep) {
-        const unsigned q = nbr[(size_t)k * cap + e];
-        const int n = q & MDT_NBR_IDX_MASK, code = q >> MDT_NBR_IDX_BITS;
-        const double dx = (xk - px[n]) - T.shift[3 * code];
-        const double dy = (yk - py[n]) - T.shift[3 * code + 1];
-        const double dz = (zk - pz[n]) - T.shift[3 * code + 2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double ri = mdt_rsqrt(r2);
-        const double r = r2 * ri;
-        if (r > rnear) return;
-        force_pair(tk, n, Gk, dx, dy, dz, r, ri, fx, fy, fz, ep);
+    // a listed pair (entry q) of the atom at (xk, yk, zk): its vector; returns r^2
+    auto listed = [&](unsigned q, double xk, double yk, double zk, const PairRec &pn, double &dx, double &dy, double &dz) {
+        const double *sft = s_sh + 4 * (q >> MDT_NBR_IDX_BITS);
+        dx = (xk - pn.x) - sft[0];
+        dy = (yk - pn.y) - sft[1];
+        dz = (zk - pn.z) - sft[2];
+        return dx * dx + dy * dy + dz * dz;
     };
-    for (int k0 = 0; k0 < N; k0 += apb) {
-        const int k = k0 + lane / TPA;
-        const int sub = lane % TPA;
-        const bool act = k < N;
-        double fx = 0.0, fy = 0.0, fz = 0.0, ep = 0.0;
-        if (act) {
-            const int tk = typ[k];
-            const double xk = px[k], yk = py[k], zk = pz[k];
-            const double Gk = G[k];
-            const int ck = cnt[k];
-            for (int e = sub; e < ck; e += TPA) pair_b(k, tk, xk, yk, zk, Gk, e, fx, fy, fz, ep);
+    // a pair's force crs d, added to n; its rounded components
+    auto add_force = [&](int n, double crs, const double *d, double g[3]) {
+        unsigned long long u[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const double tq = fma(crs, d[q], MDT_FRC_C);
+            u[q] = grid_int(tq, MDT_FRC_C);
+            g[q] = tq - MDT_FRC_C;
         }
-        fx = group_sum<TPA>(fx);
-        fy = group_sum<TPA>(fy);
-        fz = group_sum<TPA>(fz);
-        ep = group_sum<TPA>(ep);
-        if (act && sub == 0) {
-            fx_add_scaled(&fxa[k], fx, &bad_local);
-            fx_add_scaled(&fya[k], fy, &bad_local);
-            fx_add_scaled(&fza[k], fz, &bad_local);
-            E[k] -= 0.5 * ep;
+        atomicAdd(&rec[n].w, u[0]);
+        atomicAdd(&w2[n], u[1]);
+        atomicAdd(&w3[n], u[2]);
+    };
+    // a term of either pass from the fast limit on (rare): added by itself, to n and to k
+    auto add_large = [&](int k, int n, double crs, const double *d) {
+#pragma unroll 1
+        for (int q = 0; q < 3; ++q) {
+            double g;
+            const unsigned long long u = grid_any(crs * d[q], MDT_P43, &g, &bad_local);
+            unsigned long long *w = q == 0 ? &rec[n].w : (q == 1 ? w2 : w3) + n;
+            atomicAdd(w, u);
+            w = q == 0 ? &rec[k].w : (q == 1 ? w2 : w3) + k;
+            atomicAdd(w, 0ull - u);
         }
+    };
+    // a row's pair (one type, its constants uniform): the sigma term of either atom, the force terms
+    const int ub = MIXED ? 0 : bulk, ubb = ub * MDT_MAXT + ub;
+    const double u_bs0 = ecg->betas0[ub], u_etaT = -ecg->eta2[ub] * MDT_EXP_K, u_kdbT = -ecg->kappadbeta[ub] * MDT_EXP_K;
+    const double u_csig = ecg->csig[ubb], u_etad = ecg->etad[ubb], u_wv = ecg->wv[ubb], u_kdb = ecg->kappadbeta[ub];
+    const float uf_eta = -(float)(ecg->eta2[ub] * MDT_LOG2E), uf_kdbl2 = -(float)(ecg->kappadbeta[ub] * MDT_LOG2E);
+    const float uf_csig = (float)u_csig, uf_etad = (float)u_etad, uf_wv = (float)u_wv, uf_kdb = (float)u_kdb;
+    auto bulk_sigma = [&](double r) {
+        if constexpr (PREC == 1) {
+            const float th = mdt_rcpf(1.0f + cut_exp(r));
+            return (double)(uf_csig * (th * mdt_exp2f(uf_eta * (float)(r - u_bs0))));
+        } else {
+            double rt1;
+            return u_csig * (theta(r, &rt1) * mdt_exp_t(u_etaT * (r - u_bs0), T.exptab));
+        }
+    };
+    auto bulk_force = [&](double r, double G2, double &c, double &ep) {  // G2: G of both atoms
+        if constexpr (PREC == 1) {
+            const float e1 = cut_exp(r);
+            const float th = mdt_rcpf(1.0f + e1);
+            const float rt1 = acutf * e1 * th;
+            const float dr = (float)(r - u_bs0);
+            const float fs = th * mdt_exp2f(uf_eta * dr), fv = uf_wv * (th * mdt_exp2f(uf_kdbl2 * dr));
+            c = (double)(uf_csig * ((uf_etad + rt1) * fs)) * G2 + (double)((uf_kdb + rt1) * fv);
+            ep = (double)(2.0f * fv);
+        } else {
+            double rt1;
+            const double th = theta(r, &rt1);
+            const double dr = r - u_bs0;
+            const double fs = th * mdt_exp_t(u_etaT * dr, T.exptab);
+            const double fv = u_wv * (th * mdt_exp_t(u_kdbT * dr, T.exptab));
+            c = u_csig * ((u_etad + rt1) * fs) * G2 + (u_kdb + rt1) * fv;
+            ep = 2.0 * fv;
+        }
+    };
+    // the lane's piece of round rb / nthr: the wavefront with the longest pieces of
+    // one round has the shortest of the next
+    auto piece_of = [&](int rb) {
+        return rb + wl + ((rb / nthr & 1) ? nthr - 64 - 64 * wave : 64 * wave);
+    };
+    // The pairs of the lane's piece, atom k at (x, y, z): eval(n, G, r2, in) gives a
+    // pair's terms (in false: none), add(n, terms, d) adds them; a lane's terms of a
+    // `size` from lim on go to large(n, terms, d), which clears them.  Two entries at
+    // a time without a branch between them.
+    auto each_entry = [&](int r0, int k, int len, double x, double y, double z, double lim, auto eval, auto add,
+                          auto large) {
+        const uint32_t *src = stream + (direct ? 0 : s_cb[r0 >> 6]) + (r0 & 63);
+        const uint16_t *row = scan_rows + k * capg + (r0 & ((1 << sh) - 1));  // direct
+        const int last = 32 * (len - 1 & ~1);  // of the piece's words
+        uint32_t cur = direct ? 0 : r0 == lane ? word0 : src[0];
+        double d[3], g[3];
+        if (!slow && !direct) {
+            for (int e = 0; e < len; e += 2) {
+                const uint32_t q = cur;
+                cur = src[32 * e + 64 < last ? 32 * e + 64 : last];
+                const PairRec a0 = rec[q & MDT_NBR_IDX_MASK], a1 = rec[q >> 16 & MDT_NBR_IDX_MASK];
+                const double r0 = listed(q & 0xFFFF, x, y, z, a0, d[0], d[1], d[2]);
+                const double r1 = listed(q >> 16, x, y, z, a1, g[0], g[1], g[2]);
+                const int n0 = q & MDT_NBR_IDX_MASK, n1 = q >> 16 & MDT_NBR_IDX_MASK;
+                auto t0 = eval(n0, a0.g, r0, true), t1 = eval(n1, a1.g, r1, e + 1 < len);
+                if (__builtin_expect(!(fmax(t0.size, t1.size) < lim) || t0.size + t1.size != t0.size + t1.size, 0)) {
+                    if (!(t0.size < lim)) large(n0, t0, d);
+                    if (!(t1.size < lim)) large(n1, t1, g);
+                }
+                add(n0, t0, d);
+                add(n1, t1, g);
+            }
+        } else {
+            for (int e = 0; e < len; ++e) {
+                const unsigned q = direct ? row[e << sh] : e & 1 ? cur >> 16 : cur & 0xFFFF;
+                if (!direct && e & 1) cur = src[32 * (e + 1) < last ? 32 * (e + 1) : last];
+                const int n = q & MDT_NBR_IDX_MASK;
+                const PairRec pn = rec[n];
+                double r2;
+                int code;
+                if (q >> MDT_NBR_IDX_BITS == MDT_ANY_IMAGE)
+                    r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], pn, xr, N, k, n, d, &code);
+                else
+                    r2 = listed(q, x, y, z, pn, d[0], d[1], d[2]);
+                auto tm = eval(n, pn.g, r2, true);
+                if (!(tm.size < lim)) large(n, tm, d);
+                add(n, tm, d);
+            }
+        }
+    };
+    // f(n, d, r2) for the near partners of flat atom number q, one per lane from the
+    // last wavefront on, which has the shortest pieces, or none
+    auto each_flat = [&](int q, auto f) {
+        const int h = s_flat[q], c = s_fcnt[q];
+        const PairRec ph = rec[h];
+        for (int e = lane + 64 < nthr ? lane + 64 : lane + 64 - nthr; e < (c <= MDT_FLAT_CAP ? c : N); e += nthr) {
+            double d[3], r2;
+            int n = e, code;
+            if (c <= MDT_FLAT_CAP) {
+                const unsigned ent = s_flist[q * MDT_FLAT_CAP + e];
+                n = ent & MDT_NBR_IDX_MASK;
+                r2 = listed(ent, ph.x, ph.y, ph.z, rec[n], d[0], d[1], d[2]);
+            } else if (!flat_pair(h, n, d, r2, code)) {
+                continue;
+            }
+            f(n, d, r2);
+        }
+    };
+
+    // ---- phase 2: pass A, sigma ----
+    for (int rb = 0; rb < R; rb += nthr) {
+        const int r0 = piece_of(rb);
+        if (r0 >= R) continue;
+        const uint32_t info = rb == 0 ? info0 : rows[r0];
+        const int k = info & MDT_NBR_IDX_MASK, len = info >> MDT_NBR_IDX_BITS;
+        const double xk = rec[k].x, yk = rec[k].y, zk = rec[k].z;
+        const int tk = MIXED ? typ[k] : 0;
+        double s1 = 0.0, s2 = 0.0;
+        struct Sig {
+            double size, own, other;
+        };
+        each_entry(
+            r0, k, len, xk, yk, zk, MDT_SIG_FAST,
+            [&](int n, double, double r2, bool in) {
+                const double r = r2 * mdt_rsqrt(r2);
+                Sig v;
+                if constexpr (MIXED)
+                    sigma_terms(tk, typ[n], r, v.own, v.other);
+                else
+                    v.own = v.other = bulk_sigma(r);
+                const double on = in && !(r > rnear) ? 1.0 : 0.0;  // r > rnear: in the skin; a factor, not a branch
+                v.own *= on;
+                v.other *= on;
+                v.size = MIXED ? fmax(v.own, v.other) : v.own;
+                return v;
+            },
+            [&](int n, const Sig &v, const double *) {
+                double h, l;
+                unsigned long long u1, u2;
+                sig_words(v.own, &u1, &u2, &h, &l);
+                s1 += h;
+                s2 += l;
+                if constexpr (MIXED) sig_words(v.other, &u1, &u2, &h, &l);
+                atomicAdd(&rec[n].w, u1);
+                atomicAdd(&w2[n], u2);
+            },
+            [&](int n, Sig &v, const double *) {
+                sig_large(&rec[k].w, v.own, &bad_local);
+                sig_large(&rec[n].w, v.other, &bad_local);
+                v.own = v.other = 0.0;
+            });
+        add_sum(&rec[k].w, s1, MDT_P42, &bad_local);
+        add_sum(&w2[k], s2, MDT_P42 * MDT_P46, &bad_local);
+    }
+    for (int q = 0; q < nflat; ++q) {
+        const int h = s_flat[q];
+        double s1 = 0.0, s2 = 0.0;
+        each_flat(q, [&](int n, const double *d, double r2) {
+            double own, other, hi, lo;
+            unsigned long long u1, u2;
+            sigma_terms(typ[h], typ[n], r2 * mdt_rsqrt(r2), own, other);
+            if (!(own < MDT_SIG_FAST && other < MDT_SIG_FAST)) {
+                sig_large(&rec[h].w, own, &bad_local);
+                sig_large(&rec[n].w, other, &bad_local);
+                return;
+            }
+            sig_words(own, &u1, &u2, &hi, &lo);
+            s1 += hi;
+            s2 += lo;
+            sig_words(other, &u1, &u2, &hi, &lo);
+            atomicAdd(&rec[n].w, u1);
+            atomicAdd(&w2[n], u2);
+        });
+        add_uniform(&rec[h].w, s1, MDT_P42, &bad_local);
+        add_uniform(&w2[h], s2, MDT_P42 * MDT_P46, &bad_local);
     }
     __syncthreads();
 
-    // ---- the pairs beyond rnear of the tiny atoms (as in pass A) ----
-    if (anytiny) {
+    // ---- tiny atoms: sigma~ of the near pairs below MDT_SIG_TINY; their
+    // pairs beyond rnear from a minimum-image test of all atoms, a wavefront
+    // per atom (lanes over partners: an order of the atoms' own).  A tiny
+    // atom's share is summed by its own scan (below MDT_SIG_VTINY over the near
+    // pairs too, in place of its words), the other atoms' through their words.
+    int any = 0;
+    for (int k = lane; k < N; k += nthr) {
+        uint8_t ty = 0;
+        if (T.owner[typ[k]]) {
+            const double s = sig_sum(rec[k].w, w2[k]);
+            ty = s < MDT_SIG_TINY ? (s < MDT_SIG_VTINY ? 2 : 1) : 0;
+        }
+        tiny[k] = ty;
+        any |= ty;
+    }
+    const bool anytiny = __syncthreads_or(any);
+    // the partners n of tiny atom k: within the cut-off, and beyond rnear unless `near`
+    auto partner = [&](int k, int n, bool near, double d[3], double &r, double &ri) {
+        if (n == k || !T.pair_on[typ[k] * MDT_MAXT + typ[n]]) return false;
+        int code;
+        const double r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], rec[n], xr, N, k, n, d, &code);
+        ri = mdt_rsqrt(r2);
+        r = r2 * ri;
+        return (near || r > rnear) && r <= cutr;
+    };
+    // calls f(k) for every tiny atom, each on one wavefront
+    auto each_tiny = [&](auto f) {
+        int at = 0;
         for (int t0 = 0; t0 < N; t0 += 64) {
-          unsigned long long tm = __ballot(t0 + wl < N && tiny[t0 + wl] != 0);
-          while (tm) {
-            const int t = t0 + __builtin_ctzll(tm);
-            tm &= tm - 1;
-            const int tt = typ[t];
-            const double Gt = G[t];
-            double v[4] = {0.0, 0.0, 0.0, 0.0};  // fx fy fz (fixed-point units), ep
-            for (int n0 = lane; n0 < N; n0 += nthr) {
+            unsigned long long tm = __ballot(t0 + wl < N && tiny[t0 + wl] != 0);
+            for (; tm; tm &= tm - 1, ++at)
+                if (at % nwaves == wave) f(t0 + __builtin_ctzll(tm));
+        }
+    };
+    if (anytiny) {
+        each_tiny([&](int k) {
+            const int tk = typ[k];
+            const bool near = tiny[k] == 2;
+            double sig = 0.0;
+            for (int n0 = wl; n0 < N; n0 += 64) {
                 int n = n0;
                 opaque(n);
                 double d[3], r, ri;
-                if (far_partner(t, n, d, r, ri)) force_pair(tt, n, Gt, d[0], d[1], d[2], r, ri, v[0], v[1], v[2], v[3]);
+                if (!partner(k, n, near, d, r, ri)) continue;
+                double own, other, hi, lo;
+                unsigned long long u1, u2;
+                sigma_terms(tk, typ[n], r, own, other);
+                sig += own;
+                if (r > rnear && !tiny[n]) {
+                    sig_words(other, &u1, &u2, &hi, &lo);  // beyond rnear: far below MDT_SIG_FAST
+                    atomicAdd(&rec[n].w, u1);
+                    atomicAdd(&w2[n], u2);
+                }
             }
-            block_sum4_fixed(v, s_wsum, lane, nthr);
-            if (lane == 0) {
-                fx_add_scaled(&fxa[t], v[0], &bad_local);
-                fx_add_scaled(&fya[t], v[1], &bad_local);
-                fx_add_scaled(&fza[t], v[2], &bad_local);
-                E[t] -= 0.5 * v[3];
-            }
-          }
-        }
+            sig = wave_sum(sig);
+            if (wl == 0) w3[k] = __double_as_longlong(sig);
+        });
         __syncthreads();
     }
 
+    // ---- per atom: s, dens, E_coh + vref, G = dE/dsigma ----
+    double ep1 = 0.0, ep2 = 0.0;
+    auto add_energy = [&](double ep) {
+        const double h = (ep + MDT_EPR_C1) - MDT_EPR_C1;
+        ep1 += h;
+        ep2 += ((ep - h) + MDT_EPR_C2) - MDT_EPR_C2;
+    };
+    for (int k = lane; k < N; k += nthr) {
+        const int tk = typ[k];
+        double Gk = 0.0, Ek = 0.0;
+        if (T.owner[tk]) {
+            double dn;
+            const double sig = (tiny[k] == 2 ? 0.0 : sig_sum(rec[k].w, w2[k])) + __longlong_as_double(w3[k]);
+            emt_atom(T, tk, sig, &Gk, &Ek, &dn);
+            if (!JUDGE) bv.dens[doff + k] = dn;  // raw EMT density (pes_emt_mod.f90:855,861)
+        }
+        rec[k].g = Gk;
+        add_energy(-2.0 * Ek);
+        rec[k].w = w2[k] = w3[k] = 0;  // force words from here on
+    }
+    __syncthreads();
+
+    // ---- phase 3: pass B, pair forces and pair energies ----
+    // each pair's dE/dr gives +F on the owner and -F on the partner
+    // (Newton's third law)
+    for (int rb = 0; rb < R; rb += nthr) {
+        const int r0 = piece_of(rb);
+        if (r0 >= R) continue;
+        const uint32_t info = rb == 0 ? info0 : rows[r0];
+        const int k = info & MDT_NBR_IDX_MASK, len = info >> MDT_NBR_IDX_BITS;
+        const double xk = rec[k].x, yk = rec[k].y, zk = rec[k].z, Gk = rec[k].g;
+        const int tk = MIXED ? typ[k] : 0;
+        double fx = 0.0, fy = 0.0, fz = 0.0;
+        struct Frc {
+            double size, crs, ep;
+        };
+        each_entry(
+            r0, k, len, xk, yk, zk, MDT_FRC_FAST,
+            [&](int n, double Gn, double r2, bool in) {
+                const double ri = mdt_rsqrt(r2);
+                const double r = r2 * ri;
+                double c;
+                Frc v;
+                if constexpr (MIXED)
+                    force_terms(tk, typ[n], r, Gk, Gn, c, v.ep);
+                else
+                    bulk_force(r, Gk + Gn, c, v.ep);
+                const double on = in && !(r > rnear) ? 1.0 : 0.0;
+                c *= on;
+                v.ep *= on;
+                v.size = fabs(c);
+                v.crs = c * ri;
+                return v;
+            },
+            [&](int n, const Frc &v, const double *d) {
+                double g[3];
+                add_energy(v.ep);
+                add_force(n, v.crs, d, g);
+                fx -= g[0];
+                fy -= g[1];
+                fz -= g[2];
+            },
+            [&](int n, Frc &v, const double *d) {
+                add_large(k, n, v.crs, d);
+                v.crs = 0.0;
+            });
+        add_sum(&rec[k].w, fx, MDT_P43, &bad_local);
+        add_sum(&w2[k], fy, MDT_P43, &bad_local);
+        add_sum(&w3[k], fz, MDT_P43, &bad_local);
+    }
+    // the pair (k, n) of an atom k that a wavefront's lanes share: -F on k in fk
+    auto pair_forces = [&](int k, int n, const double *d, double r, double ri, double fk[3]) {
+        double c, ep, g[3];
+        force_terms(typ[k], typ[n], r, rec[k].g, rec[n].g, c, ep);
+        add_energy(ep);
+        if (!(fabs(c) < MDT_FRC_FAST)) {
+            add_large(k, n, c * ri, d);
+            return;
+        }
+        add_force(n, c * ri, d, g);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) fk[q] -= g[q];
+    };
+    for (int q = 0; q < nflat; ++q) {
+        const int h = s_flat[q];
+        double fk[3] = {0.0, 0.0, 0.0};
+        each_flat(q, [&](int n, const double *d, double r2) {
+            const double ri = mdt_rsqrt(r2);
+            pair_forces(h, n, d, r2 * ri, ri, fk);
+        });
+        add_uniform(&rec[h].w, fk[0], MDT_P43, &bad_local);
+        add_uniform(&w2[h], fk[1], MDT_P43, &bad_local);
+        add_uniform(&w3[h], fk[2], MDT_P43, &bad_local);
+    }
+    // the pairs beyond rnear of the tiny atoms, a pair of two by its owner
+    if (anytiny)
+        each_tiny([&](int k) {
+            double fk[3] = {0.0, 0.0, 0.0};
+            for (int n0 = wl; n0 < N; n0 += 64) {
+                int n = n0;
+                opaque(n);
+                double d[3], r, ri;
+                if ((tiny[n] && !owns(k, n)) || !partner(k, n, false, d, r, ri)) continue;
+                pair_forces(k, n, d, r, ri, fk);
+            }
+            add_uniform(&rec[k].w, fk[0], MDT_P43, &bad_local);
+            add_uniform(&w2[k], fk[1], MDT_P43, &bad_local);
+            add_uniform(&w3[k], fk[2], MDT_P43, &bad_local);
+        });
+    ep1 = wave_sum(ep1);
+    ep2 = wave_sum(ep2);
+    if (wl == 0) {
+        unsafeAtomicAdd(&s_ep[0], ep1);
+        unsafeAtomicAdd(&s_ep[1], ep2);
+    }
+    __syncthreads();
     // ---- judge mode: compare with the given forces, write nothing else ----
     if constexpr (JUDGE) {
         double sq = 0.0, mx = 0.0;
         for (int k = lane; k < N; k += nthr) {
             const int tk = typ[k];
             for (int cc = 0; cc < 3; ++cc) {
-                unsigned long long *acc = cc == 0 ? fxa : (cc == 1 ? fya : fza);
-                const double F = T.owner[tk] ? (double)(long long)acc[k] * MDT_F_ISCALE : 0.0;
+                const double F = T.owner[tk] ? frc_sum(cc == 0 ? rec[k].w : cc == 1 ? w2[k] : w3[k]) : 0.0;
                 const double d = F - bv.judge_f[roff + (long long)cc * N + k];
                 sq += d * d;
                 mx = fabs(d) > mx ? fabs(d) : mx;
             }
         }
-        // fixed-order block reduction through red[] (wave partials, then wave 0)
+        // fixed-order block reduction through jr[] (wave partials, then wave 0)
         for (int o = 32; o > 0; o >>= 1) {
             sq += __shfl_xor(sq, o, 64);
             const double m2 = __shfl_xor(mx, o, 64);
             mx = m2 > mx ? m2 : mx;
         }
         __shared__ double jr[32];
-        if ((lane & 63) == 0) {
-            jr[2 * (lane >> 6)] = sq;
-            jr[2 * (lane >> 6) + 1] = mx;
+        if (wl == 0) {
+            jr[2 * wave] = sq;
+            jr[2 * wave + 1] = mx;
         }
         __syncthreads();
         if (lane == 0) {
             double s2 = 0.0, m2 = 0.0;
-            for (int w = 0; w < (nthr + 63) / 64; ++w) {
+            for (int w = 0; w < nwaves; ++w) {
                 s2 += jr[2 * w];
                 m2 = jr[2 * w + 1] > m2 ? jr[2 * w + 1] : m2;
             }
@@ -943,34 +1394,23 @@ __global__ void __launch_bounds__(MAXB, 4)
 
     // ---- phase 4: set_acceleration (force.f90:89-98), outputs ----
     for (int k = lane; k < N; k += nthr) {
-        const int tk = typ[k];
-        double F[3] = {(double)(long long)fxa[k] * MDT_F_ISCALE, (double)(long long)fya[k] * MDT_F_ISCALE,
-                       (double)(long long)fza[k] * MDT_F_ISCALE};
-        if (!T.owner[tk]) F[0] = F[1] = F[2] = 0.0;
+        double F[3] = {frc_sum(rec[k].w), frc_sum(w2[k]), frc_sum(w3[k])};
+        if (!T.owner[typ[k]]) F[0] = F[1] = F[2] = 0.0;
         if (add_fin) {
             F[0] += bv.f[roff + k];
             F[1] += bv.f[roff + N + k];
             F[2] += bv.f[roff + 2 * N + k];
         }
-        const uint8_t fb = bv.fixed[doff + k];
-        const double mass = bv.mass[aoff + k];
-        const double a0 = (fb & 1) ? 0.0 : F[0] / mass;
-        const double a1 = (fb & 2) ? 0.0 : F[1] / mass;
-        const double a2 = (fb & 4) ? 0.0 : F[2] / mass;
+        const int fb = k == lane ? fixed0 : bv.fixed[doff + k];
+        const double mass = k == lane ? mass0 : bv.mass[aoff + k];
         bv.f[roff + k] = F[0];
         bv.f[roff + N + k] = F[1];
         bv.f[roff + 2 * N + k] = F[2];
-        bv.a[roff + k] = a0;
-        bv.a[roff + N + k] = a1;
-        bv.a[roff + 2 * N + k] = a2;
+        bv.a[roff + k] = (fb & 1) ? 0.0 : F[0] / mass;
+        bv.a[roff + N + k] = (fb & 2) ? 0.0 : F[1] / mass;
+        bv.a[roff + 2 * N + k] = (fb & 4) ? 0.0 : F[2] / mass;
     }
-    // ---- energy of the replica: fixed-order reduction by wave 0 ----
-    if (lane < 64) {
-        double e = 0.0;
-        for (int i = lane; i < N; i += 64) e += E[i];
-        for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
-        if (lane == 0) bv.epot[bv.traj_eoff[t] + b] = e;
-    }
+    if (lane == 0) bv.epot[bv.traj_eoff[t] + b] = -0.5 * (s_ep[0] + s_ep[1]);
     if (bad_local) atomicOr(&bv.status[t], bad_local);
 }
 
@@ -2293,51 +2733,73 @@ __global__ void __launch_bounds__(MAXB, 2)
 // ---------------------------------------------------------------------------
 // host-side launchers (C++ linkage, used by mdt_api.hip)
 // ---------------------------------------------------------------------------
-size_t mdt_replica_smem(int N, int cap, bool nbr_lds) {
-    const int c = cap < N - 1 ? cap : (N > 1 ? N - 1 : 1);
-    // px py pz | A0 A1 A2 | G | E: 8 N doubles; cnt, lists; typ, tiny
-    return sizeof(double) * (8 * (size_t)N) + sizeof(uint16_t) * ((size_t)N + (nbr_lds ? (size_t)N * c : 0)) +
-           2 * (size_t)N + 16;
+// marks one slot in `period` invalid (launch-shape tuning)
+__global__ void k_drop_lists(int2 *valid, int n, int period, int phase) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && i % period == phase) valid[i].x = 0;
 }
-
-template <bool L, int F, bool J>
-static hipError_t launch_replica_t(int tpa, dim3 g, dim3 blk, size_t smem, const EmtConst *ec, const PropConst *pc,
-                                   const BatchView &bv, int add_fin, hipStream_t st) {
-    if (blk.x > 512) {  // 1024-lane instantiations: one or two threads per atom
-        switch (tpa) {
-        case 1: hipLaunchKernelGGL((k_replica<1, L, F, J, 1024>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-        case 2: hipLaunchKernelGGL((k_replica<2, L, F, J, 1024>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    }
-    switch (tpa) {
-    case 1: hipLaunchKernelGGL((k_replica<1, L, F, J>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-    case 2: hipLaunchKernelGGL((k_replica<2, L, F, J>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-    case 4: hipLaunchKernelGGL((k_replica<4, L, F, J>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-    case 8: hipLaunchKernelGGL((k_replica<8, L, F, J>), g, blk, smem, st, ec, pc, bv, add_fin); break;
-    default: return hipErrorInvalidValue;
-    }
+hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipStream_t st) {
+    hipLaunchKernelGGL(k_drop_lists, dim3((n + 256) / 256), dim3(256), 0, st, valid, n, period, phase);
     return hipGetLastError();
 }
 
-// calc_force on every replica; ec and pc are device pointers.  The judge
-// (bv.judge_acc set) always runs the FP64 arithmetic.
+// k_replica's dynamic LDS, W2, W3, records, typ, tiny, and its HBM slot for a
+// class: nrep replicas of up to N atoms, workgroups of `block` lanes, rows of up to
+// cap entries; offsets in 4-byte words.  The stream's chunks of 64 pieces hold two
+// entries a word, padded to their first piece's length, which is at most the
+// last one's of the chunk before: 32 (longest + 1 a chunk) + half the entries -- 2
+// more a chunk for lengths of 63 to 65, which are not told apart --, or, uncut, N
+// rows of cap; and a row of slack.  The scanned rows go to LDS (scan < 0) where at
+// most REP_FEW workgroups run, about two a CU, whose number LDS then does not
+// limit, and they fit into `lds`.
+ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds) {
+    ReplicaLists l;
+    const long long chunks = (N + block) / 64 + 1;
+    l.rows = 32 * (cap + 65 + 3 * chunks) + (N + 64LL) * (cap + 1) / 2 + 64;
+    l.chunk = l.rows + N + block;
+    const size_t rows = 2 * (size_t)N * ((cap + 7) & ~7);
+    l.smem = 58 * (size_t)N;
+    l.scan = (l.chunk + chunks + 3) & ~3LL;
+    l.stride = l.scan;
+    if (nrep <= REP_FEW && l.smem + 8 + rows <= lds) {
+        l.smem += 8 + rows;
+        l.scan = -1;
+    } else {
+        l.stride += (long long)rows / 4;
+    }
+    return l;
+}
+
+template <bool M, int F, bool J>
+static hipError_t launch_replica_t(dim3 g, dim3 blk, size_t smem, const EmtConst *ec, const PropConst *pc,
+                                   const BatchView &bv, int add_fin, hipStream_t st) {
+    if (blk.x > 512)
+        hipLaunchKernelGGL((k_replica<M, F, J, 1024>), g, blk, smem, st, ec, pc, bv, add_fin);
+    else
+        hipLaunchKernelGGL((k_replica<M, F, J, 512>), g, blk, smem, st, ec, pc, bv, add_fin);
+    return hipGetLastError();
+}
+
+// calc_force on every replica; ec and pc are device pointers; tpa lanes per
+// atom scan for the rows.  The judge (bv.judge_acc set) always runs the FP64
+// arithmetic.
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
-                              const BatchView &bv, int add_fin, hipStream_t st) {
+                              const BatchView &view, int add_fin, hipStream_t st) {
     dim3 g(nrep), blk(block);
-    const bool lds = bv.nbr_global == nullptr || bv.rl_stage;  // kept lists staged in LDS: the LDS instantiation
+    BatchView bv = view;
+    bv.tpa_shift = tpa == 8 ? 3 : tpa == 4 ? 2 : tpa == 2 ? 1 : 0;
+    const bool m = bv.bulk < 0;
     if (bv.judge_acc)
-        return lds ? launch_replica_t<true, 0, true>(tpa, g, blk, smem, ec, pc, bv, add_fin, st)
-                   : launch_replica_t<false, 0, true>(tpa, g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 0, true>(g, blk, smem, ec, pc, bv, add_fin, st)
+                 : launch_replica_t<false, 0, true>(g, blk, smem, ec, pc, bv, add_fin, st);
     if (bv.precision == 1)
-        return lds ? launch_replica_t<true, 1, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st)
-                   : launch_replica_t<false, 1, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 1, false>(g, blk, smem, ec, pc, bv, add_fin, st)
+                 : launch_replica_t<false, 1, false>(g, blk, smem, ec, pc, bv, add_fin, st);
     if (bv.precision == 2)
-        return lds ? launch_replica_t<true, 2, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st)
-                   : launch_replica_t<false, 2, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st);
-    return lds ? launch_replica_t<true, 0, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st)
-               : launch_replica_t<false, 0, false>(tpa, g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 2, false>(g, blk, smem, ec, pc, bv, add_fin, st)
+                 : launch_replica_t<false, 2, false>(g, blk, smem, ec, pc, bv, add_fin, st);
+    return m ? launch_replica_t<true, 0, false>(g, blk, smem, ec, pc, bv, add_fin, st)
+             : launch_replica_t<false, 0, false>(g, blk, smem, ec, pc, bv, add_fin, st);
 }
 
 // LDS of k_mixed for trajectories of up to nmax atoms (one projectile) and

@@ -44,7 +44,9 @@
 #define NA_TRAJ (NA_CELL + NA_ALIGN(8 * 20))  // N, P, status, traj_id | soff, aoff, eoff (8-byte aligned)
 #define NA_PC (NA_TRAJ + NA_ALIGN(64))
 #define NA_NBR (NA_PC + NA_ALIGN(sizeof(PropConst)))
-#define NA_TOTAL (NA_NBR + NA_ALIGN(2 * (size_t)NOALLOC_MAX_AB * NOALLOC_NBCAP))
+// k_replica's lists (mdt_replica_lists at 96 entries per row): less than 10240 words a replica and 104 an atom
+#define NA_LIST_WORDS (10240 * (size_t)NOALLOC_MAX_BEADS + 104 * (size_t)NOALLOC_MAX_AB)
+#define NA_TOTAL (NA_NBR + NA_ALIGN(4 * NA_LIST_WORDS))
 
 static __device__ __align__(256) unsigned char scratch[NA_TOTAL];
 
@@ -136,7 +138,7 @@ __global__ void k_noalloc_unpack(const unsigned char *s, const EmtConst *ec, int
 
 }  // namespace
 
-size_t mdt_replica_smem(int N, int cap, bool nbr_lds);
+ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds);
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
                               const BatchView &bv, int add_fin, hipStream_t st);
 int mdt_noalloc_fail(int code, const char *msg);
@@ -167,12 +169,12 @@ int mdt_noalloc_compute(void *ptr, size_t lds_limit, const EmtConst *d_ec, int n
     int cap = NOALLOC_NBCAP < N - 1 ? NOALLOC_NBCAP : (N > 1 ? N - 1 : 1);
     int tpa = 8;
     while (tpa > 1 && N * tpa > 512) tpa >>= 1;
-    const size_t lds_dyn = lds_limit > 5632 ? lds_limit - 5632 : 0;  // beside k_replica's static tables (<= 4.7 KB)
-    const size_t smem_lds = mdt_replica_smem(N, cap, true);
-    const bool lds = smem_lds <= lds_dyn;
-    const size_t smem = lds ? smem_lds : mdt_replica_smem(N, cap, false);
-    if (smem > lds_dyn) return mdt_noalloc_fail(MDT_EUNSUP, "universe too large for one workgroup's LDS");
     const int block = (((N * tpa + 63) / 64) * 64) < 64 ? 64 : (((N * tpa + 63) / 64) * 64);
+    const size_t lds_dyn = lds_limit > 6656 ? lds_limit - 6656 : 0;  // beside k_replica's static tables
+    const ReplicaLists lay = mdt_replica_lists(P, N, block, cap, lds_dyn);
+    const size_t smem = lay.smem;
+    if (smem > lds_dyn) return mdt_noalloc_fail(MDT_EUNSUP, "universe too large for one workgroup's LDS");
+    if ((size_t)lay.stride * P > NA_LIST_WORDS) return mdt_noalloc_fail(MDT_EUNSUP, "universe too large for the scratch lists");
     const long long n3 = 3LL * P * N;
     const int grid = (int)((n3 + 255) / 256 < 1024 ? (n3 + 255) / 256 : 1024);
     hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(64), 0, st, s);
@@ -205,8 +207,12 @@ int mdt_noalloc_compute(void *ptr, size_t lds_limit, const EmtConst *d_ec, int n
     v.a = (double *)(s + NA_A);
     v.dens = (double *)(s + NA_DENS);
     v.epot = (double *)(s + NA_EPOT);
-    v.nbr_global = lds ? nullptr : (uint16_t *)(s + NA_NBR);
-    v.nbr_stride = lds ? 0 : (long long)N * cap;
+    v.bulk = -1;  // the types are on the device only
+    v.rl_lists = (uint32_t *)(s + NA_NBR);
+    v.rl_stride = lay.stride;
+    v.rl_rows = lay.rows;
+    v.rl_chunk = lay.chunk;
+    v.rl_scan = lay.scan;
     e = mdt_launch_replica(tpa, P, block, smem, d_ec, (const PropConst *)(s + NA_PC), v, 0, st);
     if (e != hipSuccess) return mdt_noalloc_fail(MDT_EHIP, hipGetErrorString(e));
     hipLaunchKernelGGL(k_noalloc_unpack, dim3(grid), dim3(256), 0, st, (const unsigned char *)s, d_ec, N, P, epot, f,

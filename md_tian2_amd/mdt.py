@@ -328,7 +328,7 @@ class Batch:
 
     def set_keep(self, mode):
         """k_replica's lists: -1 autotuned (default), 0 rebuilt every launch,
-        1 kept (Verlet skin) and staged in LDS, 2 kept and read from HBM."""
+        1 or 2 kept (Verlet skin)."""
         _check(lib().mdt_batch_set_keep(self.h, int(mode)))
 
     def class_shapes(self):

@@ -18,6 +18,8 @@
 #include "mdt_device.h"
 
 ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds);
+hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed,
+                               const double *src, double *dst, hipStream_t st);
 hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipStream_t st);
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
                               const BatchView &bv, int add_fin, hipStream_t st);
@@ -251,6 +253,10 @@ struct mdt_batch {
     PropChunk *d_chunk = nullptr;
     double *d_com = nullptr;
     int nchunk = 0, chunk_mode = -1;
+    // set_state / get_state: runs of atoms and one array in the caller's layout
+    StateTile *d_tile = nullptr;
+    double *d_xfer = nullptr;
+    int ntile = 0;
 
     // k_replica's pair-term arithmetic: mode 1 is full FP32 pair terms when
     // the EMT types' stiffness allows (EmtConst::fp32_ok), else only the
@@ -551,7 +557,7 @@ int mdt_batch_destroy(mdt_batch *b) {
                     b->d_tproj, b->d_tid, b->d_x, b->d_v, b->d_a, b->d_f, b->d_dens, b->d_epot,
                     b->d_cjk, b->d_status, b->d_pc, b->d_step, b->d_nnG, b->d_nnC,
                     b->d_nnflag, b->d_nnF, b->d_judge, b->d_mix, b->d_mix_nbr, b->d_mix_ref, b->d_mix_fold, b->d_mix_cnt, b->d_mix_valid, b->d_obs, b->d_done, b->d_est, b->d_eta,
-                    b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey, b->d_step_h, b->d_ident, b->d_chunk, b->d_com};
+                    b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey, b->d_step_h, b->d_ident, b->d_chunk, b->d_com, b->d_tile, b->d_xfer};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
@@ -875,17 +881,21 @@ int mdt_batch_seed(mdt_batch *b, uint32_t seed, const uint32_t *traj_id) {
     return 0;
 }
 
-// reference (3,P,N) per trajectory <-> device [b][c][i]
-static void to_device_layout(const mdt_batch *b, const double *src, std::vector<double> &dst) {
-    dst.resize(b->tot3pn);
+// k_relayout's tiles and transfer array, made once per batch
+static int build_tiles(mdt_batch *b) {
+    if (b->d_xfer) return 0;
+    std::vector<StateTile> tl;
     for (int t = 0; t < b->ntraj; ++t) {
-        const int N = b->N[t], P = b->P[t];
-        const long long o = b->soff[t];
-        for (int i = 0; i < N; ++i)
-            for (int bb = 0; bb < P; ++bb)
-                for (int c = 0; c < 3; ++c)
-                    dst[o + ((long long)bb * 3 + c) * N + i] = src[o + c + 3 * (bb + (long long)P * i)];
+        const int na = std::max(1, MDT_TILE / b->P[t]);
+        for (int i = 0; i < b->N[t]; i += na) tl.push_back({t, i, std::min(na, b->N[t] - i)});
     }
+    if (!b->d_tile) {
+        int rc = dalloc(&b->d_tile, tl.size());
+        if (rc) return rc;
+    }
+    HIPCHK(hipMemcpy(b->d_tile, tl.data(), sizeof(StateTile) * tl.size(), hipMemcpyHostToDevice));
+    b->ntile = (int)tl.size();
+    return dalloc(&b->d_xfer, (size_t)b->tot3pn);
 }
 
 // bead slot holding atom i's bead bb on the device: in mixed bead mode a
@@ -895,32 +905,20 @@ static inline int dev_bead(const mdt_batch *b, int t, int i, int bb) {
     return (b->bead_mode == 1 && b->P[t] > 1 && i > 0) ? 0 : bb;
 }
 
-static void from_device_layout(const mdt_batch *b, const std::vector<double> &src, double *dst) {
-    for (int t = 0; t < b->ntraj; ++t) {
-        const int N = b->N[t], P = b->P[t];
-        const long long o = b->soff[t];
-        for (int i = 0; i < N; ++i)
-            for (int bb = 0; bb < P; ++bb) {
-                const int sb = dev_bead(b, t, i, bb);
-                for (int c = 0; c < 3; ++c)
-                    dst[o + c + 3 * (bb + (long long)P * i)] = src[o + ((long long)sb * 3 + c) * N + i];
-            }
-    }
-}
-
 int mdt_batch_set_state(mdt_batch *b, const double *r, const double *v) {
     if (!b || !r) return fail(MDT_EINVAL, "mdt_batch_set_state: NULL argument");
-    std::vector<double> tmp;
     hipStream_t st = b->ctx->stream;
-    to_device_layout(b, r, tmp);
-    HIPCHK(hipMemcpyAsync(b->d_x, tmp.data(), sizeof(double) * b->tot3pn, hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));
-    if (v) {
-        to_device_layout(b, v, tmp);
-        HIPCHK(hipMemcpyAsync(b->d_v, tmp.data(), sizeof(double) * b->tot3pn, hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
+    int rc = build_tiles(b);
+    if (rc) return rc;
+    const double *srcs[2] = {r, v};
+    double *dsts[2] = {b->d_x, b->d_v};
+    for (int k = 0; k < 2; ++k) {
+        if (!srcs[k]) continue;
+        HIPCHK(hipMemcpyAsync(b->d_xfer, srcs[k], sizeof(double) * b->tot3pn, hipMemcpyHostToDevice, st));
+        HIPCHK(mdt_launch_relayout(false, b->ntile, b->d_tile, b->view(), 0, b->d_xfer, dsts[k], st));
     }
-    int rc = invalidate_lists(b);  // new positions: the kept lists are stale
+    HIPCHK(hipStreamSynchronize(st));
+    rc = invalidate_lists(b);  // new positions: the kept lists are stale
     if (rc) return rc;
     b->have_state = true;
     return 0;
@@ -929,15 +927,16 @@ int mdt_batch_set_state(mdt_batch *b, const double *r, const double *v) {
 int mdt_batch_get_state(mdt_batch *b, double *r, double *v, double *f, double *a, double *epot, double *dens) {
     if (!b) return fail(MDT_EINVAL, "mdt_batch_get_state: NULL batch");
     hipStream_t st = b->ctx->stream;
-    std::vector<double> tmp(b->tot3pn);
+    int rc = build_tiles(b);
+    if (rc) return rc;
     double *srcs[4] = {b->d_x, b->d_v, b->d_f, b->d_a};
     double *dsts[4] = {r, v, f, a};
     for (int k = 0; k < 4; ++k) {
         if (!dsts[k]) continue;
-        HIPCHK(hipMemcpyAsync(tmp.data(), srcs[k], sizeof(double) * b->tot3pn, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        from_device_layout(b, tmp, dsts[k]);
+        HIPCHK(mdt_launch_relayout(true, b->ntile, b->d_tile, b->view(), b->bead_mode == 1, srcs[k], b->d_xfer, st));
+        HIPCHK(hipMemcpyAsync(dsts[k], b->d_xfer, sizeof(double) * b->tot3pn, hipMemcpyDeviceToHost, st));
     }
+    HIPCHK(hipStreamSynchronize(st));
     if (epot) {
         HIPCHK(hipMemcpyAsync(epot, b->d_epot, sizeof(double) * b->totp, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));

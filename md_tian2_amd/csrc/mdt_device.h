@@ -108,6 +108,12 @@ struct PropChunk {
 };
 #define MDT_CHUNK 256
 
+// atoms i0 .. i0 + na - 1 of trajectory t with their beads, at most MDT_TILE of them (k_relayout)
+struct StateTile {
+    int t, i0, na;
+};
+#define MDT_TILE 256
+
 // k_replica's HBM slot: words per slot and where its parts start (mdt_replica_lists)
 struct ReplicaLists {
     long long stride, rows, chunk, scan;

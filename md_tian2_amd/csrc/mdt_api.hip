@@ -20,6 +20,7 @@
 ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds);
 hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed,
                                const double *src, double *dst, hipStream_t st);
+hipError_t mdt_launch_call(bool in, double *host, int N, int P, const CallArrays &a, hipStream_t st);
 hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipStream_t st);
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
                               const BatchView &bv, int add_fin, hipStream_t st);
@@ -257,6 +258,7 @@ struct mdt_batch {
     StateTile *d_tile = nullptr;
     double *d_xfer = nullptr;
     int ntile = 0;
+    double *h_call = nullptr, *d_call = nullptr;  // pinned block of a one-universe call, and its device address
 
     // k_replica's pair-term arithmetic: mode 1 is full FP32 pair terms when
     // the EMT types' stiffness allows (EmtConst::fp32_ok), else only the
@@ -560,6 +562,7 @@ int mdt_batch_destroy(mdt_batch *b) {
                     b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey, b->d_step_h, b->d_ident, b->d_chunk, b->d_com, b->d_tile, b->d_xfer};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (b->h_call) (void)hipHostFree(b->h_call);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
     for (hipGraphExec_t g : b->gexec_h)
         if (g) (void)hipGraphExecDestroy(g);
@@ -781,6 +784,20 @@ int mdt_batch_create(mdt_context *ctx, int ntraj, const int32_t *natoms, const i
     return 0;
 }
 
+// the atoms' types, and per type their number in all and the most of one trajectory
+static void set_types(mdt_batch *b, const std::vector<uint8_t> &ty) {
+    b->h_type = ty;
+    for (int a = 0; a < MDT_MAXT; ++a) b->type_total[a] = b->type_most[a] = 0;
+    for (int t = 0; t < b->ntraj; ++t) {
+        int n[MDT_MAXT] = {};
+        for (int i = 0; i < b->N[t]; ++i) ++n[ty[b->aoff[t] + i]];
+        for (int a = 0; a < MDT_MAXT; ++a) {
+            b->type_total[a] += n[a];
+            b->type_most[a] = std::max(b->type_most[a], n[a]);
+        }
+    }
+}
+
 int mdt_batch_set_atoms(mdt_batch *b, const int32_t *idx, const double *mass, const int32_t *is_fixed) {
     if (!b || !idx || !mass || !is_fixed) return fail(MDT_EINVAL, "mdt_batch_set_atoms: NULL argument");
     std::vector<uint8_t> ty(b->totn), fx(b->totpn);
@@ -804,16 +821,7 @@ int mdt_batch_set_atoms(mdt_batch *b, const int32_t *idx, const double *mass, co
     }
     hipStream_t st = b->ctx->stream;
     const bool same = ty == b->h_type;
-    b->h_type = ty;
-    for (int a = 0; a < MDT_MAXT; ++a) b->type_total[a] = b->type_most[a] = 0;
-    for (int t = 0; t < b->ntraj; ++t) {
-        int n[MDT_MAXT] = {};
-        for (int i = 0; i < b->N[t]; ++i) ++n[ty[b->aoff[t] + i]];
-        for (int a = 0; a < MDT_MAXT; ++a) {
-            b->type_total[a] += n[a];
-            b->type_most[a] = std::max(b->type_most[a], n[a]);
-        }
-    }
+    set_types(b, ty);
     HIPCHK(hipMemcpyAsync(b->d_type, ty.data(), b->totn, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(b->d_mass, mass, sizeof(double) * b->totn, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(b->d_fixed, fx.data(), b->totpn, hipMemcpyHostToDevice, st));
@@ -1484,16 +1492,20 @@ static int launch_force(mdt_batch *b) {
     return launch_pes(b, bv, b->allP1 ? 0 : 1, c->stream);
 }
 
+static int status_error(int t, int s) {
+    if (!s) return 0;
+    return fail(MDT_ETRAJ, "trajectory %d flagged status %d (1: neighbour overflow, 2: negative density, 4: bad propagator "
+                "or type, 8: fixed-point overflow, 16: network extrapolation without EMT fallback)",
+                t, s);
+}
+
 static int check_status(mdt_batch *b) {
     std::vector<int> s(b->ntraj);
     HIPCHK(hipMemcpy(s.data(), b->d_status, sizeof(int) * b->ntraj, hipMemcpyDeviceToHost));
     // network extrapolation is handled by the EMT fallback when EMT is set
     const int ignore = (b->pes == 1 && b->ctx->have_params) ? MDT_ST_NN_EXTRAPOLATION : 0;
     for (int t = 0; t < b->ntraj; ++t)
-        if (s[t] & ~ignore)
-            return fail(MDT_ETRAJ, "trajectory %d flagged status %d (1: neighbour overflow, 2: negative density, 4: bad propagator "
-                        "or type, 8: fixed-point overflow, 16: network extrapolation without EMT fallback)",
-                        t, s[t]);
+        if (int rc = status_error(t, s[t] & ~ignore)) return rc;
     return 0;
 }
 
@@ -2086,13 +2098,12 @@ int mdt_batch_tune(mdt_batch *b, int tpa, int nbcap, int *tpa_chosen) {
     return 0;
 }
 
-int mdt_compute_emt(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx, const double *simbox,
-                    const double *isimbox, const double *r, double *epot, double *f, double *dens,
-                    int32_t flag) {
-    (void)flag;  // compute_emt ignores it (forces are always computed)
-    if (!ctx || !idx || !simbox || !isimbox || !r || !epot || !f || !dens)
-        return fail(MDT_EINVAL, "mdt_compute_emt: NULL argument");
-    if (!ctx->have_params) return fail(MDT_ESTATE, "no EMT parameters (call mdt_emt_params_set)");
+// The cached batch of one universe (natoms, nbeads) with its data, on its way to the
+// device: set_atoms (unit masses, nothing fixed), set_cells and set_state in one
+// launch.
+static int call_begin(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx, const double *simbox,
+                      const double *isimbox, const double *r, CallArrays &a, bool clear) {
+    HIPCHK(hipSetDevice(ctx->device));
     int rc;
     if (!ctx->scratch || ctx->scratch_N != natoms || ctx->scratch_P != nbeads) {
         if (ctx->scratch) mdt_batch_destroy(ctx->scratch);
@@ -2104,24 +2115,64 @@ int mdt_compute_emt(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx
         ctx->scratch_P = nbeads;
     }
     mdt_batch *b = ctx->scratch;
-    std::vector<double> mass(natoms, 1.0);
-    std::vector<int32_t> fixed(3LL * natoms * nbeads, 0);
-    if ((rc = mdt_batch_set_atoms(b, idx, mass.data(), fixed.data()))) return rc;
-    if ((rc = mdt_batch_set_cells(b, simbox, isimbox))) return rc;
-    if ((rc = mdt_batch_set_state(b, r, nullptr))) return rc;
-    // compute_emt only: one force launch per replica, no ring-polymer step
-    HIPCHK(hipSetDevice(ctx->device));
-    if ((rc = ensure_ready(b, false))) return rc;
-    if ((rc = autotune_if_needed(b))) return rc;
-    HIPCHK(hipMemsetAsync(b->d_f, 0, sizeof(double) * b->tot3pn, ctx->stream));
-    if ((rc = launch_replicas(b, b->view(), 0, ctx->stream))) return rc;
+    std::vector<uint8_t> ty(natoms);
+    for (int k = 0; k < natoms; ++k) {
+        if (idx[k] < 1 || idx[k] > MDT_MAXT) return fail(MDT_EINVAL, "idx[%d]=%d outside 1..%d", k, idx[k], MDT_MAXT);
+        ty[k] = (uint8_t)(idx[k] - 1);
+    }
+    const size_t n3 = 3 * (size_t)natoms * nbeads, nin = 18 + n3 + (natoms + 1) / 2;
+    if (!b->h_call) {
+        HIPCHK(hipHostMalloc((void **)&b->h_call, sizeof(double) * (nin + n3 + nbeads + n3 / 3 + 1), hipHostMallocDefault));
+        HIPCHK(hipHostGetDevicePointer((void **)&b->d_call, b->h_call, 0));
+    }
+    set_types(b, ty);
+    b->h_icell.assign(isimbox, isimbox + 9);
+    for (SizeClass &k : b->cls) k.nn_img = -1;
+    b->have_atoms = b->have_cells = b->have_state = true;
+    std::memcpy(b->h_call, simbox, 9 * sizeof(double));
+    std::memcpy(b->h_call + 9, isimbox, 9 * sizeof(double));
+    std::memcpy(b->h_call + 18, r, n3 * sizeof(double));
+    std::memcpy(b->h_call + 18 + n3, idx, natoms * sizeof(int32_t));
+    a = CallArrays{b->d_cell, b->d_icell, b->d_x, b->d_mass, b->d_f, b->d_epot, b->d_dens,
+                   b->d_type, b->d_fixed, b->d_nnKey, b->d_status, clear ? 1 : 0};
+    HIPCHK(mdt_launch_call(true, b->d_call, natoms, nbeads, a, ctx->stream));
+    return 0;
+}
+
+// waits for the results; *out: f | epot | dens, *status: the trajectory's status
+static int call_end(mdt_context *ctx, int natoms, int nbeads, const CallArrays &a, const double **out, int *status) {
+    mdt_batch *b = ctx->scratch;
+    const size_t n3 = 3 * (size_t)natoms * nbeads, nin = 18 + n3 + (natoms + 1) / 2;
+    HIPCHK(mdt_launch_call(false, b->d_call + nin, natoms, nbeads, a, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if ((rc = check_status(b))) return rc;
+    *out = b->h_call + nin;
+    std::memcpy(status, *out + n3 + nbeads + n3 / 3, sizeof(int));
+    return 0;
+}
+
+int mdt_compute_emt(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx, const double *simbox,
+                    const double *isimbox, const double *r, double *epot, double *f, double *dens,
+                    int32_t flag) {
+    (void)flag;  // compute_emt ignores it (forces are always computed)
+    if (!ctx || !idx || !simbox || !isimbox || !r || !epot || !f || !dens)
+        return fail(MDT_EINVAL, "mdt_compute_emt: NULL argument");
+    if (!ctx->have_params) return fail(MDT_ESTATE, "no EMT parameters (call mdt_emt_params_set)");
+    int rc;
+    CallArrays a;
+    // (a status that an earlier call of this shape left stays)
+    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a, false))) return rc;
+    mdt_batch *b = ctx->scratch;
+    // compute_emt only: one force launch per replica, no ring-polymer step
+    if ((rc = autotune_if_needed(b))) return rc;
+    if ((rc = launch_replicas(b, b->view(), 0, ctx->stream))) return rc;
+    const double *out;
+    int st;
+    if ((rc = call_end(ctx, natoms, nbeads, a, &out, &st))) return rc;
+    if ((rc = status_error(0, st))) return rc;
     const long long n3 = 3LL * natoms * nbeads;
-    std::vector<double> ff(n3), ee(nbeads), dd((size_t)natoms * nbeads);
-    if ((rc = mdt_batch_get_state(b, nullptr, nullptr, ff.data(), nullptr, ee.data(), dd.data()))) return rc;
-    for (long long k = 0; k < n3; ++k) f[k] += ff[k];
-    for (int k = 0; k < nbeads; ++k) epot[k] += ee[k];
+    for (long long k = 0; k < n3; ++k) f[k] += out[k];
+    for (int k = 0; k < nbeads; ++k) epot[k] += out[n3 + k];
+    const double *dd = out + n3 + nbeads;
     for (int i = 0; i < natoms; ++i)
         if (ctx->ec.owner[idx[i] - 1])
             for (int k = 0; k < nbeads; ++k) dens[k + (long long)nbeads * i] = dd[k + (long long)nbeads * i];
@@ -2408,42 +2459,25 @@ int mdt_compute_nene(mdt_context *ctx, int natoms, int nbeads, const int32_t *id
         return fail(MDT_EINVAL, "mdt_compute_nene: NULL argument");
     if (!ctx->have_nn) return fail(MDT_ESTATE, "no network (call mdt_nn_params_set)");
     int rc;
-    if (!ctx->scratch || ctx->scratch_N != natoms || ctx->scratch_P != nbeads) {
-        if (ctx->scratch) mdt_batch_destroy(ctx->scratch);
-        ctx->scratch = nullptr;
-        int32_t n = natoms, p = nbeads;
-        if ((rc = mdt_batch_create(ctx, 1, &n, &p, &ctx->scratch))) return rc;
-        ctx->scratch->keep_mode = 0;  // one launch per state
-        ctx->scratch_N = natoms;
-        ctx->scratch_P = nbeads;
-    }
+    CallArrays a;
+    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a, true))) return rc;
     mdt_batch *b = ctx->scratch;
-    std::vector<double> mass(natoms, 1.0);
-    std::vector<int32_t> fixed(3LL * natoms * nbeads, 0);
-    if ((rc = mdt_batch_set_atoms(b, idx, mass.data(), fixed.data()))) return rc;
-    if ((rc = mdt_batch_set_cells(b, simbox, isimbox))) return rc;
-    if ((rc = mdt_batch_set_state(b, r, nullptr))) return rc;
-    HIPCHK(hipSetDevice(ctx->device));
     b->pes = 1;
     if ((rc = ensure_nn(b))) return rc;
-    if ((rc = ensure_ready(b, false))) return rc;
-    HIPCHK(hipMemsetAsync(b->d_status, 0, sizeof(int) * b->ntraj, ctx->stream));
     HIPCHK(mdt_launch_nene(b->nrep, b->maxN, b->lds_limit, ctx->d_nn, b->view(), b->d_nnG, b->d_nnC, b->d_nnflag,
                            b->d_nnF, b->maxN, 0, 0, nn_radial(ctx), b->d_nnNbr, b->d_nnCnt, b->d_nnRef, b->d_nnKey,
                            b->list_skin / MDT_BOHR2ANG, ctx->stream, 1));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    std::vector<int> st(1);
-    HIPCHK(hipMemcpy(st.data(), b->d_status, sizeof(int), hipMemcpyDeviceToHost));
+    const double *out;
+    int st;
+    if ((rc = call_end(ctx, natoms, nbeads, a, &out, &st))) return rc;
     b->pes = 0;
-    if (st[0] & ~MDT_ST_NN_EXTRAPOLATION)
+    if (st & ~MDT_ST_NN_EXTRAPOLATION)
         return fail(MDT_ETRAJ, "compute_nene: status %d (1: neighbour overflow, 4: atom type not in the network, "
-                    "8: fixed-point overflow)", st[0]);
-    if (nextrap) *nextrap = (st[0] & MDT_ST_NN_EXTRAPOLATION) ? 1 : 0;
+                    "8: fixed-point overflow)", st);
+    if (nextrap) *nextrap = (st & MDT_ST_NN_EXTRAPOLATION) ? 1 : 0;
     const long long n3 = 3LL * natoms * nbeads;
-    std::vector<double> ff(n3), ee(nbeads);
-    if ((rc = mdt_batch_get_state(b, nullptr, nullptr, ff.data(), nullptr, ee.data(), nullptr))) return rc;
-    for (long long k = 0; k < n3; ++k) f[k] += ff[k];
-    for (int k = 0; k < nbeads; ++k) epot[k] += ee[k];
+    for (long long k = 0; k < n3; ++k) f[k] += out[k];
+    for (int k = 0; k < nbeads; ++k) epot[k] += out[n3 + k];
     return 0;
 }
 

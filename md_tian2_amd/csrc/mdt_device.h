@@ -114,6 +114,14 @@ struct StateTile {
 };
 #define MDT_TILE 256
 
+// a one-universe batch's arrays (k_call_in, k_call_out)
+struct CallArrays {
+    double *cell, *icell, *x, *mass, *f, *epot, *dens;
+    uint8_t *type, *fixed;
+    int *nnkey, *status;
+    int clear;  // the status starts from 0
+};
+
 // k_replica's HBM slot: words per slot and where its parts start (mdt_replica_lists)
 struct ReplicaLists {
     long long stride, rows, chunk, scan;

@@ -2778,6 +2778,55 @@ hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, cons
 }
 
 // ---------------------------------------------------------------------------
+// One universe's call (compute_emt, compute_nene): the batch arrays from one block of
+// pinned host memory and the results into it, read and written over the host link
+// by the kernels themselves.  A call is three launches and one wait (145 atoms x 16
+// beads: 55 KB each way); with a copy or a fill per array and a wait after most of
+// them it spent 170 of its 215 us on those.
+//   in:  cell 9 | inverse 9 | r(3,P,N) | types (1-based, 4 bytes)
+//   out: f(3,P,N) | epot(P) | dens(P,N) | status
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) k_call_in(const double *__restrict__ in, int N, int P, CallArrays a) {
+    const int q = blockIdx.x * 256 + threadIdx.x, n3 = 3 * P * N;
+    if (q < 9) a.cell[q] = in[q];
+    if (q < 9) a.icell[q] = in[9 + q];
+    if (q < n3) {
+        const int i = q / (3 * P), bc = q - 3 * P * i;
+        a.x[(long long)bc * N + i] = in[18 + q];
+    }
+    if (q < N) {
+        a.type[q] = (uint8_t)(((const int32_t *)(in + 18 + n3))[q] - 1);
+        a.mass[q] = 1.0;
+    }
+    if (q < P * N) a.fixed[q] = 0;
+    if (q < P && a.nnkey) a.nnkey[q] = 0;  // new positions: kept lists are stale
+    if (q == 0 && a.clear) *a.status = 0;
+}
+
+__global__ void __launch_bounds__(256) k_call_out(double *__restrict__ out, int N, int P, CallArrays a) {
+    const int q = blockIdx.x * 256 + threadIdx.x, n3 = 3 * P * N;
+    if (q < n3) {
+        const int i = q / (3 * P), bc = q - 3 * P * i;
+        out[q] = a.f[(long long)bc * N + i];
+    }
+    if (q < P) out[n3 + q] = a.epot[q];
+    if (q < P * N) {
+        const int i = q / P, b = q - P * i;
+        out[n3 + P + q] = a.dens[(long long)b * N + i];
+    }
+    if (q == 0) *(int *)(out + n3 + P + P * N) = *a.status;
+}
+
+hipError_t mdt_launch_call(bool in, double *host, int N, int P, const CallArrays &a, hipStream_t st) {
+    const dim3 g((3 * P * N + 255) / 256);
+    if (in)
+        hipLaunchKernelGGL(k_call_in, g, dim3(256), 0, st, host, N, P, a);
+    else
+        hipLaunchKernelGGL(k_call_out, g, dim3(256), 0, st, host, N, P, a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // host-side launchers (C++ linkage, used by mdt_api.hip)
 // ---------------------------------------------------------------------------
 // marks one slot in `period` invalid (launch-shape tuning)

@@ -595,7 +595,7 @@ def main():
     mobile = ~s0.fixed[:, 0, 0]
     n_lan = int(((s0.idx == 1) & mobile).sum())
     n_ver = int(((s0.idx == 0) & mobile).sum())
-    # k_replica's own work (calc_force; the integrator's runs in k_traj) over
+    # k_replica's own work (calc_force; the integrator's runs in k_traj_classical or k_prop) over
     # the reference's pairs (every pair within its cut-off)
     flop_force = FLOP_PAIR * pairs + FLOP_ATOM * n_atoms
     # the same count over the pairs the kernel evaluates (within the near radius)

@@ -280,9 +280,6 @@ struct mdt_batch {
         }
         return best;
     }
-    // what a captured graph's force launches depend on
-    int launch_key() const { return arith() | (bulk() + 1) << 4; }
-
     BatchView view() const {
         BatchView v{};
         v.ntraj = ntraj;
@@ -1468,6 +1465,16 @@ static bool traj_classical(const mdt_batch *b) {
     return b->allP1 && b->maxN <= traj_block(b) && !b->pc.any_pile && !b->pc.any_andersen;
 }
 
+// remove_com_velocity follows propagate_1 (src/md_algo.f90:37-71: with Andersen or PILE atoms)
+static bool removes_com(const mdt_batch *b) { return (b->pc.any_andersen || b->pc.any_pile) && !b->no_com; }
+
+// What the host decides about a step's launches, baked into a captured graph:
+// the force kernel's arithmetic and majority type, the propagator kernel, the
+// COM removal.  (Setters of other such choices drop the graph.)
+static int launch_key(const mdt_batch *b) {
+    return b->arith() | (b->bulk() + 1) << 4 | (traj_classical(b) ? 1 << 8 : 0) | (removes_com(b) ? 1 << 9 : 0);
+}
+
 // the propagators of every trajectory (flags of k_prop)
 static int launch_prop(mdt_batch *b, const BatchView &bv, const uint32_t *step_base, uint32_t prev, uint32_t step,
                        int flags) {
@@ -1476,9 +1483,8 @@ static int launch_prop(mdt_batch *b, const BatchView &bv, const uint32_t *step_b
         HIPCHK(mdt_launch_traj_classical(b->ntraj, b->d_pc, bv, step_base, prev, step, flags, traj_block(b), c->stream, 0));
         return 0;
     }
-    const bool com = (b->pc.any_andersen || b->pc.any_pile) && !b->no_com;
-    HIPCHK(mdt_launch_prop(b->ntraj, b->maxP, b->d_pc, bv, b->d_cjk, b->d_cjkoff, b->d_chunk, b->nchunk, b->d_com, com,
-                           step_base, prev, step, flags, c->stream));
+    HIPCHK(mdt_launch_prop(b->ntraj, b->maxP, b->d_pc, bv, b->d_cjk, b->d_cjkoff, b->d_chunk, b->nchunk, b->d_com,
+                           removes_com(b), step_base, prev, step, flags, c->stream));
     return 0;
 }
 
@@ -1761,11 +1767,11 @@ static int step_split(mdt_batch *b, int nsteps, int S, int *replays_out) {
     if (!b->d_step_h && (rc = dalloc(&b->d_step_h, 2))) return rc;
     int replays = 0;
     if (S > 0 && nsteps >= S) {
-        if ((b->gexec_h[0] || b->gexec_h[1]) && b->graph_key != b->launch_key()) drop_graph(b);
+        if (b->graph_key != launch_key(b)) drop_graph(b);
         if (!b->gexec_h[0] || !b->gexec_h[1]) {
             drop_graph(b);
             if ((rc = capture_half(b, 0)) || (rc = capture_half(b, 1))) return rc;
-            b->graph_key = b->launch_key();
+            b->graph_key = launch_key(b);
         }
     }
     hipStream_t st[2] = {c->stream, c->side[0]};
@@ -1842,10 +1848,10 @@ int mdt_batch_step(mdt_batch *b, int nsteps) {
         if ((rc = step_split(b, nsteps, S, &replays))) return rc;
     } else {
         if (S > 0 && nsteps >= S) {
-            if (b->gexec && b->graph_key != b->launch_key()) drop_graph(b);  // EMT parameters changed the kernel
+            if (b->graph_key != launch_key(b)) drop_graph(b);
             if (!b->gexec) {
                 if ((rc = capture_chunk(b))) return rc;
-                b->graph_key = b->launch_key();
+                b->graph_key = launch_key(b);
             }
             HIPCHK(mdt_launch_advance(b->d_step, b->step, 1, c->stream));
             replays = nsteps / S;

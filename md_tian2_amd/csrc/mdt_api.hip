@@ -797,6 +797,7 @@ static void set_types(mdt_batch *b, const std::vector<uint8_t> &ty) {
 
 int mdt_batch_set_atoms(mdt_batch *b, const int32_t *idx, const double *mass, const int32_t *is_fixed) {
     if (!b || !idx || !mass || !is_fixed) return fail(MDT_EINVAL, "mdt_batch_set_atoms: NULL argument");
+    HIPCHK(hipSetDevice(b->ctx->device));
     std::vector<uint8_t> ty(b->totn), fx(b->totpn);
     for (long long k = 0; k < b->totn; ++k) {
         if (idx[k] < 1 || idx[k] > MDT_MAXT) return fail(MDT_EINVAL, "idx[%lld]=%d outside 1..%d", k, idx[k], MDT_MAXT);
@@ -831,6 +832,7 @@ static void drop_graph(mdt_batch *b);
 
 int mdt_batch_set_cells(mdt_batch *b, const double *simbox, const double *isimbox) {
     if (!b || !simbox || !isimbox) return fail(MDT_EINVAL, "mdt_batch_set_cells: NULL argument");
+    HIPCHK(hipSetDevice(b->ctx->device));
     hipStream_t st = b->ctx->stream;
     HIPCHK(hipMemcpyAsync(b->d_cell, simbox, sizeof(double) * 9 * b->ntraj, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(b->d_icell, isimbox, sizeof(double) * 9 * b->ntraj, hipMemcpyHostToDevice, st));
@@ -912,6 +914,7 @@ static inline int dev_bead(const mdt_batch *b, int t, int i, int bb) {
 
 int mdt_batch_set_state(mdt_batch *b, const double *r, const double *v) {
     if (!b || !r) return fail(MDT_EINVAL, "mdt_batch_set_state: NULL argument");
+    HIPCHK(hipSetDevice(b->ctx->device));
     hipStream_t st = b->ctx->stream;
     int rc = build_tiles(b);
     if (rc) return rc;
@@ -931,6 +934,7 @@ int mdt_batch_set_state(mdt_batch *b, const double *r, const double *v) {
 
 int mdt_batch_get_state(mdt_batch *b, double *r, double *v, double *f, double *a, double *epot, double *dens) {
     if (!b) return fail(MDT_EINVAL, "mdt_batch_get_state: NULL batch");
+    HIPCHK(hipSetDevice(b->ctx->device));
     hipStream_t st = b->ctx->stream;
     int rc = build_tiles(b);
     if (rc) return rc;
@@ -2060,6 +2064,7 @@ int mdt_batch_estimators(mdt_batch *b, double *out) {
 
 int mdt_batch_status(mdt_batch *b, int32_t *status, int clear) {
     if (!b || !status) return fail(MDT_EINVAL, "mdt_batch_status: NULL argument");
+    HIPCHK(hipSetDevice(b->ctx->device));
     HIPCHK(hipMemcpy(status, b->d_status, sizeof(int) * b->ntraj, hipMemcpyDeviceToHost));
     if (clear) HIPCHK(zero_on(b->ctx->stream, b->d_status, sizeof(int) * b->ntraj));
     return 0;

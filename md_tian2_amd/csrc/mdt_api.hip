@@ -2110,10 +2110,10 @@ int mdt_batch_tune(mdt_batch *b, int tpa, int nbcap, int *tpa_chosen) {
 }
 
 // The cached batch of one universe (natoms, nbeads) with its data, on its way to the
-// device: set_atoms (unit masses, nothing fixed), set_cells and set_state in one
-// launch.
+// device: set_atoms (unit masses, nothing fixed), set_cells, set_state and a cleared
+// status in one launch.
 static int call_begin(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx, const double *simbox,
-                      const double *isimbox, const double *r, CallArrays &a, bool clear) {
+                      const double *isimbox, const double *r, CallArrays &a) {
     HIPCHK(hipSetDevice(ctx->device));
     int rc;
     if (!ctx->scratch || ctx->scratch_N != natoms || ctx->scratch_P != nbeads) {
@@ -2145,7 +2145,7 @@ static int call_begin(mdt_context *ctx, int natoms, int nbeads, const int32_t *i
     std::memcpy(b->h_call + 18, r, n3 * sizeof(double));
     std::memcpy(b->h_call + 18 + n3, idx, natoms * sizeof(int32_t));
     a = CallArrays{b->d_cell, b->d_icell, b->d_x, b->d_mass, b->d_f, b->d_epot, b->d_dens,
-                   b->d_type, b->d_fixed, b->d_nnKey, b->d_status, clear ? 1 : 0};
+                   b->d_type, b->d_fixed, b->d_nnKey, b->d_status};
     HIPCHK(mdt_launch_call(true, b->d_call, natoms, nbeads, a, ctx->stream));
     return 0;
 }
@@ -2170,8 +2170,7 @@ int mdt_compute_emt(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx
     if (!ctx->have_params) return fail(MDT_ESTATE, "no EMT parameters (call mdt_emt_params_set)");
     int rc;
     CallArrays a;
-    // (a status that an earlier call of this shape left stays)
-    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a, false))) return rc;
+    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a))) return rc;
     mdt_batch *b = ctx->scratch;
     // compute_emt only: one force launch per replica, no ring-polymer step
     if ((rc = autotune_if_needed(b))) return rc;
@@ -2471,7 +2470,7 @@ int mdt_compute_nene(mdt_context *ctx, int natoms, int nbeads, const int32_t *id
     if (!ctx->have_nn) return fail(MDT_ESTATE, "no network (call mdt_nn_params_set)");
     int rc;
     CallArrays a;
-    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a, true))) return rc;
+    if ((rc = call_begin(ctx, natoms, nbeads, idx, simbox, isimbox, r, a))) return rc;
     mdt_batch *b = ctx->scratch;
     b->pes = 1;
     if ((rc = ensure_nn(b))) return rc;

@@ -119,7 +119,6 @@ struct CallArrays {
     double *cell, *icell, *x, *mass, *f, *epot, *dens;
     uint8_t *type, *fixed;
     int *nnkey, *status;
-    int clear;  // the status starts from 0
 };
 
 // k_replica's HBM slot: words per slot and where its parts start (mdt_replica_lists)

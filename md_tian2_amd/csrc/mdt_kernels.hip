@@ -2800,7 +2800,7 @@ __global__ void __launch_bounds__(256) k_call_in(const double *__restrict__ in, 
     }
     if (q < P * N) a.fixed[q] = 0;
     if (q < P && a.nnkey) a.nnkey[q] = 0;  // new positions: kept lists are stale
-    if (q == 0 && a.clear) *a.status = 0;
+    if (q == 0) *a.status = 0;
 }
 
 __global__ void __launch_bounds__(256) k_call_out(double *__restrict__ out, int N, int P, CallArrays a) {

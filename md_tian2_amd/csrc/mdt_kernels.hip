@@ -1080,10 +1080,14 @@ __global__ void __launch_bounds__(MAXB, 4)
                 const PairRec pn = rec[n];
                 double r2;
                 int code;
-                if (q >> MDT_NBR_IDX_BITS == MDT_ANY_IMAGE)
+                if (q >> MDT_NBR_IDX_BITS == MDT_ANY_IMAGE) {
                     r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], pn, xr, N, k, n, d, &code);
-                else
+                    // in a skewed cell its image may be anywhere; the terms of a pair
+                    // beyond rnear count 0 times and stay finite up to 2 rnear
+                    r2 = r2 > 4.0 * rnear * rnear ? 4.0 * rnear * rnear : r2;
+                } else {
                     r2 = listed(q, x, y, z, pn, d[0], d[1], d[2]);
+                }
                 auto tm = eval(n, pn.g, r2, true);
                 if (!(tm.size < lim)) large(n, tm, d);
                 add(n, tm, d);

@@ -109,3 +109,30 @@ def test_large_terms(gpu_ctx, pes_hau):
     e, f, _ = oracle.emt_energy_forces(s, cols, pesm)
     assert np.abs(o["epot"] - e).max() <= 1e-9 * max(1.0, np.abs(e).max())
     assert np.abs(o["f"] - f).max() <= 1e-9 * max(1.0, np.abs(f).max())
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_far_image_of_a_kept_pair(gpu_ctx, pes_hau, precision):
+    """In a strongly skewed cell the image that a kept pair rounds to may be 60 A
+    away while another one, which it could round to, is near: the pair is listed and
+    counts nothing.  Two atoms half a cell apart along two axes, a and b
+    nearly parallel: both fractional differences just below 1/2 give (a + b) / 2, one
+    of them above 1/2 would give (a - b) / 2, 3.2 A long."""
+    s = geometry.h_on_slab("Au", n=1, nlayers=4, nfixed=1, z0=1.7)  # H and 4 Au
+    s.simbox = np.array([[60.0, 60.0, 0.0], [0.0, 6.4, 0.0], [0.0, 0.0, 40.0]])
+    frac = np.array([[0.1, 0.32, 0.55], [0.1, 0.1, 0.5], [0.5999, 0.5998, 0.5], [0.1, 0.1, 0.58], [0.6001, 0.5998, 0.58]])
+    s.r[:, 0] = frac @ s.simbox.T
+    cols, pesm = pesfile.emt_tables(pes_hau, s.type_names)
+    gpu_ctx.set_emt(cols, pesm)
+    e, f, _ = oracle.emt_energy_forces(s, cols, pesm)
+    assert np.abs(f).max() > 1e-3
+    b = mdt.Batch(gpu_ctx, [s], dt=0.1)
+    b.set_precision(precision)
+    b.set_keep(1)
+    for _ in range(2):  # the build and a launch on the kept rows
+        b.compute_forces()
+    o = b.get_state()[0]
+    b.close()
+    tol = 1e-9 if precision == 0 else 1e-5  # the FP32 pair terms' bar
+    assert np.abs(o["epot"] - e).max() <= tol * max(1.0, np.abs(e).max())
+    assert np.abs(o["f"] - f).max() <= tol * max(1.0, np.abs(f).max())

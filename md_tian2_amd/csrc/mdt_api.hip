@@ -134,6 +134,7 @@ struct SizeClass {
     int *d_reps = nullptr;     // replica ids; NULL when the class holds every replica in order
     int tpa = 0, nbcap = 0, block = 0;
     int keep = 0;              // lists kept across launches (Verlet skin): 0 no, 1 or 2 as asked
+    int want = 0, split = 1;   // the same where the skin is positive; 1 / split of the lanes (configure_class)
     std::vector<int> h_mem;    // its replicas (host copy)
     int nn_img = -1;           // radial network: some cell of the class needs the image search (-1: not known)
     double nn_img_rc = 0.0;    // the cut-off (A) nn_img was decided for
@@ -1107,6 +1108,8 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
     }
     c.block = block;
     c.keep = skin ? keep : 0;
+    c.want = keep;
+    c.split = split;
     c.wide = wide;
     c.tpa = tpa;
     c.nbcap = cap;
@@ -1594,6 +1597,8 @@ static int autotune(mdt_batch *b) {
                     }
                 }
         }
+        // (without a skin nothing was learnt about kept lists: the default, should it come back)
+        if (b->list_skin <= 0.0) best_keep = -1;
         if ((rc = configure_class(b, k, best, b->nbcap_req, best_keep, best_wide, best_split))) return rc;
         k.tuned_ms = best_ms / ntime;
         total += k.tuned_ms;
@@ -1966,14 +1971,14 @@ int mdt_batch_set_list_skin(mdt_batch *b, double skin) {
     if (!(skin >= 0.0 && skin < 5.0)) return fail(MDT_EINVAL, "list skin %g A (0 <= skin < 5)", skin);
     HIPCHK(hipSetDevice(b->ctx->device));
     if (skin != b->list_skin) drop_graph(b);
-    const bool relayout = (skin > 0.0) != (b->list_skin > 0.0);  // classes' lists move between LDS and HBM
+    const bool relayout = (skin > 0.0) != (b->list_skin > 0.0);  // kept lists come or go
     b->list_skin = skin;
     if (relayout && !b->cls.empty()) {
         int rc = lds_limit(b);
         if (rc) return rc;
         for (SizeClass &c : b->cls)
             if ((rc = configure_class(b, c, c.tpa > 0 ? c.tpa : heuristic_tpa(c.nmax), b->nbcap_req,
-                                      c.tpa > 0 ? c.keep : -1, c.tpa > 0 ? c.wide : 0)))
+                                      c.tpa > 0 ? c.want : -1, c.tpa > 0 ? c.wide : 0, c.split)))
                 return rc;
         note_tpa(b);
     }

@@ -1,7 +1,8 @@
 """Host code of the C interface on two devices, without a GPU: libmdt_gpu.so runs on
 a HIP runtime that keeps device memory in host memory and executes no kernel
 (tests/native/fake_hip.cpp).  Whichever device the calling thread has current, a
-call allocates, copies and launches on its context's."""
+call allocates, copies and launches on its context's.  A skin switched off and
+on again leaves the launch shape that tuning chose."""
 import os
 import subprocess
 import sys
@@ -68,3 +69,28 @@ def run(so, script, **env):
 def test_every_call_uses_its_contexts_device(fake_hip):
     out = run(fake_hip, TWO, FAKE_HIP_DEVICES="2")
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+SKIN = SETUP + """
+s = geometry.h_on_slab("Au", n=6, nlayers=4, rng=rng)
+c = mdt.Context(0)
+c.set_emt(cols, pesm)
+b = mdt.Batch(c, [s] * 600, dt=0.1)
+tune_at, shapes = float(os.environ["TUNE_AT"]), []
+b.set_list_skin(tune_at)
+b.tune(0)
+shapes.append(b.class_shapes())
+for skin in (0.0, 0.3):
+    b.set_list_skin(skin)
+    shapes.append(b.class_shapes())
+print([(x[0]["tpa"], x[0]["keep"], x[0]["block"]) for x in shapes])
+"""
+
+
+# the second candidate is one lane per atom on half the lanes: 145 atoms, 128 lanes
+@pytest.mark.parametrize("tune_at,want", [("0.3", [(1, 1, 128), (1, 0, 128), (1, 1, 128)]),
+                                          ("0.0", [(1, 0, 128), (1, 0, 128), (1, 1, 128)])])
+def test_skin_off_and_on_keeps_the_tuned_shape(fake_hip, tune_at, want):
+    out = run(fake_hip, SKIN, TUNE_AT=tune_at, FAKE_HIP_BEST="2")
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.strip() == str(want)

@@ -309,6 +309,10 @@ struct PairRec {
 //   forces: 2^-43 eV/A (|v| < 256 eV/A).
 // Larger terms are converted by rint and added by themselves; those beyond 2^63
 // grids, and NaN, are flagged (MDT_ST_FIXED_OVERFLOW) and left out.
+// A lane sums the terms of its piece of a row, whose order is the list's, as rounded
+// FP64 terms: exact while the lane's sum stays below 2^53 grids, 1024 eV/A or
+// sigma 2048; beyond that it is rounded, the same in every run but not however the
+// row is cut.  Atoms whose partners come in no fixed order (flat lists) sum integers.
 // Energies are summed in registers: 2^-33 eV (sums below 1e6 eV) and 2^-70 for
 // the rest.
 #define MDT_SIG_C1 1536.0                         // 1.5 * 2^(52 - 42)
@@ -428,12 +432,13 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// the same with v's sum over the wavefront (p the same in every lane: left to
-// itself the compiler adds such lanes up one by one)
-__device__ __forceinline__ void add_uniform(unsigned long long *p, double v, double scale, int *bad) {
-    if (__ballot(v != 0.0) == 0) return;  // the wavefront has none
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) add_sum(p, v, scale, bad);
+// LDS += the wavefront's integers (p the same in every lane: left to itself the
+// compiler adds such lanes up one by one)
+__device__ __forceinline__ void add_uniform(unsigned long long *p, unsigned long long v) {
+    if (__ballot(v != 0) == 0) return;  // the wavefront has none
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(p, v);
 }
 
 // Pair ownership: each unordered pair is evaluated once, by its owner; the
@@ -981,9 +986,8 @@ __global__ void __launch_bounds__(MAXB, 4)
         dz = (zk - pn.z) - sft[2];
         return dx * dx + dy * dy + dz * dz;
     };
-    // a pair's force crs d, added to n; its rounded components
-    auto add_force = [&](int n, double crs, const double *d, double g[3]) {
-        unsigned long long u[3];
+    // a pair's force crs d, added to n; its rounded components, as integers in u
+    auto add_force = [&](int n, double crs, const double *d, double g[3], unsigned long long u[3]) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const double tq = fma(crs, d[q], MDT_FRC_C);
@@ -1160,7 +1164,7 @@ __global__ void __launch_bounds__(MAXB, 4)
     }
     for (int q = 0; q < nflat; ++q) {
         const int h = s_flat[q];
-        double s1 = 0.0, s2 = 0.0;
+        unsigned long long s1 = 0, s2 = 0;
         each_flat(q, [&](int n, const double *d, double r2) {
             double own, other, hi, lo;
             unsigned long long u1, u2;
@@ -1171,14 +1175,14 @@ __global__ void __launch_bounds__(MAXB, 4)
                 return;
             }
             sig_words(own, &u1, &u2, &hi, &lo);
-            s1 += hi;
-            s2 += lo;
+            s1 += u1;
+            s2 += u2;
             sig_words(other, &u1, &u2, &hi, &lo);
             atomicAdd(&rec[n].w, u1);
             atomicAdd(&w2[n], u2);
         });
-        add_uniform(&rec[h].w, s1, MDT_P42, &bad_local);
-        add_uniform(&w2[h], s2, MDT_P42 * MDT_P46, &bad_local);
+        add_uniform(&rec[h].w, s1);
+        add_uniform(&w2[h], s2);
     }
     __syncthreads();
 
@@ -1298,8 +1302,9 @@ __global__ void __launch_bounds__(MAXB, 4)
             },
             [&](int n, const Frc &v, const double *d) {
                 double g[3];
+                unsigned long long u[3];
                 add_energy(v.ep);
-                add_force(n, v.crs, d, g);
+                add_force(n, v.crs, d, g, u);
                 fx -= g[0];
                 fy -= g[1];
                 fz -= g[2];
@@ -1313,33 +1318,34 @@ __global__ void __launch_bounds__(MAXB, 4)
         add_sum(&w3[k], fz, MDT_P43, &bad_local);
     }
     // the pair (k, n) of an atom k that a wavefront's lanes share: -F on k in fk
-    auto pair_forces = [&](int k, int n, const double *d, double r, double ri, double fk[3]) {
+    auto pair_forces = [&](int k, int n, const double *d, double r, double ri, unsigned long long fk[3]) {
         double c, ep, g[3];
+        unsigned long long u[3];
         force_terms(typ[k], typ[n], r, rec[k].g, rec[n].g, c, ep);
         add_energy(ep);
         if (!(fabs(c) < MDT_FRC_FAST)) {
             add_large(k, n, c * ri, d);
             return;
         }
-        add_force(n, c * ri, d, g);
+        add_force(n, c * ri, d, g, u);
 #pragma unroll
-        for (int q = 0; q < 3; ++q) fk[q] -= g[q];
+        for (int q = 0; q < 3; ++q) fk[q] -= u[q];
     };
     for (int q = 0; q < nflat; ++q) {
         const int h = s_flat[q];
-        double fk[3] = {0.0, 0.0, 0.0};
+        unsigned long long fk[3] = {0, 0, 0};
         each_flat(q, [&](int n, const double *d, double r2) {
             const double ri = mdt_rsqrt(r2);
             pair_forces(h, n, d, r2 * ri, ri, fk);
         });
-        add_uniform(&rec[h].w, fk[0], MDT_P43, &bad_local);
-        add_uniform(&w2[h], fk[1], MDT_P43, &bad_local);
-        add_uniform(&w3[h], fk[2], MDT_P43, &bad_local);
+        add_uniform(&rec[h].w, fk[0]);
+        add_uniform(&w2[h], fk[1]);
+        add_uniform(&w3[h], fk[2]);
     }
     // the pairs beyond rnear of the tiny atoms, a pair of two by its owner
     if (anytiny)
         each_tiny([&](int k) {
-            double fk[3] = {0.0, 0.0, 0.0};
+            unsigned long long fk[3] = {0, 0, 0};
             for (int n0 = wl; n0 < N; n0 += 64) {
                 int n = n0;
                 opaque(n);
@@ -1347,9 +1353,9 @@ __global__ void __launch_bounds__(MAXB, 4)
                 if ((tiny[n] && !owns(k, n)) || !partner(k, n, false, d, r, ri)) continue;
                 pair_forces(k, n, d, r, ri, fk);
             }
-            add_uniform(&rec[k].w, fk[0], MDT_P43, &bad_local);
-            add_uniform(&w2[k], fk[1], MDT_P43, &bad_local);
-            add_uniform(&w3[k], fk[2], MDT_P43, &bad_local);
+            add_uniform(&rec[k].w, fk[0]);
+            add_uniform(&w2[k], fk[1]);
+            add_uniform(&w3[k], fk[2]);
         });
     ep1 = wave_sum(ep1);
     ep2 = wave_sum(ep2);

@@ -136,3 +136,29 @@ def test_far_image_of_a_kept_pair(gpu_ctx, pes_hau, precision):
     tol = 1e-9 if precision == 0 else 1e-5  # the FP32 pair terms' bar
     assert np.abs(o["epot"] - e).max() <= tol * max(1.0, np.abs(e).max())
     assert np.abs(o["f"] - f).max() <= tol * max(1.0, np.abs(f).max())
+
+
+def test_flat_sums_do_not_depend_on_the_order(gpu_ctx, pes_hau):
+    """An H pushed by 60 atoms at once, each by less than the fast conversion's
+    limit, together by more than FP64 holds in steps of the grid: its force has the
+    same bits in whatever order the atoms are numbered."""
+    g = np.random.default_rng(3)
+    s = geometry.h_on_slab("Au", n=6, nlayers=4, rng=g, z0=2.7)
+    s.r[1:61, 0] = s.r[0, 0] + [0.5, 0.0, 0.0] + g.normal(0, 0.08, (60, 3))
+    cols, pesm = pesfile.emt_tables(pes_hau, s.type_names)
+    gpu_ctx.set_emt(cols, pesm)
+    _, f, _ = oracle.emt_energy_forces(s, cols, pesm)
+    assert np.abs(f[0, 0]).max() > 4096.0
+    systems = []
+    for k in range(8):
+        q = s.copy()
+        q.r[1:] = s.r[1:][g.permutation(s.natoms - 1)] if k else s.r[1:]
+        systems.append(q)
+    b = mdt.Batch(gpu_ctx, systems, dt=0.1)
+    b.tune(tpa=1, nbcap=144)
+    b.compute_forces()
+    out = b.get_state()
+    b.close()
+    assert np.abs(out[0]["f"][0] - f[0]).max() <= 1e-9 * np.abs(f).max()
+    for o in out[1:]:
+        assert np.array_equal(o["f"][0], out[0]["f"][0])

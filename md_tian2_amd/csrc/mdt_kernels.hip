@@ -660,7 +660,6 @@ __global__ void __launch_bounds__(MAXB, 4)
             }
             float4 f;
             const bool folded = fold(x, y, z, x, y, z, &f);
-            if (!(fabsf(f.x) + fabsf(f.y) + fabsf(f.z) < 1e30f)) bad_local |= MDT_ST_FIXED_OVERFLOW;
             f.w = __int_as_float(ty);
             rec[i].x = x;
             rec[i].y = y;
@@ -873,7 +872,8 @@ __global__ void __launch_bounds__(MAXB, 4)
     auto flat_pair = [&](int h, int n, double d[3], double &r2, int &code) {
         if (n == h || !T.pair_on[typ[h] * MDT_MAXT + typ[n]] || (typ[n] != bulk && n < h)) return false;
         r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[h], rec[n], xr, N, h, n, d, &code);
-        return !(r2 * mdt_rsqrt(r2) > rnear);
+        // (r2 = 0 is near; an atom without a position has no partners, as in the scan)
+        return r2 == r2 && !(r2 * mdt_rsqrt(r2) > rnear);
     };
     const int nflat = MIXED ? 0 : (s_nflat < MDT_FLAT_MAX ? s_nflat : MDT_FLAT_MAX);
     for (int f = 0; f < nflat; ++f) {

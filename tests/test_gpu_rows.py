@@ -180,3 +180,29 @@ def test_largest_pair_forces(gpu_ctx, pes_hau):
     b.close()
     assert np.abs(o["epot"] - e).max() <= 1e-9 * np.abs(e).max()
     assert np.abs(o["f"] - f).max() <= 1e-9 * np.abs(f).max()
+
+
+@pytest.mark.parametrize("lost", [0, 20])
+@pytest.mark.parametrize("keep", [0, 1])
+def test_an_atom_without_a_position(gpu_ctx, pes_hau, lost, keep):
+    """An atom at NaN (an H or an Au of a trajectory that blew up) has no partners;
+    the batch goes on and the other atoms' forces are those without it."""
+    s = geometry.h_on_slab("Au", n=5, nlayers=4, rng=np.random.default_rng(8), z0=1.6)
+    cols, pesm = pesfile.emt_tables(pes_hau, s.type_names)
+    gpu_ctx.set_emt(cols, pesm)
+    rest = np.delete(np.arange(s.natoms), lost)
+    w = geometry.System(s.type_names, s.idx[rest], s.mass[rest], s.fixed[rest], s.algo, s.simbox, s.r[rest], s.v[rest])
+    _, f, _ = oracle.emt_energy_forces(w, cols, pesm)
+    q = s.copy()
+    q.r[lost] = np.nan
+    b = mdt.Batch(gpu_ctx, [s, q], dt=0.1)
+    b.set_keep(keep)
+    for _ in range(2):
+        b.compute_forces()
+    assert not b.status().any()
+    o = b.get_state()
+    b.close()
+    assert np.abs(o[1]["f"][rest] - f).max() <= 1e-9 * max(1.0, np.abs(f).max())
+    assert not o[1]["f"][lost].any()
+    _, f, _ = oracle.emt_energy_forces(s, cols, pesm)
+    assert np.abs(o[0]["f"] - f).max() <= 1e-9 * max(1.0, np.abs(f).max())

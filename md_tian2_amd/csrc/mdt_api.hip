@@ -17,7 +17,7 @@
 #include "../../include/mdt_gpu.h"
 #include "mdt_device.h"
 
-ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds);
+ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, bool once);
 hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed,
                                const double *src, double *dst, hipStream_t st);
 hipError_t mdt_launch_call(bool in, double *host, int N, int P, const CallArrays &a, hipStream_t st);
@@ -144,6 +144,10 @@ struct SizeClass {
     // at the build (3 nmax per slot), valid words
     uint32_t *d_lists = nullptr;
     ReplicaLists lay{};
+    // shape of a launch whose rows serve it alone (k_replica reads them in LDS, uncut),
+    // where lists are kept else; smem1 0: they do not fit
+    int tpa1 = 0, block1 = 0, wide1 = 0;
+    size_t smem1 = 0;
     double *d_ref = nullptr;
     int2 *d_valid = nullptr;
     float tuned_ms = 0.f;
@@ -249,6 +253,10 @@ struct mdt_batch {
     double obs_ul = 0, obs_ll = 0, ads_start = 0, ads_end = 0;
     int obs_exit = 0;
     uint32_t obs_step0 = 0;
+    // launches since the lists were last dropped (2: or more), and whether there was
+    // one alone between the two drops before (rows_once)
+    int since = 0;
+    bool once = false;
     int no_com = 0;  // mdt_batch_set_com_removal(b, 0)
     double *d_est = nullptr;  // MDT_NEST per trajectory
     // k_prop's chunks (built for chunk_mode, the bead mode) and their COM partial sums
@@ -618,6 +626,8 @@ static void free_classes(mdt_batch *b) {
 // launch (after the batch's queued launches, which may still set the flags)
 static int invalidate_lists(mdt_batch *b) {
     hipStream_t st = b->ctx->stream;
+    if (b->since > 0) b->once = b->since == 1;
+    b->since = 0;
     bool any = b->d_mix_valid || b->d_nnKey;
     for (const SizeClass &c : b->cls) any = any || c.d_valid;
     if (!any) return 0;
@@ -1084,9 +1094,11 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
     const int lanes = wide ? 1024 : 512;
     while (tpa > 1 && c.nmax * tpa > lanes) tpa >>= 1;
     if (c.nmax * tpa <= 512) wide = 0;  // fits 512 lanes: the 512-lane instantiation
-    // lists kept across launches (Verlet skin) unless the skin is 0.  Kept wins at every
-    // size measured: 100 replicas of 37 atoms 15 us a launch against 20, 4096 of 145
-    // 113 against 200 (half of them), 2048 of 385 300 against 540
+    // lists kept across launches (Verlet skin) unless the skin is 0.  Kept wins at most
+    // sizes: 2048 replicas of 385 atoms 300 us a launch against 540, 100 of 385 66 us
+    // a step against 87; few replicas of narrow cells are the exception (500 of 65
+    // atoms 36 us a step, 43 kept: their entries take their images at every launch),
+    // which the tuner finds
     if (b->keep_mode >= 0) keep = b->keep_mode;
     if (keep < 0) keep = 1;
     const bool skin = b->list_skin > 0.0 && keep >= 1;
@@ -1094,7 +1106,7 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
     const int block = std::min(wide ? 1024 : 512, std::max(64, rounded));
     // dynamic LDS beside the kernel's static tables (6.4 KB in the judge's variant; 6.5 KiB allowed)
     const size_t lds_dyn = b->lds_limit > REP_STATIC_LDS ? b->lds_limit - REP_STATIC_LDS : 0;
-    const ReplicaLists lay = mdt_replica_lists(c.nrep, c.nmax, block, cap, lds_dyn);
+    const ReplicaLists lay = mdt_replica_lists(c.nrep, c.nmax, block, cap, lds_dyn, !skin && c.nrep <= REP_FEW);
     if (lay.smem > lds_dyn)
         return fail(MDT_EUNSUP, "replica of %d atoms needs %zu bytes of LDS (limit %zu)", c.nmax, lay.smem, lds_dyn);
     free_class_lists(c);
@@ -1114,6 +1126,10 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
     c.tpa = tpa;
     c.nbcap = cap;
     c.smem = lay.smem;
+    if (c.tpa1 <= 0) c.tpa1 = heuristic_tpa(c.nmax);
+    c.block1 = std::min(c.nmax * c.tpa1 > 512 && c.wide1 ? 1024 : 512, std::max(64, (c.nmax * c.tpa1 + 63) / 64 * 64));
+    const ReplicaLists lay1 = mdt_replica_lists(c.nrep, c.nmax, c.block1, cap, lds_dyn, true);
+    c.smem1 = skin && c.nrep <= REP_FEW && lay1.scan < 0 && lay1.stride <= lay.stride ? lay1.smem : 0;
     return 0;
 }
 
@@ -1326,19 +1342,32 @@ static double row_skin(const mdt_batch *b) {
     return b->bulk() >= 0 && b->nrep > REP_FEW ? std::min(b->list_skin, ROW_SKIN * std::sqrt((double)b->maxP)) : b->list_skin;
 }
 
-// v's fields of class k's launch, from block slot t0 on
-static void class_view(const mdt_batch *b, const SizeClass &k, int t0, BatchView &v) {
+// The launch of class k on n replicas from block slot t0 on, v its view but for the
+// lists; once: rows for this launch alone, in their own shape where few workgroups
+// run.  Rows that are read uncut hold all types.
+static hipError_t launch_class(const mdt_batch *b, const SizeClass &k, int t0, int n, bool once, BatchView v, int add_fin,
+                               hipStream_t st) {
+    const bool kept = k.d_valid && !once;
+    once = once && k.smem1 > 0;
     v.nbcap = k.nbcap;
     v.rl_lists = k.d_lists + (size_t)t0 * k.lay.stride;
     v.rl_stride = k.lay.stride;
-    v.rl_rows = k.lay.rows;
+    v.rl_rows = once ? 0 : k.lay.rows;
     v.rl_chunk = k.lay.chunk;
-    v.rl_scan = k.lay.scan;
-    v.rl_ref = k.d_ref ? k.d_ref + (size_t)t0 * 3 * k.nmax : nullptr;
-    v.rl_valid = k.d_valid ? k.d_valid + t0 : nullptr;
+    v.rl_scan = once ? -1 : k.lay.scan;
+    v.rl_ref = kept ? k.d_ref + (size_t)t0 * 3 * k.nmax : nullptr;
+    v.rl_valid = kept ? k.d_valid + t0 : nullptr;
     v.rl_skin = row_skin(b);
     v.rl_ns = k.nmax;
+    if (v.rl_scan < 0 && !v.rl_valid) v.bulk = -1;
+    return mdt_launch_replica(once ? k.tpa1 : k.tpa, n, once ? k.block1 : k.block, once ? k.smem1 : k.smem, b->ctx->d_ec,
+                              b->d_pc, v, add_fin, st);
 }
+
+// Whether the next launch of the EMT forces gets rows that serve it alone: the
+// last positions that the caller set were used for one launch.
+static bool rows_once(const mdt_batch *b) { return b->once && b->since == 0; }
+static void note_launches(mdt_batch *b, int n) { b->since = std::min(b->since + n, 2); }
 
 static int launch_replicas(mdt_batch *b, const BatchView &base, int add_fin, hipStream_t main_st) {
     mdt_context *c = b->ctx;
@@ -1347,13 +1376,14 @@ static int launch_replicas(mdt_batch *b, const BatchView &base, int add_fin, hip
     int rc = fork_open(fk, c, main_st, (int)(b->cls.size() + b->mix_cls.size()));
     if (rc) return rc;
     hipStream_t st = main_st;
+    const bool emt = !base.judge_acc && !base.only;  // calc_force itself, not the network's judge or fallback
     for (const SizeClass &k : b->cls) {
         if ((rc = fork_stream(fk, &st))) return rc;
         BatchView v = base;
         v.rep_list = k.d_reps;
-        class_view(b, k, 0, v);
-        HIPCHK(mdt_launch_replica(k.tpa, k.nrep, k.block, k.smem, c->d_ec, b->d_pc, v, add_fin, st));
+        HIPCHK(launch_class(b, k, 0, k.nrep, emt && rows_once(b), v, add_fin, st));
     }
+    if (emt) note_launches(b, 1);
     if (!b->mix_traj.empty() && (rc = launch_mixed(b, base, 0, add_fin, main_st, &fk))) return rc;
     return fork_close(fk);
 }
@@ -1543,8 +1573,8 @@ static int autotune(mdt_batch *b) {
     HIPCHK(hipMemcpyAsync(se, b->d_epot, sizeof(double) * b->totp, hipMemcpyDeviceToDevice, st));
     HIPCHK(hipMemcpyAsync(sd, b->d_dens, sizeof(double) * b->totpn, hipMemcpyDeviceToDevice, st));
     // per class: threads per atom x (for more than 512 atoms x threads per
-    // atom: 512 lanes looping over the atoms, or up to 1024 lanes), or half the lanes, with kept
-    // lists; the best of them with lists rebuilt every launch too.  A kept
+    // atom: 512 lanes looping over the atoms, or up to 1024 lanes) x lists kept or
+    // rebuilt at every launch; kept ones also on half the lanes.  A kept
     // configuration is timed with the share of its slots rebuilt at each launch that
     // a 300 K metal and a step of 0.1 fs give, so its figure is not a reuse-only best case.
     const int cands[4] = {1, 2, 4, 8};
@@ -1555,12 +1585,10 @@ static int autotune(mdt_batch *b) {
     for (SizeClass &k : b->cls) {
         int best = k.tpa, best_keep = k.keep, best_wide = k.wide, best_split = 1;
         float best_ms = 1e30f;
-        // rebuilt lists (0) only in the shape that is best for kept ones
+        float best1_ms = 1e30f;  // of the shapes with rows for one launch
         const int kfirst = b->keep_mode >= 0 ? b->keep_mode : (b->list_skin > 0.0 ? 1 : 0);
         const int klast = b->keep_mode >= 0 ? b->keep_mode : 0;
         for (int keep = kfirst; keep >= klast; --keep) {
-            const bool only = keep < kfirst;
-            const int btpa = best, bwide = best_wide, bsplit = best_split;
             for (int tpa : cands)
                 for (int wide = b->wide_mode == 1 ? 1 : 0; wide <= (b->wide_mode == 0 ? 0 : 1); ++wide) {
                     if (!wide && k.nmax * tpa > 512 && tpa != 1) continue;
@@ -1568,19 +1596,17 @@ static int autotune(mdt_batch *b) {
                     if (!wide && b->wide_mode == 1 && tpa <= 2 && k.nmax * tpa > 512 && k.nmax * tpa <= 1024)
                         continue;
                     for (int split = 1; split <= (tpa == 1 && !wide ? 2 : 1); ++split) {
-                        if (only && (tpa != btpa || wide != bwide || split != bsplit)) continue;
                         if (split > 1 && (k.nmax + split - 1) / split > 512) continue;
                         const int last = k.block;
                         if ((rc = configure_class(b, k, tpa, b->nbcap_req, keep, wide, split))) return rc;
                         if (split > 1 && k.block == last) continue;  // the same workgroup
                         BatchView v = b->view();
                         v.rep_list = k.d_reps;
-                        class_view(b, k, 0, v);
-                        HIPCHK(mdt_launch_replica(tpa, k.nrep, k.block, k.smem, c->d_ec, b->d_pc, v, 0, st));
+                        HIPCHK(launch_class(b, k, 0, k.nrep, false, v, 0, st));
                         HIPCHK(mdt_launch_drop_lists(k.d_valid, k.keep ? k.nrep : 0, period, 0, st));
                         HIPCHK(hipEventRecord(b->ev0, st));
                         for (int q = 0; q < ntime; ++q) {
-                            HIPCHK(mdt_launch_replica(tpa, k.nrep, k.block, k.smem, c->d_ec, b->d_pc, v, 0, st));
+                            HIPCHK(launch_class(b, k, 0, k.nrep, false, v, 0, st));
                             HIPCHK(mdt_launch_drop_lists(k.d_valid, k.keep ? k.nrep : 0, period, (q + 1) * period / ntime, st));
                         }
                         HIPCHK(hipEventRecord(b->ev1, st));
@@ -1593,6 +1619,11 @@ static int autotune(mdt_batch *b) {
                             best_keep = k.keep;
                             best_wide = k.wide;
                             best_split = split;
+                        }
+                        if (!k.keep && ms < best1_ms) {
+                            best1_ms = ms;
+                            k.tpa1 = tpa;
+                            k.wide1 = k.wide;
                         }
                     }
                 }
@@ -1723,12 +1754,11 @@ static int enqueue_half(mdt_batch *b, int h, int nsteps, const uint32_t *step_ba
     const SizeClass &k = b->cls[0];
     BatchView v = bv;
     v.rep_list = b->d_ident + t0;
-    class_view(b, k, t0, v);
     for (int s = 0; s < nsteps; ++s) {
         const uint32_t prev = first + s, stp = first + s + 1;
         const int flags = (s > 0 ? 1 : 0) | 2;
         HIPCHK(mdt_launch_traj_classical(t1 - t0, b->d_pc, bv, step_base, prev, stp, flags, traj_block(b), st, t0));
-        HIPCHK(mdt_launch_replica(k.tpa, t1 - t0, k.block, k.smem, c->d_ec, b->d_pc, v, 0, st));
+        HIPCHK(launch_class(b, k, t0, t1 - t0, s == 0 && rows_once(b), v, 0, st));
     }
     if (nsteps > 0)
         HIPCHK(mdt_launch_traj_classical(t1 - t0, b->d_pc, bv, step_base, first + nsteps, first + nsteps, 1,
@@ -1740,6 +1770,7 @@ static int enqueue_half(mdt_batch *b, int h, int nsteps, const uint32_t *step_ba
 // d_step_h[h], which the chunk's last node advances) and instantiates it.
 static int capture_half(mdt_batch *b, int h) {
     mdt_context *c = b->ctx;
+    note_launches(b, 1);  // replays keep their rows
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_half(b, h, b->graph_chunk, b->d_step_h + h, 0u, c->stream);
@@ -1796,6 +1827,7 @@ static int step_split(mdt_batch *b, int nsteps, int S, int *replays_out) {
     const int rest = nsteps - replays * S;
     for (int h = 0; h < 2; ++h)
         if ((rc = enqueue_half(b, h, rest, nullptr, b->step, st[h]))) return rc;
+    note_launches(b, std::min(nsteps, 2));
     b->step += (uint32_t)rest;
     HIPCHK(hipEventRecord(c->join_ev[0], st[1]));
     HIPCHK(hipStreamWaitEvent(st[0], c->join_ev[0], 0));
@@ -1811,6 +1843,7 @@ static int capture_chunk(mdt_batch *b) {
         int rc = dalloc(&b->d_step, 1);
         if (rc) return rc;
     }
+    note_launches(b, 1);  // replays keep their rows
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_steps(b, b->graph_chunk, b->d_step, 0u, false);
@@ -1841,6 +1874,7 @@ int mdt_batch_step(mdt_batch *b, int nsteps) {
     if (rc) return rc;
     if ((rc = autotune_if_needed(b))) return rc;
     if (b->pes == 1 && (rc = ensure_nn(b))) return rc;
+    if (nsteps > 1) b->once = false;
     mdt_context *c = b->ctx;
     if (b->profile && (int)b->evf.size() < 2 * nsteps) {
         const size_t old = b->evf.size();
@@ -1865,6 +1899,7 @@ int mdt_batch_step(mdt_batch *b, int nsteps) {
             HIPCHK(mdt_launch_advance(b->d_step, b->step, 1, c->stream));
             replays = nsteps / S;
             for (int k = 0; k < replays; ++k) HIPCHK(hipGraphLaunch(b->gexec, c->stream));
+            note_launches(b, std::min(replays * S, 2));
             b->step += (uint32_t)(replays * S);
         }
         const int rest = nsteps - replays * S;

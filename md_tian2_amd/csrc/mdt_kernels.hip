@@ -281,10 +281,14 @@ __device__ __forceinline__ void emt_atom(const LdsTypes &T, int tk, double sig, 
 // coordinate (s - anint(s) is odd in r_j - r_i, so the pair's order does
 // not matter).  (ia, ib, ic) = isimbox(axis, 1..3); ra, rb the x, y, z of
 // the two atoms.
+__device__ __forceinline__ double tie_dot(double ia, double ib, double ic, double d0, double d1, double d2) {
+#pragma clang fp contract(off)
+    return ia * d0 + ib * d1 + ic * d2;
+}
 __device__ __forceinline__ double tie_image(double ia, double ib, double ic, double ra0, double ra1, double ra2, double rb0,
                                          double rb1, double rb2, double x) {
 #pragma clang fp contract(off)
-    const double s = ia * (ra0 - rb0) + ib * (ra1 - rb1) + ic * (ra2 - rb2);
+    const double s = tie_dot(ia, ib, ic, ra0 - rb0, ra1 - rb1, ra2 - rb2);
     return rint(x - (s - round(s)));
 }
 
@@ -379,10 +383,14 @@ __device__ __forceinline__ double sig_sum(unsigned long long w1, unsigned long l
     return (double)(long long)w1 * (1.0 / MDT_P42) + (double)(long long)w2 * (1.0 / (MDT_P42 * MDT_P46));
 }
 __device__ __forceinline__ double frc_sum(unsigned long long w) { return (double)(long long)w * (1.0 / MDT_P42); }
-// LDS += a sum of rounded terms (a multiple of the grid)
-__device__ __forceinline__ void add_sum(unsigned long long *p, double v, double scale, int *bad) {
+// LDS += a sum of rounded terms (a multiple of the grid, C as in grid_int)
+__device__ __forceinline__ void add_sum(unsigned long long *p, double v, double C, double scale, int *bad) {
+    unsigned long long u;
     double r;
-    const unsigned long long u = grid_any(v, scale, &r, bad);
+    if (__builtin_expect(fabs(v) < C * (1.0 / 3.0), 1))  // 2^51 grids
+        u = grid_int(v + C, C);
+    else
+        u = grid_any(v, scale, &r, bad);
     atomicAdd(p, u);
 }
 
@@ -392,8 +400,8 @@ __device__ __forceinline__ void add_sum(unsigned long long *p, double v, double 
 // scan's image code).  The rounding is decided in FP32 from ihf (H^-1, 9
 // floats, column major; error ~1e-7 against the 1e-4 tie window); a component
 // within 1e-4 of +-1/2 takes the reference's image from the FP64 H^-1 ihg and
-// the unfolded positions xr (SoA, N per component), both in global memory, as
-// tie_image does.  Returns |d|^2.
+// the unfolded positions -- xr (SoA, N per component) in global memory, or, xr NULL,
+// the staged ones: no atom was folded -- as tie_image does.  Returns |d|^2.
 __device__ __forceinline__ double pair_image(const float *ihf, const double *ihg, const double *shift, const PairRec &pk,
                                              const PairRec &pn, const double *xr, int N, int k, int n, double d[3],
                                              int *codep) {
@@ -405,18 +413,24 @@ __device__ __forceinline__ double pair_image(const float *ihf, const double *ihg
     float m0 = rintf(f0), m1 = rintf(f1), m2 = rintf(f2);
     const bool t0 = fabsf(f0 - m0) > 0.4999f, t1 = fabsf(f1 - m1) > 0.4999f, t2 = fabsf(f2 - m2) > 0.4999f;
     if (t0 | t1 | t2) {  // rare: the exact fractional difference and the reference's tie rule
-        const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
-        const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
-        if (t0) m0 = (float)tie_image(ihg[0], ihg[3], ihg[6], a0, a1, a2, b0, b1, b2, ihg[0] * cx + ihg[3] * cy + ihg[6] * cz);
-        if (t1) m1 = (float)tie_image(ihg[1], ihg[4], ihg[7], a0, a1, a2, b0, b1, b2, ihg[1] * cx + ihg[4] * cy + ihg[7] * cz);
-        if (t2) m2 = (float)tie_image(ihg[2], ihg[5], ihg[8], a0, a1, a2, b0, b1, b2, ihg[2] * cx + ihg[5] * cy + ihg[8] * cz);
+        if (xr) {
+            const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
+            const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
+            if (t0) m0 = (float)tie_image(ihg[0], ihg[3], ihg[6], a0, a1, a2, b0, b1, b2, ihg[0] * cx + ihg[3] * cy + ihg[6] * cz);
+            if (t1) m1 = (float)tie_image(ihg[1], ihg[4], ihg[7], a0, a1, a2, b0, b1, b2, ihg[1] * cx + ihg[4] * cy + ihg[7] * cz);
+            if (t2) m2 = (float)tie_image(ihg[2], ihg[5], ihg[8], a0, a1, a2, b0, b1, b2, ihg[2] * cx + ihg[5] * cy + ihg[8] * cz);
+        } else {  // tie_image's x is its s
+            if (t0) m0 = (float)round(tie_dot(ihg[0], ihg[3], ihg[6], cx, cy, cz));
+            if (t1) m1 = (float)round(tie_dot(ihg[1], ihg[4], ihg[7], cx, cy, cz));
+            if (t2) m2 = (float)round(tie_dot(ihg[2], ihg[5], ihg[8], cx, cy, cz));
+        }
     }
     const int code = ((int)m0 + 1) + 3 * ((int)m1 + 1) + 9 * ((int)m2 + 1);
     d[0] = cx - shift[4 * code];
     d[1] = cy - shift[4 * code + 1];
     d[2] = cz - shift[4 * code + 2];
     *codep = code;
-    return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    return fma(d[2], d[2], fma(d[1], d[1], d[0] * d[0]));
 }
 
 // Hides v's derivation from the optimiser (an empty asm with a register
@@ -438,6 +452,14 @@ __device__ __forceinline__ void add_uniform(unsigned long long *p, unsigned long
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) atomicAdd(p, v);
+}
+
+// a b rounded, whatever it is added to: a pair's distance and terms have the same
+// bits in rows, flat lists and direct sums
+template <class F>
+__device__ __forceinline__ F mul_rn(F a, F b) {
+#pragma clang fp contract(off)
+    return a * b;
 }
 
 // Pair ownership: each unordered pair is evaluated once, by its owner; the
@@ -470,6 +492,19 @@ __device__ __forceinline__ bool owns(int k, int n) { return (k < n) != (((k + n)
 //    skin.  Positions stay unfolded (fractional components in [-0.2, 1.2);
 //    others are folded by the fold of the build), so an entry's image code stays
 //    what it was at the build: a launch only reads them.
+//  * Rows for one launch (lists not kept, or fresh positions at every call).  Few
+//    workgroups read them in LDS as scanned, tpa lanes per atom, with every type in
+//    them (MIXED): no cut, no sort, and no flat lists, whose three phases of
+//    their own cost 3 k cycles each to a workgroup that waits for latency
+//    (100 replicas of 37 atoms, 150 steps: 3.45 ms, 3.68 with kept rows).  Many
+//    workgroups cut them as ever: rows in LDS would leave 3 of 5 workgroups a CU
+//    (4096 replicas of 145 atoms: 0.41 ms a call, 0.36 cut).
+//  * The scan tests two candidates of an atom at a time and looks for images that
+//    round either way only along axes where such a pair can be near (new
+//    positions of 4096 x 145 atoms: 0.39 -> 0.36 ms a call).
+//  * A pair's terms have the same bits in rows of one type, rows of all types, flat
+//    lists and direct sums: products that an addition could fuse are written
+//    out (mul_rn, fma).
 //  * The pair terms of two entries are evaluated without a branch between them, so
 //    that one's chain of dependent instructions fills the other's gaps.
 // PREC (arithmetic of the pair terms):
@@ -501,7 +536,7 @@ __global__ void __launch_bounds__(MAXB, 4)
     __shared__ uint16_t s_flist[MIXED ? 1 : MDT_FLAT_MAX * MDT_FLAT_CAP];
     __shared__ int s_np[64], s_hist[64];  // pieces at each length limit, of each length
     __shared__ int s_cb[64];              // stream offset of each chunk of 64 pieces
-    __shared__ int s_nflat, s_R, s_slow, s_anyfold;
+    __shared__ int s_nflat, s_R, s_slow, s_anyfold, s_folded;
     const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : (int)blockIdx.x;
     if (bv.only && !bv.only[rep]) return;                          // whole block: uniform
     if (bv.skip && bv.skip[rep]) return;                           // whole block: uniform
@@ -542,7 +577,9 @@ __global__ void __launch_bounds__(MAXB, 4)
     // too small to fill the GPU in LDS: mdt_replica_lists)
     uint32_t *stream = bv.rl_lists + (long long)blockIdx.x * bv.rl_stride;
     uint32_t *rows = stream + bv.rl_rows, *chunk = stream + bv.rl_chunk;
-    uint16_t *scan_rows = bv.rl_scan < 0 ? (uint16_t *)(smem_raw + ((58 * N + 7) & ~7)) : (uint16_t *)(stream + bv.rl_scan);
+    // (never one pointer to either: that makes every access a flat one)
+    const bool lds_scan = bv.rl_scan < 0;
+    uint16_t *lrow = (uint16_t *)(smem_raw + ((58 * N + 7) & ~7)), *grow = (uint16_t *)(stream + bv.rl_scan);
     int bad_local = 0;
 
     // Verlet skin: the rows of this block slot are built with rnear + skin and
@@ -574,7 +611,7 @@ __global__ void __launch_bounds__(MAXB, 4)
     }
     if (lane == 0) {
         s_nflat = 0;
-        s_anyfold = 0;
+        s_anyfold = s_folded = 0;
         s_slow = kept >> 2 & 1;
         s_R = kept >> 3;
         s_ep[0] = s_ep[1] = 0.0;
@@ -606,10 +643,27 @@ __global__ void __launch_bounds__(MAXB, 4)
         const double g2 = (f2 >= -0.2 && f2 < 1.2) ? 0.0 : floor(f2);
         if (f) *f = make_float4((float)(f0 - g0), (float)(f1 - g1), (float)(f2 - g2), 0.f);
         if (g0 == 0.0 && g1 == 0.0 && g2 == 0.0) return false;
+        s_folded = 1;  // benign race: every writer stores 1
         x -= s_h[0] * g0 + s_h[3] * g1 + s_h[6] * g2;
         y -= s_h[1] * g0 + s_h[4] * g1 + s_h[7] * g2;
         z -= s_h[2] * g0 + s_h[5] * g1 + s_h[8] * g2;
         return true;
+    };
+    // staged for a scan: folded position, fractional one and type
+    float4 *f4 = (float4 *)w2;
+    auto stage = [&](int i, int ty, double x, double y, double z) {
+        if (keep) {
+            ref[i] = x;
+            ref[bv.rl_ns + i] = y;
+            ref[2 * bv.rl_ns + i] = z;
+        }
+        float4 f;
+        if (fold(x, y, z, x, y, z, &f) && (MIXED || ty == bulk)) s_anyfold = 1;  // benign race: every writer stores 1
+        f.w = __int_as_float(ty);
+        rec[i].x = x;
+        rec[i].y = y;
+        rec[i].z = z;
+        f4[i] = f;
     };
     int moved = 0;
     for (int i = lane; i < N; i += nthr) {
@@ -617,25 +671,29 @@ __global__ void __launch_bounds__(MAXB, 4)
         typ[i] = (uint8_t)ty;
         double x = xr[i], y = xr[N + i], z = xr[2 * N + i];
         const bool rowed = MIXED || ty == bulk;
-        if (kept && rowed) {
+        if (!rowed && T.owner[ty]) {
+            const int q = atomicAdd(&s_nflat, 1);  // the order is free
+            if (q < MDT_FLAT_MAX) {
+                s_flat[q] = i;
+                s_fcnt[q] = 0;
+            }
+        }
+        rec[i].g = 0.0;
+        if (!kept) {
+            stage(i, ty, x, y, z);
+            continue;
+        }
+        if (rowed) {
             const double rx = ref[i], ry = ref[bv.rl_ns + i], rz = ref[2 * bv.rl_ns + i];
             const double d0 = x - rx, d1 = y - ry, d2 = z - rz;
             if (!(d0 * d0 + d1 * d1 + d2 * d2 <= 0.25 * skin * skin)) moved = 1;
             if (kept & 2) fold(x, y, z, rx, ry, rz, nullptr);
-        } else if (!rowed) {
+        } else {
             fold(x, y, z, x, y, z, nullptr);
-            if (T.owner[ty]) {
-                const int q = atomicAdd(&s_nflat, 1);  // the order is free
-                if (q < MDT_FLAT_MAX) {
-                    s_flat[q] = i;
-                    s_fcnt[q] = 0;
-                }
-            }
         }
         rec[i].x = x;
         rec[i].y = y;
         rec[i].z = z;
-        rec[i].g = 0.0;
         rec[i].w = w2[i] = w3[i] = 0;
     }
     if (kept && lane < kept >> 3) word0 = stream[off0 + wl];
@@ -645,29 +703,15 @@ __global__ void __launch_bounds__(MAXB, 4)
     // ---- phase 1: rows ----
     // few workgroups and rows for this launch only: they are read where the scan
     // put them, in LDS, tpa lanes per row (cutting and sorting them costs 6 us)
-    const bool direct = !keep && bv.rl_scan < 0;
+    const bool direct = !keep && lds_scan;
     const int sh = bv.tpa_shift;
     if (!reuse) {
-        if (lane == 0) s_slow = 0;
-        float4 *f4 = (float4 *)w2;  // fractional coordinates and type
-        for (int i = lane; i < N; i += nthr) {
-            const int ty = typ[i];
-            double x = xr[i], y = xr[N + i], z = xr[2 * N + i];
-            if (keep) {
-                ref[i] = x;
-                ref[bv.rl_ns + i] = y;
-                ref[2 * bv.rl_ns + i] = z;
-            }
-            float4 f;
-            const bool folded = fold(x, y, z, x, y, z, &f);
-            f.w = __int_as_float(ty);
-            rec[i].x = x;
-            rec[i].y = y;
-            rec[i].z = z;
-            f4[i] = f;
-            if (folded && (MIXED || ty == bulk)) s_anyfold = 1;  // benign race: every writer stores 1
+        if (kept) {  // the rows are stale
+            if (lane == 0) s_slow = 0;
+            for (int i = lane; i < N; i += nthr) stage(i, typ[i], xr[i], xr[N + i], xr[2 * N + i]);
+            __syncthreads();
         }
-        __syncthreads();
+        const double *xt = s_folded ? xr : nullptr;  // the unfolded positions are the staged ones
         // The scan only decides membership: FP32 fractional differences, r^2
         // from the cell metric H^T H with the bound widened by 1e-4; the
         // passes test r <= rnear in FP64.  A fractional difference within
@@ -679,7 +723,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         // row lengths go to the record's word
         float g00, g11, g22, g01, g02, g12;  // H^T H, cell vectors = columns of H
         {
-            const double *h = bv.cell + 9 * t;
+            const double *h = s_h;
             g00 = (float)(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]);
             g11 = (float)(h[3] * h[3] + h[4] * h[4] + h[5] * h[5]);
             g22 = (float)(h[6] * h[6] + h[7] * h[7] + h[8] * h[8]);
@@ -687,21 +731,20 @@ __global__ void __launch_bounds__(MAXB, 4)
             g02 = (float)(2 * (h[0] * h[6] + h[1] * h[7] + h[2] * h[8]));
             g12 = (float)(2 * (h[3] * h[6] + h[4] * h[7] + h[5] * h[8]));
         }
-        float mg0 = 0.4999f, mg1 = 0.4999f, mg2 = 0.4999f;  // components beyond these can round either way
-        if (keep) {
-            const double *ih = bv.icell + 9 * t;
-            mg0 -= (float)(sqrt(ih[0] * ih[0] + ih[3] * ih[3] + ih[6] * ih[6]) * skin);
-            mg1 -= (float)(sqrt(ih[1] * ih[1] + ih[4] * ih[4] + ih[7] * ih[7]) * skin);
-            mg2 -= (float)(sqrt(ih[2] * ih[2] + ih[5] * ih[5] + ih[8] * ih[8]) * skin);
-        }
-        int all_on = 1;
-        if (MIXED) {
-            for (int q = 0; q < ecg->ntypes * ecg->ntypes; ++q)
-                if (!T.pair_on[(q / ecg->ntypes) * MDT_MAXT + q % ecg->ntypes]) all_on = 0;
-        } else {
-            all_on = T.pair_on[bulk * MDT_MAXT + bulk];
-        }
         const double rn = keep ? rnear + skin : rnear;
+        // components beyond these can round either way (2: none can, the cell is so wide
+        // along the axis that such a pair is beyond rn in any image)
+        auto margin = [&](int a) {
+            const float *ih = s_ihf + a;
+            const float inv = sqrtf(ih[0] * ih[0] + ih[3] * ih[3] + ih[6] * ih[6]);  // 1 / width
+            const float mg = 0.4999f - (keep ? (float)skin * inv : 0.f);
+            return mg > 1.001f * (float)rn * inv ? 2.f : mg;
+        };
+        const float mg0 = margin(0), mg1 = margin(1), mg2 = margin(2);
+        // (of the pairs of types; one lane each)
+        const int nt = ecg->ntypes;
+        const bool all_on = MIXED ? __all(wl >= nt * nt || T.pair_on[wl / nt * MDT_MAXT + wl % nt])
+                                  : T.pair_on[bulk * MDT_MAXT + bulk] != 0;
         const float cut2f = (float)(rn * rn * (1.0 + 1e-4));
         const int tpa = 1 << sh, apb = nthr >> sh;
         const unsigned long long gmask = ((1ull << tpa) - 1ull) << ((wl >> sh) << sh);
@@ -714,60 +757,87 @@ __global__ void __launch_bounds__(MAXB, 4)
             const float4 pk = act ? f4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
             const int a_lo = (k + 1) >> 1;
             int c = 0;
-            for (int m0 = 0; m0 < mmax; m0 += tpa) {
-                const int mi = m0 + sub;
-                const int n = mi < a_lo ? ((k + 1) & 1) + 2 * mi : k + 2 + 2 * (mi - a_lo);
-                bool in = false;
-                int code = 0;
-                if (act && n < N) {
-                    const float4 pn = f4[n];
-                    const int tn = __float_as_int(pn.w);
-                    if (MIXED ? (all_on || T.pair_on[tk * MDT_MAXT + tn]) : tn == bulk) {
-                        const float e0 = pk.x - pn.x, e1 = pk.y - pn.y, e2 = pk.z - pn.z;
-                        float m0f = rintf(e0), m1f = rintf(e1), m2f = rintf(e2);
-                        float d0 = e0 - m0f, d1 = e1 - m1f, d2 = e2 - m2f;
-                        const bool t0 = fabsf(d0) > mg0, t1 = fabsf(d1) > mg1, t2 = fabsf(d2) > mg2;
-                        const bool tie = t0 | t1 | t2;
-                        if (tie && !keep) {
-                            const double a0 = xr[k], a1 = xr[N + k], a2 = xr[2 * N + k];
-                            const double b0 = xr[n], b1 = xr[N + n], b2 = xr[2 * N + n];
-                            const double cx = rec[k].x - rec[n].x, cy = rec[k].y - rec[n].y, cz = rec[k].z - rec[n].z;
-                            const double *ih = s_ih;
-                            if (t0) m0f = (float)tie_image(ih[0], ih[3], ih[6], a0, a1, a2, b0, b1, b2, ih[0] * cx + ih[3] * cy + ih[6] * cz);
-                            if (t1) m1f = (float)tie_image(ih[1], ih[4], ih[7], a0, a1, a2, b0, b1, b2, ih[1] * cx + ih[4] * cy + ih[7] * cz);
-                            if (t2) m2f = (float)tie_image(ih[2], ih[5], ih[8], a0, a1, a2, b0, b1, b2, ih[2] * cx + ih[5] * cy + ih[8] * cz);
-                            d0 = e0 - m0f;
-                            d1 = e1 - m1f;
-                            d2 = e2 - m2f;
-                        }
-                        auto metric = [&](float d0, float d1, float d2) {
-                            return d0 * (g00 * d0 + g01 * d1 + g02 * d2) + d1 * (g11 * d1 + g12 * d2) + g22 * d2 * d2;
-                        };
-                        float r2 = metric(d0, d1, d2);
-                        code = ((int)m0f + 1) + 3 * ((int)m1f + 1) + 9 * ((int)m2f + 1);
-                        if (tie && keep) {
-                            code = MDT_ANY_IMAGE;
-                            for (int q = 1; q < 8; ++q)
-                                r2 = fminf(r2, metric(d0 - (t0 && (q & 1) ? copysignf(1.f, d0) : 0.f),
-                                                      d1 - (t1 && (q & 2) ? copysignf(1.f, d1) : 0.f),
-                                                      d2 - (t2 && (q & 4) ? copysignf(1.f, d2) : 0.f)));
-                        }
-                        in = r2 <= cut2f;
+            // candidate n of this lane's atom: listed (and the entry's code)?
+            auto test = [&](int n, const float4 &pn, bool ok, int &code) {
+                const int tn = __float_as_int(pn.w);
+                ok = ok && (MIXED ? (all_on || T.pair_on[tk * MDT_MAXT + tn]) : tn == bulk);
+                const float e0 = pk.x - pn.x, e1 = pk.y - pn.y, e2 = pk.z - pn.z;
+                float m0f = rintf(e0), m1f = rintf(e1), m2f = rintf(e2);
+                float d0 = e0 - m0f, d1 = e1 - m1f, d2 = e2 - m2f;
+                const bool t0 = fabsf(d0) > mg0, t1 = fabsf(d1) > mg1, t2 = fabsf(d2) > mg2;
+                const bool tie = ok && (t0 | t1 | t2);
+                if (tie && !keep) {
+                    const PairRec ck = rec[k], cn = rec[n];
+                    const double cx = ck.x - cn.x, cy = ck.y - cn.y, cz = ck.z - cn.z;
+                    const double *ih = s_ih;
+                    if (xt) {
+                        const double a0 = xt[k], a1 = xt[N + k], a2 = xt[2 * N + k];
+                        const double b0 = xt[n], b1 = xt[N + n], b2 = xt[2 * N + n];
+                        if (t0) m0f = (float)tie_image(ih[0], ih[3], ih[6], a0, a1, a2, b0, b1, b2, ih[0] * cx + ih[3] * cy + ih[6] * cz);
+                        if (t1) m1f = (float)tie_image(ih[1], ih[4], ih[7], a0, a1, a2, b0, b1, b2, ih[1] * cx + ih[4] * cy + ih[7] * cz);
+                        if (t2) m2f = (float)tie_image(ih[2], ih[5], ih[8], a0, a1, a2, b0, b1, b2, ih[2] * cx + ih[5] * cy + ih[8] * cz);
+                    } else {
+                        if (t0) m0f = (float)round(tie_dot(ih[0], ih[3], ih[6], cx, cy, cz));
+                        if (t1) m1f = (float)round(tie_dot(ih[1], ih[4], ih[7], cx, cy, cz));
+                        if (t2) m2f = (float)round(tie_dot(ih[2], ih[5], ih[8], cx, cy, cz));
                     }
+                    d0 = e0 - m0f;
+                    d1 = e1 - m1f;
+                    d2 = e2 - m2f;
                 }
-                const unsigned long long m = __ballot(in) & gmask;
+                auto metric = [&](float d0, float d1, float d2) {
+                    return d0 * (g00 * d0 + g01 * d1 + g02 * d2) + d1 * (g11 * d1 + g12 * d2) + g22 * d2 * d2;
+                };
+                float r2 = metric(d0, d1, d2);
+                code = (int)(m0f + 3.f * m1f + (9.f * m2f + 13.f));
+                if (tie && keep) {
+                    code = MDT_ANY_IMAGE;
+                    for (int q = 1; q < 8; ++q)
+                        r2 = fminf(r2, metric(d0 - (t0 && (q & 1) ? copysignf(1.f, d0) : 0.f),
+                                              d1 - (t1 && (q & 2) ? copysignf(1.f, d1) : 0.f),
+                                              d2 - (t2 && (q & 4) ? copysignf(1.f, d2) : 0.f)));
+                }
+                return ok && r2 <= cut2f;
+            };
+            auto put = [&](int n, bool in, int code, int pos) {
                 if (in) {
-                    const int pos = c + __popcll(m & below);
                     const uint16_t ent = (uint16_t)(n | (code << MDT_NBR_IDX_BITS));
+                    const uint32_t at = (uint32_t)(k * capg + pos);
                     if (pos >= cap) {
                         bad_local |= MDT_ST_NBR_OVERFLOW;
                     } else {
-                        scan_rows[(size_t)k * capg + pos] = ent;
+                        if (lds_scan)
+                            lrow[at] = ent;
+                        else
+                            grow[at] = ent;
                         if (code == MDT_ANY_IMAGE) s_slow = 1;  // benign race: every writer stores 1
                     }
                 }
-                c += __popcll(m);
-            }
+            };
+            // two candidates at a time, so that one's reads and chain fill the other's gaps
+            const int below_k = (k + 1) & 1, above_k = k + 2 - 2 * a_lo;
+            auto scan = [&](auto one) {
+                for (int m0 = sub; m0 - sub < mmax; m0 += 2 * tpa) {
+                    const int m1 = m0 + tpa;
+                    const int na = 2 * m0 + (m0 < a_lo ? below_k : above_k), nb = 2 * m1 + (m1 < a_lo ? below_k : above_k);
+                    const float4 pa = f4[na < N ? na : N - 1], pb = f4[nb < N ? nb : N - 1];
+                    int codea, codeb;
+                    const bool ina = test(na, pa, act && na < N, codea), inb = test(nb, pb, act && nb < N, codeb);
+                    one(na, ina, codea);
+                    one(nb, inb, codeb);
+                }
+            };
+            if (sh == 0)
+                scan([&](int n, bool in, int code) {
+                    put(n, in, code, c);
+                    c += in ? 1 : 0;
+                });
+            else  // the atom's lanes in order
+                scan([&](int n, bool in, int code) {
+                    const unsigned long long m = __ballot(in) & gmask;
+                    put(n, in, code, c + __popcll(m & below));
+                    c += __popcll(m);
+                });
             c = c < cap ? c : cap;
             if (direct) {
                 const uint32_t info = k < N ? (uint32_t)(k | ((c - sub + tpa - 1) >> sh) << MDT_NBR_IDX_BITS) : 0u;
@@ -797,7 +867,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         }
         __syncthreads();
         // (few workgroups: the last wavefront is left to the flat lists)
-        const int lim0 = (N + nthr / 4 + nthr - 1) / nthr * nthr - (bv.rl_scan < 0 && nwaves > 3 ? 64 : 0);
+        const int lim0 = (N + nthr / 4 + nthr - 1) / nthr * nthr - (lds_scan && nwaves > 3 ? 64 : 0);
         const int lim = lim0 < N + nthr ? lim0 : N + nthr;
         const unsigned long long fit = __ballot(s_np[wl] <= lim);
         const int L = fit ? __builtin_ctzll(fit) + 2 : 4096;  // none fits: one piece per row
@@ -852,10 +922,13 @@ __global__ void __launch_bounds__(MAXB, 4)
                 const int st = j * l + (j > ns - m ? j - (ns - m) : 0);
                 const int p = atomicAdd(&s_hist[len < 63 ? len : 63], 1);  // the order is free
                 rows[p] = (uint32_t)(k | len << MDT_NBR_IDX_BITS);
-                const uint16_t *src = scan_rows + (size_t)k * capg + st;
+                const int src = k * capg + st;
                 uint32_t *dst = stream + s_cb[p >> 6] + (p & 63);
-                for (int e = 0; e < len; e += 2)
-                    dst[32 * e] = src[e] | (uint32_t)src[e + 1 < len ? e + 1 : e] << 16;
+                for (int e = 0; e < len; e += 2) {
+                    const int e1 = e + 1 < len ? e + 1 : e;
+                    dst[32 * e] = lds_scan ? lrow[src + e] | (uint32_t)lrow[src + e1] << 16
+                                           : grow[src + e] | (uint32_t)grow[src + e1] << 16;
+                }
             }
         }
         }
@@ -867,13 +940,14 @@ __global__ void __launch_bounds__(MAXB, 4)
                 *valid = make_int2(1 | (s_anyfold ? 2 : 0) | (s_slow ? 4 : 0) | s_R << 3, ecg->gen);
         }
     }
+    const double *xt = s_folded ? xr : nullptr;
     // ---- flat lists: the near partners of the atoms outside the majority type ----
     // (two of those atoms with each other: listed at the lower index)
     auto flat_pair = [&](int h, int n, double d[3], double &r2, int &code) {
         if (n == h || !T.pair_on[typ[h] * MDT_MAXT + typ[n]] || (typ[n] != bulk && n < h)) return false;
-        r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[h], rec[n], xr, N, h, n, d, &code);
+        r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[h], rec[n], xt, N, h, n, d, &code);
         // (r2 = 0 is near; an atom without a position has no partners, as in the scan)
-        return r2 == r2 && !(r2 * mdt_rsqrt(r2) > rnear);
+        return r2 == r2 && !(mul_rn(r2, mdt_rsqrt(r2)) > rnear);
     };
     const int nflat = MIXED ? 0 : (s_nflat < MDT_FLAT_MAX ? s_nflat : MDT_FLAT_MAX);
     for (int f = 0; f < nflat; ++f) {
@@ -907,7 +981,7 @@ __global__ void __launch_bounds__(MAXB, 4)
     // theta and, for its derivative, rt1 = acut e1 theta
     auto theta = [&](double r, double *rt1) {
         if constexpr (PREC == 0) {
-            const double e1 = mdt_exp_t((r - rcut) * (acut * MDT_EXP_K), T.exptab);
+            const double e1 = mdt_exp_ab(r - rcut, acut * MDT_EXP_K, T.exptab);
             const double th = mdt_rcp(1 + e1);
             *rt1 = acut * e1 * th;
             return th;
@@ -930,50 +1004,64 @@ __global__ void __launch_bounds__(MAXB, 4)
         } else {
             double rt1;
             const double th = theta(r, &rt1);
-            const double fsn = th * mdt_exp_t(T.etaT[tn] * (r - T.bs0[tn]), T.exptab);
-            const double fsk = (tn == tk) ? fsn : th * mdt_exp_t(T.etaT[tk] * (r - T.bs0[tk]), T.exptab);
-            own = T.csig[tk * MDT_MAXT + tn] * fsn;
-            other = T.csig[tn * MDT_MAXT + tk] * fsk;
+            const double fsn = th * mdt_exp_ab(T.etaT[tn], r - T.bs0[tn], T.exptab);
+            const double fsk = (tn == tk) ? fsn : th * mdt_exp_ab(T.etaT[tk], r - T.bs0[tk], T.exptab);
+            own = mul_rn(T.csig[tk * MDT_MAXT + tn], fsn);
+            other = mul_rn(T.csig[tn * MDT_MAXT + tk], fsk);
         }
     };
     // dE/dr of the pair: density part through G of both atoms, pair (V) part
     // directly; and the pair energy
     auto force_terms = [&](int tk, int tn, double r, double Gk, double Gn, double &c, double &ep) {
+        if (tn < tk) {  // one order of the sums, whichever of the two asks
+            const int u = tk;
+            tk = tn;
+            tn = u;
+            const double g = Gk;
+            Gk = Gn;
+            Gn = g;
+        }
         const int kn = tk * MDT_MAXT + tn, nk = tn * MDT_MAXT + tk;
         if constexpr (PREC == 1) {
             const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
-            const float rt1 = acutf * e1 * th;
+            const float rt1 = mul_rn(acutf * e1, th);
             const float drn = (float)(r - T.bs0[tn]);
             const float fsn = th * mdt_exp2f(-T.f_eta2l2[tn] * drn);
             const float fvn = th * mdt_exp2f(-T.f_kdbl2[tn] * drn);
-            float fsk = fsn, fvk = fvn;
-            if (tn != tk) {
-                const float drk = (float)(r - T.bs0[tk]);
-                fsk = th * mdt_exp2f(-T.f_eta2l2[tk] * drk);
-                fvk = th * mdt_exp2f(-T.f_kdbl2[tk] * drk);
+            if (tn == tk) {  // one element: one set of pair constants (kn == nk)
+                const float fv = T.f_wv[kn] * fvn;
+                c = fma((double)(T.f_csig[kn] * ((T.f_etad[kn] + rt1) * fsn)), Gk + Gn, (double)((T.f_kdb[tn] + rt1) * fv));
+                ep = (double)(2.0f * fv);
+                return;
             }
+            const float drk = (float)(r - T.bs0[tk]);
+            const float fsk = th * mdt_exp2f(-T.f_eta2l2[tk] * drk);
+            const float fvk = th * mdt_exp2f(-T.f_kdbl2[tk] * drk);
             const float ta = T.f_csig[kn] * ((T.f_etad[kn] + rt1) * fsn);
             const float tb = T.f_csig[nk] * ((T.f_etad[nk] + rt1) * fsk);
-            const float tv = 0.5f * (T.f_wv[kn] * ((T.f_kdb[tn] + rt1) * fvn) + T.f_wv[nk] * ((T.f_kdb[tk] + rt1) * fvk));
-            c = Gk * (double)ta + Gn * (double)tb + (double)tv;
-            ep = (double)(T.f_wv[kn] * fvn + T.f_wv[nk] * fvk);
+            const float tv = 0.5f * fmaf(T.f_wv[kn], (T.f_kdb[tn] + rt1) * fvn, T.f_wv[nk] * ((T.f_kdb[tk] + rt1) * fvk));
+            c = fma(Gk, (double)ta, fma(Gn, (double)tb, (double)tv));
+            ep = (double)fmaf(T.f_wv[kn], fvn, T.f_wv[nk] * fvk);
         } else {
             double rt1;
             const double th = theta(r, &rt1);
             const double drn = r - T.bs0[tn];
-            const double fsn = th * mdt_exp_t(T.etaT[tn] * drn, T.exptab);
-            const double fvn = th * mdt_exp_t(T.kdbT[tn] * drn, T.exptab);
-            if (tn == tk) {  // one element: one set of pair constants (kn == nk)
-                c = T.csig[kn] * ((T.etad[kn] + rt1) * fsn) * (Gk + Gn) + T.wv[kn] * ((T.kdb[tn] + rt1) * fvn);
-                ep = 2.0 * T.wv[kn] * fvn;
+            const double fsn = th * mdt_exp_ab(T.etaT[tn], drn, T.exptab);
+            const double fvn = th * mdt_exp_ab(T.kdbT[tn], drn, T.exptab);
+            if (tn == tk) {
+                const double fv = T.wv[kn] * fvn;
+                c = fma(T.csig[kn] * ((T.etad[kn] + rt1) * fsn), Gk + Gn, (T.kdb[tn] + rt1) * fv);
+                ep = 2.0 * fv;
             } else {
                 const double drk = r - T.bs0[tk];
-                const double fsk = th * mdt_exp_t(T.etaT[tk] * drk, T.exptab);
-                const double fvk = th * mdt_exp_t(T.kdbT[tk] * drk, T.exptab);
-                c = Gk * T.csig[kn] * ((T.etad[kn] + rt1) * fsn) + Gn * T.csig[nk] * ((T.etad[nk] + rt1) * fsk) +
-                    0.5 * (T.wv[kn] * ((T.kdb[tn] + rt1) * fvn) + T.wv[nk] * ((T.kdb[tk] + rt1) * fvk));
-                ep = T.wv[kn] * fvn + T.wv[nk] * fvk;
+                const double fsk = th * mdt_exp_ab(T.etaT[tk], drk, T.exptab);
+                const double fvk = th * mdt_exp_ab(T.kdbT[tk], drk, T.exptab);
+                const double vn = T.wv[kn] * fvn, vk = T.wv[nk] * fvk;
+                const double v = fma(T.kdb[tn] + rt1, vn, (T.kdb[tk] + rt1) * vk);
+                c = fma(Gk * T.csig[kn], (T.etad[kn] + rt1) * fsn,
+                        fma(Gn * T.csig[nk], (T.etad[nk] + rt1) * fsk, 0.5 * v));
+                ep = vn + vk;
             }
         }
     };
@@ -983,7 +1071,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         dx = (xk - pn.x) - sft[0];
         dy = (yk - pn.y) - sft[1];
         dz = (zk - pn.z) - sft[2];
-        return dx * dx + dy * dy + dz * dz;
+        return fma(dz, dz, fma(dy, dy, dx * dx));
     };
     // a pair's force crs d, added to n; its rounded components, as integers in u
     auto add_force = [&](int n, double crs, const double *d, double g[3], unsigned long long u[3]) {
@@ -1021,25 +1109,25 @@ __global__ void __launch_bounds__(MAXB, 4)
             return (double)(uf_csig * (th * mdt_exp2f(uf_eta * (float)(r - u_bs0))));
         } else {
             double rt1;
-            return u_csig * (theta(r, &rt1) * mdt_exp_t(u_etaT * (r - u_bs0), T.exptab));
+            return mul_rn(u_csig, theta(r, &rt1) * mdt_exp_ab(u_etaT, r - u_bs0, T.exptab));
         }
     };
     auto bulk_force = [&](double r, double G2, double &c, double &ep) {  // G2: G of both atoms
         if constexpr (PREC == 1) {
             const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
-            const float rt1 = acutf * e1 * th;
+            const float rt1 = mul_rn(acutf * e1, th);
             const float dr = (float)(r - u_bs0);
             const float fs = th * mdt_exp2f(uf_eta * dr), fv = uf_wv * (th * mdt_exp2f(uf_kdbl2 * dr));
-            c = (double)(uf_csig * ((uf_etad + rt1) * fs)) * G2 + (double)((uf_kdb + rt1) * fv);
+            c = fma((double)(uf_csig * ((uf_etad + rt1) * fs)), G2, (double)((uf_kdb + rt1) * fv));
             ep = (double)(2.0f * fv);
         } else {
             double rt1;
             const double th = theta(r, &rt1);
             const double dr = r - u_bs0;
-            const double fs = th * mdt_exp_t(u_etaT * dr, T.exptab);
-            const double fv = u_wv * (th * mdt_exp_t(u_kdbT * dr, T.exptab));
-            c = u_csig * ((u_etad + rt1) * fs) * G2 + (u_kdb + rt1) * fv;
+            const double fs = th * mdt_exp_ab(u_etaT, dr, T.exptab);
+            const double fv = u_wv * (th * mdt_exp_ab(u_kdbT, dr, T.exptab));
+            c = fma(u_csig * ((u_etad + rt1) * fs), G2, (u_kdb + rt1) * fv);
             ep = 2.0 * fv;
         }
     };
@@ -1055,14 +1143,21 @@ __global__ void __launch_bounds__(MAXB, 4)
     auto each_entry = [&](int r0, int k, int len, double x, double y, double z, double lim, auto eval, auto add,
                           auto large) {
         const uint32_t *src = stream + (direct ? 0 : s_cb[r0 >> 6]) + (r0 & 63);
-        const uint16_t *row = scan_rows + k * capg + (r0 & ((1 << sh) - 1));  // direct
+        const uint16_t *row = lrow + k * capg + (r0 & ((1 << sh) - 1));  // direct
         const int last = 32 * (len - 1 & ~1);  // of the piece's words
-        uint32_t cur = direct ? 0 : r0 == lane ? word0 : src[0];
+        // entries e and e + 1 (the last one twice in an odd piece)
+        auto word = [&](int e) {
+            if (!direct) return src[32 * e < last ? 32 * e : last];
+            const int e0 = e < len ? e : len - 1, e1 = e + 1 < len ? e + 1 : len - 1;
+            return (uint32_t)row[e0 << sh] | (uint32_t)row[e1 << sh] << 16;
+        };
+        if (len == 0) return;  // a lane without an entry of its row (direct)
+        uint32_t cur = !direct && r0 == lane ? word0 : word(0);
         double d[3], g[3];
-        if (!slow && !direct) {
+        if (!slow) {
             for (int e = 0; e < len; e += 2) {
                 const uint32_t q = cur;
-                cur = src[32 * e + 64 < last ? 32 * e + 64 : last];
+                cur = word(e + 2);
                 const PairRec a0 = rec[q & MDT_NBR_IDX_MASK], a1 = rec[q >> 16 & MDT_NBR_IDX_MASK];
                 const double r0 = listed(q & 0xFFFF, x, y, z, a0, d[0], d[1], d[2]);
                 const double r1 = listed(q >> 16, x, y, z, a1, g[0], g[1], g[2]);
@@ -1077,14 +1172,14 @@ __global__ void __launch_bounds__(MAXB, 4)
             }
         } else {
             for (int e = 0; e < len; ++e) {
-                const unsigned q = direct ? row[e << sh] : e & 1 ? cur >> 16 : cur & 0xFFFF;
-                if (!direct && e & 1) cur = src[32 * (e + 1) < last ? 32 * (e + 1) : last];
+                const unsigned q = e & 1 ? cur >> 16 : cur & 0xFFFF;
+                if (e & 1) cur = word(e + 1);
                 const int n = q & MDT_NBR_IDX_MASK;
                 const PairRec pn = rec[n];
                 double r2;
                 int code;
                 if (q >> MDT_NBR_IDX_BITS == MDT_ANY_IMAGE) {
-                    r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], pn, xr, N, k, n, d, &code);
+                    r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], pn, xt, N, k, n, d, &code);
                     // in a skewed cell its image may be anywhere; the terms of a pair
                     // beyond rnear count 0 times and stay finite up to 2 rnear
                     r2 = r2 > 4.0 * rnear * rnear ? 4.0 * rnear * rnear : r2;
@@ -1131,7 +1226,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         each_entry(
             r0, k, len, xk, yk, zk, MDT_SIG_FAST,
             [&](int n, double, double r2, bool in) {
-                const double r = r2 * mdt_rsqrt(r2);
+                const double r = mul_rn(r2, mdt_rsqrt(r2));
                 Sig v;
                 if constexpr (MIXED)
                     sigma_terms(tk, typ[n], r, v.own, v.other);
@@ -1158,8 +1253,8 @@ __global__ void __launch_bounds__(MAXB, 4)
                 sig_large(&rec[n].w, v.other, &bad_local);
                 v.own = v.other = 0.0;
             });
-        add_sum(&rec[k].w, s1, MDT_P42, &bad_local);
-        add_sum(&w2[k], s2, MDT_P42 * MDT_P46, &bad_local);
+        add_sum(&rec[k].w, s1, MDT_SIG_C1, MDT_P42, &bad_local);
+        add_sum(&w2[k], s2, MDT_SIG_C2, MDT_P42 * MDT_P46, &bad_local);
     }
     for (int q = 0; q < nflat; ++q) {
         const int h = s_flat[q];
@@ -1167,7 +1262,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         each_flat(q, [&](int n, const double *d, double r2) {
             double own, other, hi, lo;
             unsigned long long u1, u2;
-            sigma_terms(typ[h], typ[n], r2 * mdt_rsqrt(r2), own, other);
+            sigma_terms(typ[h], typ[n], mul_rn(r2, mdt_rsqrt(r2)), own, other);
             if (!(own < MDT_SIG_FAST && other < MDT_SIG_FAST)) {
                 sig_large(&rec[h].w, own, &bad_local);
                 sig_large(&rec[n].w, other, &bad_local);
@@ -1205,9 +1300,9 @@ __global__ void __launch_bounds__(MAXB, 4)
     auto partner = [&](int k, int n, bool near, double d[3], double &r, double &ri) {
         if (n == k || !T.pair_on[typ[k] * MDT_MAXT + typ[n]]) return false;
         int code;
-        const double r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], rec[n], xr, N, k, n, d, &code);
+        const double r2 = pair_image(s_ihf, bv.icell + 9 * t, s_sh, rec[k], rec[n], xt, N, k, n, d, &code);
         ri = mdt_rsqrt(r2);
-        r = r2 * ri;
+        r = mul_rn(r2, ri);
         return (near || r > rnear) && r <= cutr;
     };
     // calls f(k) for every tiny atom, each on one wavefront
@@ -1285,7 +1380,7 @@ __global__ void __launch_bounds__(MAXB, 4)
             r0, k, len, xk, yk, zk, MDT_FRC_FAST,
             [&](int n, double Gn, double r2, bool in) {
                 const double ri = mdt_rsqrt(r2);
-                const double r = r2 * ri;
+                const double r = mul_rn(r2, ri);
                 double c;
                 Frc v;
                 if constexpr (MIXED)
@@ -1312,9 +1407,9 @@ __global__ void __launch_bounds__(MAXB, 4)
                 add_large(k, n, v.crs, d);
                 v.crs = 0.0;
             });
-        add_sum(&rec[k].w, fx, MDT_P42, &bad_local);
-        add_sum(&w2[k], fy, MDT_P42, &bad_local);
-        add_sum(&w3[k], fz, MDT_P42, &bad_local);
+        add_sum(&rec[k].w, fx, MDT_FRC_C, MDT_P42, &bad_local);
+        add_sum(&w2[k], fy, MDT_FRC_C, MDT_P42, &bad_local);
+        add_sum(&w3[k], fz, MDT_FRC_C, MDT_P42, &bad_local);
     }
     // the pair (k, n) of an atom k that a wavefront's lanes share: -F on k in fk
     auto pair_forces = [&](int k, int n, const double *d, double r, double ri, unsigned long long fk[3]) {
@@ -1335,7 +1430,7 @@ __global__ void __launch_bounds__(MAXB, 4)
         unsigned long long fk[3] = {0, 0, 0};
         each_flat(q, [&](int n, const double *d, double r2) {
             const double ri = mdt_rsqrt(r2);
-            pair_forces(h, n, d, r2 * ri, ri, fk);
+            pair_forces(h, n, d, mul_rn(r2, ri), ri, fk);
         });
         add_uniform(&rec[h].w, fk[0]);
         add_uniform(&w2[h], fk[1]);
@@ -2854,19 +2949,23 @@ hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipS
 // entries a word, padded to their first piece's length, which is at most the
 // last one's of the chunk before: 32 (longest + 1 a chunk) + half the entries -- 2
 // more a chunk for lengths of 63 to 65, which are not told apart --, or, uncut, N
-// rows of cap; and a row of slack.  The scanned rows go to LDS (scan < 0) where at
-// most REP_FEW workgroups run, about two a CU, whose number LDS then does not
-// limit, and they fit into `lds`.
-ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds) {
+// rows of cap; and a row of slack.  The scanned rows go to LDS (scan < 0), if they fit
+// into `lds`, where at most REP_FEW workgroups run, about two a CU, whose number
+// LDS then does not limit, and where the rows serve one launch (once): they are
+// then read from there, by the lanes that found them, without a cut.  The table
+// holds N + block rows or pieces.
+ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, bool once) {
     ReplicaLists l;
     const long long chunks = (N + block) / 64 + 1;
     l.rows = 32 * (cap + 65 + 3 * chunks) + (N + 64LL) * (cap + 1) / 2 + 64;
-    l.chunk = l.rows + N + block;
     const size_t rows = 2 * (size_t)N * ((cap + 7) & ~7);
     l.smem = 58 * (size_t)N;
+    const bool in_lds = (once || nrep <= REP_FEW) && l.smem + 8 + rows <= lds;
+    if (in_lds && once) l.rows = 0;  // no stream
+    l.chunk = l.rows + N + block;
     l.scan = (l.chunk + chunks + 3) & ~3LL;
     l.stride = l.scan;
-    if (nrep <= REP_FEW && l.smem + 8 + rows <= lds) {
+    if (in_lds) {
         l.smem += 8 + rows;
         l.scan = -1;
     } else {

@@ -44,8 +44,9 @@
 #define NA_TRAJ (NA_CELL + NA_ALIGN(8 * 20))  // N, P, status, traj_id | soff, aoff, eoff (8-byte aligned)
 #define NA_PC (NA_TRAJ + NA_ALIGN(64))
 #define NA_NBR (NA_PC + NA_ALIGN(sizeof(PropConst)))
-// k_replica's lists (mdt_replica_lists at 96 entries per row): less than 10240 words a replica and 104 an atom
-#define NA_LIST_WORDS (10240 * (size_t)NOALLOC_MAX_BEADS + 104 * (size_t)NOALLOC_MAX_AB)
+// k_replica's lists (mdt_replica_lists at 96 entries per row, for one launch): the most,
+// 1880528 words, at 26 beads of 630 atoms, whose rows do not fit into LDS
+#define NA_LIST_WORDS 1900000
 #define NA_TOTAL (NA_NBR + NA_ALIGN(4 * NA_LIST_WORDS))
 
 static __device__ __align__(256) unsigned char scratch[NA_TOTAL];
@@ -138,7 +139,7 @@ __global__ void k_noalloc_unpack(const unsigned char *s, const EmtConst *ec, int
 
 }  // namespace
 
-ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds);
+ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, bool once);
 hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
                               const BatchView &bv, int add_fin, hipStream_t st);
 int mdt_noalloc_fail(int code, const char *msg);
@@ -171,7 +172,7 @@ int mdt_noalloc_compute(void *ptr, size_t lds_limit, const EmtConst *d_ec, int n
     while (tpa > 1 && N * tpa > 512) tpa >>= 1;
     const int block = (((N * tpa + 63) / 64) * 64) < 64 ? 64 : (((N * tpa + 63) / 64) * 64);
     const size_t lds_dyn = lds_limit > 6656 ? lds_limit - 6656 : 0;  // beside k_replica's static tables
-    const ReplicaLists lay = mdt_replica_lists(P, N, block, cap, lds_dyn);
+    const ReplicaLists lay = mdt_replica_lists(P, N, block, cap, lds_dyn, true);
     const size_t smem = lay.smem;
     if (smem > lds_dyn) return mdt_noalloc_fail(MDT_EUNSUP, "universe too large for one workgroup's LDS");
     if ((size_t)lay.stride * P > NA_LIST_WORDS) return mdt_noalloc_fail(MDT_EUNSUP, "universe too large for the scratch lists");

@@ -55,7 +55,7 @@ extern "C" {
 #define MDT_ST_NBR_OVERFLOW 1  /* neighbour list capacity exceeded */
 #define MDT_ST_NEG_DENSITY 2   /* ldfa saw a negative density (src/md_algo.f90:551-554) */
 #define MDT_ST_BAD_PROP 4      /* unknown propagator (src/md_algo.f90:66-67) */
-#define MDT_ST_FIXED_OVERFLOW 8 /* a pair term exceeded the fixed-point accumulator range */
+#define MDT_ST_FIXED_OVERFLOW 8 /* a pair term exceeded the fixed-point accumulator range (EMT forces: 1.0e6 eV/A) */
 #define MDT_ST_NN_EXTRAPOLATION 16 /* a network input left its scaling range (EMT fallback applied) */
 
 typedef struct mdt_context mdt_context;

@@ -310,11 +310,14 @@ struct PairRec {
 // of its two atoms owns a pair.  (FP64 LDS atomics would save the subtraction, but
 // on random addresses they take 21 cycles a wavefront, 64-bit integer ones 11.)
 //   sigma: 2^-42 (|v| < 512) and 2^-88 for the rest;
-//   forces: 2^-42 eV/A (|v| < 512 eV/A).
+//   forces: 2^-43 eV/A (|v| < 256 eV/A).  The words hold up to 1.05e6 eV/A, 700 times
+//   the largest pair force of the shipped parameter sets; 2^-42 would hold twice as
+//   much and double the error of a run's state (4096 x 145 atoms, 200 steps, against
+//   64 bits: 2.8e-13 with 2^-43, 5.5e-13 with 2^-42).
 // Larger terms are converted by rint and added by themselves; those beyond 2^63
 // grids, and NaN, are flagged (MDT_ST_FIXED_OVERFLOW) and left out.
 // A lane sums the terms of its piece of a row, whose order is the list's, as rounded
-// FP64 terms: exact while the lane's sum stays below 2^53 grids, 2048 eV/A or
+// FP64 terms: exact while the lane's sum stays below 2^53 grids, 1024 eV/A or
 // sigma 2048; beyond that it is rounded, the same in every run but not however the
 // row is cut.  Atoms whose partners come in no fixed order (flat lists) sum integers.
 // Energies are summed in registers: 2^-33 eV (sums below 1e6 eV) and 2^-70 for
@@ -322,11 +325,12 @@ struct PairRec {
 #define MDT_SIG_C1 1536.0                         // 1.5 * 2^(52 - 42)
 #define MDT_SIG_C2 2.1827872842550278e-11         // 1.5 * 2^(52 - 88)
 #define MDT_SIG_FAST 511.0
-#define MDT_FRC_C 1536.0                          // 1.5 * 2^(52 - 42)
-#define MDT_FRC_FAST 511.0
+#define MDT_FRC_C 768.0                           // 1.5 * 2^(52 - 43)
+#define MDT_FRC_FAST 255.0
 #define MDT_EPR_C1 786432.0                       // 1.5 * 2^(52 - 33)
 #define MDT_EPR_C2 5.7220458984375e-06            // 1.5 * 2^(52 - 70)
 #define MDT_P42 4398046511104.0
+#define MDT_P43 8796093022208.0
 #define MDT_P46 70368744177664.0
 
 // Below this sigma~ (of the near pairs) the words' absolute step shows in a
@@ -382,7 +386,7 @@ __device__ double sig_large(unsigned long long *p, double v, int *bad) {
 __device__ __forceinline__ double sig_sum(unsigned long long w1, unsigned long long w2) {
     return (double)(long long)w1 * (1.0 / MDT_P42) + (double)(long long)w2 * (1.0 / (MDT_P42 * MDT_P46));
 }
-__device__ __forceinline__ double frc_sum(unsigned long long w) { return (double)(long long)w * (1.0 / MDT_P42); }
+__device__ __forceinline__ double frc_sum(unsigned long long w) { return (double)(long long)w * (1.0 / MDT_P43); }
 // LDS += a sum of rounded terms (a multiple of the grid, C as in grid_int)
 __device__ __forceinline__ void add_sum(unsigned long long *p, double v, double C, double scale, int *bad) {
     unsigned long long u;
@@ -1090,7 +1094,7 @@ __global__ void __launch_bounds__(MAXB, 4)
 #pragma unroll 1
         for (int q = 0; q < 3; ++q) {
             double g;
-            const unsigned long long u = grid_any(crs * d[q], MDT_P42, &g, &bad_local);
+            const unsigned long long u = grid_any(crs * d[q], MDT_P43, &g, &bad_local);
             unsigned long long *w = q == 0 ? &rec[n].w : (q == 1 ? w2 : w3) + n;
             atomicAdd(w, u);
             w = q == 0 ? &rec[k].w : (q == 1 ? w2 : w3) + k;
@@ -1407,9 +1411,9 @@ __global__ void __launch_bounds__(MAXB, 4)
                 add_large(k, n, v.crs, d);
                 v.crs = 0.0;
             });
-        add_sum(&rec[k].w, fx, MDT_FRC_C, MDT_P42, &bad_local);
-        add_sum(&w2[k], fy, MDT_FRC_C, MDT_P42, &bad_local);
-        add_sum(&w3[k], fz, MDT_FRC_C, MDT_P42, &bad_local);
+        add_sum(&rec[k].w, fx, MDT_FRC_C, MDT_P43, &bad_local);
+        add_sum(&w2[k], fy, MDT_FRC_C, MDT_P43, &bad_local);
+        add_sum(&w3[k], fz, MDT_FRC_C, MDT_P43, &bad_local);
     }
     // the pair (k, n) of an atom k that a wavefront's lanes share: -F on k in fk
     auto pair_forces = [&](int k, int n, const double *d, double r, double ri, unsigned long long fk[3]) {

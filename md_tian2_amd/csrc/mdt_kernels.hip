@@ -1029,22 +1029,22 @@ __global__ void __launch_bounds__(MAXB, 4)
         if constexpr (PREC == 1) {
             const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
-            const float rt1 = mul_rn(acutf * e1, th);
+            const float ae = acutf * e1;  // theta' / theta = ae th
             const float drn = (float)(r - T.bs0[tn]);
             const float fsn = th * mdt_exp2f(-T.f_eta2l2[tn] * drn);
             const float fvn = th * mdt_exp2f(-T.f_kdbl2[tn] * drn);
             if (tn == tk) {  // one element: one set of pair constants (kn == nk)
                 const float fv = T.f_wv[kn] * fvn;
-                c = fma((double)(T.f_csig[kn] * ((T.f_etad[kn] + rt1) * fsn)), Gk + Gn, (double)((T.f_kdb[tn] + rt1) * fv));
+                c = fma((double)(T.f_csig[kn] * (fmaf(ae, th, T.f_etad[kn]) * fsn)), Gk + Gn, (double)(fmaf(ae, th, T.f_kdb[tn]) * fv));
                 ep = (double)(2.0f * fv);
                 return;
             }
             const float drk = (float)(r - T.bs0[tk]);
             const float fsk = th * mdt_exp2f(-T.f_eta2l2[tk] * drk);
             const float fvk = th * mdt_exp2f(-T.f_kdbl2[tk] * drk);
-            const float ta = T.f_csig[kn] * ((T.f_etad[kn] + rt1) * fsn);
-            const float tb = T.f_csig[nk] * ((T.f_etad[nk] + rt1) * fsk);
-            const float tv = 0.5f * fmaf(T.f_wv[kn], (T.f_kdb[tn] + rt1) * fvn, T.f_wv[nk] * ((T.f_kdb[tk] + rt1) * fvk));
+            const float ta = T.f_csig[kn] * (fmaf(ae, th, T.f_etad[kn]) * fsn);
+            const float tb = T.f_csig[nk] * (fmaf(ae, th, T.f_etad[nk]) * fsk);
+            const float tv = 0.5f * fmaf(T.f_wv[kn], fmaf(ae, th, T.f_kdb[tn]) * fvn, T.f_wv[nk] * (fmaf(ae, th, T.f_kdb[tk]) * fvk));
             c = fma(Gk, (double)ta, fma(Gn, (double)tb, (double)tv));
             ep = (double)fmaf(T.f_wv[kn], fvn, T.f_wv[nk] * fvk);
         } else {
@@ -1120,10 +1120,10 @@ __global__ void __launch_bounds__(MAXB, 4)
         if constexpr (PREC == 1) {
             const float e1 = cut_exp(r);
             const float th = mdt_rcpf(1.0f + e1);
-            const float rt1 = mul_rn(acutf * e1, th);
+            const float ae = acutf * e1;  // theta' / theta = ae th
             const float dr = (float)(r - u_bs0);
             const float fs = th * mdt_exp2f(uf_eta * dr), fv = uf_wv * (th * mdt_exp2f(uf_kdbl2 * dr));
-            c = fma((double)(uf_csig * ((uf_etad + rt1) * fs)), G2, (double)((uf_kdb + rt1) * fv));
+            c = fma((double)(uf_csig * (fmaf(ae, th, uf_etad) * fs)), G2, (double)(fmaf(ae, th, uf_kdb) * fv));
             ep = (double)(2.0f * fv);
         } else {
             double rt1;

@@ -18,7 +18,7 @@
 #include "mdt_device.h"
 
 ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, bool once);
-hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed,
+hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed, long long from,
                                const double *src, double *dst, hipStream_t st);
 hipError_t mdt_launch_call(bool in, double *host, int N, int P, const CallArrays &a, hipStream_t st);
 hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipStream_t st);
@@ -126,11 +126,19 @@ struct mdt_context {
 // LDS, neighbour buffer), so that small slabs in a mixed batch do not run
 // with the largest slab's shape.
 #define ROW_SKIN 0.1         // A, per sqrt(beads) (row_skin)
+#define LIST_SLOTS 8192       // of a class whose lists do not all fit into memory: 32 workgroups a CU
 #define REP_STATIC_LDS 6656   // k_replica's static LDS, rounded up
+
+// tiles first .. first + n - 1 of a state's transfer: words from .. to - 1 of the caller's array
+struct XferPart {
+    int first, n;
+    long long from, to;
+};
 
 struct SizeClass {
     int nmax = 0;              // largest replica of the class
     int nrep = 0;
+    int slots = 0;             // list slots: one per replica, or fewer that its launches take in turn
     int *d_reps = nullptr;     // replica ids; NULL when the class holds every replica in order
     int tpa = 0, nbcap = 0, block = 0;
     int keep = 0;              // lists kept across launches (Verlet skin): 0 no, 1 or 2 as asked
@@ -266,7 +274,7 @@ struct mdt_batch {
     // set_state / get_state: runs of atoms and one array in the caller's layout
     StateTile *d_tile = nullptr;
     double *d_xfer = nullptr;
-    int ntile = 0;
+    std::vector<XferPart> xfer_part;
     double *h_call = nullptr, *d_call = nullptr;  // pinned block of a one-universe call, and its device address
 
     // k_replica's pair-term arithmetic: mode 1 is full FP32 pair terms when
@@ -912,8 +920,25 @@ static int build_tiles(mdt_batch *b) {
         if (rc) return rc;
     }
     HIPCHK(hipMemcpy(b->d_tile, tl.data(), sizeof(StateTile) * tl.size(), hipMemcpyHostToDevice));
-    b->ntile = (int)tl.size();
-    return dalloc(&b->d_xfer, (size_t)b->tot3pn);
+    // an array as large as the caller's, or, on a GPU that is nearly full, a smaller
+    // one that the tiles pass through in several parts
+    long long cap = b->tot3pn;
+    int rc = dalloc(&b->d_xfer, (size_t)cap);
+    while (rc && cap > 65536) {
+        (void)hipGetLastError();
+        cap = (cap + 1) / 2;
+        rc = dalloc(&b->d_xfer, (size_t)cap);
+    }
+    if (rc) return rc;
+    b->xfer_part.clear();
+    for (size_t k = 0; k < tl.size(); ++k) {
+        const StateTile &w = tl[k];
+        const long long from = b->soff[w.t] + 3LL * b->P[w.t] * w.i0, to = from + 3LL * b->P[w.t] * w.na;
+        if (b->xfer_part.empty() || to - b->xfer_part.back().from > cap) b->xfer_part.push_back({(int)k, 0, from, to});
+        ++b->xfer_part.back().n;
+        b->xfer_part.back().to = to;
+    }
+    return 0;
 }
 
 // bead slot holding atom i's bead bb on the device: in mixed bead mode a
@@ -933,8 +958,10 @@ int mdt_batch_set_state(mdt_batch *b, const double *r, const double *v) {
     double *dsts[2] = {b->d_x, b->d_v};
     for (int k = 0; k < 2; ++k) {
         if (!srcs[k]) continue;
-        HIPCHK(hipMemcpyAsync(b->d_xfer, srcs[k], sizeof(double) * b->tot3pn, hipMemcpyHostToDevice, st));
-        HIPCHK(mdt_launch_relayout(false, b->ntile, b->d_tile, b->view(), 0, b->d_xfer, dsts[k], st));
+        for (const XferPart &p : b->xfer_part) {
+            HIPCHK(hipMemcpyAsync(b->d_xfer, srcs[k] + p.from, sizeof(double) * (p.to - p.from), hipMemcpyHostToDevice, st));
+            HIPCHK(mdt_launch_relayout(false, p.n, b->d_tile + p.first, b->view(), 0, p.from, b->d_xfer, dsts[k], st));
+        }
     }
     HIPCHK(hipStreamSynchronize(st));
     rc = invalidate_lists(b);  // new positions: the kept lists are stale
@@ -953,8 +980,11 @@ int mdt_batch_get_state(mdt_batch *b, double *r, double *v, double *f, double *a
     double *dsts[4] = {r, v, f, a};
     for (int k = 0; k < 4; ++k) {
         if (!dsts[k]) continue;
-        HIPCHK(mdt_launch_relayout(true, b->ntile, b->d_tile, b->view(), b->bead_mode == 1, srcs[k], b->d_xfer, st));
-        HIPCHK(hipMemcpyAsync(dsts[k], b->d_xfer, sizeof(double) * b->tot3pn, hipMemcpyDeviceToHost, st));
+        for (const XferPart &p : b->xfer_part) {
+            HIPCHK(mdt_launch_relayout(true, p.n, b->d_tile + p.first, b->view(), b->bead_mode == 1, p.from, srcs[k],
+                                       b->d_xfer, st));
+            HIPCHK(hipMemcpyAsync(dsts[k] + p.from, b->d_xfer, sizeof(double) * (p.to - p.from), hipMemcpyDeviceToHost, st));
+        }
     }
     HIPCHK(hipStreamSynchronize(st));
     if (epot) {
@@ -1101,7 +1131,7 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
     // which the tuner finds
     if (b->keep_mode >= 0) keep = b->keep_mode;
     if (keep < 0) keep = 1;
-    const bool skin = b->list_skin > 0.0 && keep >= 1;
+    bool skin = b->list_skin > 0.0 && keep >= 1;
     const int rounded = ((c.nmax * tpa + split - 1) / split + 63) / 64 * 64;
     const int block = std::min(wide ? 1024 : 512, std::max(64, rounded));
     // dynamic LDS beside the kernel's static tables (6.4 KB in the judge's variant; 6.5 KiB allowed)
@@ -1111,13 +1141,17 @@ static int configure_class(mdt_batch *b, SizeClass &c, int tpa, int nbcap, int k
         return fail(MDT_EUNSUP, "replica of %d atoms needs %zu bytes of LDS (limit %zu)", c.nmax, lay.smem, lds_dyn);
     free_class_lists(c);
     c.lay = lay;
+    c.slots = c.nrep;
     int rc = dalloc(&c.d_lists, (size_t)c.lay.stride * c.nrep);
-    if (rc) return rc;
-    if (skin) {
-        rc = dalloc(&c.d_ref, 3 * (size_t)c.nmax * c.nrep) | dalloc(&c.d_valid, (size_t)c.nrep);
-        if (rc) return rc;
-        HIPCHK(zero_on(b->ctx->stream, c.d_valid, sizeof(int2) * c.nrep));
+    if (!rc && skin) rc = dalloc(&c.d_ref, 3 * (size_t)c.nmax * c.nrep) | dalloc(&c.d_valid, (size_t)c.nrep);
+    if (rc) {  // a GPU that is nearly full: rebuilt lists, in slots that the launches take in turn
+        (void)hipGetLastError();
+        free_class_lists(c);
+        skin = false;
+        c.slots = std::min(c.nrep, LIST_SLOTS);
+        if ((rc = dalloc(&c.d_lists, (size_t)c.lay.stride * c.slots))) return rc;
     }
+    if (skin) HIPCHK(zero_on(b->ctx->stream, c.d_valid, sizeof(int2) * c.nrep));
     c.block = block;
     c.keep = skin ? keep : 0;
     c.want = keep;
@@ -1360,8 +1394,16 @@ static hipError_t launch_class(const mdt_batch *b, const SizeClass &k, int t0, i
     v.rl_skin = row_skin(b);
     v.rl_ns = k.nmax;
     if (v.rl_scan < 0 && !v.rl_valid) v.bulk = -1;
-    return mdt_launch_replica(once ? k.tpa1 : k.tpa, n, once ? k.block1 : k.block, once ? k.smem1 : k.smem, b->ctx->d_ec,
-                              b->d_pc, v, add_fin, st);
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < n && e == hipSuccess; q += k.slots) {
+        e = mdt_launch_replica(once ? k.tpa1 : k.tpa, std::min(n - q, k.slots), once ? k.block1 : k.block,
+                               once ? k.smem1 : k.smem, b->ctx->d_ec, b->d_pc, v, add_fin, st);
+        if (v.rep_list)
+            v.rep_list += k.slots;
+        else
+            v.rep0 += k.slots;
+    }
+    return e;
 }
 
 // Whether the next launch of the EMT forces gets rows that serve it alone: the
@@ -1738,7 +1780,7 @@ static int enqueue_steps(mdt_batch *b, int nsteps, const uint32_t *step_base, ui
 static bool use_split(const mdt_batch *b) {
     if (b->split_mode == 0 || b->profile) return false;
     if (!(b->allP1 && traj_classical(b) && b->pes == 0 && b->cls.size() == 1 && b->mix_traj.empty() &&
-          b->cls[0].d_reps == nullptr && b->ntraj >= 2))
+          b->cls[0].d_reps == nullptr && b->cls[0].slots == b->cls[0].nrep && b->ntraj >= 2))
         return false;
     return b->split_mode == 1 || b->ntraj >= 1024;
 }

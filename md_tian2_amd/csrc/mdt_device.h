@@ -153,6 +153,7 @@ struct BatchView {
     uint16_t *nbr_global;   // k_mixed's neighbour lists, nbr_stride entries per listed trajectory
     long long nbr_stride;
     const int *rep_list;    // non-NULL: block k works on replica rep_list[k] (size-class launches)
+    int rep0;               // without a list block k works on replica rep0 + k (k_replica)
     const int *only;        // non-NULL: calc_force only on replicas with only[rep] != 0
     const int *skip;        // non-NULL: no calc_force on replicas with skip[rep] != 0
     // judge mode (judge_acc non-NULL): replicas with rep % judge_mod ==

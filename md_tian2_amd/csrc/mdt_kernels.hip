@@ -541,7 +541,7 @@ __global__ void __launch_bounds__(MAXB, 4)
     __shared__ int s_np[64], s_hist[64];  // pieces at each length limit, of each length
     __shared__ int s_cb[64];              // stream offset of each chunk of 64 pieces
     __shared__ int s_nflat, s_R, s_slow, s_anyfold, s_folded;
-    const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : (int)blockIdx.x;
+    const int rep = bv.rep_list ? bv.rep_list[blockIdx.x] : bv.rep0 + (int)blockIdx.x;
     if (bv.only && !bv.only[rep]) return;                          // whole block: uniform
     if (bv.skip && bv.skip[rep]) return;                           // whole block: uniform
     if (JUDGE && (rep % bv.judge_mod) != bv.judge_phase) return;   // whole block: uniform
@@ -2850,12 +2850,12 @@ __global__ void __launch_bounds__(MAXB, 2)
 template <bool OUT>
 __global__ void __launch_bounds__(256)
     k_relayout(const StateTile *__restrict__ tiles, const int *__restrict__ traj_N, const int *__restrict__ traj_P,
-               const long long *__restrict__ traj_soff, int mixed, const double *__restrict__ src,
+               const long long *__restrict__ traj_soff, int mixed, long long from, const double *__restrict__ src,
                double *__restrict__ dst) {
     __shared__ double s[3 * MDT_TILE];
     const StateTile w = tiles[blockIdx.x];
     const int N = traj_N[w.t], P3 = 3 * traj_P[w.t], n = P3 * w.na;
-    const long long dev = traj_soff[w.t] + w.i0, ref = traj_soff[w.t] + (long long)P3 * w.i0;
+    const long long dev = traj_soff[w.t] + w.i0, ref = traj_soff[w.t] + (long long)P3 * w.i0 - from;
     const bool first = mixed && P3 > 3;
     if (OUT) {
         for (int q = threadIdx.x; q < n; q += 256) {
@@ -2874,14 +2874,15 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed,
+// from: the first word of the caller's array that src (in) or dst (out) holds
+hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, const BatchView &v, int mixed, long long from,
                                const double *src, double *dst, hipStream_t st) {
     if (out)
         hipLaunchKernelGGL((k_relayout<true>), dim3(ntile), dim3(256), 0, st, tiles, v.traj_N, v.traj_P, v.traj_soff,
-                           mixed, src, dst);
+                           mixed, from, src, dst);
     else
         hipLaunchKernelGGL((k_relayout<false>), dim3(ntile), dim3(256), 0, st, tiles, v.traj_N, v.traj_P, v.traj_soff,
-                           mixed, src, dst);
+                           mixed, from, src, dst);
     return hipGetLastError();
 }
 

@@ -94,3 +94,28 @@ def test_skin_off_and_on_keeps_the_tuned_shape(fake_hip, tune_at, want):
     out = run(fake_hip, SKIN, TUNE_AT=tune_at, FAKE_HIP_BEST="2")
     assert out.returncode == 0, out.stderr
     assert out.stdout.strip() == str(want)
+
+
+FULL = SETUP + """
+s = geometry.h_on_slab("Au", n=3, nlayers=4, rng=rng)
+c = mdt.Context(0)
+c.set_emt(cols, pesm)
+b = mdt.Batch(c, [s] * 20000, dt=0.1)
+b.compute_forces()
+n0 = hip.fake_hip_launches()
+b.compute_forces()
+n1 = hip.fake_hip_launches()
+b.step(2)
+b.get_state()
+print(b.class_shapes()[0]["keep"], n1 - n0)
+"""
+
+
+# 20000 trajectories of 37 atoms: 125 MB of state, 540 MB of lists
+@pytest.mark.parametrize("mb,want", [(800, "1 1"), (360, "0 3")])
+def test_a_batch_whose_lists_do_not_fit_still_runs(fake_hip, mb, want):
+    """Without room for a list slot per replica the lists are rebuilt in fewer slots, a
+    slice of the batch at a time."""
+    out = run(fake_hip, FULL, FAKE_HIP_BYTES=str(mb << 20))
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.strip() == want

@@ -22,8 +22,8 @@ hipError_t mdt_launch_relayout(bool out, int ntile, const StateTile *tiles, cons
                                const double *src, double *dst, hipStream_t st);
 hipError_t mdt_launch_call(bool in, double *host, int N, int P, const CallArrays &a, hipStream_t st);
 hipError_t mdt_launch_drop_lists(int2 *valid, int n, int period, int phase, hipStream_t st);
-hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
-                              const BatchView &bv, int add_fin, hipStream_t st);
+hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const BatchView &bv,
+                              int add_fin, hipStream_t st);
 hipError_t mdt_launch_estimators(int ntraj, const PropConst *pc, const BatchView &bv, double *out, hipStream_t st);
 hipError_t mdt_launch_traj_classical(int ntraj, const PropConst *pc, const BatchView &bv, const uint32_t *step_base,
                                      uint32_t step_prev, uint32_t step, int flags, int block, hipStream_t st,
@@ -1081,7 +1081,6 @@ static int ensure_ready(mdt_batch *b, bool need_prop) {
         if (rc) return rc;
     }
     b->pc.mixed = b->bead_mode == 1 ? 1 : 0;
-    b->pc.no_com = b->no_com;
     if (!traj_classical(b)) {
         int rc = build_chunks(b);
         if (rc) return rc;
@@ -1397,7 +1396,7 @@ static hipError_t launch_class(const mdt_batch *b, const SizeClass &k, int t0, i
     hipError_t e = hipSuccess;
     for (int q = 0; q < n && e == hipSuccess; q += k.slots) {
         e = mdt_launch_replica(once ? k.tpa1 : k.tpa, std::min(n - q, k.slots), once ? k.block1 : k.block,
-                               once ? k.smem1 : k.smem, b->ctx->d_ec, b->d_pc, v, add_fin, st);
+                               once ? k.smem1 : k.smem, b->ctx->d_ec, v, add_fin, st);
         if (v.rep_list)
             v.rep_list += k.slots;
         else

@@ -94,7 +94,6 @@ struct PropConst {
     int any_langevin, any_pile, any_andersen;
     int mixed;  // 1: atoms of non-projectile types are classical (one bead, kept in bead 0)
     uint32_t seed;
-    int no_com;  // 1: no remove_com_velocity after propagate_1 (an extension; see mdt_batch_set_com_removal)
 };
 
 // A run of one trajectory's atoms with all their beads: the work of one

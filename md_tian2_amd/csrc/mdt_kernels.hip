@@ -529,7 +529,7 @@ __device__ __forceinline__ bool owns(int k, int n) { return (k < n) != (((k + n)
 // would otherwise leave each CU two waves per SIMD.
 template <bool MIXED, int PREC, bool JUDGE, int MAXB>
 __global__ void __launch_bounds__(MAXB, 4)
-    k_replica(const EmtConst *__restrict__ ecg, const PropConst *__restrict__ pcg, BatchView bv, int add_fin) {
+    k_replica(const EmtConst *__restrict__ ecg, BatchView bv, int add_fin) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ LdsTypes T;
     __shared__ double s_sh[27 * 4];  // lattice translations of the image codes, 32 bytes each
@@ -1822,7 +1822,6 @@ k_prop(const PropConst *__restrict__ pcg, BatchView bv, const double *cjk_all, c
     const bool lan = act && algo == MDT_PROP_LANGEVIN;
     const double temp_k = pc.is_proj[ty] ? tproj : tsurf;
     LanCoef L;
-    bool have_l = false;
     if (flags & 3) {
         if ((flags & 1) && lan) {
             int bad = 0;
@@ -1842,7 +1841,6 @@ k_prop(const PropConst *__restrict__ pcg, BatchView bv, const double *cjk_all, c
         if (lan) {
             const double temp = MDT_KB * nb * temp_k / mass;
             L = lan_coef(dn, dt, temp, big && temp > MDT_TOLERANCE);
-            have_l = true;
         }
     }
     if ((flags & 1) && act) {  // propagate_2 of step step_prev
@@ -2980,35 +2978,35 @@ ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, 
 }
 
 template <bool M, int F, bool J>
-static hipError_t launch_replica_t(dim3 g, dim3 blk, size_t smem, const EmtConst *ec, const PropConst *pc,
-                                   const BatchView &bv, int add_fin, hipStream_t st) {
+static hipError_t launch_replica_t(dim3 g, dim3 blk, size_t smem, const EmtConst *ec, const BatchView &bv, int add_fin,
+                                   hipStream_t st) {
     if (blk.x > 512)
-        hipLaunchKernelGGL((k_replica<M, F, J, 1024>), g, blk, smem, st, ec, pc, bv, add_fin);
+        hipLaunchKernelGGL((k_replica<M, F, J, 1024>), g, blk, smem, st, ec, bv, add_fin);
     else
-        hipLaunchKernelGGL((k_replica<M, F, J, 512>), g, blk, smem, st, ec, pc, bv, add_fin);
+        hipLaunchKernelGGL((k_replica<M, F, J, 512>), g, blk, smem, st, ec, bv, add_fin);
     return hipGetLastError();
 }
 
-// calc_force on every replica; ec and pc are device pointers; tpa lanes per
+// calc_force on every replica; ec is a device pointer; tpa lanes per
 // atom scan for the rows.  The judge (bv.judge_acc set) always runs the FP64
 // arithmetic.
-hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
-                              const BatchView &view, int add_fin, hipStream_t st) {
+hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const BatchView &view,
+                              int add_fin, hipStream_t st) {
     dim3 g(nrep), blk(block);
     BatchView bv = view;
     bv.tpa_shift = tpa == 8 ? 3 : tpa == 4 ? 2 : tpa == 2 ? 1 : 0;
     const bool m = bv.bulk < 0;
     if (bv.judge_acc)
-        return m ? launch_replica_t<true, 0, true>(g, blk, smem, ec, pc, bv, add_fin, st)
-                 : launch_replica_t<false, 0, true>(g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 0, true>(g, blk, smem, ec, bv, add_fin, st)
+                 : launch_replica_t<false, 0, true>(g, blk, smem, ec, bv, add_fin, st);
     if (bv.precision == 1)
-        return m ? launch_replica_t<true, 1, false>(g, blk, smem, ec, pc, bv, add_fin, st)
-                 : launch_replica_t<false, 1, false>(g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 1, false>(g, blk, smem, ec, bv, add_fin, st)
+                 : launch_replica_t<false, 1, false>(g, blk, smem, ec, bv, add_fin, st);
     if (bv.precision == 2)
-        return m ? launch_replica_t<true, 2, false>(g, blk, smem, ec, pc, bv, add_fin, st)
-                 : launch_replica_t<false, 2, false>(g, blk, smem, ec, pc, bv, add_fin, st);
-    return m ? launch_replica_t<true, 0, false>(g, blk, smem, ec, pc, bv, add_fin, st)
-             : launch_replica_t<false, 0, false>(g, blk, smem, ec, pc, bv, add_fin, st);
+        return m ? launch_replica_t<true, 2, false>(g, blk, smem, ec, bv, add_fin, st)
+                 : launch_replica_t<false, 2, false>(g, blk, smem, ec, bv, add_fin, st);
+    return m ? launch_replica_t<true, 0, false>(g, blk, smem, ec, bv, add_fin, st)
+             : launch_replica_t<false, 0, false>(g, blk, smem, ec, bv, add_fin, st);
 }
 
 // LDS of k_mixed for trajectories of up to nmax atoms (one projectile) and

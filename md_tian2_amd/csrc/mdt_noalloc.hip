@@ -140,8 +140,8 @@ __global__ void k_noalloc_unpack(const unsigned char *s, const EmtConst *ec, int
 }  // namespace
 
 ReplicaLists mdt_replica_lists(int nrep, int N, int block, int cap, size_t lds, bool once);
-hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const PropConst *pc,
-                              const BatchView &bv, int add_fin, hipStream_t st);
+hipError_t mdt_launch_replica(int tpa, int nrep, int block, size_t smem, const EmtConst *ec, const BatchView &bv,
+                              int add_fin, hipStream_t st);
 int mdt_noalloc_fail(int code, const char *msg);
 
 // The array's address on the current device (taken once per device).
@@ -214,7 +214,7 @@ int mdt_noalloc_compute(void *ptr, size_t lds_limit, const EmtConst *d_ec, int n
     v.rl_rows = lay.rows;
     v.rl_chunk = lay.chunk;
     v.rl_scan = lay.scan;
-    e = mdt_launch_replica(tpa, P, block, smem, d_ec, (const PropConst *)(s + NA_PC), v, 0, st);
+    e = mdt_launch_replica(tpa, P, block, smem, d_ec, v, 0, st);
     if (e != hipSuccess) return mdt_noalloc_fail(MDT_EHIP, hipGetErrorString(e));
     hipLaunchKernelGGL(k_noalloc_unpack, dim3(grid), dim3(256), 0, st, (const unsigned char *)s, d_ec, N, P, epot, f,
                        dens, status);

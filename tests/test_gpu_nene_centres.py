@@ -93,3 +93,33 @@ def test_workgroup_sizes_agree_bitwise(gpu_ctx):
     for out in got[1:]:
         for k, o in enumerate(out):
             assert np.array_equal(o["f"], got[0][k % 5]["f"]) and np.array_equal(o["epot"], got[0][k % 5]["epot"])
+
+
+def test_forces_keep_single_precision(gpu_ctx):
+    """The shipped angular network on thermal slabs, against 64 bits: forces to 1e-5 and
+    energies to 2e-6 eV/atom.  A pair's terms round some 12 times (2^-24 each) and its
+    exponent, up to 30, once (2^-24 30 = 2e-6); sums over many pairs average, and the
+    network, whose operands keep 24 bits, adds a few 2^-24 a layer, so the
+    2-norm stays some 3e-6 and below 1e-5.  Operands of 16 bits (two bf16 parts: 2^-17
+    = 8e-6 each, over three layers and the way back) or the hardware's sine and
+    cosine (2^-18 absolute) give 2e-5."""
+    import os
+
+    g = np.random.default_rng(33)
+    m = nene.load(os.path.join(os.path.dirname(mdt.LIB_PATH), "nn", "hau"))
+    om = no.Model(m)
+    gpu_ctx.set_nn(m, TYPES)
+    diff = norm = 0.0
+    for n in (3, 5, 6):
+        for z in (1.6, 3.0):
+            s = geometry.h_on_slab("Au", n=n, nlayers=4, rng=g, z0=z)
+            u = _universe(s.r[:, 0] + g.normal(0, 0.05, s.r[:, 0].shape), s.simbox)
+            e, f, _ = gpu_ctx.compute_nene(u)
+            E, _, F, _ = om.energy_forces(om.elem_index([1] + [79] * (u.natoms - 1)), u.r[:, 0] / nene.BOHR2ANG,
+                                          u.simbox.T / nene.BOHR2ANG)
+            F = F * nene.HABOHR2EVANG
+            diff += ((f[:, 0] - F) ** 2).sum()
+            norm += (F ** 2).sum()
+            assert abs(e[0] - E * nene.HA2EV) / u.natoms <= 2e-6
+    print("network forces: relative error %.2e" % np.sqrt(diff / norm))
+    assert np.sqrt(diff / norm) <= 1e-5

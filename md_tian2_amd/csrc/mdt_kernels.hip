@@ -707,7 +707,8 @@ __global__ void __launch_bounds__(MAXB, 4)
     // ---- phase 1: rows ----
     // few workgroups and rows for this launch only: they are read where the scan
     // put them, in LDS, tpa lanes per row (cutting and sorting them costs 6 us)
-    const bool direct = !keep && lds_scan;
+    // (launches that want this hold all types in their rows: the row loop of one type has no test for it)
+    const bool direct = MIXED && !keep && lds_scan;
     const int sh = bv.tpa_shift;
     if (!reuse) {
         if (kept) {  // the rows are stale

@@ -1619,7 +1619,7 @@ static int autotune(mdt_batch *b) {
     // configuration is timed with the share of its slots rebuilt at each launch that
     // a 300 K metal and a step of 0.1 fs give, so its figure is not a reuse-only best case.
     const int cands[4] = {1, 2, 4, 8};
-    const int ntime = 5;
+    const int ntime = 5;  // rebuilt lists: 2, every launch does the same
     // launches between two rebuilds of a slot (row_skin)
     const int period = std::max(ntime, (int)(1250 * row_skin(b) / std::sqrt((double)b->maxP)));
     float total = 0.f;
@@ -1646,7 +1646,8 @@ static int autotune(mdt_batch *b) {
                         HIPCHK(launch_class(b, k, 0, k.nrep, false, v, 0, st));
                         HIPCHK(mdt_launch_drop_lists(k.d_valid, k.keep ? k.nrep : 0, period, 0, st));
                         HIPCHK(hipEventRecord(b->ev0, st));
-                        for (int q = 0; q < ntime; ++q) {
+                        const int nq = k.keep ? ntime : 2;
+                        for (int q = 0; q < nq; ++q) {
                             HIPCHK(launch_class(b, k, 0, k.nrep, false, v, 0, st));
                             HIPCHK(mdt_launch_drop_lists(k.d_valid, k.keep ? k.nrep : 0, period, (q + 1) * period / ntime, st));
                         }
@@ -1654,6 +1655,7 @@ static int autotune(mdt_batch *b) {
                         HIPCHK(hipEventSynchronize(b->ev1));
                         float ms = 0.f;
                         HIPCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
+                        ms *= (float)ntime / nq;
                         if (ms < best_ms) {
                             best_ms = ms;
                             best = tpa;

@@ -108,7 +108,7 @@ int mdt_compute_emt(mdt_context *ctx, int natoms, int nbeads, const int32_t *idx
  * every array a DEVICE pointer in the same layout (idx(N), simbox(3,3),
  * isimbox(3,3), r(3,P,N), epot(P), f(3,P,N), dens(P,N)); status (device,
  * may be NULL) receives the call's MDT_ST_* bits.  The universe is staged
- * in a fixed scratch array of about 4.7 MB per GPU, held until the process
+ * in a fixed scratch array of about 9 MB per GPU, held until the process
  * ends: natoms <= 2048, nbeads <= 64, natoms * nbeads <= 16384 (larger
  * universes return MDT_EINVAL).  Launches go to `stream` (a hipStream_t;
  * NULL: the context's stream) and are not waited for; the call allocates

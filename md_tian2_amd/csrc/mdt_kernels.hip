@@ -474,11 +474,11 @@ __device__ __forceinline__ bool owns(int k, int n) { return (k < n) != (((k + n)
 // calc_force for one replica per workgroup.
 //
 // What bounds it: with enough replicas the issue of vector instructions (about 60 %
-// of the cycles; 165 a pair and lane in both passes together) beside the LDS (45 %:
+// of the cycles; about 165 a pair and lane in both passes together) beside the LDS (51 %:
 // positions, exponential table, atomics), with few of them the latency of its
-// phases.  H/Au 6x6x4, 4096 replicas of 3 k near pairs: 180 us a step with the
-// propagator, 263 before rows were sorted pieces; H/Pt 8x8x6, 2048 replicas: 300 us
-// a launch, 494 before.
+// phases.  H/Au 6x6x4, 4096 replicas of 3 k near pairs: 166 us a step with the
+// propagator, 263 before rows were sorted pieces; H/Pt 8x8x6, 2048 replicas: 281 us
+// a launch (mean, builds included), 494 before.
 //  * Rows.  The owned half lists hold the near pairs (r <= rnear) of the
 //    atoms of one EMT type, the majority (bv.bulk); their constants are
 //    uniform, so a pair needs no type.  A row is cut into equal pieces, one a

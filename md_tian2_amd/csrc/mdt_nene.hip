@@ -500,7 +500,7 @@ __device__ void mlp_tile(const NnConst &M, int e, const int *rows, const float *
 // and queues those that count, and evaluates the queue 64 at a time with
 // every lane at work.  With one centre per wavefront every parameter of its
 // functions is wavefront-uniform (scalar registers, no tables in LDS).
-// H/Au 6x6x4, 512 replicas: k_nene_g 1017 -> 439 us, k_nene_f 1570 -> 615 us,
+// H/Au 6x6x4, 512 replicas: k_nene_g 1017 -> 433 us, k_nene_f 1570 -> 610 us,
 // issuing vector instructions 85 % of the time; the training gradient over
 // 256 frames of 37 atoms: k_nn_frame 2240 -> 167 us.  The error against FP64
 // fell too (forces 2.1e-5 -> 3.3e-6 relative, gradient 2.7e-3 -> 3.9e-4): the

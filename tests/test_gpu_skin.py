@@ -1,27 +1,24 @@
 """Neighbour lists kept across force calls (Verlet skin) in k_replica.
 
-Size classes of more than 256 atoms (and smaller ones where the autotuner
-finds it faster) keep their owned half lists in HBM, built with the near
-radius + skin (the lists hold the pairs within the near radius r_near,
-beyond which a pair weighs less than 2^-56; the pairs beyond it of atoms
-whose near sigma is tiny come from a direct scan), while no atom of the
-replica moved more than skin / 2 since the build; a kept list gets the
-image of every entry recomputed from the current positions.  The reference visits every pair
-under the minimum image at every call (src/pes_emt_mod.f90:1204-1206), so
-parity is what a rebuild at every call gives:
+Half lists are kept in HBM, built with the near radius + skin (the lists hold
+the pairs within the near radius r_near, beyond which a pair weighs less than
+2^-56; the pairs beyond it of atoms whose near sigma is tiny come from a direct
+scan), while no atom of the replica moved more than skin / 2 since the build; a
+kept list gets the image of every entry recomputed from the current positions.
+The reference visits every pair under the minimum image at every call
+(src/pes_emt_mod.f90:1204-1206), so parity is what a rebuild at every call gives:
 
 * skins 0 (rebuild every call), 0.3 A (default) and 0.02 A (a rebuild every
-  few steps) give the same trajectories to rounding (only the summation
-  order of sigma in registers can differ), over 200 steps in which the
+  few steps) give the same trajectories to rounding, over 200 steps in which the
   atoms move beyond half the default skin;
 * the forces of the final state equal the oracle's;
 * a projectile starting 6.5 A above the surface (tiny sigma: its pairs
   beyond r_near come from the direct scan) moves into the near region on
   kept lists;
 * a 4x4 cell (10 A wide, below 2 (r_near + skin), half-cell ties inside the
-  cut-off) rebuilds at every call: there the rounded image of a pair need not
-  be its nearest, so a list built for one image could miss the pair after it
-  rounds to another; the skins agree to rounding there too;
+  cut-off): there the image of a pair can change between builds, and entries
+  whose image is not the only one within reach search it again at every launch;
+  the skins agree to rounding there too;
 * new positions from set_state drop the kept lists."""
 import numpy as np
 import pytest
@@ -125,10 +122,9 @@ def test_autotuned_keep_equals_rebuilt_lists(gpu_ctx, pes_hau):
 
 @pytest.mark.parametrize("metal,n,nlayers", [("Au", 6, 4), ("Pt", 8, 4)])
 def test_list_modes_agree(gpu_ctx, pes_hau, pes_hpt, metal, n, nlayers):
-    """mdt_batch_set_keep: lists rebuilt every launch (0), kept and staged in
-    LDS during a launch (1), kept and read from HBM (2) give the same
-    trajectories to rounding over 150 steps, with the same threads per
-    atom; mode 1 runs staged where the lists fit in LDS."""
+    """mdt_batch_set_keep: lists rebuilt every launch (0) and kept and read
+    from HBM (1 and 2, the same) give the same trajectories to rounding over
+    150 steps, with the same threads per atom."""
     rng = np.random.default_rng(85 + n)
     pes = pes_hau if metal == "Au" else pes_hpt
     systems = [geometry.h_on_slab(metal, n=n, nlayers=nlayers, rng=rng, z0=z, einc=1.0, tsurf=300.0)
@@ -158,7 +154,7 @@ def test_list_modes_agree(gpu_ctx, pes_hau, pes_hpt, metal, n, nlayers):
 
 
 def test_skin_switch_keeps_batch_usable(gpu_ctx, pes_hpt):
-    """Switching the skin off and on moves the lists between LDS and HBM;
+    """Switching the skin off and on switches between rebuilt and kept lists;
     the forces stay the oracle's."""
     rng = np.random.default_rng(70)
     systems = [geometry.h_on_slab("Pt", n=8, nlayers=4, rng=rng, z0=2.0, tsurf=300.0) for _ in range(3)]
